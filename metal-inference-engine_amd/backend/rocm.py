@@ -23,10 +23,10 @@ Method -> kernel:
                          linear-attention prefill (src/models/qwen3_5.py:144-162) in four launches
   attention_prep         rk_attn_prep: q / k RMSNorm + partial RoPE (+ the decode KV write) of a gated-attention
                          layer (src/models/qwen3_5.py:251-262, 100-110) in one launch
-  linear, embedding      rk_linear_rows (bf16 / INT8 / INT4 weights, up to 32 rows), rk_dequant_rows (+ a BLAS GEMM
-                         beyond 32 rows; embedding rows), src/backend/metal.py:50-133
+  linear, embedding      rk_linear_rows (bf16 / INT8 / INT4 weights, up to 32 rows), rk_linear_gemm (more rows),
+                         rk_dequant_rows (embedding rows), src/backend/metal.py:50-133
   swiglu                 rk_swiglu_rows: the linear on the stacked [gate; up] weight with silu * up of each gate / up
-                         output pair in its epilogue (one launch; beyond 32 rows the linear then rk_silu_mul)
+                         output pair in its epilogue (one launch; beyond 32 rows rk_linear_gemm with the same)
   rms_norm_swiglu        rk_swiglu_rows with the RMSNorm applied while x is staged (the MLP of a decode step)
   silu_mul               rk_silu_mul on the two halves of a gate_up output, in place
   silu_mul_linear        rk_linear_rows_ex: SwiGLU's silu * up applied while the down projection stages its
@@ -214,8 +214,8 @@ class RocmBackend:
     # ---- decode-time linears
     def linear(self, x, w, b=None, residual=None):
         """Backend.linear (src/backend/base.py:19-21) on a bf16 weight or a block-quantized QuantTensor
-        (src/backend/metal.py:59-133): up to 32 rows through rk_linear_rows (16 per launch), beyond that an fp32
-        GEMM on row chunks of the weight dequantized by rk_dequant_rows -> [M, N] fp32."""
+        (src/backend/metal.py:59-133): up to 32 rows through rk_linear_rows (16 per launch), beyond that
+        rk_linear_gemm -> [M, N] fp32."""
         return kernels.linear(x, w, b, residual)
 
     def embedding(self, table, ids):
@@ -229,7 +229,7 @@ class RocmBackend:
         """silu(x @ gate.T) * (x @ up.T) for w_gate_up = [gate; up] stacked [2F, K] (src/backend/base.py:40-41): up
         to 32 rows one rk_swiglu_rows launch per 16 (the linear over the stacked weight with silu * up of each gate /
         up output pair in its epilogue, as MetalBackend.swiglu's fused matvec_swiglu_bf16, src/backend/metal.py:
-        145-157); beyond, the linear then silu * up over the two column halves of its output, read in place."""
+        145-157); beyond, rk_linear_gemm with silu * up in its epilogue."""
         return kernels.swiglu(x, w_gate_up)
 
     def rms_norm_swiglu(self, x, ss, norm_w, eps, w_gate_up):

@@ -704,7 +704,7 @@ def attn_prep(y, q_w, k_w, eps: float, positions, theta: float, rot: int, dims, 
 
 W_TYPES = {"int8": RK_W_INT8, "int4": RK_W_INT4}
 LINEAR_ROWS = 16            # activation rows per rk_linear_rows launch (the MFMA's 16 columns)
-KERNEL_ROWS = 32            # up to here: the matvec kernel in groups of 16; beyond: dequantize + GEMM
+KERNEL_ROWS = 32            # up to here: the matvec kernel in groups of 16; beyond: rk_linear_gemm
 LINEAR_LONG_ROWS = 65536    # rk_linear_rows' persistent kernel for INT8 weights from this many rows (M <= 8)
 
 
@@ -880,14 +880,18 @@ def _swiglu_fused(w, K: int) -> bool:
 def swiglu(x, w) -> torch.Tensor:
     """Backend.swiglu (src/backend/base.py:40-41): silu(x @ gate^T) * (x @ up^T) for w = [gate; up] stacked [2F, K]
     (bf16 or a QuantTensor) -> [M, F] fp32. Up to KERNEL_ROWS rows: rk_swiglu_rows, one launch per 16 rows (the
-    linear's sums, then silu * up on each gate / up pair in the same launch); beyond that, or for F % 8 != 0, the
-    linear and then silu_mul on its two halves (the same results within 1e-5)."""
+    linear's sums, then silu * up on each gate / up pair in the same launch); beyond that rk_linear_gemm with the
+    product in its epilogue. Up to KERNEL_ROWS rows with F % 8 != 0, and rows that are not whole blocks: the linear
+    and then silu_mul on its two halves (the same results within 1e-5)."""
     N, K = w.shape
     M = x.shape[0]
     if x.dim() != 2 or x.shape[1] != K or N % 2:
         raise ValueError(f"swiglu: x {tuple(x.shape)} for a [{N}, {K}] stacked [gate; up] weight")
     from quant import QuantTensor
-    if M > KERNEL_ROWS or not (isinstance(w, QuantTensor) or w.dtype == torch.bfloat16) or not _swiglu_fused(w, K):
+    fused = isinstance(w, QuantTensor) or w.dtype == torch.bfloat16
+    if fused and M > KERNEL_ROWS and K % 32 == 0:
+        return _gemm(x, w, glu=True)
+    if not fused or not _swiglu_fused(w, K):
         y = linear(x, w)
         return silu_mul(y[:, :N // 2], y[:, N // 2:])
     _need_cuda("swiglu", x, w.data if isinstance(w, QuantTensor) else w)
@@ -955,31 +959,48 @@ def dequantize(w, rows=None, row0: int = 0, n_rows: int | None = None) -> torch.
     return out
 
 
-DEQUANT_CHUNK = 1 << 23     # weights expanded per prefill GEMM piece (32 MB fp32), as the reference
+def _gemm(x, w, bias=None, residual=None, glu: bool = False) -> torch.Tensor:
+    """rk_linear_gemm: any number of rows against a bf16 / quantized weight whose rows are whole blocks of 32; glu:
+    w = [gate; up], silu(x gate^T) * (x up^T). bias [N] and residual [M, N] fp32, contiguous, or None."""
+    wt, data, scales, mins, N, K = _weight_args(w)
+    dev = _need_cuda("linear", x, data)
+    x, ld = _rows_k(x, K)
+    if data.data_ptr() % 16:                    # rows are read as 16-byte vectors
+        data = data.clone()
+    M = x.shape[0]
+    out = torch.empty(M, N // 2 if glu else N, dtype=torch.float32, device=dev)
+    lib = load()
+    # a tensor of the call's own, not the shared workspace: it grows with the rows
+    ws = torch.empty(lib.lib.rk_linear_gemm_workspace_bytes(M, N, K, wt, int(glu)), dtype=torch.uint8, device=dev)
+    lib.call("rk_linear_gemm", out.data_ptr(), x.data_ptr(), ld, M, N, K, data.data_ptr(), wt,
+             scales.data_ptr() if scales is not None else None, mins.data_ptr() if mins is not None else None,
+             bias.data_ptr() if bias is not None else None, residual.data_ptr() if residual is not None else None,
+             int(glu), ws.data_ptr(), ws.numel(), _stream(dev))
+    return out
 
 
 def linear(x, w, bias=None, residual=None) -> torch.Tensor:
     """The reference's decode / prefill linear on a bf16 or quantized weight (src/backend/metal.py:59-133): up to 32
-    rows through the matvec kernel, beyond that an fp32 GEMM (the ROCm BLAS through torch) on row chunks of the
-    dequantized weight, so the full-size fp32 weight never exists. fp32 / other-dtype weights: x @ w.T in fp32."""
+    rows through the matvec kernel, beyond that rk_linear_gemm. fp32 / other-dtype weights, and bf16 rows that are not
+    whole blocks of 32: x @ w.T in fp32."""
     from quant import QuantTensor
     M = x.shape[0]
-    if not isinstance(w, QuantTensor) and w.dtype != torch.bfloat16:
+    if not isinstance(w, QuantTensor) and (w.dtype != torch.bfloat16 or w.shape[1] % 32):
         y = x.float() @ w.float().T
-    elif M <= KERNEL_ROWS and w.shape[1] % 32 == 0:
+    elif M <= KERNEL_ROWS:
         return linear_rows(x, w, bias, residual)
     else:
         N, K = w.shape
-        x = x.float()
-        y = torch.empty(M, N, dtype=torch.float32, device=x.device)
-        step = max(1, DEQUANT_CHUNK // K)
-        for r in range(0, N, step):
-            n = min(step, N - r)
-            if isinstance(w, QuantTensor) or K % 32 == 0:
-                wr = dequantize(w, row0=r, n_rows=n)
-            else:
-                wr = w[r:r + n].float()
-            y[:, r:r + n] = x @ wr.T
+        if x.dim() != 2 or x.shape[1] != K:
+            raise ValueError(f"linear: x {tuple(x.shape)} for a [{N}, {K}] weight")
+        # added in the kernel where they are what it reads, else (broadcast shapes) below
+        rows = lambda t: t.to(device=x.device, dtype=torch.float32).contiguous()
+        b = rows(bias) if bias is not None and bias.shape == (N,) else None
+        r = rows(residual) if residual is not None and residual.shape == (M, N) and (bias is None or b is not None) \
+            else None
+        y = _gemm(x, w, b, r)
+        bias = None if b is not None else bias
+        residual = None if r is not None else residual
     if bias is not None:
         y = y + bias.float()
     return y + residual.float() if residual is not None else y

@@ -1,0 +1,555 @@
+// Linears of many rows (prefill tokens, decode batches past the row kernels' 32), gfx950.
+//
+// Semantics (reference): MetalBackend.linear / _qlinear for M > 32 rows (src/backend/metal.py:55-133), which expands
+// the weight to fp32 and runs an fp32 GEMM: y [M, N] = x [M, K] @ dequant(W)^T (+ bias) (+ residual), fp32, W bf16 or
+// block-quantized (src/quant.py:1-10, 45-56); and Backend.swiglu (src/backend/base.py:40-41) over a stacked
+// [gate; up] weight.
+//
+// Design: the fp32 matrix rate of gfx950 is 1/16 of its 16-bit rate, so an fp32 product is worth two 16-bit ones if
+// two carry enough bits. Here they do:
+//   x  enters as two fp16 pieces hi + lo of x * 2^a, with 2^a (per row) placing the row's largest value in
+//      [2^14, 2^15): hi = fp16(x 2^a), lo = fp16(x 2^a - hi). A value keeps a relative error of 2^-24, what one fp32
+//      rounding costs, down to 2^-16 of its row's largest, and below that an absolute one of 2^-40 of the largest.
+//   W  is one fp16 operand: INT8 / INT4 codes are exact, a bf16 row times its own 2^b (largest in [2^14, 2^15)) is
+//      exact down to 2^-32 of the row's largest and within 2^-40 of it below.
+// Every product of two pieces is exact in fp32 and accumulates in fp32. A quantization block is one MFMA's k-extent
+// (32), so its scale multiplies the block's sums on the VALU. The powers of two leave in the epilogue (ldexp), exactly.
+//
+// W is expanded to fp16 rows, a slab at a time, and the product runs on LDS tiles of both. An INT4 weight is
+// s (q - 8) + (8 s + min): the codes enter as q - 8 (small partial sums), and min and 8 s as K / 16 more columns, (min,
+// s) against the block's activation sum (1, 8): pairs in one MFMA, whose near-equal terms of opposite sign cancel
+// inside it. Three launches per slab: split_rows, slab_weights, gemm_rows.
+//
+// Measured against the fp32 GEMM on the expanded weight (1777 rows, bf16): 12288 x 2048 with silu * up 740 -> 235 us
+// in all (gemm_rows 200 us = 890 TFLOP/s of 16-bit products; a large bf16 GEMM of the BLAS reaches 1270 on this
+// card), 2048 x 6144 440 -> 157 us; error against 64 bits 1.4e-6 -> 2.7e-7 of the result at K 6144. What bounds
+// gemm_rows: matrix-core issue and the fp32 joins beside it (copies without the loads, without the LDS reads or with a
+// quarter of the joins are each about 10 % faster), and whole tiles: 224 workgroups on 256 CUs at 2048 columns.
+#include "rk_device.h"
+#include "rk_internal.h"
+
+namespace rk {
+namespace {
+
+constexpr int kQB = 32;                            // weights per quantization block = one MFMA's k-extent
+constexpr int kBK = 32;                            // k per step
+constexpr int kTop = 14;                           // a row's largest value lies in [2^kTop, 2^(kTop + 1))
+constexpr int kSumShift = 8;                       // 8 block sums (of 32 values) are scaled by 2^-kSumShift
+constexpr long long kSlabElems = 1ll << 25;        // fp16 weights expanded at a time (64 MiB)
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ f32x4 mfma_f16(u32x4 a, u32x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0,
+                                                  0);
+}
+
+__device__ __forceinline__ uint32_t pack_f16(float a, float b) {   // round to nearest even
+    return __builtin_bit_cast(uint32_t, (f16x2){(_Float16)a, (_Float16)b});
+}
+
+// 16 bytes per lane from src into LDS at dst (wave-uniform) + 16 * lane
+__device__ __forceinline__ void load_to_lds(const void* src, char* dst) {
+    __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+
+__device__ __forceinline__ void load4_to_lds(const void* src, char* dst) {   // the same, 4 bytes per lane
+    __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)dst, 4, 0, 0);
+}
+
+__device__ __forceinline__ float half_to_f32(uint32_t h) { return (float)__builtin_bit_cast(_Float16, (uint16_t)h); }
+
+// the power of two that puts the magnitude m into [2^kTop, 2^(kTop + 1)): its exponent (0 for m = 0; inf and NaN as
+// the largest finite exponent, so that they stay inf and NaN in the pieces)
+__device__ __forceinline__ int top_exponent(float m) {
+    const int e = (int)(__float_as_uint(m) >> 23) - 127;
+    return m == 0.0f ? 0 : kTop - max(min(e, 127), -112);
+}
+
+// hi and lo pieces of v (already scaled): hi = fp16(v), lo = fp16(v - hi); an infinite hi has no rest
+__device__ __forceinline__ void split2(float v, float& hi, float& lo) {
+    hi = (float)(_Float16)v;
+    lo = __builtin_isinf(hi) ? 0.0f : v - hi;
+}
+
+// largest |v| of a 256-thread workgroup, in every thread
+__device__ __forceinline__ float block_absmax(float m, float* red) {
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    return fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+}
+
+// Operand layout of gemm_rows, shared by both operands: rows cut into steps of 32 values, [step][rows][32] fp16 (x:
+// [step][piece][rows][32]), so that a stage of a tile is one contiguous run per operand. The 16-byte unit u of row R
+// sits at u ^ swizzle(R): an operand read (lane l: row l % 16, unit l / 16) is served 16 lanes at a time, rows 0-3 and
+// 12-15 of one unit with rows 4-11 of the next, and these then lie on all 16 units of the 256-byte bank line.
+// Rows past the matrix (up to whole tiles) are not written: their products are never stored.
+__device__ __forceinline__ int swizzle(int R) { return (0x78 >> (2 * ((R >> 2) & 3))) & 3; }
+__device__ __forceinline__ size_t unit_at(size_t slice, int rows, int R, int u) {
+    return (slice * rows + R) * kBK + 8 * (u ^ swizzle(R));
+}
+
+// One workgroup per row m of x: the row's pieces and its exponent ex[m]. With SUMS, columns K + 2b and K + 2b + 1 are
+// the pieces of block b's sum and of 8 times it, both * 2^-kSumShift, then zeros to the end of the last step. The
+// second pass reads the row from the caches.
+template <bool SUMS>
+__global__ __launch_bounds__(256) void split_rows(uint16_t* a, int* ex, const float* x, long long x_ld, int Mp, int K,
+                                                  int steps) {
+    __shared__ float red[4];
+    const int m = blockIdx.x, tid = threadIdx.x;
+    const float* xr = x + (size_t)m * x_ld;
+    float big = 0.0f;
+    for (int c = tid; c < K / 8; c += 256) {
+        const f32x4 v0 = *reinterpret_cast<const f32x4*>(xr + 8 * c), v1 = *reinterpret_cast<const f32x4*>(xr + 8 * c + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) big = fmaxf(big, fmaxf(fabsf(v0[e]), fabsf(v1[e])));
+    }
+    big = block_absmax(big, red);
+    const int k = top_exponent(big);
+    if (tid == 0) ex[m] = k;
+    for (int c = tid; c < K / 8; c += 256) {
+        const f32x4 v0 = *reinterpret_cast<const f32x4*>(xr + 8 * c), v1 = *reinterpret_cast<const f32x4*>(xr + 8 * c + 4);
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[e] = ldexpf(v0[e], k);
+            v[4 + e] = ldexpf(v1[e], k);
+        }
+        u32x4 ph, pl;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float h0, l0, h1, l1;
+            split2(v[2 * e], h0, l0);
+            split2(v[2 * e + 1], h1, l1);
+            ph[e] = pack_f16(h0, h1);
+            pl[e] = pack_f16(l0, l1);
+        }
+        *reinterpret_cast<u32x4*>(a + unit_at(2 * (size_t)(c >> 2), Mp, m, c & 3)) = ph;
+        *reinterpret_cast<u32x4*>(a + unit_at(2 * (size_t)(c >> 2) + 1, Mp, m, c & 3)) = pl;
+        if constexpr (SUMS) {                      // the four threads of a block are neighbours in one wave
+            float sum = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) sum += v[e];
+            sum += __shfl_xor(sum, 1);
+            sum += __shfl_xor(sum, 2);
+            if ((c & 3) == 0) {
+                const int b = c >> 2;              // sixteen blocks' pairs to a step
+                float h, l;
+                split2(ldexpf(sum, -kSumShift), h, l);
+                const size_t sl = 2 * (size_t)(K / kBK + (b >> 4));
+                *reinterpret_cast<uint32_t*>(a + unit_at(sl, Mp, m, (b & 15) >> 2) + 2 * (b & 3)) = pack_f16(h, 8.0f * h);
+                *reinterpret_cast<uint32_t*>(a + unit_at(sl + 1, Mp, m, (b & 15) >> 2) + 2 * (b & 3)) =
+                    pack_f16(l, 8.0f * l);
+            }
+        }
+    }
+    if constexpr (SUMS)
+        for (int b = K / kBK + tid; b < 16 * (steps - K / kBK); b += 256) {
+            const size_t sl = 2 * (size_t)(K / kBK + (b >> 4));
+            *reinterpret_cast<uint32_t*>(a + unit_at(sl, Mp, m, (b & 15) >> 2) + 2 * (b & 3)) = 0u;
+            *reinterpret_cast<uint32_t*>(a + unit_at(sl + 1, Mp, m, (b & 15) >> 2) + 2 * (b & 3)) = 0u;
+        }
+}
+
+struct SlabArgs {
+    uint16_t* out;                 // [steps][Np][32] fp16
+    float* sc;                     // quantized: [steps][Np] scales
+    int* ew;                       // bf16: [rows] exponents
+    const void* w;
+    const uint16_t* scales;
+    const uint16_t* mins;
+    int Np, row0, K, steps;        // padded slab rows; the slab's first weight row (glu: its first gate row)
+    int F;                         // glu: rows of each half; 0: plain
+};
+
+// the weight row behind slab row j: row0 + j, or with glu sixteen gate rows, then the sixteen up rows of the same
+// outputs, in turn, so that an output's gate and up sums meet in one lane (rows past F, in the last pair of
+// sixteens, repeat row F - 1: their outputs are not stored)
+__device__ __forceinline__ size_t slab_row(const SlabArgs& a, int j) {
+    if (!a.F) return (size_t)(a.row0 + j);
+    const int f = min(a.row0 + 16 * (j >> 5) + (j & 15), a.F - 1);
+    return (size_t)((j & 16) ? a.F + f : f);
+}
+
+// One workgroup per slab row: fp16 operands of the row (codes, or bf16 * 2^b) and its scales; INT4 codes minus 8, then
+// the row's (min, scale) pairs.
+template <int WT>
+__global__ __launch_bounds__(256) void slab_weights(SlabArgs a) {
+    __shared__ float red[4];
+    const int j = blockIdx.x, tid = threadIdx.x;
+    const size_t n = slab_row(a, j);
+    const int nblk = a.K / kQB;
+    int k = 0;
+    if constexpr (WT == RK_W_BF16) {
+        const uint16_t* w = static_cast<const uint16_t*>(a.w) + n * a.K;
+        float big = 0.0f;
+        for (int c = tid; c < a.K / 8; c += 256) {
+            const u32x4 q = *reinterpret_cast<const u32x4*>(w + 8 * c);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) big = fmaxf(big, fmaxf(fabsf(bf16_lo(q[e])), fabsf(bf16_hi(q[e]))));
+        }
+        k = top_exponent(block_absmax(big, red));
+        if (tid == 0) a.ew[j] = k;
+    }
+    for (int c = tid; c < a.K / 8; c += 256) {
+        u32x4 o;
+        if constexpr (WT == RK_W_BF16) {
+            const u32x4 q = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.w) + n * a.K + 8 * c);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = pack_f16(ldexpf(bf16_lo(q[e]), k), ldexpf(bf16_hi(q[e]), k));
+        } else if constexpr (WT == RK_W_INT8) {
+            const u32x2 q = *reinterpret_cast<const u32x2*>(static_cast<const int8_t*>(a.w) + n * a.K + 8 * c);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                o[e] = pack_f16((float)(int)__builtin_amdgcn_sbfe(q[e >> 1], 16 * (e & 1), 8),
+                                (float)(int)__builtin_amdgcn_sbfe(q[e >> 1], 16 * (e & 1) + 8, 8));
+        } else {
+            const uint32_t q = *reinterpret_cast<const uint32_t*>(static_cast<const uint8_t*>(a.w) + n * (a.K / 2) + 4 * c);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                o[e] = pack_f16((float)__builtin_amdgcn_ubfe(q, 8 * e, 4) - 8.0f,
+                                (float)__builtin_amdgcn_ubfe(q, 8 * e + 4, 4) - 8.0f);
+        }
+        *reinterpret_cast<u32x4*>(a.out + unit_at(c >> 2, a.Np, j, c & 3)) = o;
+    }
+    if constexpr (WT != RK_W_BF16) {
+        const uint16_t* s = a.scales + n * nblk;
+        for (int t = tid; t < a.steps; t += 256)   // the pairs' steps: 2^kSumShift
+            a.sc[(size_t)t * a.Np + j] = t < nblk ? half_to_f32(s[t]) : (float)(1 << kSumShift);
+        if constexpr (WT == RK_W_INT4) {
+            const uint16_t* mn = a.mins + n * nblk;
+            for (int b = tid; b < 16 * (a.steps - nblk); b += 256)
+                *reinterpret_cast<uint32_t*>(a.out + unit_at(nblk + (b >> 4), a.Np, j, (b & 15) >> 2) + 2 * (b & 3)) =
+                    b < nblk ? mn[b] | (uint32_t)s[b] << 16 : 0u;
+        }
+    }
+}
+
+struct GemmArgs {
+    float* y;
+    const uint16_t* a;             // [steps][2][Mp][32]
+    const uint16_t* w;             // [steps][Np][32], the slab
+    const float* sc;               // [steps][Np]
+    const int* ex;
+    const int* ew;
+    const float* bias;             // [columns of y] or null
+    const float* res;              // as y, or null
+    long long y_ld;
+    int M, N, Mp, Np, steps;
+    int col0, cols;                // first column of y this slab gives; columns of y
+    int tm, tn;                    // tiles
+};
+
+__device__ __forceinline__ float silu_times(float g, float u) {
+    return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-g * kLog2e)) * u;
+}
+
+// Workgroup of WM x WN waves, each a 16 TI x 64 tile of y. A stage is one step of 32: 2 BM piece rows and BN
+// weight rows of 64 bytes (and each wave's 64 scales), straight from memory into LDS by global_load_lds, 1 KB per
+// instruction, kStages buffers in turn. Per stage and wave 12 operand reads feed 32 MFMAs, each read one group of
+// sixteen rows ahead, across the stages' barriers too. The loop has no other memory reads, and a wave's loads complete
+// in order, so waiting for all but the newest (kStages - 3) x loads-per-stage leaves this stage and the next in LDS.
+template <int WM, int WN, int TI, bool SCALED>
+struct Tile {
+    static constexpr int NW = WM * WN, BM = 16 * TI * WM, BN = 64 * WN, ROWS = 2 * BM + BN, NI = ROWS / 16 / NW;
+    static constexpr int kLoads = NI + (SCALED ? 1 : 0);
+    static constexpr int kBytes = ROWS * 2 * kBK + (SCALED ? 256 * NW : 0);
+    static constexpr int kStages = 160 * 1024 / kBytes < 6 ? 160 * 1024 / kBytes : 6;
+    static_assert(NI * 16 * NW == ROWS, "whole load instructions");
+    static_assert(kStages * kBytes <= 160 * 1024, "LDS");
+};
+
+template <int WM, int WN, int TI, bool SCALED, bool GLU>
+__global__ __launch_bounds__(64 * WM * WN) void gemm_rows(GemmArgs g) {
+    using TL = Tile<WM, WN, TI, SCALED>;
+    constexpr int BM = TL::BM, BN = TL::BN, NI = TL::NI, ST = TL::kStages;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, grp = lane >> 4;
+    const int wm = wave / WN, wn = wave % WN;
+
+    // tile order: workgroups go to the 8 XCDs in turn, so XCD x takes a contiguous run of tiles, walked in groups of
+    // 8 row tiles by all column tiles: the run's weight rows and pieces stay in the XCD's L2
+    const int T = g.tm * g.tn, per = T / 8, rem = T % 8, xcd = blockIdx.x % 8;
+    const int id = xcd * per + min(xcd, rem) + blockIdx.x / 8;
+    const int group = 8 * g.tn, gi = id / group, first = 8 * gi, height = min(8, g.tm - first);
+    const int m0 = BM * (first + (id % group) % height), n0 = BN * ((id % group) / height);
+
+    // load instruction i of this wave: stage rows 16 (NI wave + i) .. + 15 (hi piece rows, lo piece rows, weight rows);
+    // wave-uniform addresses, 16 bytes per lane from there
+    const char* src[NI];
+    size_t hop[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int R = 16 * (NI * wave + i);
+        const bool pc = R < 2 * BM;
+        const size_t row = pc ? (size_t)(R / BM) * g.Mp + m0 + R % BM : (size_t)(n0 + R - 2 * BM);
+        src[i] = reinterpret_cast<const char*>((pc ? g.a : g.w) + row * kBK);
+        hop[i] = (size_t)(pc ? 2 * g.Mp : g.Np) * kBK * 2;
+    }
+    const char* scp = reinterpret_cast<const char*>(g.sc + n0 + 64 * wn);
+    const int S = g.steps;
+    int ahead = 0;                                 // the next stage to request; past the last, the last again
+    auto request = [&](int buf) {
+        char* dst = smem + buf * TL::kBytes;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) load_to_lds(src[i] + 16 * lane, dst + 1024 * (NI * wave + i));
+        if constexpr (SCALED) load4_to_lds(scp + 4 * lane, dst + TL::ROWS * 2 * kBK + 256 * wave);
+        if (++ahead < S) {                         // uniform
+#pragma unroll
+            for (int i = 0; i < NI; ++i) src[i] += hop[i];
+            if constexpr (SCALED) scp += (size_t)g.Np * 4;
+        }
+    };
+#pragma unroll
+    for (int b = 0; b < ST - 1; ++b) request(b);
+
+    // operand reads: lane (r, grp) takes unit grp of row R0 + r; R0 is a multiple of 16, so the unit's place is the
+    // lane's alone
+    const int at = 64 * r + 16 * (grp ^ swizzle(r));
+    const int at_a = at + 64 * 16 * TI * wm, at_b = at + 64 * (2 * BM + 64 * wn);
+    const int at_s = TL::ROWS * 2 * kBK + 256 * wave + 4 * r;
+    auto rd = [&](const char* p) { return *reinterpret_cast<const u32x4*>(p); };
+    f32x4 acc[TI][4], d[2][4];
+    u32x4 b[4], bn[4], h[2], l[2];
+    float f[4], fn[4], fd[4];                      // scales: of this stage, of the next, of d[1]'s stage
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        d[1][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        f[t] = fn[t] = fd[t] = 0.0f;
+#pragma unroll
+        for (int i = 0; i < TI; ++i) acc[i][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    }
+    // a stage's sums start from zero and join the running ones by an fp32 addition (or fma): a third of the error of
+    // MFMAs on the running sums (bf16, K 6144: 2.7e-7 of the result against 7.1e-7; an fp32 GEMM: 1.4e-6)
+    auto join = [&](f32x4 (&to)[4], const f32x4 (&from)[4], const float (&by)[4]) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if constexpr (SCALED) to[t][e] = fmaf(by[t], from[t][e], to[t][e]);
+                else to[t][e] += from[t][e];
+            }
+    };
+    auto landed = [&] {
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((ST - 3) * TL::kLoads) : "memory");
+    };
+    landed();
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        b[t] = rd(smem + at_b + 1024 * t);
+        if constexpr (SCALED) f[t] = *reinterpret_cast<const float*>(smem + at_s + 64 * t);
+    }
+    h[0] = rd(smem + at_a);
+    l[0] = rd(smem + at_a + 64 * BM);
+
+    int buf = 0;
+    for (int s = 0; s < S; ++s) {
+        // behind this barrier stages s and s + 1 are in LDS, and stage s - 1, whose buffer the request fills, is done
+        // with (its last operands were taken before it)
+        if (s) landed();
+        request(buf == 0 ? ST - 1 : buf - 1);
+        const char* cur = smem + buf * TL::kBytes;
+        buf = buf == ST - 1 ? 0 : buf + 1;
+        const char* nxt = smem + buf * TL::kBytes;
+        // rows 16 i: their MFMAs, while the operands of the next sixteen (at the end the next stage's) are read and
+        // the sums of the sixteen before are joined
+#pragma unroll
+        for (int i = 0; i < TI; ++i) {
+            const int c = i & 1, o = c ^ 1;
+            if (i < TI - 1) {
+                h[o] = rd(cur + at_a + 1024 * (i + 1));
+                l[o] = rd(cur + at_a + 64 * BM + 1024 * (i + 1));
+            } else {
+                h[o] = rd(nxt + at_a);
+                l[o] = rd(nxt + at_a + 64 * BM);
+            }
+            if (i >= TI - 2) {
+#pragma unroll
+                for (int t = 2 * (i - TI + 2); t < 2 * (i - TI + 3); ++t) {
+                    bn[t] = rd(nxt + at_b + 1024 * t);
+                    if constexpr (SCALED) fn[t] = *reinterpret_cast<const float*>(nxt + at_s + 64 * t);
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < 4; ++t) d[c][t] = mfma_f16(l[c], b[t], (f32x4){0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+            for (int t = 0; t < 4; ++t) d[c][t] = mfma_f16(h[c], b[t], d[c][t]);
+            if (i == 0) join(acc[TI - 1], d[1], fd);
+            else join(acc[i - 1], d[o], f);
+            if (i < TI - 2) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            else __builtin_amdgcn_sched_group_barrier(0x100, SCALED ? 6 : 4, 0);
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            b[t] = bn[t];
+            if constexpr (SCALED) {
+                fd[t] = f[t];
+                f[t] = fn[t];
+            }
+        }
+    }
+    join(acc[TI - 1], d[1], fd);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the requests past the last stage
+
+    // lane (r, grp) holds rows 4 grp + e, column r of each 16 x 16 tile
+#pragma unroll
+    for (int i = 0; i < TI; ++i) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int m = m0 + 16 * TI * wm + 16 * i + 4 * grp + e;
+            if (m >= g.M) continue;
+            const int em = g.ex[m];
+            float v[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                int ee = -em;
+                if constexpr (!SCALED) ee -= g.ew[min(n0 + 64 * wn + 16 * t + r, g.N - 1)];
+                v[t] = ldexpf(acc[i][t][e], ee);
+            }
+            if constexpr (GLU) {
+#pragma unroll
+                for (int t = 0; t < 4; t += 2) {
+                    const int c = g.col0 + ((n0 + 64 * wn + 16 * t) >> 1) + r;
+                    if (c < g.cols && n0 + 64 * wn + 16 * t < g.N) g.y[(size_t)m * g.y_ld + c] = silu_times(v[t], v[t + 1]);
+                }
+            } else {
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const int n = n0 + 64 * wn + 16 * t + r;
+                    if (n >= g.N) continue;
+                    const int c = g.col0 + n;
+                    float o = v[t];
+                    if (g.bias) o = __fadd_rn(o, g.bias[c]);
+                    if (g.res) o = __fadd_rn(o, g.res[(size_t)m * g.y_ld + c]);
+                    g.y[(size_t)m * g.y_ld + c] = o;
+                }
+            }
+        }
+    }
+}
+
+struct Layout {
+    int Mp, Np, steps, slab;       // slab: output columns expanded at a time; Np: its weight rows, in whole tiles
+    size_t pieces, ex, slab_w, slab_sc, ew, total;
+};
+
+size_t up256(size_t n) { return (n + 255) / 256 * 256; }
+
+// rows of W behind `cols` output columns (glu: whole pairs of sixteens)
+int slab_rows(int cols, bool glu) { return glu ? (cols + 15) / 16 * 32 : cols; }
+
+Layout layout(int M, int N, int K, int w_type, bool glu) {
+    Layout l;
+    l.Mp = (M + 127) / 128 * 128;
+    l.steps = K / kBK + (w_type == RK_W_INT4 ? (K / 16 + kBK - 1) / kBK : 0);
+    const int cols = glu ? N / 2 : N;
+    long long s = kSlabElems / (l.steps * kBK) / (glu ? 2 : 1) / 256 * 256;
+    if (s < 256) s = 256;
+    l.slab = s < cols ? (int)s : cols;
+    const size_t rows = (size_t)slab_rows(l.slab, glu);
+    l.Np = (int)up256(rows);
+    l.pieces = 0;
+    l.ex = (size_t)l.steps * 2 * l.Mp * kBK * 2;
+    l.slab_w = l.ex + up256((size_t)M * 4);
+    l.slab_sc = l.slab_w + (size_t)l.steps * l.Np * kBK * 2;
+    l.ew = l.slab_sc + (w_type == RK_W_BF16 ? 0 : (size_t)l.steps * l.Np * 4);
+    l.total = l.ew + up256(rows * 4);
+    return l;
+}
+
+template <int WM, int WN, int TI>
+int launch_gemm(const GemmArgs& in, bool scaled, bool glu, hipStream_t s) {
+    GemmArgs g = in;
+    constexpr int BM = 16 * TI * WM, BN = 64 * WN;
+    const size_t lds = scaled ? Tile<WM, WN, TI, true>::kStages * Tile<WM, WN, TI, true>::kBytes
+                              : Tile<WM, WN, TI, false>::kStages * Tile<WM, WN, TI, false>::kBytes;
+    g.tm = (g.M + BM - 1) / BM;
+    g.tn = (g.N + BN - 1) / BN;
+    const auto fn = scaled ? (glu ? gemm_rows<WM, WN, TI, true, true> : gemm_rows<WM, WN, TI, true, false>)
+                           : (glu ? gemm_rows<WM, WN, TI, false, true> : gemm_rows<WM, WN, TI, false, false>);
+    if (int rc = allow_dynamic_lds((const void*)fn, lds)) return rc;
+    if ((long long)g.tm * g.tn >= (1ll << 31)) return fail(RK_ERR_ARG, "rk_linear_gemm: M %d too large", g.M);
+    hipLaunchKernelGGL(fn, dim3((unsigned)(g.tm * g.tn)), dim3(64 * WM * WN), lds, s, g);
+    return check_launch("gemm_rows");
+}
+
+}  // namespace
+}  // namespace rk
+
+using namespace rk;
+
+extern "C" {
+
+size_t rk_linear_gemm_workspace_bytes(int M, int N, int K, int w_type, int glu) {
+    if (M < 1 || N < 1 || K < kQB || K % kQB) return 0;
+    return layout(M, N, K, w_type, glu != 0).total;
+}
+
+int rk_linear_gemm(float* y, const float* x, long long x_ld, int M, int N, int K, const void* w, int w_type,
+                   const void* scales, const void* mins, const float* bias, const float* residual, int glu,
+                   void* workspace, size_t workspace_bytes, void* stream) {
+    if (M == 0 || N == 0) return RK_OK;
+    const bool quant = w_type == RK_W_INT8 || w_type == RK_W_INT4;
+    if (!y || !x || !w || (quant && !scales) || (w_type == RK_W_INT4 && !mins))
+        return fail(RK_ERR_ARG, "rk_linear_gemm: null pointer");
+    if (w_type != RK_W_BF16 && !quant) return fail(RK_ERR_UNSUPPORTED, "rk_linear_gemm: weight type %d", w_type);
+    if (M < 0 || N < 0 || K < kQB || K % kQB || K > (1 << 24) || (glu && N % 2))
+        return fail(RK_ERR_ARG, "rk_linear_gemm: M %d, N %d, K %d (a multiple of %d)", M, N, K, kQB);
+    if (glu && (bias || residual)) return fail(RK_ERR_ARG, "rk_linear_gemm: no bias or residual with glu");
+    if (reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(w) % 16 || x_ld < K || x_ld % 4)
+        return fail(RK_ERR_ARG, "rk_linear_gemm: x and w must be 16-byte aligned, x rows at a stride >= K of 4n");
+    const Layout l = layout(M, N, K, w_type, glu != 0);
+    if (!workspace || workspace_bytes < l.total)
+        return fail(RK_ERR_WORKSPACE, "rk_linear_gemm: workspace %zu bytes (need %zu)", workspace_bytes, l.total);
+    char* ws = static_cast<char*>(workspace);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    uint16_t* pieces = reinterpret_cast<uint16_t*>(ws + l.pieces);
+    int* ex = reinterpret_cast<int*>(ws + l.ex);
+    const auto split = w_type == RK_W_INT4 ? split_rows<true> : split_rows<false>;
+    hipLaunchKernelGGL(split, dim3((unsigned)M), dim3(256), 0, st, pieces, ex, x, x_ld, l.Mp, K, l.steps);
+    if (int rc = check_launch("split_rows")) return rc;
+    const int cols = glu ? N / 2 : N;
+    int cus = device_cus();
+    if (cus <= 0) cus = 256;
+    for (int c0 = 0; c0 < cols; c0 += l.slab) {
+        const int nc = l.slab < cols - c0 ? l.slab : cols - c0;
+        SlabArgs sa{};
+        sa.out = reinterpret_cast<uint16_t*>(ws + l.slab_w);
+        sa.sc = reinterpret_cast<float*>(ws + l.slab_sc);
+        sa.ew = reinterpret_cast<int*>(ws + l.ew);
+        sa.w = w; sa.scales = static_cast<const uint16_t*>(scales); sa.mins = static_cast<const uint16_t*>(mins);
+        sa.Np = l.Np; sa.row0 = c0; sa.K = K; sa.steps = l.steps; sa.F = glu ? cols : 0;
+        const int rows = slab_rows(nc, glu != 0);
+        const auto expand = w_type == RK_W_BF16 ? slab_weights<RK_W_BF16>
+                            : w_type == RK_W_INT8 ? slab_weights<RK_W_INT8> : slab_weights<RK_W_INT4>;
+        hipLaunchKernelGGL(expand, dim3((unsigned)rows), dim3(256), 0, st, sa);
+        if (int rc = check_launch("slab_weights")) return rc;
+        GemmArgs g{};
+        g.y = y; g.a = pieces; g.w = sa.out; g.sc = sa.sc; g.ex = ex; g.ew = sa.ew; g.bias = bias; g.res = residual;
+        g.y_ld = cols; g.M = M; g.N = rows; g.Mp = l.Mp; g.Np = l.Np; g.steps = l.steps; g.col0 = c0; g.cols = cols;
+        // 128 x 256 tiles where they give every CU two of them, else 128 x 128 (1777 x 2048 outputs: 112 tiles of 256
+        // columns leave half the CUs idle), else 64 x 128; eight waves of 32 x 64 beat four of 64 x 64 there (157
+        // against 168 us at 1777 x 2048 x 6144: two waves per SIMD)
+        auto tiles = [&](int bm, int bn) {
+            return (long long)((M + bm - 1) / bm) * ((rows + bn - 1) / bn);
+        };
+        int rc;
+        if (tiles(128, 256) >= 2 * cus) rc = launch_gemm<2, 4, 4>(g, quant, glu != 0, st);
+        else if (M > 64) rc = launch_gemm<4, 2, 2>(g, quant, glu != 0, st);
+        else rc = launch_gemm<2, 2, 2>(g, quant, glu != 0, st);
+        if (rc) return rc;
+    }
+    return RK_OK;
+}
+
+}  // extern "C"

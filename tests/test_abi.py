@@ -322,3 +322,28 @@ def test_linear_ex2_checked_on_host(lib):
     ex = dict(y=fake, x=fake, xld=2048, op=2, aux=fake, auxld=2048, M=8, N=2048, K=2048, w=fake, wt=3, s=fake, m=fake,
               b=None, r=None, p=fake, pb=1 << 30, c=fake, nc=1024)
     assert L.rk_linear_rows_ex(*ex.values(), None) == 1 and "input transform 2" in lib.last_error()
+
+
+def test_linear_gemm_checked_on_host(lib):
+    fake = 4096
+    L = lib.lib
+
+    def call(**kw):
+        a = dict(y=fake, x=fake, xld=2048, M=64, N=2048, K=2048, w=fake, wt=3, s=fake, m=fake, b=None, r=None, glu=0,
+                 ws=fake, wsb=1 << 40)
+        a.update(kw)
+        return L.rk_linear_gemm(*a.values(), None)
+
+    assert call(x=None) == 1 and "null pointer" in lib.last_error()
+    assert call(m=None) == 1 and "null pointer" in lib.last_error()
+    assert call(wt=9) == 2 and "weight type 9" in lib.last_error()
+    assert call(K=2040) == 1 and call(xld=2044) == 1 and call(x=fake + 4) == 1
+    assert call(glu=1, N=2047) == 1 and call(glu=1, b=fake) == 1
+    assert call(M=0) == 0
+    for M, N, K, wt, glu in ((33, 2048, 2048, 3, 0), (64, 12288, 2048, 1, 1), (5000, 300000, 2048, 2, 0)):
+        need = L.rk_linear_gemm_workspace_bytes(M, N, K, wt, glu)
+        assert need > 4 * M * K and call(M=M, N=N, K=K, xld=K, wt=wt, glu=glu, wsb=need - 1) == 3
+        assert "workspace" in lib.last_error()
+    assert L.rk_linear_gemm_workspace_bytes(0, 64, 64, 1, 0) == 0
+    # weights are expanded a slab at a time: 64 MiB of them at most, however many there are
+    assert L.rk_linear_gemm_workspace_bytes(64, 1 << 22, 2048, 1, 0) < 80 << 20

@@ -249,3 +249,55 @@ def test_long_int8_matrix_on_the_persistent_grid(backend, N, K):
         assert rel_err(ss, tile_sums(y.cpu().double()).float()) < 1e-6
         rows[M] = got.cpu()
     assert torch.equal(rows[1][0], rows[8][0]) and torch.equal(rows[3], rows[8][:3])
+
+
+@pytest.mark.parametrize("kind", ["bf16", "int8", "int4"])
+@pytest.mark.parametrize("M,N,K,glu", [(33, 100, 96, False), (64, 130, 2080, False), (65, 272, 64, False),
+                                       (129, 1000, 512, False), (257, 515, 1056, False), (600, 4352, 256, False),
+                                       (33, 2 * 20, 256, True), (140, 2 * 1000, 544, True), (513, 2 * 2200, 128, True)])
+def test_many_row_linears_against_64_bits(backend, kind, M, N, K, glu):
+    """rk_linear_gemm at the edges of its tiles (rows and columns around 64, 128 and 256, odd numbers of 32-value
+    steps, glu halves that are not whole sixteens), with rows of very different magnitude and values of very different
+    magnitude in one row, against the products in 64 bits. Bound: each output's sum of |x w| times 2^-24 for the
+    rounding of x and the same for every 32-value partial sum's fp32 rounding, of which there are K / 32 in sequence."""
+    w, deq = weight(kind, N, K, N + K)
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K, generator=g) * torch.exp2(torch.randint(-60, 40, (M, 1), generator=g).float())
+    x[:, ::7] *= 2.0 ** -20
+    x[M // 2] = 0.0
+    b, r = (None, None) if glu else (torch.randn(N, generator=g), torch.randn(M, N, generator=g))
+    if glu:
+        x = x.sign() * x.abs().clamp(1e-6, 1e3)         # silu's tails are not what is tested
+    want = x.double() @ deq.double().T
+    bound = (x.double().abs() @ deq.double().abs().T) * (2 + K / 32) * 2.0 ** -24
+    if glu:
+        F = N // 2
+        gate, up, bg, bu = want[:, :F], want[:, F:], bound[:, :F], bound[:, F:]
+        got = backend.swiglu(x.to(DEV), to_dev(w))
+        want, sg = gate * torch.sigmoid(gate) * up, (gate * torch.sigmoid(gate)).abs()
+        bound = 1.1 * bg * up.abs() + sg * bu + bg * bu + 1e-6 * want.abs() + 1e-30    # |silu'| < 1.1
+    else:
+        got = backend.linear(x.to(DEV), to_dev(w), b.to(DEV), r.to(DEV))
+        want = want + b.double() + r.double()
+        bound = bound + 2.0 ** -23 * (want.abs() + b.double().abs() + r.double().abs())
+    over = ((got.cpu().double() - want).abs() / bound.clamp(min=1e-38)).max()
+    print(f"gemm {kind} {M}x{N}x{K} glu {glu}: {over:.3f} of the bound")
+    assert over < 1.0
+
+
+def test_many_row_linears_take_what_the_row_kernels_take(backend):
+    """33 rows with strided activations, a bias and residual that broadcast, and a weight at an odd address; a row that
+    holds an infinity gives infinities or NaN and leaves its neighbours alone."""
+    w, deq = weight("bf16", 48, 64, 5)
+    g = torch.Generator().manual_seed(5)
+    x = torch.randn(33, 128, generator=g)
+    b, r = torch.randn(1, 48, generator=g), torch.randn(48, generator=g)
+    flat = torch.empty(48 * 64 + 1, dtype=torch.bfloat16, device=DEV)
+    odd = flat[1:].view(48, 64).copy_(w)
+    got = backend.linear(x.to(DEV)[:, ::2], odd, b.to(DEV), r.to(DEV))
+    assert rel_err(got, x[:, ::2] @ deq.T + b + r) < TOL
+    x[7, 6] = float("inf")
+    bad = backend.linear(x.to(DEV)[:, ::2], odd, b.to(DEV), r.to(DEV))
+    assert not torch.isfinite(bad[7]).any()
+    keep = [i for i in range(33) if i != 7]
+    assert torch.equal(bad[keep], got[keep])
