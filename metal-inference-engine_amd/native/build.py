@@ -16,7 +16,8 @@ PROBE_LIB = HERE / "librk_probe.so"       # measurement probes (include/rk_probe
 OBJ_DIR = HERE / "_obj"
 SOURCES = ["rk_abi.cpp", "paged_decode.hip", "kv_cache.hip", "page_table.hip", "deltanet_step.hip", "paged_prefill.hip",
            "chunked_delta.hip", "chunked_delta_cols.hip", "deltanet_prefill.hip", "attn_prep.hip",
-           "linear.hip", "linear_gemm.hip", "decode_ops.hip"]
+           "linear.hip", "linear_gemm.hip", "linear_mid.hip",
+           "decode_ops.hip"]
 PROBE_SOURCES = ["probes.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
@@ -32,7 +33,8 @@ FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Wall", "-Wno-
 _ROUNDED = ["-ffp-contract=on"]
 SOURCE_FLAGS = {"chunked_delta_cols.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "deltanet_step.hip": _ROUNDED,
                 "decode_ops.hip": _ROUNDED, "deltanet_prefill.hip": _ROUNDED, "attn_prep.hip": _ROUNDED,
-                "linear.hip": _ROUNDED, "linear_gemm.hip": _ROUNDED + ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+                "linear.hip": _ROUNDED, "linear_gemm.hip": _ROUNDED + ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+                "linear_mid.hip": _ROUNDED + ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 def _compile(src: str, verbose: bool) -> Path:

@@ -18,36 +18,22 @@
 // W is expanded to fp16 rows, a slab at a time, and the product runs on LDS tiles of both. An INT4 weight is
 // s (q - 8) + (8 s + min): the codes enter as q - 8 (small partial sums), and min and 8 s as K / 16 more columns, (min,
 // s) against the block's activation sum (1, 8): pairs in one MFMA, whose near-equal terms of opposite sign cancel
-// inside it. Three launches per slab: split_rows, slab_weights, gemm_rows.
+// inside it. Three launches per slab: split_rows, slab_weights, gemm_rows (four with K-splits: gemm_finish). Up to a few
+// hundred rows linear_mid.hip reads W as stored instead.
 //
 // Measured against the fp32 GEMM on the expanded weight (1777 rows, bf16): 12288 x 2048 with silu * up 740 -> 235 us
 // in all (gemm_rows 200 us = 890 TFLOP/s of 16-bit products; a large bf16 GEMM of the BLAS reaches 1270 on this
 // card), 2048 x 6144 440 -> 157 us; error against 64 bits 1.4e-6 -> 2.7e-7 of the result at K 6144. What bounds
 // gemm_rows: matrix-core issue and the fp32 joins beside it (copies without the loads, without the LDS reads or with a
 // quarter of the joins are each about 10 % faster), and whole tiles: 224 workgroups on 256 CUs at 2048 columns.
-#include "rk_device.h"
-#include "rk_internal.h"
+#include "linear_pieces.h"
 
 namespace rk {
 namespace {
 
-constexpr int kQB = 32;                            // weights per quantization block = one MFMA's k-extent
 constexpr int kBK = 32;                            // k per step
-constexpr int kTop = 14;                           // a row's largest value lies in [2^kTop, 2^(kTop + 1))
 constexpr int kSumShift = 8;                       // 8 block sums (of 32 values) are scaled by 2^-kSumShift
 constexpr long long kSlabElems = 1ll << 25;        // fp16 weights expanded at a time (64 MiB)
-
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ f32x4 mfma_f16(u32x4 a, u32x4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0,
-                                                  0);
-}
-
-__device__ __forceinline__ uint32_t pack_f16(float a, float b) {   // round to nearest even
-    return __builtin_bit_cast(uint32_t, (f16x2){(_Float16)a, (_Float16)b});
-}
 
 // 16 bytes per lane from src into LDS at dst (wave-uniform) + 16 * lane
 __device__ __forceinline__ void load_to_lds(const void* src, char* dst) {
@@ -56,30 +42,6 @@ __device__ __forceinline__ void load_to_lds(const void* src, char* dst) {
 
 __device__ __forceinline__ void load4_to_lds(const void* src, char* dst) {   // the same, 4 bytes per lane
     __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)dst, 4, 0, 0);
-}
-
-__device__ __forceinline__ float half_to_f32(uint32_t h) { return (float)__builtin_bit_cast(_Float16, (uint16_t)h); }
-
-// the power of two that puts the magnitude m into [2^kTop, 2^(kTop + 1)): its exponent (0 for m = 0; inf and NaN as
-// the largest finite exponent, so that they stay inf and NaN in the pieces)
-__device__ __forceinline__ int top_exponent(float m) {
-    const int e = (int)(__float_as_uint(m) >> 23) - 127;
-    return m == 0.0f ? 0 : kTop - max(min(e, 127), -112);
-}
-
-// hi and lo pieces of v (already scaled): hi = fp16(v), lo = fp16(v - hi); an infinite hi has no rest
-__device__ __forceinline__ void split2(float v, float& hi, float& lo) {
-    hi = (float)(_Float16)v;
-    lo = __builtin_isinf(hi) ? 0.0f : v - hi;
-}
-
-// largest |v| of a 256-thread workgroup, in every thread
-__device__ __forceinline__ float block_absmax(float m, float* red) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-    __syncthreads();
-    return fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
 }
 
 // Operand layout of gemm_rows, shared by both operands: rows cut into steps of 32 values, [step][rows][32] fp16 (x:
@@ -241,10 +203,35 @@ struct GemmArgs {
     int M, N, Mp, Np, steps;
     int col0, cols;                // first column of y this slab gives; columns of y
     int tm, tn;                    // tiles
+    int S;                         // K-splits
+    float* part;                   // S > 1: [S][M][Np] sums, to be finished by gemm_finish
 };
 
-__device__ __forceinline__ float silu_times(float g, float u) {
-    return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-g * kLog2e)) * u;
+// weight columns 32 q + r and 32 q + 16 + r (v, u) of row m: powers of two, then bias and residual or silu * up
+template <bool SCALED, bool GLU>
+__device__ __forceinline__ void gemm_store(const GemmArgs& g, int m, int n, float v, float u) {
+    const int em = g.ex[m];
+    int ev = -em, eu = -em;
+    if constexpr (!SCALED) {
+        ev -= g.ew[min(n, g.N - 1)];
+        eu -= g.ew[min(n + 16, g.N - 1)];
+    }
+    v = ldexpf(v, ev);
+    u = ldexpf(u, eu);
+    if constexpr (GLU) {
+        const int c = g.col0 + ((n & ~31) >> 1) + (n & 15);
+        if (c < g.cols && n < g.N) g.y[(size_t)m * g.y_ld + c] = silu_times(v, u);
+    } else {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            if (n + 16 * h >= g.N) continue;
+            const int c = g.col0 + n + 16 * h;
+            float o = h ? u : v;
+            if (g.bias) o = __fadd_rn(o, g.bias[c]);
+            if (g.res) o = __fadd_rn(o, g.res[(size_t)m * g.y_ld + c]);
+            g.y[(size_t)m * g.y_ld + c] = o;
+        }
+    }
 }
 
 // Workgroup of WM x WN waves, each a 16 TI x 64 tile of y. A stage is one step of 32: 2 BM piece rows and BN
@@ -278,6 +265,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_rows(GemmArgs g) {
     const int group = 8 * g.tn, gi = id / group, first = 8 * gi, height = min(8, g.tm - first);
     const int m0 = BM * (first + (id % group) % height), n0 = BN * ((id % group) / height);
 
+    // this split's steps
+    const int s0 = (int)((long long)g.steps * blockIdx.y / g.S), S = (int)((long long)g.steps * (blockIdx.y + 1) / g.S) - s0;
     // load instruction i of this wave: stage rows 16 (NI wave + i) .. + 15 (hi piece rows, lo piece rows, weight rows);
     // wave-uniform addresses, 16 bytes per lane from there
     const char* src[NI];
@@ -289,9 +278,9 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_rows(GemmArgs g) {
         const size_t row = pc ? (size_t)(R / BM) * g.Mp + m0 + R % BM : (size_t)(n0 + R - 2 * BM);
         src[i] = reinterpret_cast<const char*>((pc ? g.a : g.w) + row * kBK);
         hop[i] = (size_t)(pc ? 2 * g.Mp : g.Np) * kBK * 2;
+        src[i] += s0 * hop[i];
     }
-    const char* scp = reinterpret_cast<const char*>(g.sc + n0 + 64 * wn);
-    const int S = g.steps;
+    const char* scp = reinterpret_cast<const char*>(g.sc + n0 + 64 * wn) + (size_t)s0 * g.Np * 4;
     int ahead = 0;                                 // the next stage to request; past the last, the last again
     auto request = [&](int buf) {
         char* dst = smem + buf * TL::kBytes;
@@ -406,41 +395,39 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_rows(GemmArgs g) {
     for (int i = 0; i < TI; ++i) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const int m = m0 + 16 * TI * wm + 16 * i + 4 * grp + e;
+            const int m = m0 + 16 * TI * wm + 16 * i + 4 * grp + e, n = n0 + 64 * wn + r;
             if (m >= g.M) continue;
-            const int em = g.ex[m];
-            float v[4];
+            if (g.S > 1) {                         // uniform; the part rows hold whole tiles
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                int ee = -em;
-                if constexpr (!SCALED) ee -= g.ew[min(n0 + 64 * wn + 16 * t + r, g.N - 1)];
-                v[t] = ldexpf(acc[i][t][e], ee);
-            }
-            if constexpr (GLU) {
-#pragma unroll
-                for (int t = 0; t < 4; t += 2) {
-                    const int c = g.col0 + ((n0 + 64 * wn + 16 * t) >> 1) + r;
-                    if (c < g.cols && n0 + 64 * wn + 16 * t < g.N) g.y[(size_t)m * g.y_ld + c] = silu_times(v[t], v[t + 1]);
-                }
+                for (int t = 0; t < 4; ++t) g.part[((size_t)blockIdx.y * g.M + m) * g.Np + n + 16 * t] = acc[i][t][e];
             } else {
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const int n = n0 + 64 * wn + 16 * t + r;
-                    if (n >= g.N) continue;
-                    const int c = g.col0 + n;
-                    float o = v[t];
-                    if (g.bias) o = __fadd_rn(o, g.bias[c]);
-                    if (g.res) o = __fadd_rn(o, g.res[(size_t)m * g.y_ld + c]);
-                    g.y[(size_t)m * g.y_ld + c] = o;
-                }
+                gemm_store<SCALED, GLU>(g, m, n, acc[i][0][e], acc[i][1][e]);
+                gemm_store<SCALED, GLU>(g, m, n + 32, acc[i][2][e], acc[i][3][e]);
             }
         }
     }
 }
 
+// The splits' sums of row blockIdx.y, in order; a thread per pair of columns 16 apart.
+template <bool SCALED, bool GLU>
+__global__ __launch_bounds__(256) void gemm_finish(GemmArgs g) {
+    const int q = 256 * blockIdx.x + threadIdx.x, m = blockIdx.y;
+    const int n = 32 * (q >> 4) + (q & 15);
+    if (n >= g.N) return;
+    const float* p = g.part + (size_t)m * g.Np + n;
+    float v = p[0], u = p[16];                     // Np is a multiple of 32
+    for (int s = 1; s < g.S; ++s) {
+        p += (size_t)g.M * g.Np;
+        v += p[0];
+        u += p[16];
+    }
+    gemm_store<SCALED, GLU>(g, m, n, v, u);
+}
+
 struct Layout {
     int Mp, Np, steps, slab;       // slab: output columns expanded at a time; Np: its weight rows, in whole tiles
-    size_t pieces, ex, slab_w, slab_sc, ew, total;
+    int form, S;                   // gemm_rows' tile: 0 128 x 256, 1 128 x 128, 2 64 x 128; K-splits
+    size_t pieces, ex, slab_w, slab_sc, ew, part, total;
 };
 
 size_t up256(size_t n) { return (n + 255) / 256 * 256; }
@@ -463,7 +450,20 @@ Layout layout(int M, int N, int K, int w_type, bool glu) {
     l.slab_w = l.ex + up256((size_t)M * 4);
     l.slab_sc = l.slab_w + (size_t)l.steps * l.Np * kBK * 2;
     l.ew = l.slab_sc + (w_type == RK_W_BF16 ? 0 : (size_t)l.steps * l.Np * 4);
-    l.total = l.ew + up256(rows * 4);
+    l.part = l.ew + up256(rows * 4);
+    // 128 x 256 tiles where they give every CU two of them, else 128 x 128 (1777 x 2048 outputs: 112 tiles of 256
+    // columns leave half the CUs idle), else 64 x 128; eight waves of 32 x 64 beat four of 64 x 64 there (157 against
+    // 168 us at 1777 x 2048 x 6144: two waves per SIMD). Fewer than half as many tiles as CUs: K-splits of at least
+    // 16 steps, until the tiles fill the CUs (2048 columns, K 6144: 384 rows 133 -> 56 us, 256 rows 132 -> 45)
+    int cus = device_cus();
+    if (cus <= 0) cus = 256;
+    auto tiles = [&](int bm, int bn) { return (long long)((M + bm - 1) / bm) * (((long long)rows + bn - 1) / bn); };
+    l.form = tiles(128, 256) >= 2 * cus ? 0 : M > 64 ? 1 : 2;
+    const long long t = l.form == 1 ? tiles(128, 128) : tiles(64, 128);
+    l.S = 1;
+    if (l.form && 2 * t <= cus) l.S = (int)(cus / t < l.steps / 16 ? cus / t : l.steps / 16);
+    if (l.S < 1) l.S = 1;
+    l.total = l.part + (l.S > 1 ? (size_t)l.S * M * l.Np * 4 : 0);
     return l;
 }
 
@@ -479,8 +479,13 @@ int launch_gemm(const GemmArgs& in, bool scaled, bool glu, hipStream_t s) {
                            : (glu ? gemm_rows<WM, WN, TI, false, true> : gemm_rows<WM, WN, TI, false, false>);
     if (int rc = allow_dynamic_lds((const void*)fn, lds)) return rc;
     if ((long long)g.tm * g.tn >= (1ll << 31)) return fail(RK_ERR_ARG, "rk_linear_gemm: M %d too large", g.M);
-    hipLaunchKernelGGL(fn, dim3((unsigned)(g.tm * g.tn)), dim3(64 * WM * WN), lds, s, g);
-    return check_launch("gemm_rows");
+    hipLaunchKernelGGL(fn, dim3((unsigned)(g.tm * g.tn), (unsigned)g.S), dim3(64 * WM * WN), lds, s, g);
+    if (int rc = check_launch("gemm_rows")) return rc;
+    if (g.S == 1) return RK_OK;
+    const auto fin = scaled ? (glu ? gemm_finish<true, true> : gemm_finish<true, false>)
+                            : (glu ? gemm_finish<false, true> : gemm_finish<false, false>);
+    hipLaunchKernelGGL(fin, dim3((unsigned)((g.Np / 2 + 255) / 256), (unsigned)g.M), dim3(256), 0, s, g);
+    return check_launch("gemm_finish");
 }
 
 }  // namespace
@@ -492,7 +497,10 @@ extern "C" {
 
 size_t rk_linear_gemm_workspace_bytes(int M, int N, int K, int w_type, int glu) {
     if (M < 1 || N < 1 || K < kQB || K % kQB) return 0;
-    return layout(M, N, K, w_type, glu != 0).total;
+    // either form may run (an odd address of the scales sends a call to the other one)
+    const size_t tiles = layout(M, N, K, w_type, glu != 0).total;
+    const size_t mid = mid_takes(M, K, w_type, nullptr, nullptr) ? mid_workspace_bytes(M, N, K, w_type, glu) : 0;
+    return tiles > mid ? tiles : mid;
 }
 
 int rk_linear_gemm(float* y, const float* x, long long x_ld, int M, int N, int K, const void* w, int w_type,
@@ -508,9 +516,13 @@ int rk_linear_gemm(float* y, const float* x, long long x_ld, int M, int N, int K
     if (glu && (bias || residual)) return fail(RK_ERR_ARG, "rk_linear_gemm: no bias or residual with glu");
     if (reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(w) % 16 || x_ld < K || x_ld % 4)
         return fail(RK_ERR_ARG, "rk_linear_gemm: x and w must be 16-byte aligned, x rows at a stride >= K of 4n");
+    const size_t need = rk_linear_gemm_workspace_bytes(M, N, K, w_type, glu);
+    if (!workspace || workspace_bytes < need)
+        return fail(RK_ERR_WORKSPACE, "rk_linear_gemm: workspace %zu bytes (need %zu)", workspace_bytes, need);
+    if (mid_takes(M, K, w_type, scales, mins))
+        return mid_linear(y, x, x_ld, M, N, K, w, w_type, scales, mins, bias, residual, glu, workspace,
+                          static_cast<hipStream_t>(stream));
     const Layout l = layout(M, N, K, w_type, glu != 0);
-    if (!workspace || workspace_bytes < l.total)
-        return fail(RK_ERR_WORKSPACE, "rk_linear_gemm: workspace %zu bytes (need %zu)", workspace_bytes, l.total);
     char* ws = static_cast<char*>(workspace);
     hipStream_t st = static_cast<hipStream_t>(stream);
     uint16_t* pieces = reinterpret_cast<uint16_t*>(ws + l.pieces);
@@ -519,8 +531,6 @@ int rk_linear_gemm(float* y, const float* x, long long x_ld, int M, int N, int K
     hipLaunchKernelGGL(split, dim3((unsigned)M), dim3(256), 0, st, pieces, ex, x, x_ld, l.Mp, K, l.steps);
     if (int rc = check_launch("split_rows")) return rc;
     const int cols = glu ? N / 2 : N;
-    int cus = device_cus();
-    if (cus <= 0) cus = 256;
     for (int c0 = 0; c0 < cols; c0 += l.slab) {
         const int nc = l.slab < cols - c0 ? l.slab : cols - c0;
         SlabArgs sa{};
@@ -537,15 +547,11 @@ int rk_linear_gemm(float* y, const float* x, long long x_ld, int M, int N, int K
         GemmArgs g{};
         g.y = y; g.a = pieces; g.w = sa.out; g.sc = sa.sc; g.ex = ex; g.ew = sa.ew; g.bias = bias; g.res = residual;
         g.y_ld = cols; g.M = M; g.N = rows; g.Mp = l.Mp; g.Np = l.Np; g.steps = l.steps; g.col0 = c0; g.cols = cols;
-        // 128 x 256 tiles where they give every CU two of them, else 128 x 128 (1777 x 2048 outputs: 112 tiles of 256
-        // columns leave half the CUs idle), else 64 x 128; eight waves of 32 x 64 beat four of 64 x 64 there (157
-        // against 168 us at 1777 x 2048 x 6144: two waves per SIMD)
-        auto tiles = [&](int bm, int bn) {
-            return (long long)((M + bm - 1) / bm) * ((rows + bn - 1) / bn);
-        };
+        g.S = l.S;
+        g.part = reinterpret_cast<float*>(ws + l.part);
         int rc;
-        if (tiles(128, 256) >= 2 * cus) rc = launch_gemm<2, 4, 4>(g, quant, glu != 0, st);
-        else if (M > 64) rc = launch_gemm<4, 2, 2>(g, quant, glu != 0, st);
+        if (l.form == 0) rc = launch_gemm<2, 4, 4>(g, quant, glu != 0, st);
+        else if (l.form == 1) rc = launch_gemm<4, 2, 2>(g, quant, glu != 0, st);
         else rc = launch_gemm<2, 2, 2>(g, quant, glu != 0, st);
         if (rc) return rc;
     }

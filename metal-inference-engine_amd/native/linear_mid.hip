@@ -1,0 +1,456 @@
+// Linears of a full decode batch or a short prompt (33 to a few hundred rows), gfx950; semantics in linear_gemm.hip.
+//
+// What bounds them is reading W (2048 x 6144 INT4: 7.9 MB, 1.5 us at a copy's rate) and the latency of a chain of
+// launches, so W is read once, as stored, straight into MFMA operands, and the whole chip shares it: a workgroup takes
+// 16 NT weight rows and one K-split, its eight waves an eighth of the split each, and every wave multiplies its blocks
+// with all the activation rows of a row block (48 or 64). The activations come as operand-ready pieces from memory
+// (the L2s hold them: 4 bytes per value, 0.5 MB for 64 x 2048), written once by split_operands; they pass through no
+// LDS, since no two waves of a workgroup use the same ones. INT8 / INT4: two fp16 pieces, codes exact in fp16, a
+// block's scale (and INT4 min times the block's activation sum) on the VALU, as linear.hip; bf16: three bf16 pieces
+// (exact), so that W needs no conversion. The waves' sums meet in LDS; K-splits meet in memory, added in order by
+// mid_finish.
+//
+// Measured (64 rows, INT4, all launches): 12288 x 2048 with silu * up 26 us, 2048 x 6144 26 us (gemm_rows 46 and 34, the
+// fp32 GEMM on the expanded weight 100 and 110); mid_rows itself 24 and 18 us in a trace, of which the activations'
+// 0.5 MB per CU from the L2 (64 bytes per cycle) and the VALU's scales and mins are about 4 us each, the MFMAs 4.
+#include "linear_pieces.h"
+
+namespace rk {
+namespace {
+
+constexpr int kWaves = 8;
+
+template <int WT> constexpr int pieces_of() { return WT == RK_W_BF16 ? 3 : 2; }
+
+struct MidArgs {
+    float* y;
+    const uint16_t* a;             // [row block][K / 32][piece][MT][64 lanes][8]: MFMA operands
+    const float* sums;             // INT4: [row block][K / 32][16 MT] block sums of the scaled activations
+    const int* ex;                 // [M] exponents (INT8 / INT4)
+    const void* w;
+    const uint16_t* scales;
+    const uint16_t* mins;
+    const float* bias;
+    const float* res;
+    f32x4* part;                   // S > 1: [row block][row group][split][item]
+    int M, N, K;                   // N: weight rows (glu: both halves)
+    int S, SB, WB;                 // splits; blocks per split and per wave
+    int MB, G, glu;                // row blocks; groups of 16 NT weight rows
+};
+
+// Row m of x as operands of the row block m / (16 MT): lane (r, g) of tile i takes row 16 i + r's values 8g .. 8g + 7
+// of a block. fp16 pairs of x * 2^ex (INT4: in the order of int4_f16) or bf16 thirds.
+template <int WT, int MT>
+__global__ __launch_bounds__(256) void split_operands(uint16_t* a, float* sums, int* ex, const float* x, long long x_ld,
+                                                      int K) {
+    constexpr int P = pieces_of<WT>();
+    __shared__ float red[4];
+    const int m = blockIdx.x, tid = threadIdx.x;
+    const int mb = m / (16 * MT), i = m % (16 * MT) / 16, r = m % 16, nblk = K / kQB;
+    const float* xr = x + (size_t)m * x_ld;
+    int k = 0;
+    if constexpr (WT != RK_W_BF16) {
+        float big = 0.0f;
+        for (int c = tid; c < K / 8; c += 256) {
+            const f32x4 v0 = *reinterpret_cast<const f32x4*>(xr + 8 * c), v1 = *reinterpret_cast<const f32x4*>(xr + 8 * c + 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) big = fmaxf(big, fmaxf(fabsf(v0[e]), fabsf(v1[e])));
+        }
+        k = top_exponent(block_absmax(big, red));
+        if (tid == 0) ex[m] = k;
+    }
+    for (int c = tid; c < K / 8; c += 256) {
+        const f32x4 v0 = *reinterpret_cast<const f32x4*>(xr + 8 * c), v1 = *reinterpret_cast<const f32x4*>(xr + 8 * c + 4);
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[e] = WT == RK_W_BF16 ? v0[e] : ldexpf(v0[e], k);
+            v[4 + e] = WT == RK_W_BF16 ? v1[e] : ldexpf(v1[e], k);
+        }
+        u32x4 pc[P];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int e0 = WT == RK_W_INT4 ? q : 2 * q, e1 = WT == RK_W_INT4 ? q + 4 : 2 * q + 1;
+            if constexpr (WT == RK_W_BF16) {
+                Split3 s0 = split3(v[e0]), s1 = split3(v[e1]);
+                if (!__builtin_isfinite(v[e0])) s0.mid = s0.lo = 0u;   // an infinity has no rest
+                if (!__builtin_isfinite(v[e1])) s1.mid = s1.lo = 0u;
+                pc[0][q] = pack_hi2(s0.hi, s1.hi);
+                pc[1][q] = pack_hi2(s0.mid, s1.mid);
+                pc[2][q] = pack_hi2(s0.lo, s1.lo);
+            } else {
+                float h0, l0, h1, l1;
+                split2(v[e0], h0, l0);
+                split2(v[e1], h1, l1);
+                pc[0][q] = pack_f16(h0, h1);
+                pc[1][q] = pack_f16(l0, l1);
+            }
+        }
+        const size_t blk = (size_t)mb * nblk + (c >> 2);
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+            *reinterpret_cast<u32x4*>(a + (((blk * P + p) * MT + i) * 64 + 16 * (c & 3) + r) * 8) = pc[p];
+        if constexpr (WT == RK_W_INT4) {           // the four threads of a block are neighbours in one wave
+            float sum = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) sum += v[e];
+            sum += __shfl_xor(sum, 1);
+            sum += __shfl_xor(sum, 2);
+            if ((c & 3) == 0) sums[blk * (16 * MT) + 16 * i + r] = sum;
+        }
+    }
+}
+
+// weight row behind row lr of the tiles: lr, or with glu gate rows 8T .. 8T + 7 then their up rows in tile T
+__device__ __forceinline__ size_t mid_row(const MidArgs& a, int lr) {
+    if (!a.glu) return (size_t)min(lr, a.N - 1);
+    const int F = a.N >> 1, f = min(8 * (lr >> 4) + (lr & 7), F - 1);
+    return (size_t)((lr & 8) ? F + f : f);
+}
+
+// rows 4g .. 4g + 3 of tile i, column c of tile t (lane l = 16 g + c of item (i, t)): powers of two, bias, residual or
+// silu * up, store; whole waves enter
+template <int WT, int MT, int NT>
+__device__ __forceinline__ void mid_store(const MidArgs& a, f32x4 v, int mb, int rg, int item) {
+    const int i = item / (64 * NT), t = item / 64 % NT, l = item & 63, c = l & 15;
+    const int m0 = 16 * MT * mb + 16 * i + 4 * (l >> 4);
+    if constexpr (WT != RK_W_BF16) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = ldexpf(v[e], -a.ex[min(m0 + e, a.M - 1)]);
+    }
+    if (a.glu) {                                   // uniform
+        f32x4 u;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) u[e] = __shfl_xor(v[e], 8);
+        const int F = a.N >> 1, n = 8 * (rg * NT + t) + (c & 7);
+        if (c < 8 && n < F) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (m0 + e < a.M) a.y[(size_t)(m0 + e) * F + n] = silu_times(v[e], u[e]);
+        }
+        return;
+    }
+    const int n = 16 * (rg * NT + t) + c;
+    if (n >= a.N) return;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        if (m0 + e >= a.M) continue;
+        float o = v[e];
+        if (a.bias) o = __fadd_rn(o, a.bias[n]);
+        if (a.res) o = __fadd_rn(o, a.res[(size_t)(m0 + e) * a.N + n]);
+        a.y[(size_t)(m0 + e) * a.N + n] = o;
+    }
+}
+
+// 4 x 4 transpose over the wave's 16-lane groups: register d of group g <- register g of group d
+__device__ __forceinline__ u32x4 xpose4(uint32_t a0, uint32_t a1, uint32_t a2, uint32_t a3) {
+    const auto s02 = __builtin_amdgcn_permlane32_swap(a0, a2, false, false);
+    const auto s13 = __builtin_amdgcn_permlane32_swap(a1, a3, false, false);
+    const auto s01 = __builtin_amdgcn_permlane16_swap(s02[0], s13[0], false, false);
+    const auto s23 = __builtin_amdgcn_permlane16_swap(s02[1], s13[1], false, false);
+    return (u32x4){s01[0], s01[1], s23[0], s23[1]};
+}
+
+// 8 INT4 codes minus 8 as fp16, in the order 0 4 1 5 2 6 3 7: a code q as the low bits of 0x6400 is the fp16 value
+// 1024 + q; the subtraction is exact
+__device__ __forceinline__ u32x4 int4_f16(uint32_t v) {
+    const f16x2 off = {(_Float16)1032.0f, (_Float16)1032.0f};
+    u32x4 o;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const uint32_t p = (v >> (4 * q) & 0x000F000Fu) | 0x64006400u;
+        o[q] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, p) - off);
+    }
+    return o;
+}
+
+// 8 INT8 codes as fp16: q + 128 as the low byte of 0x6400 is the fp16 value 1152 + q; the subtraction is exact
+__device__ __forceinline__ u32x4 int8_f16(uint32_t lo, uint32_t hi) {
+    const f16x2 off = {(_Float16)1152.0f, (_Float16)1152.0f};
+    u32x4 o;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const uint32_t u = (q < 2 ? lo : hi) ^ 0x80808080u;
+        const uint32_t p = __builtin_amdgcn_perm(0x64646464u, u, q & 1 ? 0x04030402u : 0x04010400u);
+        o[q] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, p) - off);
+    }
+    return o;
+}
+
+// One workgroup per (row group, K-split, row block). A wave walks its blocks four at a time (a chunk: 16-byte weight
+// loads of whole blocks, transposed over the lane groups as in linear.hip), the next chunk's weights and scales and the
+// next block's activations requested ahead. Chunks past the wave's range repeat loaded addresses and enter with
+// weight 0, so the loop body has no branch.
+template <int WT, int MT, int NT>
+__global__ __launch_bounds__(64 * kWaves) void mid_rows(MidArgs a) {
+    constexpr int P = pieces_of<WT>();
+    constexpr int CH = WT == RK_W_INT4 ? 1 : WT == RK_W_INT8 ? 2 : 4;   // 16-byte loads per tile and chunk
+    constexpr bool QUANT = WT != RK_W_BF16;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, grp = lane >> 4;
+    const int nblk = a.K / kQB;
+    // row blocks of one (row group, split) are 8 workgroups apart: on one XCD, whose L2 keeps the weights for them
+    const int oct = blockIdx.x / (8 * a.MB), in8 = blockIdx.x % (8 * a.MB);
+    const int t_id = 8 * oct + in8 % 8, mb = in8 / 8;
+    if (t_id >= a.G * a.S) return;
+    const int rg = t_id / a.S, sp = t_id % a.S;
+    const int k0 = sp * a.SB + wave * a.WB;
+    const int k1 = min(min(nblk, (sp + 1) * a.SB), k0 + a.WB);
+
+    const uint8_t* wrow[NT];
+    const uint16_t* srow[NT];
+    const uint16_t* mrow[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const size_t n = mid_row(a, 16 * (rg * NT + t) + r);
+        wrow[t] = static_cast<const uint8_t*>(a.w) + n * ((size_t)nblk * (WT == RK_W_BF16 ? 64 : WT == RK_W_INT8 ? 32 : 16));
+        if constexpr (QUANT) srow[t] = a.scales + n * nblk;
+        if constexpr (WT == RK_W_INT4) mrow[t] = a.mins + n * nblk;
+    }
+    u32x4 wn[NT][CH];
+    uint32_t sn[QUANT ? NT : 1][2], mn[WT == RK_W_INT4 ? NT : 1][2];
+    auto load_w = [&](int kb) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+#pragma unroll
+            for (int c = 0; c < CH; ++c) {
+                size_t off;
+                if constexpr (WT == RK_W_BF16) off = (size_t)min(kb + c, nblk - 1) * 64 + 16 * grp;
+                else if constexpr (WT == RK_W_INT8) off = (size_t)min(kb + grp, nblk - 1) * 32 + 16 * c;
+                else off = (size_t)min(kb + grp, nblk - 1) * 16;
+                wn[t][c] = *reinterpret_cast<const u32x4*>(wrow[t] + off);
+            }
+            if constexpr (QUANT) {                 // nblk and kb are even
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int kk = min(kb + 2 * h, nblk - 2);
+                    sn[t][h] = *reinterpret_cast<const uint32_t*>(srow[t] + kk);
+                    if constexpr (WT == RK_W_INT4) mn[t][h] = *reinterpret_cast<const uint32_t*>(mrow[t] + kk);
+                }
+            }
+        }
+    };
+    u32x4 xa[2][P][MT];
+    f32x4 bs[2][WT == RK_W_INT4 ? MT : 1];
+    auto load_x = [&](int kb, int slot) {
+        const size_t blk = (size_t)mb * nblk + min(kb, nblk - 1);
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+                xa[slot][p][i] = *reinterpret_cast<const u32x4*>(a.a + (((blk * P + p) * MT + i) * 64 + lane) * 8);
+        if constexpr (WT == RK_W_INT4) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+                bs[slot][i] = *reinterpret_cast<const f32x4*>(a.sums + blk * (16 * MT) + 16 * i + 4 * grp);
+        }
+    };
+    f32x4 acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[i][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+    if (k0 < k1) {
+        load_w(k0);
+        load_x(k0, 0);
+    }
+    for (int kc = k0; kc < k1; kc += 4) {
+        u32x4 wc[NT][CH];
+        uint32_t sc[QUANT ? NT : 1][2], mc[WT == RK_W_INT4 ? NT : 1][2];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            if constexpr (WT == RK_W_INT4) wc[t][0] = xpose4(wn[t][0][0], wn[t][0][1], wn[t][0][2], wn[t][0][3]);
+            else if constexpr (WT == RK_W_INT8) {
+                const u32x4 lo = xpose4(wn[t][0][0], wn[t][0][2], wn[t][1][0], wn[t][1][2]);
+                const u32x4 hi = xpose4(wn[t][0][1], wn[t][0][3], wn[t][1][1], wn[t][1][3]);
+                wc[t][0] = (u32x4){lo[0], hi[0], lo[1], hi[1]};
+                wc[t][1] = (u32x4){lo[2], hi[2], lo[3], hi[3]};
+            } else {
+#pragma unroll
+                for (int c = 0; c < CH; ++c) wc[t][c] = wn[t][c];
+            }
+            if constexpr (QUANT) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    sc[t][h] = sn[t][h];
+                    if constexpr (WT == RK_W_INT4) mc[t][h] = mn[t][h];
+                }
+            }
+        }
+        load_w(kc + 4 < k1 ? kc + 4 : kc);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            const int s = d & 1;
+            // past the wave's range: zero scales and mins, zero bf16 weights (a mask; a condition becomes a branch)
+            const uint32_t in = kc + d < k1 ? 0xffffffffu : 0u;
+            load_x(min(kc + d + 1, k1 - 1), s ^ 1);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                u32x4 b;
+                if constexpr (WT == RK_W_INT4) b = int4_f16(wc[t][0][d]);
+                else if constexpr (WT == RK_W_INT8) b = int8_f16(wc[t][d >> 1][2 * (d & 1)], wc[t][d >> 1][2 * (d & 1) + 1]);
+                else b = wc[t][d] & (u32x4){in, in, in, in};
+                float f = 0.0f, mi = 0.0f;
+                if constexpr (QUANT) f = half_to_f32((sc[t][d >> 1] & in) >> (16 * (d & 1)));
+                // INT4: s (q - 8) + (8 s + min), whose two terms stay small (s q and min nearly cancel over a block)
+                if constexpr (WT == RK_W_INT4) mi = fmaf(8.0f, f, half_to_f32((mc[t][d >> 1] & in) >> (16 * (d & 1))));
+#pragma unroll
+                for (int i = 0; i < MT; ++i) {
+                    f32x4 p = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int q = P - 1; q >= 0; --q)
+                        p = QUANT ? mfma_f16(xa[s][q][i], b, p) : mfma16x16x32(xa[s][q][i], b, p);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        if constexpr (QUANT) acc[i][t][e] = fmaf(f, p[e], acc[i][t][e]);
+                        else acc[i][t][e] += p[e];
+                        if constexpr (WT == RK_W_INT4) acc[i][t][e] = fmaf(mi, bs[s][i][e], acc[i][t][e]);
+                    }
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);     // one block ahead: more in flight does not fit the registers
+        }
+    }
+
+    // the waves' sums, in wave order
+    constexpr int ITEMS = 64 * MT * NT;
+    f32x4* red = reinterpret_cast<f32x4*>(smem);
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) red[wave * ITEMS + (i * NT + t) * 64 + lane] = acc[i][t];
+    __syncthreads();
+    for (int item = threadIdx.x; item < ITEMS; item += 64 * kWaves) {
+        f32x4 v = red[item];
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) {
+            const f32x4 o = red[w * ITEMS + item];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] += o[e];
+        }
+        if (a.S == 1) mid_store<WT, MT, NT>(a, v, mb, rg, item);
+        else a.part[((size_t)(mb * a.G + rg) * a.S + sp) * ITEMS + item] = v;
+    }
+}
+
+// The splits of one (row block, row group, wave of items), in order.
+template <int WT, int MT, int NT>
+__global__ __launch_bounds__(256) void mid_finish(MidArgs a) {
+    constexpr int ITEMS = 64 * MT * NT;
+    const int item = 256 * blockIdx.y + threadIdx.x;
+    if (item >= ITEMS) return;                     // whole waves
+    const f32x4* p = a.part + (size_t)blockIdx.x * a.S * ITEMS + item;
+    f32x4 v = p[0];
+    for (int s = 1; s < a.S; ++s) {
+        const f32x4 o = p[(size_t)s * ITEMS];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] += o[e];
+    }
+    mid_store<WT, MT, NT>(a, v, blockIdx.x / a.G, blockIdx.x % a.G, item);
+}
+
+struct MidPlan {
+    int MB, MT, NT, G, S, SB, WB;
+    size_t sums, ex, part, total;
+};
+
+// Rows up to which this form is the faster one (12288 x 2048 with silu * up, 2048 x 6144, 8224 x 2048; us, this form
+// against gemm_rows): INT4 at 128 rows 48 / 33 / 46 against 52 / 39 / 41 and at 160 rows 68 / 46 / 66 against
+// 71 / 43 / 65; INT8 at 256 rows 69 / 41 / 56 against 74 / 44 / 66 and at 384 rows 111 / 59 / 84 against 109 / 54 / 68;
+// bf16 at 96 rows 46 / 29 / 43 against 51 / 37 / 39 and at 128 rows 54 / 33 / 50 against 52 / 38 / 41. INT4 has its mins
+// on the VALU here, bf16 three pieces and two bytes of W per value.
+int mid_rows_max(int w_type) { return w_type == RK_W_INT8 ? 256 : w_type == RK_W_INT4 ? 128 : 96; }
+
+// NT, S: the least estimated time over the rounds of one workgroup per CU: a block costs a wave its activations from
+// the L2 (1 KB per 16 cycles and CU) or its MFMAs (19 cycles each, two waves per SIMD), whichever is longer, a
+// workgroup a start and an end, a split its partials
+MidPlan mid_plan(int M, int N, int K, int w_type, int glu) {
+    MidPlan p{};
+    const int nblk = K / kQB, P = w_type == RK_W_BF16 ? 3 : 2;
+    const int tiles = glu ? (N / 2 + 7) / 8 : (N + 15) / 16;
+    p.MB = (M + 63) / 64;
+    p.MT = (M + 16 * p.MB - 1) / (16 * p.MB) <= 3 ? 3 : 4;
+    int cus = device_cus();
+    if (cus <= 0) cus = 256;
+    double best = 0;
+    for (int nt = 1; nt <= (w_type == RK_W_BF16 ? 2 : w_type == RK_W_INT4 && p.MT == 4 ? 3 : 4); ++nt)
+        for (int s = 1; s <= 16 && s <= (nblk + 31) / 32 * 2; ++s) {
+            const int sb = ((nblk + s - 1) / s + 1) / 2 * 2;
+            const int wb = ((sb + kWaves - 1) / kWaves + 1) / 2 * 2;
+            const int g = (tiles + nt - 1) / nt, used = (nblk + sb - 1) / sb;
+            const double rounds = (double)((long long)g * used * p.MB + cus - 1) / cus;
+            const double blk = 128.0 * P * p.MT > 38.0 * P * p.MT * nt ? 128.0 * P * p.MT : 38.0 * P * p.MT * nt;
+            const double cost = (double)(long long)rounds * ((wb + 3) / 4 * 4 * (blk + 60.0 * nt) + 3000.0) +
+                                (used > 1 ? 5000.0 + 20.0 * used * p.MB * g * nt * p.MT / 16 : 0.0);
+            if (best == 0 || cost < best) {
+                best = cost;
+                p.NT = nt; p.G = g; p.S = used; p.SB = sb; p.WB = wb;
+            }
+        }
+    const size_t rows = (size_t)p.MB * 16 * p.MT;
+    auto up = [](size_t n) { return (n + 255) / 256 * 256; };
+    p.sums = up(rows * K * 2 * P);
+    p.ex = p.sums + (w_type == RK_W_INT4 ? up(rows * nblk * 4) : 0);
+    p.part = p.ex + up(rows * 4);
+    p.total = p.part + (p.S > 1 ? (size_t)p.MB * p.G * p.S * 64 * p.MT * p.NT * sizeof(f32x4) : 0);
+    return p;
+}
+
+}  // namespace
+
+bool mid_takes(int M, int K, int w_type, const void* scales, const void* mins) {
+    // scales and mins are read two blocks at a time
+    return M <= mid_rows_max(w_type) && K % (2 * kQB) == 0 && reinterpret_cast<uintptr_t>(scales) % 4 == 0 &&
+           reinterpret_cast<uintptr_t>(mins) % 4 == 0;
+}
+
+size_t mid_workspace_bytes(int M, int N, int K, int w_type, int glu) { return mid_plan(M, N, K, w_type, glu).total; }
+
+int mid_linear(float* y, const float* x, long long x_ld, int M, int N, int K, const void* w, int w_type,
+               const void* scales, const void* mins, const float* bias, const float* residual, int glu,
+               void* workspace, hipStream_t stream) {
+    const MidPlan p = mid_plan(M, N, K, w_type, glu);
+    char* ws = static_cast<char*>(workspace);
+    uint16_t* ops = reinterpret_cast<uint16_t*>(ws);
+    float* sums = reinterpret_cast<float*>(ws + p.sums);
+    int* ex = reinterpret_cast<int*>(ws + p.ex);
+    MidArgs a{};
+    a.y = y; a.a = ops; a.sums = sums; a.ex = ex; a.w = w;
+    a.scales = static_cast<const uint16_t*>(scales); a.mins = static_cast<const uint16_t*>(mins);
+    a.bias = bias; a.res = residual; a.part = reinterpret_cast<f32x4*>(ws + p.part);
+    a.M = M; a.N = N; a.K = K; a.S = p.S; a.SB = p.SB; a.WB = p.WB; a.MB = p.MB; a.G = p.G; a.glu = glu ? 1 : 0;
+    using Split = void (*)(uint16_t*, float*, int*, const float*, long long, int);
+    using Fn = void (*)(MidArgs);
+    Split split = nullptr;
+    Fn rows = nullptr, fin = nullptr;
+#define RK_MID(W, T, C)                                                                                        \
+    if (w_type == W && p.MT == T && p.NT == C) {                                                               \
+        split = split_operands<W, T>;                                                                          \
+        rows = mid_rows<W, T, C>;                                                                              \
+        fin = mid_finish<W, T, C>;                                                                             \
+    }
+#define RK_MIDS(T)                                                                                             \
+    RK_MID(RK_W_INT4, T, 1) RK_MID(RK_W_INT4, T, 2) RK_MID(RK_W_INT4, T, 3)                                    \
+    RK_MID(RK_W_INT8, T, 1) RK_MID(RK_W_INT8, T, 2) RK_MID(RK_W_INT8, T, 3) RK_MID(RK_W_INT8, T, 4)            \
+    RK_MID(RK_W_BF16, T, 1) RK_MID(RK_W_BF16, T, 2)
+    RK_MIDS(3) RK_MIDS(4) RK_MID(RK_W_INT4, 3, 4)
+#undef RK_MIDS
+#undef RK_MID
+    if (!rows) return fail(RK_ERR_ARG, "rk_linear_gemm: no kernel for %d x %d tiles", p.MT, p.NT);
+    hipLaunchKernelGGL(split, dim3((unsigned)M), dim3(256), 0, stream, ops, sums, ex, x, x_ld, K);
+    if (int rc = check_launch("split_operands")) return rc;
+    const size_t lds = (size_t)kWaves * 64 * p.MT * p.NT * sizeof(f32x4);
+    if (int rc = allow_dynamic_lds((const void*)rows, lds)) return rc;
+    const long long ids = ((long long)p.G * p.S + 7) / 8 * 8 * p.MB;
+    if (ids >= (1ll << 31)) return fail(RK_ERR_ARG, "rk_linear_gemm: N %d too large", N);
+    hipLaunchKernelGGL(rows, dim3((unsigned)ids), dim3(64 * kWaves), lds, stream, a);
+    if (int rc = check_launch("mid_rows")) return rc;
+    if (p.S == 1) return RK_OK;
+    hipLaunchKernelGGL(fin, dim3((unsigned)(p.MB * p.G), (unsigned)((64 * p.MT * p.NT + 255) / 256)), dim3(256), 0, stream, a);
+    return check_launch("mid_finish");
+}
+
+}  // namespace rk

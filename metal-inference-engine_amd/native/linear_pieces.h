@@ -1,0 +1,59 @@
+// Shared by the linears of many rows (linear_gemm.hip, linear_mid.hip): fp16 pieces of fp32 values.
+#pragma once
+
+#include "rk_device.h"
+#include "rk_internal.h"
+
+namespace rk {
+
+// linear_mid.hip: the form for up to a few hundred rows, behind rk_linear_gemm
+bool mid_takes(int M, int K, int w_type, const void* scales, const void* mins);
+size_t mid_workspace_bytes(int M, int N, int K, int w_type, int glu);
+int mid_linear(float* y, const float* x, long long x_ld, int M, int N, int K, const void* w, int w_type,
+               const void* scales, const void* mins, const float* bias, const float* residual, int glu,
+               void* workspace, hipStream_t stream);
+
+constexpr int kQB = 32;                            // weights per quantization block = one MFMA's k-extent
+constexpr int kTop = 14;                           // a row's largest value lies in [2^kTop, 2^(kTop + 1))
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ f32x4 mfma_f16(u32x4 a, u32x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0,
+                                                  0);
+}
+
+__device__ __forceinline__ uint32_t pack_f16(float a, float b) {   // round to nearest even
+    return __builtin_bit_cast(uint32_t, (f16x2){(_Float16)a, (_Float16)b});
+}
+
+__device__ __forceinline__ float half_to_f32(uint32_t h) { return (float)__builtin_bit_cast(_Float16, (uint16_t)h); }
+
+// the power of two that puts the magnitude m into [2^kTop, 2^(kTop + 1)): its exponent (0 for m = 0; inf and NaN as
+// the largest finite exponent, so that they stay inf and NaN in the pieces)
+__device__ __forceinline__ int top_exponent(float m) {
+    const int e = (int)(__float_as_uint(m) >> 23) - 127;
+    return m == 0.0f ? 0 : kTop - max(min(e, 127), -112);
+}
+
+// hi and lo pieces of v (already scaled): hi = fp16(v), lo = fp16(v - hi); an infinite hi has no rest
+__device__ __forceinline__ void split2(float v, float& hi, float& lo) {
+    hi = (float)(_Float16)v;
+    lo = __builtin_isinf(hi) ? 0.0f : v - hi;
+}
+
+// largest |v| of a 256-thread workgroup, in every thread
+__device__ __forceinline__ float block_absmax(float m, float* red) {
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    return fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+}
+
+__device__ __forceinline__ float silu_times(float g, float u) {
+    return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-g * kLog2e)) * u;
+}
+
+}  // namespace rk

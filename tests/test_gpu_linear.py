@@ -254,10 +254,11 @@ def test_long_int8_matrix_on_the_persistent_grid(backend, N, K):
 @pytest.mark.parametrize("kind", ["bf16", "int8", "int4"])
 @pytest.mark.parametrize("M,N,K,glu", [(33, 100, 96, False), (64, 130, 2080, False), (65, 272, 64, False),
                                        (129, 1000, 512, False), (257, 515, 1056, False), (600, 4352, 256, False),
-                                       (33, 2 * 20, 256, True), (140, 2 * 1000, 544, True), (513, 2 * 2200, 128, True)])
+                                       (48, 17, 192, False), (49, 300, 3072, False), (97, 2064, 448, False),
+                                       (33, 2 * 20, 256, True), (96, 2 * 700, 1920, True), (250, 2 * 36, 320, True), (140, 2 * 1000, 544, True), (513, 2 * 2200, 128, True)])
 def test_many_row_linears_against_64_bits(backend, kind, M, N, K, glu):
-    """rk_linear_gemm at the edges of its tiles (rows and columns around 64, 128 and 256, odd numbers of 32-value
-    steps, glu halves that are not whole sixteens), with rows of very different magnitude and values of very different
+    """rk_linear_gemm at the edges of its forms and tiles (rows and columns around 48, 64, 96, 128 and 256, odd numbers
+    of 32-value steps, glu halves that are not whole sixteens, K-splits and wave shares with a remainder), with rows of very different magnitude and values of very different
     magnitude in one row, against the products in 64 bits. Bound: each output's sum of |x w| times 2^-24 for the
     rounding of x and the same for every 32-value partial sum's fp32 rounding, of which there are K / 32 in sequence."""
     w, deq = weight(kind, N, K, N + K)
