@@ -1,4 +1,5 @@
-// Shared by the linears of many rows (linear_gemm.hip, linear_mid.hip): fp16 pieces of fp32 values.
+// fp16 pieces of fp32 values: shared by the linears of many rows (linear_gemm.hip, linear_mid.hip) and the fp32
+// prefill attention (paged_prefill.hip).
 #pragma once
 
 #include "rk_device.h"
@@ -37,10 +38,21 @@ __device__ __forceinline__ int top_exponent(float m) {
     return m == 0.0f ? 0 : kTop - max(min(e, 127), -112);
 }
 
-// hi and lo pieces of v (already scaled): hi = fp16(v), lo = fp16(v - hi); an infinite hi has no rest
-__device__ __forceinline__ void split2(float v, float& hi, float& lo) {
-    hi = (float)(_Float16)v;
-    lo = __builtin_isinf(hi) ? 0.0f : v - hi;
+// hi and lo pieces of a pair (already scaled), packed: hi = fp16(v), lo = fp16(v - hi)
+struct Pieces {
+    uint32_t hi, lo;
+};
+__device__ __forceinline__ Pieces split_pair(float a, float b) {
+    const f16x2 h = __builtin_convertvector((f32x2_t){a, b}, f16x2);
+    const f16x2 l = __builtin_convertvector((f32x2_t){a - (float)h[0], b - (float)h[1]}, f16x2);
+    return {__builtin_bit_cast(uint32_t, h), __builtin_bit_cast(uint32_t, l)};
+}
+// the same where a value may be infinite: an infinite hi has no rest (inf - inf would make it NaN)
+__device__ __forceinline__ uint32_t rest_of(Pieces p) {
+    const uint32_t e = p.hi & 0x7c007c00u, m = p.hi & 0x03ff03ffu;   // exponent 31 with mantissa 0
+    const uint32_t drop = ((e & 0xffffu) == 0x7c00u && !(m & 0xffffu) ? 0xffffu : 0u) |
+                          (e >> 16 == 0x7c00u && !(m >> 16) ? 0xffff0000u : 0u);
+    return p.lo & ~drop;
 }
 
 // largest |v| of a 256-thread workgroup, in every thread
@@ -55,5 +67,11 @@ __device__ __forceinline__ float block_absmax(float m, float* red) {
 __device__ __forceinline__ float silu_times(float g, float u) {
     return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-g * kLog2e)) * u;
 }
+
+
+// Rows of 32 fp16 (64 bytes) in LDS: the 16-byte unit u of row R sits at u ^ swizzle(R). A read of lane l: row l % 16,
+// unit l / 16, is served 16 lanes at a time, rows 0-3 and 12-15 of one unit with rows 4-11 of the next, and these then
+// lie on all 16 units of the 256-byte bank line.
+__device__ __forceinline__ int swizzle(int R) { return (0x78 >> (2 * ((R >> 2) & 3))) & 3; }
 
 }  // namespace rk

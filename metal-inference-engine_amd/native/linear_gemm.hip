@@ -26,7 +26,7 @@
 // card), 2048 x 6144 440 -> 157 us; error against 64 bits 1.4e-6 -> 2.7e-7 of the result at K 6144. What bounds
 // gemm_rows: matrix-core issue and the fp32 joins beside it (copies without the loads, without the LDS reads or with a
 // quarter of the joins are each about 10 % faster), and whole tiles: 224 workgroups on 256 CUs at 2048 columns.
-#include "linear_pieces.h"
+#include "fp16_pieces.h"
 
 namespace rk {
 namespace {
@@ -46,10 +46,8 @@ __device__ __forceinline__ void load4_to_lds(const void* src, char* dst) {   // 
 
 // Operand layout of gemm_rows, shared by both operands: rows cut into steps of 32 values, [step][rows][32] fp16 (x:
 // [step][piece][rows][32]), so that a stage of a tile is one contiguous run per operand. The 16-byte unit u of row R
-// sits at u ^ swizzle(R): an operand read (lane l: row l % 16, unit l / 16) is served 16 lanes at a time, rows 0-3 and
-// 12-15 of one unit with rows 4-11 of the next, and these then lie on all 16 units of the 256-byte bank line.
+// sits at u ^ swizzle(R).
 // Rows past the matrix (up to whole tiles) are not written: their products are never stored.
-__device__ __forceinline__ int swizzle(int R) { return (0x78 >> (2 * ((R >> 2) & 3))) & 3; }
 __device__ __forceinline__ size_t unit_at(size_t slice, int rows, int R, int u) {
     return (slice * rows + R) * kBK + 8 * (u ^ swizzle(R));
 }
@@ -83,11 +81,9 @@ __global__ __launch_bounds__(256) void split_rows(uint16_t* a, int* ex, const fl
         u32x4 ph, pl;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            float h0, l0, h1, l1;
-            split2(v[2 * e], h0, l0);
-            split2(v[2 * e + 1], h1, l1);
-            ph[e] = pack_f16(h0, h1);
-            pl[e] = pack_f16(l0, l1);
+            const Pieces p = split_pair(v[2 * e], v[2 * e + 1]);
+            ph[e] = p.hi;
+            pl[e] = rest_of(p);
         }
         *reinterpret_cast<u32x4*>(a + unit_at(2 * (size_t)(c >> 2), Mp, m, c & 3)) = ph;
         *reinterpret_cast<u32x4*>(a + unit_at(2 * (size_t)(c >> 2) + 1, Mp, m, c & 3)) = pl;
@@ -99,8 +95,9 @@ __global__ __launch_bounds__(256) void split_rows(uint16_t* a, int* ex, const fl
             sum += __shfl_xor(sum, 2);
             if ((c & 3) == 0) {
                 const int b = c >> 2;              // sixteen blocks' pairs to a step
-                float h, l;
-                split2(ldexpf(sum, -kSumShift), h, l);
+                sum = ldexpf(sum, -kSumShift);
+                const Pieces p = split_pair(sum, 0.0f);
+                const float h = half_to_f32(p.hi & 0xffffu), l = half_to_f32(rest_of(p) & 0xffffu);
                 const size_t sl = 2 * (size_t)(K / kBK + (b >> 4));
                 *reinterpret_cast<uint32_t*>(a + unit_at(sl, Mp, m, (b & 15) >> 2) + 2 * (b & 3)) = pack_f16(h, 8.0f * h);
                 *reinterpret_cast<uint32_t*>(a + unit_at(sl + 1, Mp, m, (b & 15) >> 2) + 2 * (b & 3)) =

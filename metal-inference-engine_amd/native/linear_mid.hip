@@ -13,7 +13,7 @@
 // Measured (64 rows, INT4, all launches): 12288 x 2048 with silu * up 26 us, 2048 x 6144 26 us (gemm_rows 46 and 34, the
 // fp32 GEMM on the expanded weight 100 and 110); mid_rows itself 24 and 18 us in a trace, of which the activations'
 // 0.5 MB per CU from the L2 (64 bytes per cycle) and the VALU's scales and mins are about 4 us each, the MFMAs 4.
-#include "linear_pieces.h"
+#include "fp16_pieces.h"
 
 namespace rk {
 namespace {
@@ -79,11 +79,9 @@ __global__ __launch_bounds__(256) void split_operands(uint16_t* a, float* sums, 
                 pc[1][q] = pack_hi2(s0.mid, s1.mid);
                 pc[2][q] = pack_hi2(s0.lo, s1.lo);
             } else {
-                float h0, l0, h1, l1;
-                split2(v[e0], h0, l0);
-                split2(v[e1], h1, l1);
-                pc[0][q] = pack_f16(h0, h1);
-                pc[1][q] = pack_f16(l0, l1);
+                const Pieces p = split_pair(v[e0], v[e1]);
+                pc[0][q] = p.hi;
+                pc[1][q] = rest_of(p);
             }
         }
         const size_t blk = (size_t)mb * nblk + (c >> 2);

@@ -13,7 +13,7 @@
 //      range through a 2-stage LDS ring with 4 tiles of 32 keys in flight in their registers) or, at every other
 //      bf16 shape, prefill_attention_b16 (16 queries per consumer wave); both on bf16 operands (q, k, v as stored;
 //      p rounded; fp32 accumulation), so results carry bf16-level error. For an fp32 q or pool, or an exact
-//      request, prefill_attention_f32 (fp32 products and probabilities). Details at each kernel.
+//      request, prefill_attention_f32 (fp32-level products and probabilities). Details at each kernel.
 //   3. The output is divided by the softmax sum, gated and written as fp32 [N, Hq, D].
 // With a window W (causal only), query i also sees only keys above position p[s]+i-W (src/ops.py:77-81, 97-98): a
 // work item starts at the tile holding its first query's first visible key, so whole tiles below every query's
@@ -23,9 +23,9 @@
 // Backend.attention's contiguous K / V run here (one block holding all S positions).
 // Bounds: key positions past a segment's length are clamped for addressing (and masked), table entries clamped to
 // the pool, query rows past the segment clamped for loading (and not stored).
-#include "rk_device.h"
-#include "rk_internal.h"
+#include "fp16_pieces.h"
 
+#include <cfloat>
 #include <climits>
 
 namespace rk {
@@ -570,42 +570,72 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 }
 
 // ---- 3. attention with fp32 operands: the same work list, masks, splits and gate as prefill_attention, for an
-// fp32 q or pool and for exact requests (any group size, D = 64 / 128 / 256). The reference computes
-// attention in fp32 on widened inputs (src/ops.py:84-87, 91-103), so the products here are fp32 products:
-// v_mfma_f32_16x16x4_f32, bf16 pool rows widened exactly when staged, the probabilities kept in fp32.
+// fp32 q or pool and for exact requests (any group size, D = 64 / 128 / 256). The reference computes attention in fp32
+// on widened inputs (src/ops.py:84-87, 91-103). The fp32 matrix rate is 1/16 of the fp16 one, so the products are made
+// of fp16 pieces (fp16_pieces.h): every operand x, scaled by a power of two that puts its neighbourhood's largest value
+// into [2^14, 2^15), is hi + lo to 2^-24 of itself (2^-40 of that largest value where it is tiny), and a product is
+// lo hi + hi lo + hi hi (lo lo, 2^-24 of the product, is the rounding an fp32 product has too), summed in fp32:
+// 3/16 of the fp32 matrix time. The neighbourhoods: a query row; a group of 4 keys (its exponent multiplies the group's
+// scores, held 4 to a lane); a group of 4 value rows, whose exponent, with a common one E for the accumulators, scales
+// the group's probabilities. Probabilities enter as two pieces as well.
 // blockDim = 512: wave w takes query head (chunk * 4 + w % 4) of the group (none past the group's end: that
 // wave only helps stage) and queries 16 (w / 4) .. + 15 of the work item's 32. All 8 waves stage each tile of 32
-// keys into a 2-stage LDS ring, requested a whole tile ahead: K row-major ([32 keys][D + 4 floats]) and V transposed
-// ([D dims][32 + 4 floats]), both fp32. A staging unit is one 16-byte piece of 4 consecutive key rows (4 loads);
-// the V unit's 4 x 4 (fp32) or 4 x 8 (bf16) values are transposed in registers into 16-byte V^T writes. Per wave and
-// tile, on 16 x 16 accumulators (lane l: query l % 16, rows 4 (l / 16) .. + 3):
-//   S^T = K Q^T:  A = 16 keys x 4 dims from LDS (one 16-byte read feeds four MFMAs: quarter l / 16 takes dims
-//                 16 c + 4 (l / 16) + j of MFMA j), B = Q^T from registers (the same dims of the lane's query);
-//   O^T += V^T P^T: A = 16 dims x 4 keys from V^T (one 16-byte read of V^T[16 dt + l % 16][16 kt + 4 (l / 16) ..
-//                 + 3] feeds MFMAs r = 0 .. 3: keys 4 (l / 16) + r), B = P^T, the score accumulator's register r.
-// So every lane keeps its own query's softmax state (one reduction over the 4 quarters per tile), and O^T is
-// rescaled per lane. LDS reads are conflict-free: keys and dims are stored in permuted row orders (at the kernel)
-// under which the 16 rows a wave's lanes read lie an effective 2 (mod 4) 16-byte units apart, in lane order (the
-// rule measured for 16-byte reads on gfx950, at the 16-query bf16 kernel). Staging writes are conflict-free
-// for V^T (consecutive lanes take consecutive key groups of one piece) and at most 2-way for K (consecutive lanes
-// take consecutive pieces of one row group).
+// keys into a 2-stage LDS ring, requested a whole tile ahead, split into pieces on the way: K rows and V^T rows
+// ([dim][32 keys]), 8 bytes per value as in fp32. A staging unit is one 16-byte piece of 4 consecutive key rows (4
+// loads). Per wave and tile, on 16 x 16 accumulators (lane l: query l % 16, rows 4 (l / 16) .. + 3):
+//   S^T = K Q^T:  A = 16 keys x 32 dims, one 16-byte read per piece, B = Q^T from registers;
+//   O^T += V^T P^T: A = 16 dims x 32 keys, k-slot 8 (l / 16) + j standing for key 4 (l / 16) + j (j < 4) or
+//                 16 + 4 (l / 16) + j - 4, the keys of the lane's own scores, so B is the lane's 8 probabilities.
+// So every lane keeps its own query's softmax state, and O^T is rescaled per lane. LDS reads are conflict-free.
+// Measured (8 packed segments, 8/2 heads x 256, up to 2,048 new tokens on up to 16,384 cached ones; fp32): 4,985 us on
+// fp32 MFMA (111 TFLOP/s of 157) -> 2,050 us; error against 64 bits 1.2e-6 -> 7.2e-7 of the result. What bounds it: per
+// tile the MFMAs take 43 % of the time, the LDS reads (64 KB per wave) and the VALU (softmax, splits, addresses) as
+// much each; copies without the loads / the splits / the LDS writes / the softmax are 13 / 11 / 8 / 6 % faster, one
+// without staging 30 %.
 constexpr int kF32QW = 16;      // queries per wave
 constexpr int kF32Heads = 4;    // query heads per workgroup
-constexpr int kF32Pad = 4;      // fp32 padding of an LDS row
 
-__device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+// largest x over groups of N neighbouring lanes (8, 16, 32 or 64), in every lane
+template <int N>
+__device__ __forceinline__ float lanes_max(float x) {
+    x = fmaxf(x, dpp_f32<0xb1>(x));                  // quad_perm 1 0 3 2
+    x = fmaxf(x, dpp_f32<0x4e>(x));                  // quad_perm 2 3 0 1
+    x = fmaxf(x, dpp_f32<0x141>(x));                 // row_half_mirror: the other four of eight
+    if constexpr (N >= 16) x = fmaxf(x, dpp_f32<0x140>(x));   // row_mirror: the other eight of sixteen
+    if constexpr (N >= 32) {
+        const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+        x = fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
+    }
+    if constexpr (N >= 64) {
+        const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+        x = fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
+    }
+    return x;
+}
+
+// LDS rows of prefill_attention_f32's operands, 16-byte reads by lane l of row l % 16, unit l / 16 (+ 4 c): served 16
+// lanes at a time, rows 0-3 and 12-15 of one unit with rows 4-11 of the next; each order puts these on all 16 units of
+// the 256-byte bank line. K row `row` (D fp16): unit u at u ^ row, or at u ^ (row / 2) where a row is half a line.
+template <int D>
+__device__ __forceinline__ int k_unit(int row, int u) {
+    return D == 64 ? u ^ ((row >> 1) & 7) : u ^ (row & 15);
+}
+// V^T rows (32 keys, 64 bytes; units swizzled as fp16_pieces.h's rows): dim 4 i + j sits in row j D / 4 + i, so that
+// the lanes of a staging write, 4 dims apart, write consecutive rows
+template <int D>
+__device__ __forceinline__ int v_row(int dim) {
+    return (dim & 3) * (D / 4) + (dim >> 2);
 }
 
 // The lazy running maximum of a 16-query wave (scores s[kt][r] of lane l: query l % 16, keys 16 kt + 4 (l / 16) + r):
-// m is raised to the tile's maximum (scaled by qscale) only where that exceeds m by more than kLazy, so
-// p = 2^(s qscale - m) stays <= 2^kLazy (exact in fp32, representable in bf16). Each lane first compares its own 8
+// m is raised to the tile's maximum (sub-tile kt scaled by scale_kt > 0) only where that exceeds m by more than kLazy, so
+// p = 2^(s scale - m) stays <= 2^kLazy (exact in fp32, representable in bf16). Each lane first compares its own 8
 // scores; only when some lane of the wave exceeds the bound is the maximum over the query's 4 lanes formed, so the
-// result equals max-then-compare over all 32 keys while the common case needs no cross-lane exchange (scaling by
-// qscale > 0 is monotonic, so it commutes with max).
-__device__ __forceinline__ void lazy_max(const f32x4 (&s)[2], float& m, float qscale) {
-    float t = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])),
-                    fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3]))) * qscale;
+// result equals max-then-compare over all 32 keys while the common case needs no cross-lane exchange (scaling by a
+// positive factor is monotonic, so it commutes with max).
+__device__ __forceinline__ void lazy_max(const f32x4 (&s)[2], float& m, float scale0, float scale1) {
+    float t = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])) * scale0,
+                    fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])) * scale1);
     if (__any(t > m + kLazy)) {
         t = fmaxf(t, __shfl_xor(t, 16));
         t = fmaxf(t, __shfl_xor(t, 32));
@@ -613,16 +643,17 @@ __device__ __forceinline__ void lazy_max(const f32x4 (&s)[2], float& m, float qs
     }
 }
 
-// The end of a 16-query wave of the fp32- and bf16-operand kernels: o[dt] holds O^T[16 dt + 4 (lane / 16) + r][query
-// lane % 16] for D / 16 dim tiles, with the running (m, l) of the lane's query. Split items: the piece's (o, m, l) per
+// The end of a 16-query wave of the fp32- and bf16-operand kernels: o[dt] holds 4 consecutive dims of query lane % 16,
+// from 16 dt + 4 (lane / 16) on or, PERM, from 64 (dt / 4) + 16 (lane / 16) + 4 (dt % 4) on, with the running (m, l). Split items: the piece's (o, m, l) per
 // (slot, head, half) of 16 queries, then the arrival count; the last piece combines all of them in piece order (the
 // protocol and memory ordering of prefill_attention above). Then the rows are divided by l, gated and stored.
-template <int D>
+template <int D, bool PERM>
 __device__ __forceinline__ void finish_queries(const PrefillArgs& a, const int32_t* we, f32x4 (&o)[D / 16],
                                                float m_run, float l_run, int head, int half, int row0, int nq) {
     constexpr int NC = D / 16;
     const int lane = threadIdx.x & 63, qc = lane & 15, qq = lane >> 4;
     const int qi = half * kF32QW + qc;
+    auto dim_of = [&](int dt) { return PERM ? 64 * (dt >> 2) + 16 * qq + 4 * (dt & 3) : 16 * dt + 4 * qq; };
     const int piece = we[4] >> 16, pieces = we[4] & 0xffff;
     const int first = we[3] >= 0 && piece < pieces && we[3] + pieces <= a.n_slots ? we[3] : -1;
     if (first >= 0) {
@@ -636,7 +667,7 @@ __device__ __forceinline__ void finish_queries(const PrefillArgs& a, const int32
             return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(((unsigned long long)hi << 32) | lo),
                                                      (short)0, REC * 4, 0x00020000);
         };
-        auto o_off = [&](int dt) { return 4 * (qc * D + 16 * dt + 4 * qq); };
+        auto o_off = [&](int dt) { return 4 * (qc * D + dim_of(dt)); };
         const int m_off = 4 * (kF32QW * D + qc), l_off = 4 * (kF32QW * D + kF32QW + qc);
         {
             const auto rs = rsrc_of(piece);
@@ -683,16 +714,16 @@ __device__ __forceinline__ void finish_queries(const PrefillArgs& a, const int32
         float4 gv[NC];
         if (a.gate) {
             if (a.gate_dtype == RK_BF16) {
-                const uint16_t* gp = reinterpret_cast<const uint16_t*>(a.gate) + orow * D + 4 * qq;
+                const uint16_t* gp = reinterpret_cast<const uint16_t*>(a.gate) + orow * D;
 #pragma unroll
                 for (int dt = 0; dt < NC; ++dt) {
-                    const u32x2 w = *reinterpret_cast<const u32x2*>(gp + 16 * dt);
+                    const u32x2 w = *reinterpret_cast<const u32x2*>(gp + dim_of(dt));
                     gv[dt] = make_float4(bf16_lo(w[0]), bf16_hi(w[0]), bf16_lo(w[1]), bf16_hi(w[1]));
                 }
             } else {
-                const float* gp = reinterpret_cast<const float*>(a.gate) + orow * D + 4 * qq;
+                const float* gp = reinterpret_cast<const float*>(a.gate) + orow * D;
 #pragma unroll
-                for (int dt = 0; dt < NC; ++dt) gv[dt] = *reinterpret_cast<const float4*>(gp + 16 * dt);
+                for (int dt = 0; dt < NC; ++dt) gv[dt] = *reinterpret_cast<const float4*>(gp + dim_of(dt));
             }
         }
 #pragma unroll
@@ -703,17 +734,15 @@ __device__ __forceinline__ void finish_queries(const PrefillArgs& a, const int32
 #pragma unroll
                 for (int i = 0; i < 4; ++i) v[i] = v[i] * (1.0f / (1.0f + expf(-g[i])));
             }
-            *reinterpret_cast<float4*>(a.out + orow * D + 16 * dt + 4 * qq) = make_float4(v[0], v[1], v[2], v[3]);
+            *reinterpret_cast<float4*>(a.out + orow * D + dim_of(dt)) = make_float4(v[0], v[1], v[2], v[3]);
         }
     }
 }
 
 template <int D, typename TP, bool TAB_LDS>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_attention_f32(PrefillArgs a) {
-    constexpr int ROW = D + kF32Pad;                 // K row stride (floats)
-    constexpr int ROWT = kBKP + kF32Pad;             // V^T row stride (floats)
-    constexpr int KST = kBKP * ROW;                  // K floats per stage
-    constexpr int STAGE = KST + D * ROWT;            // K rows, then V^T rows
+    constexpr int KPC = kBKP * D * 2;                // bytes of one piece of a tile's K rows, and of its V^T rows
+    constexpr int STAGE = 4 * KPC;                   // K hi, K lo, V^T hi, V^T lo
     constexpr int EL = 16 / (int)sizeof(TP);         // elements per 16-byte load
     constexpr int PER_ROW = D / EL;                  // 16-byte pieces per row
     constexpr int GROUPS = kBKP / 4;                 // groups of 4 key rows per tile
@@ -721,10 +750,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     constexpr int NU = (2 * UNITS_T + 511) / 512;    // units per thread per tile
     static_assert(UNITS_T % 64 == 0 && (UNITS_T % 512 == 0 || 512 % UNITS_T == 0),
                   "each unit slot of a wave must take one tensor");
-    constexpr int NC = D / 16;                       // 16-dim groups
+    constexpr int NC = D / 32, ND = D / 16;          // 32-dim steps of the scores, 16-dim tiles of the output
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    float* lds = reinterpret_cast<float*>(smem);                               // [2 stages][K rows; V^T rows]
-    int* tab = reinterpret_cast<int*>(smem + 2 * STAGE * sizeof(float));       // [kTabCache] block ids
+    float* ksc = reinterpret_cast<float*>(smem + 2 * STAGE);                   // [2 stages][8] 2^-(a key group's exponent)
+    int* vex = reinterpret_cast<int*>(ksc + 2 * GROUPS);                       // [2 stages][8] a value group's exponent
+    int* tab = vex + 2 * GROUPS;                                               // [kTabCache] block ids
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const WorkSlot ws = work_slot(a.Hkv, (a.G + kF32Heads - 1) / kF32Heads);
@@ -764,24 +794,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         __syncthreads();
     }
 
-    // ---- staging: unit u = tid + 512 j (u < 2 UNITS_T) of tensor u / UNITS_T (K, V), e = u % UNITS_T; K: piece
-    // e % PER_ROW of rows 4 (e / PER_ROW) .. + 3, V: piece e / GROUPS of rows 4 (e % GROUPS) .. + 3. Load r of a unit
-    // is row 4 g + r; every load of a wave reads whole 128-byte row segments.
+    // ---- staging: unit u = tid + 512 j (u < 2 UNITS_T) of tensor u / UNITS_T (K, V): piece e % PER_ROW of rows
+    // 4 (e / PER_ROW) .. + 3, e = u % UNITS_T. Load r of a unit is row 4 g + r. The PER_ROW lanes of a group of 4 rows
+    // are neighbours in one wave, so the group's largest value is a shuffle tree.
     u32x4 st[NU][4];
-    // LDS rows are permuted so that the 16 rows a wave's lanes read for one 16-byte operand (lane l: row l % 16,
-    // column piece l / 16) lie 2 (mod 4) 16-byte units apart, in lane order, which gfx950 serves without bank
-    // conflicts: key 16 kt + i of a tile sits in K row 2 i + kt, dim 32 a + 16 b + i in V^T row 32 a + 2 i + b, so
-    // with the odd 16-byte strides (D + 4 and 36 floats) lane i's row is 2 i rows (2 x odd units) from lane 0's.
-    auto k_row = [](int key) { return 2 * (key & 15) + (key >> 4); };
-    auto v_row = [](int dim) { return (dim & ~31) + 2 * (dim & 15) + ((dim >> 4) & 1); };
     auto unit_of = [&](int j, int& g, int& pc) {
         const int u = tid + 512 * j, e = u % UNITS_T;
-        const bool is_v = u >= UNITS_T;
-        g = is_v ? e % GROUPS : e / PER_ROW;
-        pc = is_v ? e / GROUPS : e % PER_ROW;
-        return is_v;
+        g = e / PER_ROW;
+        pc = e % PER_ROW;
+        return UNITS_T == 512 ? j >= 1 : u >= UNITS_T;
     };
-    auto issue = [&](int t_rel) {
+    auto issue = [&](int t_rel) __attribute__((always_inline)) {
         const int tile = t_first + t_rel;
         // all block ids of the tile first (one wait for them), then the row loads
         int blk[NU][4], rr[NU][4];
@@ -817,41 +840,70 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             }
         }
     };
-    auto stash = [&](int stage) {
-        float* s = lds + stage * STAGE;
+    auto stash = [&](int stage) __attribute__((always_inline)) {
+        char* s = smem + stage * STAGE;
 #pragma unroll
         for (int j = 0; j < NU; ++j) {
             if (tid + 512 * j >= 2 * UNITS_T) continue;
             int g, pc;
-            if (unit_of(j, g, pc)) {                 // V^T[v_row(pc EL + d)][4 g .. + 3]
-                float* dst = s + KST + 4 * g;
-                if constexpr (sizeof(TP) == 4) {
+            const bool is_v = unit_of(j, g, pc);
+            float v[4][EL];
+            float big = 0.0f;
 #pragma unroll
-                    for (int d = 0; d < 4; ++d)
-                        *reinterpret_cast<f32x4*>(dst + v_row(pc * EL + d) * ROWT) = f32x4{
-                            __uint_as_float(st[j][0][d]), __uint_as_float(st[j][1][d]),
-                            __uint_as_float(st[j][2][d]), __uint_as_float(st[j][3][d])};
-                } else {                             // bf16 -> fp32, exact
+            for (int r = 0; r < 4; ++r)
 #pragma unroll
-                    for (int d = 0; d < 4; ++d) {
-                        *reinterpret_cast<f32x4*>(dst + v_row(pc * EL + 2 * d) * ROWT) = f32x4{
-                            bf16_lo(st[j][0][d]), bf16_lo(st[j][1][d]), bf16_lo(st[j][2][d]), bf16_lo(st[j][3][d])};
-                        *reinterpret_cast<f32x4*>(dst + v_row(pc * EL + 2 * d + 1) * ROWT) = f32x4{
-                            bf16_hi(st[j][0][d]), bf16_hi(st[j][1][d]), bf16_hi(st[j][2][d]), bf16_hi(st[j][3][d])};
-                    }
+                for (int d = 0; d < EL; ++d) {
+                    if constexpr (sizeof(TP) == 4) v[r][d] = __uint_as_float(st[j][r][d]);
+                    else v[r][d] = d & 1 ? bf16_hi(st[j][r][d >> 1]) : bf16_lo(st[j][r][d >> 1]);
+                    big = fmaxf(big, fabsf(v[r][d]));
                 }
-            } else {                                 // K[k_row(4 g + r)][pc EL ..]
-                float* dst = s + pc * EL;
+            // the group's exponent, from its finite values: an infinity stays one without taking its neighbours along
+            const bool odd = __any(big == INFINITY);
+            if (odd) {
+                big = 0.0f;
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+#pragma unroll
+                    for (int d = 0; d < EL; ++d) big = fmaxf(big, __builtin_isfinite(v[r][d]) ? fabsf(v[r][d]) : 0.0f);
+            }
+            big = lanes_max<PER_ROW>(big);
+            const int e = big == 0.0f && is_v ? 126 : top_exponent(big);   // zero values: no bound on the others
+            const float f = __uint_as_float((uint32_t)(127 + e) << 23);
+            if (pc == 0) {
+                if (is_v) vex[stage * GROUPS + g] = e;
+                else ksc[stage * GROUPS + g] = __uint_as_float((uint32_t)(127 - e) << 23);
+            }
+            // pieces of pairs: values of two keys (V^T rows hold keys side by side), of two dims (K)
+            Pieces pr[2 * EL];
+#pragma unroll
+            for (int i = 0; i < 2 * EL; ++i) {
+                const int d = i >> 1, r = 2 * (i & 1);          // V: dim d, keys r, r + 1
+                const int kr = i / (EL / 2), kd = 2 * (i % (EL / 2));   // K: key kr, dims kd, kd + 1
+                pr[i] = is_v ? split_pair(v[r][d] * f, v[r + 1][d] * f) : split_pair(v[kr][kd] * f, v[kr][kd + 1] * f);
+            }
+            if (odd) {
+#pragma unroll
+                for (int i = 0; i < 2 * EL; ++i) pr[i].lo = rest_of(pr[i]);
+            }
+            if (is_v) {                              // V^T[row of the dim][the group's 4 keys]
+                char* dst = s + 2 * KPC + 8 * (g >> 2);
+#pragma unroll
+                for (int d = 0; d < EL; ++d) {
+                    const int R = v_row<D>(pc * EL + d);
+                    char* q = dst + 64 * R + 16 * ((g & 3) ^ swizzle(R));
+                    *reinterpret_cast<u32x2*>(q) = (u32x2){pr[2 * d].hi, pr[2 * d + 1].hi};
+                    *reinterpret_cast<u32x2*>(q + KPC) = (u32x2){pr[2 * d].lo, pr[2 * d + 1].lo};
+                }
+            } else {                                 // K[key][dims pc EL ..]
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    if constexpr (sizeof(TP) == 4) {
-                        *reinterpret_cast<u32x4*>(dst + k_row(4 * g + r) * ROW) = st[j][r];
-                    } else {
-                        const u32x4 w = st[j][r];
-                        *reinterpret_cast<f32x4*>(dst + k_row(4 * g + r) * ROW) =
-                            f32x4{bf16_lo(w[0]), bf16_hi(w[0]), bf16_lo(w[1]), bf16_hi(w[1])};
-                        *reinterpret_cast<f32x4*>(dst + k_row(4 * g + r) * ROW + 4) =
-                            f32x4{bf16_lo(w[2]), bf16_hi(w[2]), bf16_lo(w[3]), bf16_hi(w[3])};
+                    const int row = 4 * g + r;
+                    char* q = s + 2 * D * row + 16 * k_unit<D>(row, pc * EL / 8) + 2 * (pc * EL % 8);
+#pragma unroll
+                    for (int d = 0; d < EL; d += 4) {
+                        const int i = (r * EL + d) / 2;
+                        *reinterpret_cast<u32x2*>(q + 2 * d) = (u32x2){pr[i].hi, pr[i + 1].hi};
+                        *reinterpret_cast<u32x2*>(q + 2 * d + KPC) = (u32x2){pr[i].lo, pr[i + 1].lo};
                     }
                 }
             }
@@ -866,41 +918,77 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int qfirst = a.causal ? p0 + half * kF32QW : n_keys - 1;
     const int qlast = a.causal ? p0 + min(half * kF32QW + kF32QW, nq) - 1 : n_keys - 1;
     const int lo_edge = a.window > 0 ? qlast - a.window : INT_MIN;
-    f32x4 qv[NC];                                    // Q[query][16 c + 4 qq .. + 3]
-    f32x4 o[NC];                                     // O^T[16 dt + 4 qq + r][query]
-    float m_run = -INFINITY, l_run = 0.0f;
+    u32x4 qh[NC], ql[NC];                            // Q[query][32 c + 8 qq .. + 7] * 2^(its exponent), two pieces
+    f32x4 o[ND];                                     // O^T[row 16 dt + 4 qq + r][query] * 2^E
+    float m_run = -INFINITY, l_run = 0.0f, qs = a.qscale;
+    int E = 0;
     if (active) {
-        const long long qb = ((long long)(row0 + (qi < nq ? qi : nq - 1)) * a.Hq + head) * D + 4 * qq;
-        if (a.q_dtype == RK_BF16) {
-            const uint16_t* qp = reinterpret_cast<const uint16_t*>(a.q) + qb;
+        const long long qb = ((long long)(row0 + (qi < nq ? qi : nq - 1)) * a.Hq + head) * D + 8 * qq;
+        float q[NC][8], big = 0.0f;
 #pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                const u32x2 w = *reinterpret_cast<const u32x2*>(qp + 16 * c);
-                qv[c] = f32x4{bf16_lo(w[0]), bf16_hi(w[0]), bf16_lo(w[1]), bf16_hi(w[1])};
+        for (int c = 0; c < NC; ++c) {
+            if (a.q_dtype == RK_BF16) {
+                const u32x4 w = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(a.q) + qb + 32 * c);
+#pragma unroll
+                for (int d = 0; d < 8; ++d) q[c][d] = d & 1 ? bf16_hi(w[d >> 1]) : bf16_lo(w[d >> 1]);
+            } else {
+                const f32x4* w = reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(a.q) + qb + 32 * c);
+                const f32x4 w0 = w[0], w1 = w[1];
+#pragma unroll
+                for (int d = 0; d < 8; ++d) q[c][d] = d < 4 ? w0[d] : w1[d - 4];
             }
-        } else {
-            const float* qp = reinterpret_cast<const float*>(a.q) + qb;
 #pragma unroll
-            for (int c = 0; c < NC; ++c) qv[c] = *reinterpret_cast<const f32x4*>(qp + 16 * c);
+            for (int d = 0; d < 8; ++d) big = fmaxf(big, fabsf(q[c][d]));
         }
+        big = fmaxf(big, __shfl_xor(big, 16));
+        big = fmaxf(big, __shfl_xor(big, 32));
+        const int e = top_exponent(big);
+        qs = ldexpf(a.qscale, -e);
 #pragma unroll
-        for (int c = 0; c < NC; ++c) o[c] = f32x4{};
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+                const Pieces p = split_pair(ldexpf(q[c][2 * d], e), ldexpf(q[c][2 * d + 1], e));
+                qh[c][d] = p.hi;
+                ql[c][d] = rest_of(p);
+            }
+#pragma unroll
+        for (int dt = 0; dt < ND; ++dt) o[dt] = f32x4{};
     }
 
     auto consume = [&](int t_rel, int stage) {
-        const float* ks = lds + stage * STAGE;
-        const float* vs = ks + KST;
+        const char* ks = smem + stage * STAGE;
+        const char* vs = ks + 2 * KPC;
         const int k0 = (t_first + t_rel) * kBKP;
-        f32x4 s[2] = {f32x4{}, f32x4{}};
+        // the cross products and the products of the leading pieces in sums of their own, added at the end
+        f32x4 s[2] = {f32x4{}, f32x4{}}, x[2] = {f32x4{}, f32x4{}};
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
+            u32x4 kh[2], kl[2];
 #pragma unroll
             for (int kt = 0; kt < 2; ++kt) {
-                const f32x4 kv = *reinterpret_cast<const f32x4*>(ks + (2 * qc + kt) * ROW + 16 * c + 4 * qq);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) s[kt] = mfma_f32(kv[j], qv[c][j], s[kt]);
+                const char* kp = ks + 2 * D * (16 * kt + qc) + 16 * k_unit<D>(qc, 4 * c + qq);
+                kh[kt] = *reinterpret_cast<const u32x4*>(kp);
+                kl[kt] = *reinterpret_cast<const u32x4*>(kp + KPC);
             }
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) x[kt] = mfma_f16(kl[kt], qh[c], x[kt]);
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) s[kt] = mfma_f16(kh[kt], qh[c], s[kt]);
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) x[kt] = mfma_f16(kh[kt], ql[c], x[kt]);
         }
+        // never 0: a masked score's product must stay -inf
+        const float f0 = fmaxf(qs * ksc[stage * GROUPS + qq], FLT_MIN);
+        const float f1 = fmaxf(qs * ksc[stage * GROUPS + 4 + qq], FLT_MIN);
+        int ve[GROUPS], vmin = 126;
+#pragma unroll
+        for (int g = 0; g < GROUPS; ++g) {
+            ve[g] = __builtin_amdgcn_readfirstlane(vex[stage * GROUPS + g]);
+            vmin = min(vmin, ve[g]);
+        }
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt) s[kt] += x[kt];
         // lane (qc, qq), register r of sub-tile kt: key k0 + 16 kt + 4 qq + r
         if (k0 + kBKP - 1 > qfirst || k0 <= lo_edge) {
 #pragma unroll
@@ -912,61 +1000,99 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 }
         }
         const float m_prev = m_run;
-        lazy_max(s, m_run, a.qscale);
+        lazy_max(s, m_run, f0, f1);
         const float mb = m_run == -INFINITY ? 0.0f : m_run;
+        // probabilities (at most 2^kLazy) enter as p 2^(E - a value group's exponent) < 2^(kTop + 1): E falls when a
+        // group of larger values comes
+        const int e_new = min(E, vmin + kTop + 1 - (int)kLazy);
+        const bool first = t_rel == 0;
+        if (first) E = vmin + kTop + 1 - (int)kLazy;
+        else if (e_new < E) {                        // uniform
+#pragma unroll
+            for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o[dt][r] = ldexpf(o[dt][r], e_new - E);
+            E = e_new;
+        }
         if (__any(m_run != m_prev)) {
             const float alpha = fast_exp2(m_prev - mb);     // 0 on the first tile (m_prev = -inf)
             l_run *= alpha;
 #pragma unroll
-            for (int dt = 0; dt < NC; ++dt) o[dt] *= alpha;
+            for (int dt = 0; dt < ND; ++dt) o[dt] *= alpha;
         }
+        u32x4 ph, pl;
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
+        for (int kt = 0; kt < 2; ++kt) {
+            int g = ve[4 * kt];
+#pragma unroll
+            for (int i = 1; i < 4; ++i) g = qq == i ? ve[4 * kt + i] : g;
+            float p[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                s[kt][r] = fast_exp2(fmaf(s[kt][r], a.qscale, -mb));
-                l_run += s[kt][r];                   // this lane's keys; the 4 lanes of a query are summed at the end
+                p[r] = fast_exp2(fmaf(s[kt][r], kt ? f1 : f0, -mb));
+                l_run += p[r];                       // this lane's keys; the 4 lanes of a query are summed at the end
+                p[r] = ldexpf(p[r], E - g);
             }
-        // V^T reads one dim group ahead of their MFMAs (group i: dims 16 (i % NC) + qc, keys 16 (i / NC) + 4 qq ..)
-        const float* vt = vs + 2 * qc * ROWT + 4 * qq;
-        auto vread = [&](int i) {
-            const int dt = i % NC, kt = i / NC;
-            return *reinterpret_cast<const f32x4*>(vt + (32 * (dt >> 1) + (dt & 1)) * ROWT + 16 * kt);
-        };
-        f32x4 vv = vread(0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);       // the first read,
 #pragma unroll
-        for (int i = 0; i < 2 * NC; ++i) {
-            const int kt = i / NC, dt = i % NC;
-            const f32x4 cur = vv;
-            if (i + 1 < 2 * NC) vv = vread(i + 1);
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // the next read,
-            __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);   // then this group's four MFMAs
+            for (int r = 0; r < 2; ++r) {
+                const Pieces pp = split_pair(p[2 * r], p[2 * r + 1]);
+                ph[2 * kt + r] = pp.hi;
+                pl[2 * kt + r] = pp.lo;
+            }
+        }
 #pragma unroll
-            for (int r = 0; r < 4; ++r) o[dt] = mfma_f32(cur[r], s[kt][r], o[dt]);
+        for (int d0 = 0; d0 < ND; d0 += 2) {
+            u32x4 vh[2], vl[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const char* vp = vs + 64 * (16 * (d0 + i) + qc) + 16 * (qq ^ swizzle(qc));
+                vh[i] = *reinterpret_cast<const u32x4*>(vp);
+                vl[i] = *reinterpret_cast<const u32x4*>(vp + KPC);
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i) o[d0 + i] = mfma_f16(vl[i], ph, o[d0 + i]);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) o[d0 + i] = mfma_f16(vh[i], pl, o[d0 + i]);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) o[d0 + i] = mfma_f16(vh[i], ph, o[d0 + i]);
         }
     };
 
-    // Stage t's rows are written after tile t - 1 is computed (stage (t - 1) & 1 is free once every wave passed the
-    // barrier that ended tile t - 2), then tile t + 1 is requested; one LDS-only barrier per tile.
+    // Stage t + 1's rows are written while tile t is computed (its buffer is free since the barrier that ended tile
+    // t - 1), then tile t + 2 is requested; one LDS-only barrier per tile. Waves w and w + 4 share a SIMD: one half
+    // stages before it computes, the other after, so that one's splits (VALU) run beside the other's MFMAs.
     if (n_tiles > 0) {
         issue(0);
         stash(0);
         if (n_tiles > 1) issue(1);
         lds_barrier();
-        for (int t = 0; t < n_tiles; ++t) {
-            if (active) consume(t, t & 1);
+        auto produce = [&](int t) __attribute__((always_inline)) {
             if (t + 1 < n_tiles) {
                 stash((t + 1) & 1);
                 if (t + 2 < n_tiles) issue(t + 2);
             }
+        };
+        for (int t = 0; t < n_tiles; ++t) {
+            if (half == 0) produce(t);
+            __builtin_amdgcn_s_setprio(1);           // the wave with MFMAs first (a staging wave fills the gaps)
+            if (active) consume(t, t & 1);
+            __builtin_amdgcn_s_setprio(0);
+            if (half == 1) produce(t);
             lds_barrier();
         }
     }
     if (!active) return;
     l_run += __shfl_xor(l_run, 16);
     l_run += __shfl_xor(l_run, 32);
-    finish_queries<D>(a, we, o, m_run, l_run, head, half, row0, nq);
+    // row 16 dt + 4 qq + r is dim 4 (row % (D / 4)) + row / (D / 4): four tiles D / 64 apart hold 4 consecutive dims
+    f32x4 od[ND];
+#pragma unroll
+    for (int q = 0; q < D / 64; ++q)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) od[4 * q + r][i] = ldexpf(o[q + D / 64 * i][r], -E);
+    finish_queries<D, true>(a, we, od, m_run, l_run, head, half, row0, nq);
 }
 
 // ---- 4. attention on bf16 operands, 16 queries per consumer wave, for bf16 q and pool (v_mfma_f32_16x16x32_bf16).
@@ -1206,7 +1332,7 @@ __global__ __launch_bounds__(kB16Threads) void prefill_attention_b16(PrefillArgs
         for (int i = 0; i < kB16Ahead; ++i) va[i] = vread(i);
         __builtin_amdgcn_sched_barrier(0);
         const float m_prev = m_run;
-        lazy_max(s, m_run, a.qscale);
+        lazy_max(s, m_run, a.qscale, a.qscale);
         const float mb = m_run == -INFINITY ? 0.0f : m_run;
         if (__any(m_run != m_prev)) {
             const float alpha = fast_exp2(m_prev - mb);     // 0 on the first tile (m_prev = -inf)
@@ -1241,7 +1367,7 @@ __global__ __launch_bounds__(kB16Threads) void prefill_attention_b16(PrefillArgs
     if (!active) return;
     l_run += __shfl_xor(l_run, 16);                  // each lane summed the probabilities of its own keys
     l_run += __shfl_xor(l_run, 32);
-    finish_queries<D>(a, we, o, m_run, l_run, head, half, row0, nq);
+    finish_queries<D, false>(a, we, o, m_run, l_run, head, half, row0, nq);
 }
 
 }  // namespace
@@ -1343,7 +1469,7 @@ int rk_paged_prefill(float* out, const void* q, int q_dtype, const void* k_new, 
         hipLaunchKernelGGL(fn, dim3(n_work * Hkv * chunks), dim3(kB16Threads), lds, s, a);
         return check_launch("prefill_attention_b16");
     }
-    const size_t lds = (size_t)2 * (kBKP * (D + kF32Pad) + D * (kBKP + kF32Pad)) * sizeof(float) +
+    const size_t lds = (size_t)2 * 4 * kBKP * D * sizeof(uint16_t) + 2 * (kBKP / 4) * 2 * sizeof(int) +
                        (tab_lds ? kTabCache * sizeof(int) : 0);
     const bool f32_pool = pool_dtype == RK_F32;
 #define RK_F32_PICK(DD)                                                                                      \

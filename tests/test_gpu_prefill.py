@@ -203,3 +203,46 @@ def test_split_item_with_an_empty_piece(backend, dtype, Hq, Hkv, d, tol):
     print(f"empty split piece, {which} {Hq}/{Hkv}x{d}: rel err {err:.2e}")
     assert torch.isfinite(out).all() and err < tol
     assert int(cnt.abs().sum()) == 0
+
+
+@pytest.mark.parametrize("Hq,Hkv,d,pool", [(8, 2, 256, torch.float32), (16, 4, 128, torch.float32),
+                                           (14, 2, 64, torch.float32), (8, 2, 256, torch.bfloat16),
+                                           (4, 4, 64, torch.bfloat16)])
+def test_fp32_operands_over_magnitudes(backend, Hq, Hkv, d, pool):
+    """The fp32-operand kernel on keys, values and queries whose rows differ by powers of two (its operands are scaled by
+    row and by group of four rows), with groups of zero values, large values that come late, and an infinite value,
+    against attention in 64 bits. Bound, per output: the scores' rounding (each |q k| to 2^-22, the sum of D of them in
+    D / 32 steps) moves every probability by that much twice (numerator and sum), and the products p v are rounded to
+    2^-22 each and summed in as many fp32 steps as there are tiles."""
+    g = torch.Generator().manual_seed(d + Hq)
+    n, p = 75, 141
+    S = n + p
+    case = wl.prefill_case([n], [p], Hq, Hkv, d, 16, torch.float32, seed=d)
+    two = lambda lo, hi, *shape: torch.exp2(torch.randint(lo, hi, shape, generator=g).float())
+    rows = (case.tables[0].long()[:, None] * 16 + torch.arange(16)).flatten()[:S]
+    k, v = torch.randn(S, Hkv, d, generator=g) * two(-14, 1, S, Hkv, 1), torch.randn(S, Hkv, d, generator=g)
+    v = v * two(-10, 3, S, Hkv, 1)
+    v[8:16] = 0.0
+    v[150:] *= 64.0
+    case.q.mul_(two(-20, 2, n, Hq, 1))
+    k, v, q = k.to(pool), v.to(pool), case.q
+    v[20, 0, 3] = float("inf")
+    case.k_pool, case.v_pool = case.k_pool.to(pool), case.v_pool.to(pool)
+    case.k_pool.view(-1, Hkv, d)[rows[:p]], case.v_pool.view(-1, Hkv, d)[rows[:p]] = k[:p], v[:p]
+    case.k_new, case.v_new = k[p:].clone(), v[p:].clone()
+    got, _, _ = run_gpu(backend, case, gate=False, exact=True)
+    G = Hq // Hkv
+    kd, vd, qd = k.double().repeat_interleave(G, 1), v.double().repeat_interleave(G, 1), q.double()
+    hidden = torch.arange(S)[None, :] > torch.arange(p, S)[:, None]
+    for h in range(Hq):
+        vh = vd[:, h].clone()
+        held = torch.isinf(vh).any(0)
+        vh[torch.isinf(vh)] = 0.0
+        s = (qd[:, h] @ kd[:, h].T) / d ** 0.5
+        ds = (qd[:, h].abs() @ kd[:, h].abs().T) / d ** 0.5 * (4 + d / 32) * 2.0 ** -24
+        pr = torch.softmax(s.masked_fill(hidden, float("-inf")), -1)
+        want, mass = pr @ vh, pr @ vh.abs()
+        bound = (2 * ds.masked_fill(hidden, 0.0).amax(1, keepdim=True) + (8 + 3 * S / 32) * 2.0 ** -24) * mass
+        over = ((got[:, h].double() - want).abs() / bound)[:, ~held].max()
+        assert over < 1.0, (h, float(over))
+        assert not torch.isfinite(got[:, h][:, held]).any()
