@@ -63,13 +63,37 @@ def _link(lib: Path, objs: list[Path], verbose: bool) -> None:
     os.replace(tmp, lib)
 
 
+CALLS = HERE / "rk_calls.so"              # call_paths.cpp: a CPython extension against torch's C++ API, host code only
+
+
+def _build_calls(verbose: bool) -> None:
+    import sysconfig
+
+    import torch
+    root = Path(torch.__file__).resolve().parent
+    tmp = CALLS.with_suffix(".so.tmp")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-missing-field-initializers",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{root / 'include'}",
+           f"-I{root / 'include/torch/csrc/api/include'}", f"-I{sysconfig.get_paths()['include']}",
+           str(HERE / "call_paths.cpp"), "-o", str(tmp), f"-L{root / 'lib'}", "-ltorch_python", "-ltorch",
+           "-ltorch_cpu", "-lc10"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("g++ failed on call_paths.cpp:\n" + r.stderr)
+    os.replace(tmp, CALLS)
+
+
 def build(verbose: bool = False) -> Path:
-    """Compile every source and link librk_path.so and librk_probe.so (always rebuilds). Returns the path
-    library."""
+    """Compile every source, link librk_path.so and librk_probe.so, and build rk_calls.so (always rebuilds). Returns
+    the path library."""
     OBJ_DIR.mkdir(exist_ok=True)
     srcs = SOURCES + PROBE_SOURCES
     with ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
+        calls = ex.submit(_build_calls, verbose)
         objs = dict(zip(srcs, ex.map(lambda s: _compile(s, verbose), srcs)))
+        calls.result()
     _link(LIB, [objs[s] for s in SOURCES], verbose)
     _link(PROBE_LIB, [objs[s] for s in PROBE_SOURCES] + [objs["rk_abi.cpp"]], verbose)
     return LIB

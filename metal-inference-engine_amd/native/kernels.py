@@ -4,11 +4,15 @@ PyTorch is used here only for device memory and the stream: every computation is
 Checks mirror the reference's host-side refusals (MetalBackend._kv_kernel raises TypeError for a KV dtype it has no
 kernel for, src/backend/metal.py:189-195) and turn shape mistakes into ValueError before anything is launched.
 """
+import ctypes
+import importlib.util
 import math
+from pathlib import Path
 
 import torch
 
-from native.rocm_native import RK_BF16, RK_F32, RK_W_BF16, RK_W_INT4, RK_W_INT8, load
+from native.rocm_native import ERROR_NAMES, RK_BF16, RK_F32, RK_W_BF16, RK_W_INT4, RK_W_INT8, RocmKernelError, load
+from quant import QuantTensor
 
 DTYPE_CODES = {torch.float32: RK_F32, torch.bfloat16: RK_BF16}
 KV_DTYPES = (torch.float32, torch.bfloat16)
@@ -31,6 +35,36 @@ def to_device(t: torch.Tensor, device) -> torch.Tensor:
 
 def _stream(dev: torch.device) -> int:
     return torch.cuda.current_stream(dev).cuda_stream
+
+
+CALLS_PATH = Path(__file__).resolve().parent / "rk_calls.so"
+CALLED = ("rk_linear_workspace_bytes", "rk_linear_rows_ex2", "rk_swiglu_rows", "rk_rms_norm", "rk_layer_norm",
+          "rk_paged_decode_workspace_bytes", "rk_paged_decode", "rk_paged_decode_planned", "rk_deltanet_decode",
+          "rk_attn_prep")
+_native_calls = None
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)      # the current stream's handle of a device index
+
+
+def _calls():
+    """call_paths.cpp: the decode step's calls with their checks in C++, on the entry points of the loaded library. Each
+    returns None where a tensor would have to be converted, copied or refused; the functions below then go on as if it
+    had not been asked."""
+    global _native_calls
+    if _native_calls is None:
+        if not CALLS_PATH.exists():
+            raise FileNotFoundError(f"{CALLS_PATH} is missing: build it with `python metal-inference-engine_amd/native/"
+                                    "build.py` (or __graft_entry__.build())")
+        lib = load()
+
+        def on_error(name, rc):
+            raise RocmKernelError(f"{name}: {ERROR_NAMES.get(rc, rc)}: {lib.last_error()}")
+
+        spec = importlib.util.spec_from_file_location("rk_calls", CALLS_PATH)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        mod.init({n: ctypes.cast(getattr(lib.lib, n), ctypes.c_void_p).value for n in CALLED}, on_error)
+        _native_calls = mod
+    return _native_calls
 
 
 def _need_cuda(name: str, *ts: torch.Tensor) -> torch.device:
@@ -115,6 +149,14 @@ def paged_decode(q, k_pool, v_pool, tables, lens, block_size: int, window: int |
     tables and lens (rk_paged_decode_planned; the same bits, a shorter start). phase 0 / 1 runs one of the two
     launches (for timing)."""
     name = "paged_attention"
+    if out is None and phase is None and q.is_cuda and (
+            plan is None or plan.key == _plan_key(tables, lens, block_size, q.shape[1], k_pool.shape[2], q.shape[2],
+                                                  k_pool.shape[0], window)):
+        idx = q.get_device()
+        y = _calls().paged_decode(q, k_pool, v_pool, tables, lens, int(block_size), int(window or 0), gate,
+                                  plan.buf if plan is not None else None, _workspaces.get(idx), _raw_stream(idx))
+        if y is not None:
+            return y
     if k_pool.dtype != v_pool.dtype or k_pool.dtype not in KV_DTYPES:
         raise TypeError(f"{name}: keys and values must both be float32 or bfloat16, not "
                         f"{k_pool.dtype} / {v_pool.dtype}")
@@ -209,6 +251,11 @@ def deltanet_decode(qkv, z, b, a, conv_state, S, seq_index, slot: int, conv_w, A
     [seq_index[i], slot]."""
     name = "deltanet_decode"
     H, dk, dv, key_dim = dims
+    if qkv.is_cuda:
+        y = _calls().deltanet_decode(qkv, z, b, a, conv_state, S, seq_index, int(slot), conv_w, A_log, dt_bias, norm_w,
+                                     float(eps), H, dk, dv, key_dim, _raw_stream(qkv.get_device()))
+        if y is not None:
+            return y
     if key_dim != H * dk:
         raise ValueError(f"{name}: key_dim {key_dim} != H * dk = {H * dk}")
     B, C = qkv.shape
@@ -665,6 +712,12 @@ def attn_prep(y, q_w, k_w, eps: float, positions, theta: float, rot: int, dims, 
     (q, k, v) fp32 are returned."""
     name = "attn_prep"
     Hq, Hkv, d = dims
+    if k_pool is not None and v_pool is not None and slots is not None and y.is_cuda:
+        idx = y.get_device()
+        q = _calls().attn_prep(y, q_w, k_w, float(eps), positions, rope_inv_freq(theta, rot, y.device) if rot else None,
+                               int(rot), Hq, Hkv, d, k_pool, v_pool, slots, _raw_stream(idx))
+        if q is not None:
+            return q
     if y.dim() != 2 or y.shape[1] < (Hq + 2 * Hkv) * d or q_w.numel() != d or k_w.numel() != d:
         raise ValueError(f"{name}: y {tuple(y.shape)}, norm weights {q_w.numel()} / {k_w.numel()} for {dims}")
     if not 0 <= rot <= d:
@@ -710,9 +763,27 @@ KERNEL_ROWS = 32            # up to here: the matvec kernel in groups of 16; bey
 LINEAR_LONG_ROWS = 65536    # rk_linear_rows' persistent kernel for INT8 weights from this many rows (M <= 8)
 
 
+def _native_linear(x, w, bias=None, residual=None, ss=None, norm_w=None, eps: float = 0.0, want_ss: bool = False,
+                   glu: bool = False):
+    """call_paths.cpp's linear, or None."""
+    if not x.is_cuda:
+        return None
+    idx = x.get_device()
+    if type(w) is QuantTensor:
+        wt, data, scales, mins = W_TYPES.get(w.scheme), w.data, w.scales, w.mins
+        if wt is None or w.block != 32:
+            return None
+    else:
+        wt, data, scales, mins = RK_W_BF16, w, None, None
+        if not isinstance(w, torch.Tensor) or w.dim() != 2:
+            return None
+    N, K = w.shape
+    return _calls().linear(x, wt, data, scales, mins, N, K, bias, residual, ss, norm_w, float(eps), want_ss, glu,
+                           _workspaces.get(idx), _linear_cnt.get(idx), _raw_stream(idx))
+
+
 def _weight_args(w):
     """(w_type, data, scales, mins, N, K) of a bf16 tensor or a QuantTensor, checked."""
-    from quant import QuantTensor
     if isinstance(w, QuantTensor):
         if w.scheme not in W_TYPES or w.block != 32:
             raise TypeError(f"linear: quantized scheme {w.scheme} / block {w.block} has no kernel")
@@ -734,6 +805,10 @@ def _weight_args(w):
 def linear_rows(x, w, bias=None, residual=None, out=None) -> torch.Tensor:
     """y [M, N] = x [M, K] @ dequant(w)^T (+ bias) (+ residual), fp32, for M <= KERNEL_ROWS (rk_linear_rows, 16 rows
     per launch): the decode-time linear of src/backend/metal.py:59-133. w: bf16 [N, K] or a QuantTensor."""
+    if out is None:
+        y = _native_linear(x, w, bias, residual)
+        if y is not None:
+            return y
     wt, data, scales, mins, N, K = _weight_args(w)
     M = x.shape[0]
     if x.dim() != 2 or x.shape[1] != K or M > KERNEL_ROWS or K % 32:
@@ -807,6 +882,9 @@ def linear_ss(x, w, bias=None, residual=None):
     """linear(x, w, bias, residual) -> (y, ss): with up to 16 rows (rk_linear_rows_ex2) also the sums of squares of
     y's 16-column tiles [M, ceil(N / 16)], which let the RMSNorm before the next linear run inside it
     (rms_norm_linear); beyond 16 rows (or K % 32 != 0) the plain linear and ss = None."""
+    y = _native_linear(x, w, bias, residual, want_ss=True)
+    if y is not None:
+        return y
     wt, data, scales, mins, N, K = _weight_args(w)
     M = x.shape[0]
     if x.dim() != 2 or x.shape[1] != K or M > LINEAR_ROWS or K % 32:
@@ -838,6 +916,10 @@ def rms_norm_linear(x, ss, norm_w, eps: float, w, bias=None, residual=None) -> t
     (N > 16384 outside the persistent INT8 kernel's shapes: every workgroup recomputes the rows' rms, which costs
     more than the separate launch there):
     rms_norm, then linear (the same results within 1e-5)."""
+    if ss is not None:
+        y = _native_linear(x, w, bias, residual, ss, norm_w, eps)
+        if y is not None:
+            return y
     wt, data, scales, mins, N, K = _weight_args(w)
     M = x.shape[0]
     long_int8 = wt == RK_W_INT8 and N >= LINEAR_LONG_ROWS and K % 1024 == 0      # the persistent kernel's shapes
@@ -886,10 +968,12 @@ def swiglu(x, w) -> torch.Tensor:
     product in its epilogue. Up to KERNEL_ROWS rows with F % 8 != 0, and rows that are not whole blocks: the linear
     and then silu_mul on its two halves (the same results within 1e-5)."""
     N, K = w.shape
+    y = _native_linear(x, w, glu=True)
+    if y is not None:
+        return y
     M = x.shape[0]
     if x.dim() != 2 or x.shape[1] != K or N % 2:
         raise ValueError(f"swiglu: x {tuple(x.shape)} for a [{N}, {K}] stacked [gate; up] weight")
-    from quant import QuantTensor
     fused = isinstance(w, QuantTensor) or w.dtype == torch.bfloat16
     if fused and M > KERNEL_ROWS and K % 32 == 0:
         return _gemm(x, w, glu=True)
@@ -909,9 +993,12 @@ def rms_norm_swiglu(x, ss, norm_w, eps: float, w) -> torch.Tensor:
     ss = the sums of squares of x's 16-column tiles that the linear producing x wrote; the cases rms_norm_linear
     sends to the separate norm (no ss, more than 8 rows, K % 256 != 0 or K > 2048, more than 16384 weight rows)
     and the weights swiglu does not fuse: rms_norm, then swiglu (the same results within 1e-5)."""
+    if ss is not None:
+        y = _native_linear(x, w, ss=ss, norm_w=norm_w, eps=eps, glu=True)
+        if y is not None:
+            return y
     N, K = w.shape
     M = x.shape[0]
-    from quant import QuantTensor
     if (ss is None or x.dim() != 2 or x.shape[1] != K or M > 8 or K % 256 or K > 2048 or N > 16384
             or ss.shape != (M, K // 16) or norm_w.numel() != K
             or not (isinstance(w, QuantTensor) or w.dtype == torch.bfloat16) or not _swiglu_fused(w, K)):
@@ -985,7 +1072,6 @@ def linear(x, w, bias=None, residual=None) -> torch.Tensor:
     """The reference's decode / prefill linear on a bf16 or quantized weight (src/backend/metal.py:59-133): up to 32
     rows through the matvec kernel, beyond that rk_linear_gemm. fp32 / other-dtype weights, and bf16 rows that are not
     whole blocks of 32: x @ w.T in fp32."""
-    from quant import QuantTensor
     M = x.shape[0]
     if not isinstance(w, QuantTensor) and (w.dtype != torch.bfloat16 or w.shape[1] % 32):
         y = x.float() @ w.float().T
@@ -1011,6 +1097,10 @@ def linear(x, w, bias=None, residual=None) -> torch.Tensor:
 def _norm(entry: str, x, w, eps: float) -> torch.Tensor:
     """Rows of any length D: up to 4096 values (a multiple of 4, aligned) stay in registers, one wave per row; any
     other row takes a workgroup of its own (rk_rms_norm / rk_layer_norm choose)."""
+    if x.is_cuda:
+        y = _calls().norm(entry == "rk_layer_norm", x, w, float(eps), _raw_stream(x.get_device()))
+        if y is not None:
+            return y
     name = entry[3:]
     D = x.shape[-1]
     if w.numel() != D or D < 1:
