@@ -21,12 +21,15 @@
 // inside it. Three launches per slab: split_rows, slab_weights, gemm_rows (four with K-splits: gemm_finish). Up to a few
 // hundred rows linear_mid.hip reads W as stored instead.
 //
-// Measured against the fp32 GEMM on the expanded weight (1777 rows, bf16): 12288 x 2048 with silu * up 740 -> 235 us
-// in all (gemm_rows 200 us = 890 TFLOP/s of 16-bit products; a large bf16 GEMM of the BLAS reaches 1270 on this
-// card), 2048 x 6144 440 -> 157 us; error against 64 bits 1.4e-6 -> 2.7e-7 of the result at K 6144. What bounds
-// gemm_rows: matrix-core issue and the fp32 joins beside it (copies without the loads, without the LDS reads or with a
-// quarter of the joins are each about 10 % faster), and whole tiles: 224 workgroups on 256 CUs at 2048 columns.
+// Measured against the fp32 GEMM on the expanded weight, an MLP of 1777 rows, bf16 weights (12288 x 2048 with silu * up,
+// then 2048 x 6144): 1188 -> 355 us in all; gemm_rows 212 us there (840 TFLOP/s of 16-bit products; a large bf16 GEMM of
+// the BLAS reaches 1270 on this card) and 133 us, the expansions 20 us each, the splits 7 and 20. Error against 64 bits
+// 9.6e-7 -> 1.6e-7 of the result. What bounds gemm_rows: matrix-core issue and the fp32 joins beside it (joins after
+// every stage instead of every other: 374 against 349 us in all; copies without the loads or without the LDS reads were
+// each about 10 % faster), and whole tiles: 224 workgroups on 256 CUs at 2048 columns, 672 at 12288.
 #include "fp16_pieces.h"
+
+#include <type_traits>
 
 namespace rk {
 namespace {
@@ -299,18 +302,21 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_rows(GemmArgs g) {
     const int at_a = at + 64 * 16 * TI * wm, at_b = at + 64 * (2 * BM + 64 * wn);
     const int at_s = TL::ROWS * 2 * kBK + 256 * wave + 4 * r;
     auto rd = [&](const char* p) { return *reinterpret_cast<const u32x4*>(p); };
-    f32x4 acc[TI][4], d[2][4];
+    // the sums in the making: of one group of sixteen rows and the one before (SCALED), or of every group (two stages)
+    constexpr int ND = SCALED ? 2 : TI;
+    f32x4 acc[TI][4], d[ND][4];
     u32x4 b[4], bn[4], h[2], l[2];
     float f[4], fn[4], fd[4];                      // scales: of this stage, of the next, of d[1]'s stage
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-        d[1][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        d[ND - 1][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
         f[t] = fn[t] = fd[t] = 0.0f;
 #pragma unroll
         for (int i = 0; i < TI; ++i) acc[i][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
     }
-    // a stage's sums start from zero and join the running ones by an fp32 addition (or fma): a third of the error of
-    // MFMAs on the running sums (bf16, K 6144: 2.7e-7 of the result against 7.1e-7; an fp32 GEMM: 1.4e-6)
+    // a stage's sums (a pair of stages' where no scales stand between them) start from zero and join the running ones by
+    // an fp32 addition (or fma): a third of the error of MFMAs on the running sums (1777 rows, bf16, K 6144: 2.0e-7 of the
+    // result against 7.1e-7; an fp32 GEMM: 1.4e-6)
     auto join = [&](f32x4 (&to)[4], const f32x4 (&from)[4], const float (&by)[4]) {
 #pragma unroll
         for (int t = 0; t < 4; ++t)
@@ -333,7 +339,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_rows(GemmArgs g) {
     l[0] = rd(smem + at_a + 64 * BM);
 
     int buf = 0;
-    for (int s = 0; s < S; ++s) {
+    auto stage = [&](int s, auto odd_c) __attribute__((always_inline)) {
+        constexpr bool kOdd = decltype(odd_c)::value;           // the second stage of a pair: goes on from the first
         // behind this barrier stages s and s + 1 are in LDS, and stage s - 1, whose buffer the request fills, is done
         // with (its last operands were taken before it)
         if (s) landed();
@@ -345,7 +352,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_rows(GemmArgs g) {
         // the sums of the sixteen before are joined
 #pragma unroll
         for (int i = 0; i < TI; ++i) {
-            const int c = i & 1, o = c ^ 1;
+            const int c = i & 1, o = c ^ 1, di = SCALED ? c : i;
             if (i < TI - 1) {
                 h[o] = rd(cur + at_a + 1024 * (i + 1));
                 l[o] = rd(cur + at_a + 64 * BM + 1024 * (i + 1));
@@ -360,12 +367,14 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_rows(GemmArgs g) {
                     if constexpr (SCALED) fn[t] = *reinterpret_cast<const float*>(nxt + at_s + 64 * t);
                 }
             }
+            // the last group of the stage (pair) before, whose sums this one's overwrite
+            if (i == 0 && (SCALED || !kOdd)) join(acc[TI - 1], d[ND - 1], fd);
 #pragma unroll
-            for (int t = 0; t < 4; ++t) d[c][t] = mfma_f16(l[c], b[t], (f32x4){0.f, 0.f, 0.f, 0.f});
+            for (int t = 0; t < 4; ++t)
+                d[di][t] = mfma_f16(l[c], b[t], kOdd ? d[di][t] : (f32x4){0.f, 0.f, 0.f, 0.f});
 #pragma unroll
-            for (int t = 0; t < 4; ++t) d[c][t] = mfma_f16(h[c], b[t], d[c][t]);
-            if (i == 0) join(acc[TI - 1], d[1], fd);
-            else join(acc[i - 1], d[o], f);
+            for (int t = 0; t < 4; ++t) d[di][t] = mfma_f16(h[c], b[t], d[di][t]);
+            if (i && (SCALED || kOdd)) join(acc[i - 1], d[SCALED ? o : i - 1], f);
             if (i < TI - 2) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
             else __builtin_amdgcn_sched_group_barrier(0x100, SCALED ? 6 : 4, 0);
 #pragma unroll
@@ -383,8 +392,22 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_rows(GemmArgs g) {
                 f[t] = fn[t];
             }
         }
+    };
+    int s = 0;
+    if constexpr (SCALED) {
+        for (; s < S; ++s) stage(s, std::false_type{});
+    } else {
+        for (; s + 1 < S; s += 2) {
+            stage(s, std::false_type{});
+            stage(s + 1, std::true_type{});
+        }
+        if (s < S) {                               // an odd last stage: no group of it is joined yet
+            stage(s, std::false_type{});
+#pragma unroll
+            for (int i = 0; i < TI - 1; ++i) join(acc[i], d[i], fd);
+        }
     }
-    join(acc[TI - 1], d[1], fd);
+    join(acc[TI - 1], d[ND - 1], fd);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the requests past the last stage
 
     // lane (r, grp) holds rows 4 grp + e, column r of each 16 x 16 tile
@@ -450,7 +473,7 @@ Layout layout(int M, int N, int K, int w_type, bool glu) {
     l.part = l.ew + up256(rows * 4);
     // 128 x 256 tiles where they give every CU two of them, else 128 x 128 (1777 x 2048 outputs: 112 tiles of 256
     // columns leave half the CUs idle), else 64 x 128; eight waves of 32 x 64 beat four of 64 x 64 there (157 against
-    // 168 us at 1777 x 2048 x 6144: two waves per SIMD). Fewer than half as many tiles as CUs: K-splits of at least
+    // 168 us in all at 1777 x 2048 x 6144: two waves per SIMD). Fewer than half as many tiles as CUs: K-splits of at least
     // 16 steps, until the tiles fill the CUs (2048 columns, K 6144: 384 rows 133 -> 56 us, 256 rows 132 -> 45)
     int cus = device_cus();
     if (cus <= 0) cus = 256;

@@ -43,3 +43,31 @@ def test_loader_waits_count_its_register_requests(tmp_path):
         assert n == int(m.group(1)), f"wait at line {i}: vmcnt({m.group(1)}) but {n} loads after the last direct load"
         checked += 1
     assert checked == 4, f"expected the 4 loader waits (2 waves x prologue / loop), found {checked}"
+
+
+@pytest.mark.skipif(shutil.which(HIPCC) is None, reason="hipcc not installed")
+def test_gemm_waits_count_its_loads(tmp_path):
+    """gemm_rows waits with `s_waitcnt vmcnt(N)` for all but the loads of its newest stages, which is right only if
+    every stage between two waits is the same number L of direct loads, the start is N + 2 L of them (this stage and the
+    next are waited for), and no other memory access stands between the first wait and the last."""
+    asm = tmp_path / "gemm.s"
+    cmd = [HIPCC, "-x", "hip", "-S", "--offload-device-only", str(NATIVE / "linear_gemm.hip"), "-o", str(asm)]
+    cmd += build.FLAGS + build.SOURCE_FLAGS.get("linear_gemm.hip", [])
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    kernels = re.findall(r"^(_Z\S*gemm_rows\S*):(.*?)^\.Lfunc_end", asm.read_text(), flags=re.S | re.M)
+    assert len(kernels) == 12
+    for name, body in kernels:
+        lines = [ln.strip() for ln in body.splitlines()]
+        waits = [i for i, ln in enumerate(lines) if re.match(r"s_waitcnt vmcnt\(\d+\)$", ln) and lines[i + 1] == "s_barrier"]
+        n = {int(re.search(r"\d+", lines[i][10:]).group()) for i in waits}
+        assert len(waits) >= 2 and len(n) == 1, name
+        loads = lambda a, b: sum(ln.startswith("global_load_lds") for ln in lines[a:b])
+        last_mfma = max(i for i, ln in enumerate(lines) if ln.startswith("v_mfma"))
+        per = {loads(a, b) for a, b in zip(waits, waits[1:])} | {loads(waits[-1], last_mfma)}
+        assert len(per - {0}) == 1, (name, per)
+        L = max(per)
+        assert loads(0, waits[0]) == n.copy().pop() + 2 * L, name
+        other = [ln for ln in lines[waits[0]:last_mfma]
+                 if re.match(r"(global|buffer|flat|scratch)_", ln) and not ln.startswith("global_load_lds")]
+        assert not other, (name, other[:3])
