@@ -6,13 +6,13 @@
 // with all the activation rows of a row block (48 or 64). The activations come as operand-ready pieces from memory
 // (the L2s hold them: 4 bytes per value, 0.5 MB for 64 x 2048), written once by split_operands; they pass through no
 // LDS, since no two waves of a workgroup use the same ones. INT8 / INT4: two fp16 pieces, codes exact in fp16, a
-// block's scale (and INT4 min times the block's activation sum) on the VALU, as linear.hip; bf16: three bf16 pieces
+// block's scale on the VALU, INT4 mins and 8 scales as one more MFMA per 8 blocks; bf16: three bf16 pieces
 // (exact), so that W needs no conversion. The waves' sums meet in LDS; K-splits meet in memory, added in order by
 // mid_finish.
 //
-// Measured (64 rows, INT4, all launches): 12288 x 2048 with silu * up 26 us, 2048 x 6144 26 us (gemm_rows 46 and 34, the
-// fp32 GEMM on the expanded weight 100 and 110); mid_rows itself 24 and 18 us in a trace, of which the activations'
-// 0.5 MB per CU from the L2 (64 bytes per cycle) and the VALU's scales and mins are about 4 us each, the MFMAs 4.
+// Measured (64 rows, INT4, all launches): 12288 x 2048 with silu * up 23 us, 2048 x 6144 23 us (gemm_rows 45 and 36, the
+// fp32 GEMM on the expanded weight 100 and 110); mid_rows itself 20.6 and 15.4 us in a trace. The mins on the VALU, four
+// fmas a block and tile, had cost 10 of 55 us for the two; one chunk of weights in flight instead of two 2.
 #include "fp16_pieces.h"
 
 namespace rk {
@@ -25,7 +25,7 @@ template <int WT> constexpr int pieces_of() { return WT == RK_W_BF16 ? 3 : 2; }
 struct MidArgs {
     float* y;
     const uint16_t* a;             // [row block][K / 32][piece][MT][64 lanes][8]: MFMA operands
-    const float* sums;             // INT4: [row block][K / 32][16 MT] block sums of the scaled activations
+    const uint16_t* sums;          // INT4: [row block][K / 64][16 MT rows][2 blocks][4] block sums (split_operands)
     const int* ex;                 // [M] exponents (INT8 / INT4)
     const void* w;
     const uint16_t* scales;
@@ -39,19 +39,34 @@ struct MidArgs {
 };
 
 // Row m of x as operands of the row block m / (16 MT): lane (r, g) of tile i takes row 16 i + r's values 8g .. 8g + 7
-// of a block. fp16 pairs of x * 2^ex (INT4: in the order of int4_f16) or bf16 thirds.
+// of a block. fp16 pairs of x * 2^ex (INT4: in the order of int4_f16) or bf16 thirds. INT4: also each block's sum b of the
+// scaled values, as the fp16 pieces (b hi, 8 b hi, b lo, 8 b lo) * 2^-kSumShift, against (min, scale, min, scale).
+constexpr int kSumShift = 8;
 template <int WT, int MT>
-__global__ __launch_bounds__(256) void split_operands(uint16_t* a, float* sums, int* ex, const float* x, long long x_ld,
+__global__ __launch_bounds__(256) void split_operands(uint16_t* a, uint16_t* sums, int* ex, const float* x, long long x_ld,
                                                       int K) {
     constexpr int P = pieces_of<WT>();
     __shared__ float red[4];
     const int m = blockIdx.x, tid = threadIdx.x;
     const int mb = m / (16 * MT), i = m % (16 * MT) / 16, r = m % 16, nblk = K / kQB;
     const float* xr = x + (size_t)m * x_ld;
+    // a thread's first kHeld groups of 8 values stay in registers (rows of up to 8192: read once, all at the start)
+    constexpr int kHeld = 4;
+    f32x4 held[kHeld][2];
+#pragma unroll
+    for (int j = 0; j < kHeld; ++j) {
+        const float* p = xr + 8 * min(tid + 256 * j, K / 8 - 1);
+        held[j][0] = *reinterpret_cast<const f32x4*>(p);
+        held[j][1] = *reinterpret_cast<const f32x4*>(p + 4);
+    }
     int k = 0;
     if constexpr (WT != RK_W_BF16) {
         float big = 0.0f;
-        for (int c = tid; c < K / 8; c += 256) {
+#pragma unroll
+        for (int j = 0; j < kHeld; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) big = fmaxf(big, fmaxf(fabsf(held[j][0][e]), fabsf(held[j][1][e])));
+        for (int c = tid + 256 * kHeld; c < K / 8; c += 256) {
             const f32x4 v0 = *reinterpret_cast<const f32x4*>(xr + 8 * c), v1 = *reinterpret_cast<const f32x4*>(xr + 8 * c + 4);
 #pragma unroll
             for (int e = 0; e < 4; ++e) big = fmaxf(big, fmaxf(fabsf(v0[e]), fabsf(v1[e])));
@@ -59,8 +74,7 @@ __global__ __launch_bounds__(256) void split_operands(uint16_t* a, float* sums, 
         k = top_exponent(block_absmax(big, red));
         if (tid == 0) ex[m] = k;
     }
-    for (int c = tid; c < K / 8; c += 256) {
-        const f32x4 v0 = *reinterpret_cast<const f32x4*>(xr + 8 * c), v1 = *reinterpret_cast<const f32x4*>(xr + 8 * c + 4);
+    auto put = [&](int c, f32x4 v0, f32x4 v1) __attribute__((always_inline)) {
         float v[8];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -94,9 +108,20 @@ __global__ __launch_bounds__(256) void split_operands(uint16_t* a, float* sums, 
             for (int e = 0; e < 8; ++e) sum += v[e];
             sum += __shfl_xor(sum, 1);
             sum += __shfl_xor(sum, 2);
-            if ((c & 3) == 0) sums[blk * (16 * MT) + 16 * i + r] = sum;
+            if ((c & 3) == 0) {
+                const Pieces p = split_pair(ldexpf(sum, -kSumShift), 0.0f);
+                const float h = half_to_f32(p.hi & 0xffffu), l = half_to_f32(rest_of(p) & 0xffffu);
+                const size_t pair = (size_t)mb * (nblk / 2) + (c >> 3);
+                *reinterpret_cast<u32x2*>(sums + (pair * (16 * MT) + 16 * i + r) * 8 + 4 * ((c >> 2) & 1)) =
+                    (u32x2){pack_f16(h, 8.0f * h), pack_f16(l, 8.0f * l)};
+            }
         }
-    }
+    };
+#pragma unroll
+    for (int j = 0; j < kHeld; ++j)
+        if (tid + 256 * j < K / 8) put(tid + 256 * j, held[j][0], held[j][1]);   // the four threads of a block together
+    for (int c = tid + 256 * kHeld; c < K / 8; c += 256)
+        put(c, *reinterpret_cast<const f32x4*>(xr + 8 * c), *reinterpret_cast<const f32x4*>(xr + 8 * c + 4));
 }
 
 // weight row behind row lr of the tiles: lr, or with glu gate rows 8T .. 8T + 7 then their up rows in tile T
@@ -206,9 +231,10 @@ __global__ __launch_bounds__(64 * kWaves) void mid_rows(MidArgs a) {
         if constexpr (QUANT) srow[t] = a.scales + n * nblk;
         if constexpr (WT == RK_W_INT4) mrow[t] = a.mins + n * nblk;
     }
-    u32x4 wn[NT][CH];
-    uint32_t sn[QUANT ? NT : 1][2], mn[WT == RK_W_INT4 ? NT : 1][2];
-    auto load_w = [&](int kb) {
+    constexpr int DEPTH = WT == RK_W_INT4 ? 2 : 1;   // chunks of weights in flight
+    u32x4 wn[DEPTH][NT][CH];
+    uint32_t sn[DEPTH][QUANT ? NT : 1][2];
+    auto load_w = [&](int kb, int set) __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
 #pragma unroll
@@ -217,20 +243,17 @@ __global__ __launch_bounds__(64 * kWaves) void mid_rows(MidArgs a) {
                 if constexpr (WT == RK_W_BF16) off = (size_t)min(kb + c, nblk - 1) * 64 + 16 * grp;
                 else if constexpr (WT == RK_W_INT8) off = (size_t)min(kb + grp, nblk - 1) * 32 + 16 * c;
                 else off = (size_t)min(kb + grp, nblk - 1) * 16;
-                wn[t][c] = *reinterpret_cast<const u32x4*>(wrow[t] + off);
+                wn[set][t][c] = *reinterpret_cast<const u32x4*>(wrow[t] + off);
             }
             if constexpr (QUANT) {                 // nblk and kb are even
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
-                    const int kk = min(kb + 2 * h, nblk - 2);
-                    sn[t][h] = *reinterpret_cast<const uint32_t*>(srow[t] + kk);
-                    if constexpr (WT == RK_W_INT4) mn[t][h] = *reinterpret_cast<const uint32_t*>(mrow[t] + kk);
+                    sn[set][t][h] = *reinterpret_cast<const uint32_t*>(srow[t] + min(kb + 2 * h, nblk - 2));
                 }
             }
         }
     };
     u32x4 xa[2][P][MT];
-    f32x4 bs[2][WT == RK_W_INT4 ? MT : 1];
     auto load_x = [&](int kb, int slot) {
         const size_t blk = (size_t)mb * nblk + min(kb, nblk - 1);
 #pragma unroll
@@ -238,11 +261,6 @@ __global__ __launch_bounds__(64 * kWaves) void mid_rows(MidArgs a) {
 #pragma unroll
             for (int i = 0; i < MT; ++i)
                 xa[slot][p][i] = *reinterpret_cast<const u32x4*>(a.a + (((blk * P + p) * MT + i) * 64 + lane) * 8);
-        if constexpr (WT == RK_W_INT4) {
-#pragma unroll
-            for (int i = 0; i < MT; ++i)
-                bs[slot][i] = *reinterpret_cast<const f32x4*>(a.sums + blk * (16 * MT) + 16 * i + 4 * grp);
-        }
     };
     f32x4 acc[MT][NT];
 #pragma unroll
@@ -250,39 +268,72 @@ __global__ __launch_bounds__(64 * kWaves) void mid_rows(MidArgs a) {
 #pragma unroll
         for (int t = 0; t < NT; ++t) acc[i][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
+    const int k_last = k0 + (k1 - 1 - k0) / 4 * 4;   // the wave's last chunk
     if (k0 < k1) {
-        load_w(k0);
+#pragma unroll
+        for (int i = 0; i < DEPTH; ++i) load_w(min(k0 + 4 * i, k_last), i);
         load_x(k0, 0);
+        // INT4 is s (q - 8) + (8 s + min): the second terms of 8 blocks are one MFMA per tile, with the block sums' pieces
+        // against (min, s) pairs, whose near-equal products of opposite sign cancel inside it
+        if constexpr (WT == RK_W_INT4) {
+            for (int kb = k0; kb < k1; kb += 8) {
+                const int kp = kb + 2 * grp;       // the lane group's two blocks
+                const int kc = min(kp, nblk - 2);
+                const uint32_t in = kp < k1 ? 0xffffffffu : 0u;   // k0 and k1 are even
+                u32x4 sa[MT];
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+                    sa[i] = *reinterpret_cast<const u32x4*>(a.sums + (((size_t)mb * (nblk / 2) + kc / 2) * (16 * MT) + 16 * i + r) * 8);
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    const uint32_t m = *reinterpret_cast<const uint32_t*>(mrow[t] + kc) & in;
+                    const uint32_t f = *reinterpret_cast<const uint32_t*>(srow[t] + kc) & in;
+                    const uint32_t b0 = __builtin_amdgcn_perm(f, m, 0x05040100u), b1 = __builtin_amdgcn_perm(f, m, 0x07060302u);
+                    const u32x4 b = {b0, b0, b1, b1};
+#pragma unroll
+                    for (int i = 0; i < MT; ++i) {
+                        const f32x4 p = mfma_f16(sa[i], b, (f32x4){0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) acc[i][t][e] = fmaf((float)(1 << kSumShift), p[e], acc[i][t][e]);
+                    }
+                }
+            }
+        }
     }
     for (int kc = k0; kc < k1; kc += 4) {
         u32x4 wc[NT][CH];
-        uint32_t sc[QUANT ? NT : 1][2], mc[WT == RK_W_INT4 ? NT : 1][2];
+        uint32_t sc[QUANT ? NT : 1][2];
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-            if constexpr (WT == RK_W_INT4) wc[t][0] = xpose4(wn[t][0][0], wn[t][0][1], wn[t][0][2], wn[t][0][3]);
+            if constexpr (WT == RK_W_INT4) wc[t][0] = xpose4(wn[0][t][0][0], wn[0][t][0][1], wn[0][t][0][2], wn[0][t][0][3]);
             else if constexpr (WT == RK_W_INT8) {
-                const u32x4 lo = xpose4(wn[t][0][0], wn[t][0][2], wn[t][1][0], wn[t][1][2]);
-                const u32x4 hi = xpose4(wn[t][0][1], wn[t][0][3], wn[t][1][1], wn[t][1][3]);
+                const u32x4 lo = xpose4(wn[0][t][0][0], wn[0][t][0][2], wn[0][t][1][0], wn[0][t][1][2]);
+                const u32x4 hi = xpose4(wn[0][t][0][1], wn[0][t][0][3], wn[0][t][1][1], wn[0][t][1][3]);
                 wc[t][0] = (u32x4){lo[0], hi[0], lo[1], hi[1]};
                 wc[t][1] = (u32x4){lo[2], hi[2], lo[3], hi[3]};
             } else {
 #pragma unroll
-                for (int c = 0; c < CH; ++c) wc[t][c] = wn[t][c];
+                for (int c = 0; c < CH; ++c) wc[t][c] = wn[0][t][c];
             }
             if constexpr (QUANT) {
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    sc[t][h] = sn[t][h];
-                    if constexpr (WT == RK_W_INT4) mc[t][h] = mn[t][h];
+                for (int h = 0; h < 2; ++h) sc[t][h] = sn[0][t][h];
+            }
+            if constexpr (DEPTH == 2) {
+#pragma unroll
+                for (int c = 0; c < CH; ++c) wn[0][t][c] = wn[1][t][c];
+                if constexpr (QUANT) {
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) sn[0][t][h] = sn[1][t][h];
                 }
             }
         }
-        load_w(kc + 4 < k1 ? kc + 4 : kc);
+        load_w(min(kc + 4 * DEPTH, k_last), DEPTH - 1);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
             const int s = d & 1;
-            // past the wave's range: zero scales and mins, zero bf16 weights (a mask; a condition becomes a branch)
+            // past the wave's range: zero scales, zero bf16 weights (a mask; a condition becomes a branch)
             const uint32_t in = kc + d < k1 ? 0xffffffffu : 0u;
             load_x(min(kc + d + 1, k1 - 1), s ^ 1);
 #pragma unroll
@@ -291,10 +342,8 @@ __global__ __launch_bounds__(64 * kWaves) void mid_rows(MidArgs a) {
                 if constexpr (WT == RK_W_INT4) b = int4_f16(wc[t][0][d]);
                 else if constexpr (WT == RK_W_INT8) b = int8_f16(wc[t][d >> 1][2 * (d & 1)], wc[t][d >> 1][2 * (d & 1) + 1]);
                 else b = wc[t][d] & (u32x4){in, in, in, in};
-                float f = 0.0f, mi = 0.0f;
+                float f = 0.0f;
                 if constexpr (QUANT) f = half_to_f32((sc[t][d >> 1] & in) >> (16 * (d & 1)));
-                // INT4: s (q - 8) + (8 s + min), whose two terms stay small (s q and min nearly cancel over a block)
-                if constexpr (WT == RK_W_INT4) mi = fmaf(8.0f, f, half_to_f32((mc[t][d >> 1] & in) >> (16 * (d & 1))));
 #pragma unroll
                 for (int i = 0; i < MT; ++i) {
                     f32x4 p = {0.f, 0.f, 0.f, 0.f};
@@ -305,7 +354,6 @@ __global__ __launch_bounds__(64 * kWaves) void mid_rows(MidArgs a) {
                     for (int e = 0; e < 4; ++e) {
                         if constexpr (QUANT) acc[i][t][e] = fmaf(f, p[e], acc[i][t][e]);
                         else acc[i][t][e] += p[e];
-                        if constexpr (WT == RK_W_INT4) acc[i][t][e] = fmaf(mi, bs[s][i][e], acc[i][t][e]);
                     }
                 }
             }
@@ -356,11 +404,11 @@ struct MidPlan {
 };
 
 // Rows up to which this form is the faster one (12288 x 2048 with silu * up, 2048 x 6144, 8224 x 2048; us, this form
-// against gemm_rows): INT4 at 128 rows 48 / 33 / 46 against 52 / 39 / 41 and at 160 rows 68 / 46 / 66 against
-// 71 / 43 / 65; INT8 at 256 rows 69 / 41 / 56 against 74 / 44 / 66 and at 384 rows 111 / 59 / 84 against 109 / 54 / 68;
-// bf16 at 96 rows 46 / 29 / 43 against 51 / 37 / 39 and at 128 rows 54 / 33 / 50 against 52 / 38 / 41. INT4 has its mins
-// on the VALU here, bf16 three pieces and two bytes of W per value.
-int mid_rows_max(int w_type) { return w_type == RK_W_INT8 ? 256 : w_type == RK_W_INT4 ? 128 : 96; }
+// against gemm_rows): INT4 at 192 rows 60 / 40 / 58 against 74 / 44 / 67 and at 256 rows 80 / 42 / 61 against
+// 73 / 47 / 68; INT8 at 256 rows 69 / 41 / 56 against 74 / 44 / 66 and at 384 rows 111 / 59 / 84 against 109 / 54 / 68;
+// bf16 (three pieces and two bytes of W per value here) at 96 rows 46 / 29 / 43 against 51 / 37 / 39 and at 128 rows
+// 54 / 33 / 50 against 52 / 38 / 41.
+int mid_rows_max(int w_type) { return w_type == RK_W_INT8 ? 256 : w_type == RK_W_INT4 ? 192 : 96; }
 
 // NT, S: the least estimated time over the rounds of one workgroup per CU: a block costs a wave its activations from
 // the L2 (1 KB per 16 cycles and CU) or its MFMAs (19 cycles each, two waves per SIMD), whichever is longer, a
@@ -391,7 +439,7 @@ MidPlan mid_plan(int M, int N, int K, int w_type, int glu) {
     const size_t rows = (size_t)p.MB * 16 * p.MT;
     auto up = [](size_t n) { return (n + 255) / 256 * 256; };
     p.sums = up(rows * K * 2 * P);
-    p.ex = p.sums + (w_type == RK_W_INT4 ? up(rows * nblk * 4) : 0);
+    p.ex = p.sums + (w_type == RK_W_INT4 ? up(rows * nblk * 8) : 0);
     p.part = p.ex + up(rows * 4);
     p.total = p.part + (p.S > 1 ? (size_t)p.MB * p.G * p.S * 64 * p.MT * p.NT * sizeof(f32x4) : 0);
     return p;
@@ -413,14 +461,14 @@ int mid_linear(float* y, const float* x, long long x_ld, int M, int N, int K, co
     const MidPlan p = mid_plan(M, N, K, w_type, glu);
     char* ws = static_cast<char*>(workspace);
     uint16_t* ops = reinterpret_cast<uint16_t*>(ws);
-    float* sums = reinterpret_cast<float*>(ws + p.sums);
+    uint16_t* sums = reinterpret_cast<uint16_t*>(ws + p.sums);
     int* ex = reinterpret_cast<int*>(ws + p.ex);
     MidArgs a{};
     a.y = y; a.a = ops; a.sums = sums; a.ex = ex; a.w = w;
     a.scales = static_cast<const uint16_t*>(scales); a.mins = static_cast<const uint16_t*>(mins);
     a.bias = bias; a.res = residual; a.part = reinterpret_cast<f32x4*>(ws + p.part);
     a.M = M; a.N = N; a.K = K; a.S = p.S; a.SB = p.SB; a.WB = p.WB; a.MB = p.MB; a.G = p.G; a.glu = glu ? 1 : 0;
-    using Split = void (*)(uint16_t*, float*, int*, const float*, long long, int);
+    using Split = void (*)(uint16_t*, uint16_t*, int*, const float*, long long, int);
     using Fn = void (*)(MidArgs);
     Split split = nullptr;
     Fn rows = nullptr, fin = nullptr;
