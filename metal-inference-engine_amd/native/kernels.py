@@ -1071,12 +1071,15 @@ def _gemm(x, w, bias=None, residual=None, glu: bool = False) -> torch.Tensor:
 def linear(x, w, bias=None, residual=None) -> torch.Tensor:
     """The reference's decode / prefill linear on a bf16 or quantized weight (src/backend/metal.py:59-133): up to 32
     rows through the matvec kernel, beyond that rk_linear_gemm. fp32 / other-dtype weights, and bf16 rows that are not
-    whole blocks of 32: x @ w.T in fp32."""
+    whole blocks of 32: x @ w.T in fp32. Where a gradient of x, bias or residual is asked for beyond 32 rows, the same
+    product on the dequantized weight."""
     M = x.shape[0]
     if not isinstance(w, QuantTensor) and (w.dtype != torch.bfloat16 or w.shape[1] % 32):
         y = x.float() @ w.float().T
     elif M <= KERNEL_ROWS:
         return linear_rows(x, w, bias, residual)
+    elif torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x, bias, residual)):
+        y = x.float() @ dequantize(w).T         # differentiable, as the row kernels are not
     else:
         N, K = w.shape
         if x.dim() != 2 or x.shape[1] != K:

@@ -255,11 +255,12 @@ def test_long_int8_matrix_on_the_persistent_grid(backend, N, K):
 @pytest.mark.parametrize("M,N,K,glu", [(33, 100, 96, False), (64, 130, 2080, False), (65, 272, 64, False),
                                        (129, 1000, 512, False), (257, 515, 1056, False), (600, 4352, 256, False),
                                        (48, 17, 192, False), (49, 300, 3072, False), (97, 2064, 448, False),
-                                       (33, 2 * 20, 256, True), (96, 2 * 700, 1920, True), (250, 2 * 36, 320, True), (140, 2 * 1000, 544, True), (513, 2 * 2200, 128, True)])
+                                       (33, 2 * 20, 256, True), (96, 2 * 700, 1920, True), (250, 2 * 36, 320, True),
+                                       (140, 2 * 1000, 544, True), (513, 2 * 2200, 128, True)])
 def test_many_row_linears_against_64_bits(backend, kind, M, N, K, glu):
     """rk_linear_gemm at the edges of its forms and tiles (rows and columns around 48, 64, 96, 128 and 256, odd numbers
-    of 32-value steps, glu halves that are not whole sixteens, K-splits and wave shares with a remainder), with rows of very different magnitude and values of very different
-    magnitude in one row, against the products in 64 bits. Bound: each output's sum of |x w| times 2^-24 for the
+    of 32-value steps, glu halves that are not whole sixteens, K-splits and wave shares with a remainder), with rows of
+    very different magnitude and values of very different magnitude in one row, against the products in 64 bits. Bound: each output's sum of |x w| times 2^-24 for the
     rounding of x and the same for every 32-value partial sum's fp32 rounding, of which there are K / 32 in sequence."""
     w, deq = weight(kind, N, K, N + K)
     g = torch.Generator().manual_seed(M)
@@ -302,3 +303,18 @@ def test_many_row_linears_take_what_the_row_kernels_take(backend):
     assert not torch.isfinite(bad[7]).any()
     keep = [i for i in range(33) if i != 7]
     assert torch.equal(bad[keep], got[keep])
+
+
+@pytest.mark.parametrize("kind", ["bf16", "int4"])
+def test_many_row_linear_carries_gradients(backend, kind):
+    """Beyond the row kernels a linear is differentiable in x, bias and residual. Bound: fp32 sums of 64 products."""
+    w, deq = weight(kind, 64, 96, 3)
+    g = torch.Generator().manual_seed(3)
+    x, b, r = (torch.randn(*s, generator=g) for s in ((40, 96), (64,), (40, 64)))
+    xd, bd, rd = (t.to(DEV).requires_grad_() for t in (x, b, r))
+    y = backend.linear(xd, to_dev(w), bd, rd)
+    assert rel_err(y.detach(), x @ deq.T + b + r) < TOL
+    dy = torch.randn(40, 64, generator=g)
+    y.backward(dy.to(DEV))
+    assert rel_err(xd.grad, dy @ deq) < TOL
+    assert rel_err(bd.grad, dy.sum(0)) < TOL and torch.equal(rd.grad.cpu(), dy)
