@@ -307,9 +307,9 @@ def prefill_split_tiles(spans: list[int], heads: int, n_cu: int, balance: bool =
     unless balance: then blocks longer than 1/PREFILL_BALANCE_PIECES of a CU's share are cut to that size (at least
     2 PREFILL_MIN_SPLIT tiles), so that the last workgroups to start end close together. balance is for the
     fp32-operand kernel (one workgroup per CU, where a packed batch like config 5's 632 uneven workgroups on 256
-    CUs leaves ~14% of the CU time idle at the end): that batch takes 2,056-2,157 us at a whole share, 2,070-2,077 at
-    a half, 2,121-2,210 at a quarter, 2,276-2,285 at an eighth; 4 segments at 16/4 heads x 128 879-902 / 894-898 / 919 /
-    965. A piece costs a partial record and its share of the merge, and on the bf16-operand kernel the longer start-up
+    CUs leaves ~14% of the CU time idle at the end): 8 segments of 552 GFLOP take 2,056-2,157 us at a whole share,
+    2,070-2,077 at a half, 2,121-2,210 at a quarter, 2,276-2,285 at an eighth; 4 segments at 16/4 heads x 128 879-902 /
+    894-898 / 919 / 965. A piece costs a partial record and its share of the merge, and on the bf16-operand kernel the longer start-up
     of its producer pipeline outweighs the gain."""
     if not spans:
         return 0

@@ -91,9 +91,10 @@ __device__ __forceinline__ float row16_sum(float x) {
 }
 
 // x of lane l plus that of lane l ^ 16 or l ^ 32, in both: a register swap (v_permlane*_swap_b32) and an addition. As
-// __shfl_xor they were ds_bpermute_b32, whose round trip through the LDS unit stood in every such chain. Rows of 16 lanes
-// (xor 16) or halves (xor 32) enter whole, in pairs. The same bits. In the linears and norms of an 8-sequence decode step
-// 1425 -> 1398 us, an INT4 MLP of 8 rows 24.96 -> 24.63, of 64 rows 48.5 -> 47.9 (paged decode's own sums gained nothing and keep the shuffles).
+// __shfl_xor they were ds_bpermute_b32, whose round trip through the LDS unit stood in every such chain; the bits are
+// the same. Rows of 16 lanes (xor 16) or halves (xor 32) enter whole, in pairs. Measured over the linears and norms: a
+// decode step of 8 sequences 1425 -> 1398 us, an INT4 MLP of 8 rows 24.96 -> 24.63, of 64 rows 48.5 -> 47.9 (paged
+// decode's own sums gained nothing and keep the shuffles).
 __device__ __forceinline__ float xor16_sum(float x) {
     const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
     return __uint_as_float(p[0]) + __uint_as_float(p[1]);
