@@ -4,7 +4,9 @@
 // is: plain torch tensors on one device with the types, shapes, strides and alignments the kernel reads. Then it makes
 // the output and launches through the same C ABI entry point (addresses handed over once, by init). Anything else
 // returns None and goes the general way, which converts, copies or refuses as it always did. Nothing is kept between
-// calls: workspaces and counters are kernels.py's, passed in.
+// calls: workspaces and counters are kernels.py's, passed in. C++ exceptions become Python's as torch's own bindings
+// make them (an allocation that fails is torch.OutOfMemoryError, as from torch.empty).
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/ATen.h>
@@ -109,7 +111,7 @@ bool rows_k(const at::Tensor& x, long long K, long long& ld) {
 //   -> y, or (y, tile sums of squares) with want_ss; ss given: the RMSNorm of x is applied; glu: y = silu * up
 PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 17) return PyErr_Format(PyExc_TypeError, "linear: 17 arguments");
-    try {
+    HANDLE_TH_ERRORS
         const at::Tensor* x = tensor(a[0]);
         const int wt = (int)PyLong_AsLong(a[1]);
         Weight w;
@@ -161,15 +163,13 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
             out = t;
         }
         return finish(glu ? "rk_swiglu_rows" : "rk_linear_rows_ex2", rc, out);
-    } catch (const std::exception& e) {
-        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
-    }
+    END_HANDLE_TH_ERRORS
 }
 
 // norm(layer, x, w, eps, stream): rk_layer_norm (layer True) or rk_rms_norm of 2-D fp32 rows, fp32 weights
 PyObject* norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 5) return PyErr_Format(PyExc_TypeError, "norm: 5 arguments");
-    try {
+    HANDLE_TH_ERRORS
         const at::Tensor* x = tensor(a[1]);
         const at::Tensor* w;
         if (!x || x->dim() != 2 || !is(*x, at::kFloat) || x->size(0) < 1 || x->size(1) < 1 || x->size(0) > INT_MAX ||
@@ -185,9 +185,7 @@ PyObject* norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const int rc = fn(y.data_ptr<float>(), x->data_ptr(), RK_F32, ld, w->data_ptr(), RK_F32, (int)x->size(0),
                           (int)x->size(1), eps, stream);
         return finish(a[0] == Py_True ? "rk_layer_norm" : "rk_rms_norm", rc, THPVariable_Wrap(y));
-    } catch (const std::exception& e) {
-        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
-    }
+    END_HANDLE_TH_ERRORS
 }
 
 int code(const at::Tensor& t) { return is(t, at::kFloat) ? RK_F32 : is(t, at::kBFloat16) ? RK_BF16 : -1; }
@@ -201,7 +199,7 @@ bool pools(const at::Tensor* k, const at::Tensor* v) {
 // paged_decode(q, k_pool, v_pool, tables, lens, block_size, window, gate, plan buffer, workspace, stream) -> [B, Hq, d]
 PyObject* paged_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 11) return PyErr_Format(PyExc_TypeError, "paged_decode: 11 arguments");
-    try {
+    HANDLE_TH_ERRORS
         const at::Tensor *q = tensor(a[0]), *k = tensor(a[1]), *v = tensor(a[2]), *tb = tensor(a[3]), *ln = tensor(a[4]);
         if (!q || !tb || !ln || !pools(k, v) || q->dim() != 3 || !is(*q, at::kFloat) || !q->is_contiguous() ||
             !same(*q, *k) || !same(*q, *tb) || !same(*q, *ln) || !is(*tb, at::kInt) || !is(*ln, at::kInt) ||
@@ -240,16 +238,14 @@ PyObject* paged_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                      (int)tb->size(1), (int)k->size(0), (int)window, g, gld, ws->data_ptr(),
                                      (size_t)ws->numel(), stream);
         return finish(plan ? "rk_paged_decode_planned" : "rk_paged_decode", rc, THPVariable_Wrap(out));
-    } catch (const std::exception& e) {
-        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
-    }
+    END_HANDLE_TH_ERRORS
 }
 
 // deltanet_decode(qkv, z, b, a, conv_state, S, seq_index, slot, conv_w, A_log, dt_bias, norm_w, eps, H, dk, dv, key_dim,
 // stream) -> [B, H dv]
 PyObject* deltanet_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 18) return PyErr_Format(PyExc_TypeError, "deltanet_decode: 18 arguments");
-    try {
+    HANDLE_TH_ERRORS
         const at::Tensor *qkv = tensor(a[0]), *z = tensor(a[1]), *b = tensor(a[2]), *aa = tensor(a[3]),
                          *conv = tensor(a[4]), *S = tensor(a[5]), *seq = tensor(a[6]);
         const at::Tensor *w = tensor(a[8]), *A = tensor(a[9]), *dt = tensor(a[10]), *nw = tensor(a[11]);
@@ -283,16 +279,14 @@ PyObject* deltanet_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                             f(S), f(w), f(A), f(dt), f(nw), static_cast<const int32_t*>(seq->data_ptr()),
                                             (int)B, (int)H, (int)dk, (int)dv, (int)K, (int)nl, (int)slot, eps, stream);
         return finish("rk_deltanet_decode", rc, THPVariable_Wrap(out));
-    } catch (const std::exception& e) {
-        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
-    }
+    END_HANDLE_TH_ERRORS
 }
 
 // attn_prep(y, q_w, k_w, eps, positions, inv_freq, rot, Hq, Hkv, d, k_pool, v_pool, slots, stream) -> q [N, Hq, d]:
 // the decode form, which writes the pool
 PyObject* attn_prep(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 14) return PyErr_Format(PyExc_TypeError, "attn_prep: 14 arguments");
-    try {
+    HANDLE_TH_ERRORS
         const at::Tensor *y = tensor(a[0]), *pos = tensor(a[4]), *k = tensor(a[10]), *v = tensor(a[11]), *sl = tensor(a[12]);
         const at::Tensor *inv = a[5] == Py_None ? nullptr : tensor(a[5]), *qw, *kw;
         const long long rot = PyLong_AsLongLong(a[6]), Hq = PyLong_AsLongLong(a[7]), Hkv = PyLong_AsLongLong(a[8]),
@@ -318,9 +312,7 @@ PyObject* attn_prep(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                       static_cast<const int32_t*>(pos->data_ptr()), (const float*)ptr(inv), (int)rot, (int)N,
                                       (int)Hq, (int)Hkv, (int)d, stream);
         return finish("rk_attn_prep", rc, THPVariable_Wrap(q));
-    } catch (const std::exception& e) {
-        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
-    }
+    END_HANDLE_TH_ERRORS
 }
 
 #define METHOD(f) {#f, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f)), METH_FASTCALL, nullptr}

@@ -163,3 +163,33 @@ def test_deltanet_step_and_attention_prep(backend, monkeypatch):
             assert used == want and equal(fast, slow)
     with pytest.raises(ValueError):
         prep(yp, p=pos.long())
+
+
+@pytest.mark.gpu
+def test_out_of_memory_is_torchs_own_exception(backend):
+    """An engine catches torch.OutOfMemoryError to evict and try again. Each call below is answered in C++ and its
+    output (16 MiB) does not fit the limit set for the process; the workspaces it needs exist already."""
+    x, nw = torch.zeros(2048, 2048, device=DEV), torch.ones(2048, device=DEV)
+    w, xr = torch.zeros(1 << 18, 32, dtype=torch.bfloat16, device=DEV), torch.zeros(16, 32, device=DEV)
+    q, pool = torch.zeros(1024, 16, 256, device=DEV), torch.zeros(1, 16, 4, 256, device=DEV)
+    tables, lens = (f(1024, *s, dtype=torch.int32, device=DEV) for f, s in ((torch.zeros, (1,)), (torch.ones, ())))
+    calls = [lambda: backend.rms_norm(x, nw, 1e-6), lambda: backend.linear(xr, w),
+             lambda: backend.paged_attention(q, pool, pool, tables, lens, 16)]
+    for f in calls:
+        f()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    torch.cuda.set_per_process_memory_fraction(torch.cuda.memory_reserved() / torch.cuda.mem_get_info()[1])
+    held = []
+    try:
+        with pytest.raises(torch.OutOfMemoryError):
+            while True:                                         # what is left of segments in use
+                held.append(torch.empty(1 << 22, device=DEV))
+        for f in calls:
+            with pytest.raises(torch.OutOfMemoryError):
+                f()
+    finally:
+        held.clear()
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    for f in calls:
+        f()
