@@ -55,6 +55,13 @@ bool is(const at::Tensor& t, at::ScalarType ty) { return t.scalar_type() == ty; 
 bool at_(const at::Tensor& t, uintptr_t align) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % align == 0; }
 bool same(const at::Tensor& a, const at::Tensor& b) { return a.device() == b.device(); }
 void* ptr(const at::Tensor* t) { return t ? t->data_ptr() : nullptr; }
+// The output's allocation and the launch run without the GIL, as torch.empty and a ctypes call do: either may wait (for
+// memory to come free, for room in the device's queue), and other Python threads go on meanwhile. Whole statements: the
+// scope ends before anything of Python's is touched.
+struct Unlocked {
+    PyThreadState* state = PyEval_SaveThread();
+    ~Unlocked() { PyEval_RestoreThread(state); }
+};
 at::Tensor make(at::IntArrayRef sizes, const at::Tensor& like) { return at::empty(sizes, like.options().dtype(at::kFloat)); }
 
 // fp32, contiguous, on x's device, of `n` values in the given shape; None gives true and null
@@ -139,21 +146,26 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
         void* stream = PyLong_AsVoidPtr(a[16]);
         const float eps = (float)PyFloat_AsDouble(a[11]);
         if (PyErr_Occurred()) return nullptr;
-        at::Tensor y = make({M, glu ? N / 2 : N}, *x), sums;
-        if (want_ss) sums = make({M, (N + 15) / 16}, *x);
+        at::Tensor y, sums;
         int rc;
         const int op = norm ? RK_X_RMS_NORM : RK_X_PLAIN;
         float* part = need ? static_cast<float*>(ws->data_ptr()) : nullptr;
         const size_t pb = need ? (size_t)ws->numel() : 0;
-        if (glu)
-            rc = p_rk_swiglu_rows(y.data_ptr<float>(), x->data_ptr<float>(), ld, op, (const float*)ptr(ss), ss_ld,
-                                  (const float*)ptr(nw), eps, (int)M, (int)(N / 2), (int)K, ptr(w.data), wt, ptr(w.scales),
-                                  ptr(w.mins), part, pb, (uint32_t*)ptr(cnt), (int)cnt->numel(), stream);
-        else
-            rc = p_rk_linear_rows_ex2(y.data_ptr<float>(), want_ss ? sums.data_ptr<float>() : nullptr, x->data_ptr<float>(),
-                                      ld, op, (const float*)ptr(ss), ss_ld, (const float*)ptr(nw), eps, (int)M, (int)N,
-                                      (int)K, ptr(w.data), wt, ptr(w.scales), ptr(w.mins), (const float*)ptr(bias),
-                                      (const float*)ptr(res), part, pb, (uint32_t*)ptr(cnt), (int)cnt->numel(), stream);
+        {
+            Unlocked scope;
+            y = make({M, glu ? N / 2 : N}, *x);
+            if (want_ss) sums = make({M, (N + 15) / 16}, *x);
+            if (glu)
+                rc = p_rk_swiglu_rows(y.data_ptr<float>(), x->data_ptr<float>(), ld, op, (const float*)ptr(ss), ss_ld,
+                                      (const float*)ptr(nw), eps, (int)M, (int)(N / 2), (int)K, ptr(w.data), wt,
+                                      ptr(w.scales), ptr(w.mins), part, pb, (uint32_t*)ptr(cnt), (int)cnt->numel(), stream);
+            else
+                rc = p_rk_linear_rows_ex2(y.data_ptr<float>(), want_ss ? sums.data_ptr<float>() : nullptr,
+                                          x->data_ptr<float>(), ld, op, (const float*)ptr(ss), ss_ld, (const float*)ptr(nw),
+                                          eps, (int)M, (int)N, (int)K, ptr(w.data), wt, ptr(w.scales), ptr(w.mins),
+                                          (const float*)ptr(bias), (const float*)ptr(res), part, pb, (uint32_t*)ptr(cnt),
+                                          (int)cnt->numel(), stream);
+        }
         PyObject* out = THPVariable_Wrap(y);
         if (want_ss && out) {
             PyObject* s = THPVariable_Wrap(sums);
@@ -179,11 +191,16 @@ PyObject* norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
         void* stream = PyLong_AsVoidPtr(a[4]);
         const float eps = (float)PyFloat_AsDouble(a[3]);
         if (PyErr_Occurred()) return nullptr;
-        at::Tensor y = make(x->sizes(), *x);
+        at::Tensor y;
         const auto fn = a[0] == Py_True ? p_rk_layer_norm : p_rk_rms_norm;
         const long long ld = x->size(0) > 1 ? x->stride(0) : x->size(1);
-        const int rc = fn(y.data_ptr<float>(), x->data_ptr(), RK_F32, ld, w->data_ptr(), RK_F32, (int)x->size(0),
-                          (int)x->size(1), eps, stream);
+        int rc;
+        {
+            Unlocked scope;
+            y = make(x->sizes(), *x);
+            rc = fn(y.data_ptr<float>(), x->data_ptr(), RK_F32, ld, w->data_ptr(), RK_F32, (int)x->size(0),
+                    (int)x->size(1), eps, stream);
+        }
         return finish(a[0] == Py_True ? "rk_layer_norm" : "rk_rms_norm", rc, THPVariable_Wrap(y));
     END_HANDLE_TH_ERRORS
 }
@@ -223,20 +240,24 @@ PyObject* paged_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
         if (!ws || !same(*ws, *q) || (size_t)ws->numel() < need || (a[8] != Py_None && !plan)) Py_RETURN_NONE;
         void* stream = PyLong_AsVoidPtr(a[10]);
         if (PyErr_Occurred()) return nullptr;
-        at::Tensor out = make({B, Hq, d}, *q);
-        float* o = out.data_ptr<float>();
+        at::Tensor out;
         const float* g = static_cast<const float*>(ptr(gate));
         const long long gld = gate ? gate->stride(0) : 0;
-        const int rc =
-            plan ? p_rk_paged_decode_planned(o, (const float*)ptr(q), ptr(k), ptr(v), code(*k), (const int32_t*)ptr(tb),
-                                             (const int32_t*)ptr(ln), (int)B, (int)Hq, (int)k->size(2), (int)d, (int)bs,
-                                             (int)tb->size(1), (int)k->size(0), (int)window, g, gld,
-                                             (int32_t*)ptr(plan), (size_t)plan->numel(), ws->data_ptr(),
-                                             (size_t)ws->numel(), stream)
-                 : p_rk_paged_decode(o, (const float*)ptr(q), ptr(k), ptr(v), code(*k), (const int32_t*)ptr(tb),
-                                     (const int32_t*)ptr(ln), (int)B, (int)Hq, (int)k->size(2), (int)d, (int)bs,
-                                     (int)tb->size(1), (int)k->size(0), (int)window, g, gld, ws->data_ptr(),
-                                     (size_t)ws->numel(), stream);
+        int rc;
+        {
+            Unlocked scope;
+            out = make({B, Hq, d}, *q);
+            float* o = out.data_ptr<float>();
+            rc = plan ? p_rk_paged_decode_planned(o, (const float*)ptr(q), ptr(k), ptr(v), code(*k), (const int32_t*)ptr(tb),
+                                                  (const int32_t*)ptr(ln), (int)B, (int)Hq, (int)k->size(2), (int)d, (int)bs,
+                                                  (int)tb->size(1), (int)k->size(0), (int)window, g, gld,
+                                                  (int32_t*)ptr(plan), (size_t)plan->numel(), ws->data_ptr(),
+                                                  (size_t)ws->numel(), stream)
+                      : p_rk_paged_decode(o, (const float*)ptr(q), ptr(k), ptr(v), code(*k), (const int32_t*)ptr(tb),
+                                          (const int32_t*)ptr(ln), (int)B, (int)Hq, (int)k->size(2), (int)d, (int)bs,
+                                          (int)tb->size(1), (int)k->size(0), (int)window, g, gld, ws->data_ptr(),
+                                          (size_t)ws->numel(), stream);
+        }
         return finish(plan ? "rk_paged_decode_planned" : "rk_paged_decode", rc, THPVariable_Wrap(out));
     END_HANDLE_TH_ERRORS
 }
@@ -273,11 +294,16 @@ PyObject* deltanet_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
             if (t->stride(1) != 1) Py_RETURN_NONE;
         auto ld = [&](const at::Tensor* t) { return B > 1 ? t->stride(0) : t->size(1); };
         if (ld(b) != ld(aa)) Py_RETURN_NONE;
-        at::Tensor out = make({B, H * dv}, *qkv);
+        at::Tensor out;
         auto f = [](const at::Tensor* t) { return static_cast<float*>(t->data_ptr()); };
-        const int rc = p_rk_deltanet_decode(out.data_ptr<float>(), f(qkv), f(z), f(b), f(aa), ld(qkv), ld(z), ld(b), f(conv),
-                                            f(S), f(w), f(A), f(dt), f(nw), static_cast<const int32_t*>(seq->data_ptr()),
-                                            (int)B, (int)H, (int)dk, (int)dv, (int)K, (int)nl, (int)slot, eps, stream);
+        int rc;
+        {
+            Unlocked scope;
+            out = make({B, H * dv}, *qkv);
+            rc = p_rk_deltanet_decode(out.data_ptr<float>(), f(qkv), f(z), f(b), f(aa), ld(qkv), ld(z), ld(b), f(conv),
+                                      f(S), f(w), f(A), f(dt), f(nw), static_cast<const int32_t*>(seq->data_ptr()),
+                                      (int)B, (int)H, (int)dk, (int)dv, (int)K, (int)nl, (int)slot, eps, stream);
+        }
         return finish("rk_deltanet_decode", rc, THPVariable_Wrap(out));
     END_HANDLE_TH_ERRORS
 }
@@ -305,12 +331,17 @@ PyObject* attn_prep(PyObject*, PyObject* const* a, Py_ssize_t n) {
             sl->numel() != N || !sl->is_contiguous() || k->size(2) != Hkv || k->size(3) != d || (rot > 0) != (inv != nullptr) ||
             (inv && (!is(*inv, at::kFloat) || inv->numel() != rot / 2 || !inv->is_contiguous())))
             Py_RETURN_NONE;
-        at::Tensor q = make({N, Hq, d}, *y);
-        const int rc = p_rk_attn_prep(q.data_ptr<float>(), nullptr, nullptr, ptr(k), ptr(v), code(*k),
-                                      static_cast<const int64_t*>(sl->data_ptr()), (int)k->size(0), (int)k->size(1),
-                                      y->data_ptr(), RK_F32, y->stride(0), (const float*)ptr(qw), (const float*)ptr(kw), eps,
-                                      static_cast<const int32_t*>(pos->data_ptr()), (const float*)ptr(inv), (int)rot, (int)N,
-                                      (int)Hq, (int)Hkv, (int)d, stream);
+        at::Tensor q;
+        int rc;
+        {
+            Unlocked scope;
+            q = make({N, Hq, d}, *y);
+            rc = p_rk_attn_prep(q.data_ptr<float>(), nullptr, nullptr, ptr(k), ptr(v), code(*k),
+                                static_cast<const int64_t*>(sl->data_ptr()), (int)k->size(0), (int)k->size(1),
+                                y->data_ptr(), RK_F32, y->stride(0), (const float*)ptr(qw), (const float*)ptr(kw), eps,
+                                static_cast<const int32_t*>(pos->data_ptr()), (const float*)ptr(inv), (int)rot, (int)N,
+                                (int)Hq, (int)Hkv, (int)d, stream);
+        }
         return finish("rk_attn_prep", rc, THPVariable_Wrap(q));
     END_HANDLE_TH_ERRORS
 }

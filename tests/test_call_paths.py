@@ -1,6 +1,12 @@
 """call_paths.cpp (the decode step's calls with their checks in C++) against the general way of kernels.py: over the
 forms both accept the results are the same bits; forms that need a conversion or a copy, and wrong ones, are left to the
 general way, which gives the results and exceptions it always gave."""
+import ctypes
+import signal
+import sys
+import threading
+import time
+
 import pytest
 import torch
 
@@ -193,3 +199,45 @@ def test_out_of_memory_is_torchs_own_exception(backend):
         torch.cuda.set_per_process_memory_fraction(1.0)
     for f in calls:
         f()
+
+
+@pytest.mark.gpu
+def test_other_threads_run_during_a_launch(backend, monkeypatch):
+    """A launch may wait for room in the device's queue. pause() in the place of rk_rms_norm stands for that: it returns
+    only when a signal comes, which another Python thread sends (a timer ends it if that thread cannot run)."""
+    x, w = torch.zeros(2, 64, device=DEV), torch.ones(64, device=DEV)
+    mod, lib = kernels._calls(), kernels.load().lib
+    address = lambda f: ctypes.cast(f, ctypes.c_void_p).value
+    real = {n: address(getattr(lib, n)) for n in kernels.CALLED}
+
+    def failed(entry, status):
+        raise RuntimeError(f"{entry}: {status}")
+    order, main, sent = [], threading.get_ident(), threading.Event()
+
+    def other():
+        sent.wait()
+        order.append("other thread")
+        time.sleep(0.2)                                         # the main thread gets to pause()
+        signal.pthread_kill(main, signal.SIGUSR1)
+    interval = sys.getswitchinterval()
+    old = [signal.signal(s, lambda *a: None) for s in (signal.SIGUSR1, signal.SIGALRM)]
+    thread = threading.Thread(target=other)
+    try:
+        mod.init({**real, "rk_rms_norm": address(ctypes.CDLL(None).pause)}, failed)
+        thread.start()
+        signal.setitimer(signal.ITIMER_REAL, 5.0)
+        sys.setswitchinterval(60.0)                             # the GIL changes hands only where it is given up
+        sent.set()
+        with pytest.raises(RuntimeError, match="rk_rms_norm: -1"):
+            mod.norm(False, x, w, 1e-6, 0)
+        order.append("call returned")
+    finally:
+        sys.setswitchinterval(interval)
+        signal.setitimer(signal.ITIMER_REAL, 0)
+        sent.set()
+        thread.join()
+        for s, h in zip((signal.SIGUSR1, signal.SIGALRM), old):
+            signal.signal(s, h)
+        monkeypatch.setattr(kernels, "_native_calls", None)
+        kernels._calls()                                        # the entry points again
+    assert order == ["other thread", "call returned"]
