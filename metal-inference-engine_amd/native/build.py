@@ -66,7 +66,8 @@ def _link(lib: Path, objs: list[Path], verbose: bool) -> None:
 CALLS = HERE / "rk_calls.so"              # call_paths.cpp: a CPython extension against torch's C++ API, host code only
 
 
-def _build_calls(verbose: bool) -> None:
+def _build_calls(verbose: bool) -> Path:
+    """call_paths.cpp compiled beside CALLS: build() puts it in place once the library it calls is there."""
     import sysconfig
 
     import torch
@@ -82,7 +83,7 @@ def _build_calls(verbose: bool) -> None:
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("g++ failed on call_paths.cpp:\n" + r.stderr)
-    os.replace(tmp, CALLS)
+    return tmp
 
 
 def build(verbose: bool = False) -> Path:
@@ -93,8 +94,9 @@ def build(verbose: bool = False) -> Path:
     with ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
         calls = ex.submit(_build_calls, verbose)
         objs = dict(zip(srcs, ex.map(lambda s: _compile(s, verbose), srcs)))
-        calls.result()
+        calls_tmp = calls.result()
     _link(LIB, [objs[s] for s in SOURCES], verbose)
+    os.replace(calls_tmp, CALLS)
     _link(PROBE_LIB, [objs[s] for s in PROBE_SOURCES] + [objs["rk_abi.cpp"]], verbose)
     return LIB
 

@@ -24,19 +24,25 @@ ENTRIES(DECLARE)
 #undef DECLARE
 PyObject* on_error = nullptr;                      // on_error(entry, status) raises
 
-// init({name: address}, on_error)
+// init({name: address}, on_error): the addresses of one library, whose interface must be the one compiled in here
 PyObject* init(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 2 || !PyDict_Check(a[0])) return PyErr_Format(PyExc_TypeError, "init(dict, callable)");
+    auto address = [&](const char* name) -> void* {
+        PyObject* v = PyDict_GetItemString(a[0], name);
+        return v ? PyLong_AsVoidPtr(v) : nullptr;
+    };
     bool ok = true;
-#define FETCH(f)                                                                                                    \
-    {                                                                                                               \
-        PyObject* v = PyDict_GetItemString(a[0], #f);                                                               \
-        p_##f = v ? reinterpret_cast<decltype(&::f)>(PyLong_AsVoidPtr(v)) : nullptr;                                \
-        ok = ok && p_##f;                                                                                           \
-    }
+#define CHECK(f) ok = ok && address(#f);
+    CHECK(rk_abi_version) ENTRIES(CHECK)
+#undef CHECK
+    if (!ok) return PyErr_Occurred() ? nullptr : PyErr_Format(PyExc_KeyError, "init: an entry point is missing");
+    const int version = reinterpret_cast<decltype(&::rk_abi_version)>(address("rk_abi_version"))();
+    if (version != RK_ABI_VERSION)
+        return PyErr_Format(PyExc_ImportError, "rk_calls.so was built for ABI version %d, the library has %d: build both again",
+                            RK_ABI_VERSION, version);
+#define FETCH(f) p_##f = reinterpret_cast<decltype(&::f)>(address(#f));
     ENTRIES(FETCH)
 #undef FETCH
-    if (!ok) return PyErr_Occurred() ? nullptr : PyErr_Format(PyExc_KeyError, "init: an entry point is missing");
     Py_XINCREF(a[1]);
     Py_XSETREF(on_error, a[1]);
     Py_RETURN_NONE;

@@ -71,3 +71,23 @@ def test_gemm_waits_count_its_loads(tmp_path):
         other = [ln for ln in lines[waits[0]:last_mfma]
                  if re.match(r"(global|buffer|flat|scratch)_", ln) and not ln.startswith("global_load_lds")]
         assert not other, (name, other[:3])
+
+
+def test_a_failed_build_leaves_the_libraries_as_they_were(tmp_path, monkeypatch):
+    """rk_calls.so calls librk_path.so through prototypes compiled in: a build whose HIP part fails must not leave a new one
+    beside the old library."""
+    libs = [tmp_path / n for n in ("librk_path.so", "rk_calls.so")]
+    for p, name in zip(libs, ("LIB", "CALLS")):
+        p.write_text("old")
+        monkeypatch.setattr(build, name, p)
+    monkeypatch.setattr(build, "OBJ_DIR", tmp_path / "obj")
+
+    def run(cmd, **kw):
+        ok = cmd[0] == "g++"
+        if ok:
+            Path(cmd[cmd.index("-o") + 1]).write_text("new")
+        return subprocess.CompletedProcess(cmd, 0 if ok else 1, "", "hipcc failed")
+    monkeypatch.setattr(build.subprocess, "run", run)
+    with pytest.raises(RuntimeError):
+        build.build()
+    assert [p.read_text() for p in libs] == ["old", "old"]

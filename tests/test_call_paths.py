@@ -65,6 +65,17 @@ def test_host_tensors_and_wrong_counts_are_not_answered():
         mod.linear(x)
 
 
+def test_a_library_of_another_interface_is_refused():
+    """The addresses come from whichever library is loaded: the prototypes compiled in must be that library's."""
+    mod, lib = kernels._calls(), kernels.load().lib
+    real = {n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in kernels.CALLED}
+    other = ctypes.CFUNCTYPE(ctypes.c_int)(lambda: lib.rk_abi_version() - 1)
+    with pytest.raises(ImportError, match="ABI version"):
+        mod.init({**real, "rk_abi_version": ctypes.cast(other, ctypes.c_void_p).value}, print)
+    with pytest.raises(KeyError):
+        mod.init({n: a for n, a in real.items() if n != "rk_abi_version"}, print)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["bf16", "int8", "int4"])
 @pytest.mark.parametrize("M,N,K", [(1, 96, 256), (5, 2048, 2048), (8, 4096, 512), (16, 100, 1056), (3, 64, 6144)])
