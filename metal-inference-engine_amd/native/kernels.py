@@ -10,6 +10,7 @@ import math
 from pathlib import Path
 
 import torch
+from torch.autograd import forward_ad
 
 from native.rocm_native import ERROR_NAMES, RK_BF16, RK_F32, RK_W_BF16, RK_W_INT4, RK_W_INT8, RocmKernelError, load
 from quant import QuantTensor
@@ -1068,17 +1069,28 @@ def _gemm(x, w, bias=None, residual=None, glu: bool = False) -> torch.Tensor:
     return out
 
 
+def _seen_by_torch(*ts) -> bool:
+    """Whether torch has to see the operations on any of these tensors (or None): a gradient is asked for, a forward-mode
+    tangent carried (which requires_grad does not say), or a subclass defines them."""
+    for t in ts:
+        if t is not None and (type(t) not in (torch.Tensor, torch.nn.Parameter) or
+                              (torch.is_grad_enabled() and t.requires_grad) or
+                              forward_ad.unpack_dual(t).tangent is not None):
+            return True
+    return False
+
+
 def linear(x, w, bias=None, residual=None) -> torch.Tensor:
     """The reference's decode / prefill linear on a bf16 or quantized weight (src/backend/metal.py:59-133): up to 32
     rows through the matvec kernel, beyond that rk_linear_gemm. fp32 / other-dtype weights, and bf16 rows that are not
-    whole blocks of 32: x @ w.T in fp32. Where a gradient of x, bias or residual is asked for beyond 32 rows, the same
-    product on the dequantized weight."""
+    whole blocks of 32: x @ w.T in fp32. Where torch has to see the product beyond 32 rows (a gradient or tangent of x,
+    bias or residual), torch's on the dequantized weight."""
     M = x.shape[0]
     if not isinstance(w, QuantTensor) and (w.dtype != torch.bfloat16 or w.shape[1] % 32):
         y = x.float() @ w.float().T
     elif M <= KERNEL_ROWS:
         return linear_rows(x, w, bias, residual)
-    elif torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x, bias, residual)):
+    elif _seen_by_torch(x, bias, residual):
         y = x.float() @ dequantize(w).T         # differentiable, as the row kernels are not
     else:
         N, K = w.shape

@@ -8,6 +8,7 @@ tests/test_quant.py:46-55 there), Qwen3.5-2B's, and ragged ones (rows not a mult
 K-tile)."""
 import pytest
 import torch
+from torch.autograd import forward_ad
 
 import quant
 from helpers import rel_err
@@ -318,3 +319,24 @@ def test_many_row_linear_carries_gradients(backend, kind):
     y.backward(dy.to(DEV))
     assert rel_err(xd.grad, dy @ deq) < TOL
     assert rel_err(bd.grad, dy.sum(0)) < TOL and torch.equal(rd.grad.cpu(), dy)
+
+
+@pytest.mark.parametrize("kind", ["bf16", "int4"])
+def test_many_row_linear_carries_tangents(backend, kind):
+    """Forward mode sees the product too (a dual tensor's requires_grad does not say so), and a tensor subclass its
+    operations. Bound: fp32 sums of 96 products."""
+    w, deq = weight(kind, 64, 96, 3)
+    g = torch.Generator().manual_seed(4)
+    x, tx, r, tr = (torch.randn(*s, generator=g) for s in ((40, 96), (40, 96), (40, 64), (40, 64)))
+    wd, dev = to_dev(w), [t.to(DEV) for t in (x, tx, r, tr)]
+    f = lambda a, b: backend.linear(a, wd, None, b)
+    with forward_ad.dual_level():
+        y = forward_ad.unpack_dual(f(forward_ad.make_dual(dev[0], dev[1]), dev[2]))
+        z = forward_ad.unpack_dual(f(dev[0], forward_ad.make_dual(dev[2], dev[3])))
+    assert rel_err(y.primal, x @ deq.T + r) < TOL and rel_err(y.tangent, tx @ deq.T) < TOL
+    assert rel_err(z.primal, x @ deq.T + r) < TOL and torch.equal(z.tangent.cpu(), tr)
+
+    class Marked(torch.Tensor):
+        pass
+    sub = f(dev[0].as_subclass(Marked), dev[2])
+    assert type(sub) is Marked and rel_err(sub.as_subclass(torch.Tensor), x @ deq.T + r) < TOL
