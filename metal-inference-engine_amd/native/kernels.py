@@ -1080,18 +1080,35 @@ def _seen_by_torch(*ts) -> bool:
     return False
 
 
+EXPAND_CHUNK = 1 << 23      # weights expanded to fp32 at a time beside torch's product (32 MB), as the reference
+
+
+def _linear_torch(x, w) -> torch.Tensor:
+    """x @ dequant(w)^T by torch, differentiable in x, on row pieces of the expanded weight, so that the full-size fp32
+    weight exists only where a gradient of x keeps it."""
+    N, K = w.shape
+    x = x.float()
+    y = torch.empty(x.shape[0], N, dtype=torch.float32, device=x.device)
+    step = max(1, EXPAND_CHUNK // K)
+    for r in range(0, N, step):
+        n = min(step, N - r)
+        wr = w[r:r + n].float() if not isinstance(w, QuantTensor) and K % 32 else dequantize(w, row0=r, n_rows=n)
+        y[:, r:r + n] = x @ wr.T
+    return y
+
+
 def linear(x, w, bias=None, residual=None) -> torch.Tensor:
     """The reference's decode / prefill linear on a bf16 or quantized weight (src/backend/metal.py:59-133): up to 32
     rows through the matvec kernel, beyond that rk_linear_gemm. fp32 / other-dtype weights, and bf16 rows that are not
     whole blocks of 32: x @ w.T in fp32. Where torch has to see the product beyond 32 rows (a gradient or tangent of x,
     bias or residual), torch's on the dequantized weight."""
     M = x.shape[0]
-    if not isinstance(w, QuantTensor) and (w.dtype != torch.bfloat16 or w.shape[1] % 32):
+    if not isinstance(w, QuantTensor) and w.dtype != torch.bfloat16:
         y = x.float() @ w.float().T
-    elif M <= KERNEL_ROWS:
+    elif M <= KERNEL_ROWS and w.shape[1] % 32 == 0:
         return linear_rows(x, w, bias, residual)
-    elif _seen_by_torch(x, bias, residual):
-        y = x.float() @ dequantize(w).T         # differentiable, as the row kernels are not
+    elif w.shape[1] % 32 or _seen_by_torch(x, bias, residual):
+        y = _linear_torch(x, w)
     else:
         N, K = w.shape
         if x.dim() != 2 or x.shape[1] != K:
