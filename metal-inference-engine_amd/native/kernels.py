@@ -1113,11 +1113,11 @@ def linear(x, w, bias=None, residual=None) -> torch.Tensor:
         N, K = w.shape
         if x.dim() != 2 or x.shape[1] != K:
             raise ValueError(f"linear: x {tuple(x.shape)} for a [{N}, {K}] weight")
-        # added in the kernel where they are what it reads, else (broadcast shapes) below
-        rows = lambda t: t.to(device=x.device, dtype=torch.float32).contiguous()
-        b = rows(bias) if bias is not None and bias.shape == (N,) else None
-        r = rows(residual) if residual is not None and residual.shape == (M, N) and (bias is None or b is not None) \
-            else None
+        # added in the kernel where they are what it reads, else (broadcast shapes, or for torch to refuse) below
+        takes = lambda t, *shape: t is not None and t.shape == shape and t.device == x.device
+        rows = lambda t: t.to(torch.float32).contiguous()
+        b = rows(bias) if takes(bias, N) else None
+        r = rows(residual) if takes(residual, M, N) and (bias is None or b is not None) else None
         y = _gemm(x, w, b, r)
         bias = None if b is not None else bias
         residual = None if r is not None else residual

@@ -304,6 +304,9 @@ def test_many_row_linears_take_what_the_row_kernels_take(backend):
     assert not torch.isfinite(bad[7]).any()
     keep = [i for i in range(33) if i != 7]
     assert torch.equal(bad[keep], got[keep])
+    for args in ((r, None), (None, torch.zeros(33, 48))):       # on the host: refused
+        with pytest.raises(RuntimeError):
+            backend.linear(x.to(DEV)[:, ::2], odd, *args)
 
 
 @pytest.mark.parametrize("kind", ["bf16", "int4"])
