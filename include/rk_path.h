@@ -339,10 +339,9 @@ int rk_swiglu_rows(float* y, const float* x, long long x_ld, int x_op, const flo
  * fp32 GEMM on a dequantized weight of src/backend/metal.py:55-133): y [M, N] fp32 = x @ dequant(W)^T (+ bias)
  * (+ residual), or with glu y [M, N / 2] = silu(x gate^T) * (x up^T) for W = [gate; up] (no bias or residual).
  *   x rows at a stride x_ld >= K (a multiple of 4), x and w 16-byte aligned; w per w_type with scales / mins as
- *   rk_linear_rows; K a multiple of 32. fp32-level results: x enters as two fp16 pieces of 24 bits together relative
- *   to each value (40 bits relative to its row's largest), INT8 / INT4 codes exactly, bf16 weights exactly down to
- *   2^-32 of their row's largest; products are exact, sums fp32. An infinite or NaN value makes its row's outputs
- *   infinite or NaN.
+ *   rk_linear_rows; K a multiple of 32. x and the weights enter exactly (three bf16 pieces of every x; bf16 weights and
+ *   INT8 / INT4 codes as they are), products are exact, sums fp32. An infinite or NaN value of x makes its row's outputs
+ *   infinite or NaN, one of W its column's.
  *   workspace: rk_linear_gemm_workspace_bytes(M, N, K, w_type, glu) bytes, 256-byte aligned, no zeroing needed. */
 size_t rk_linear_gemm_workspace_bytes(int M, int N, int K, int w_type, int glu);
 int rk_linear_gemm(float* y, const float* x, long long x_ld, int M, int N, int K, const void* w, int w_type,

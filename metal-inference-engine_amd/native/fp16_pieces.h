@@ -1,5 +1,4 @@
-// fp16 pieces of fp32 values: shared by the linears of many rows (linear_gemm.hip, linear_mid.hip) and the fp32
-// prefill attention (paged_prefill.hip).
+// fp16 pieces of fp32 values, for the fp32 prefill attention (paged_prefill.hip).
 #pragma once
 
 #include "rk_device.h"
@@ -7,14 +6,6 @@
 
 namespace rk {
 
-// linear_mid.hip: the form for up to a few hundred rows, behind rk_linear_gemm
-bool mid_takes(int M, int K, int w_type, const void* scales, const void* mins);
-size_t mid_workspace_bytes(int M, int N, int K, int w_type, int glu);
-int mid_linear(float* y, const float* x, long long x_ld, int M, int N, int K, const void* w, int w_type,
-               const void* scales, const void* mins, const float* bias, const float* residual, int glu,
-               void* workspace, hipStream_t stream);
-
-constexpr int kQB = 32;                            // weights per quantization block = one MFMA's k-extent
 constexpr int kTop = 14;                           // a row's largest value lies in [2^kTop, 2^(kTop + 1))
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
@@ -24,12 +15,6 @@ __device__ __forceinline__ f32x4 mfma_f16(u32x4 a, u32x4 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0,
                                                   0);
 }
-
-__device__ __forceinline__ uint32_t pack_f16(float a, float b) {   // round to nearest even
-    return __builtin_bit_cast(uint32_t, (f16x2){(_Float16)a, (_Float16)b});
-}
-
-__device__ __forceinline__ float half_to_f32(uint32_t h) { return (float)__builtin_bit_cast(_Float16, (uint16_t)h); }
 
 // the power of two that puts the magnitude m into [2^kTop, 2^(kTop + 1)): its exponent (0 for m = 0; inf and NaN as
 // the largest finite exponent, so that they stay inf and NaN in the pieces)
@@ -54,23 +39,6 @@ __device__ __forceinline__ uint32_t rest_of(Pieces p) {
                           (e >> 16 == 0x7c00u && !(m >> 16) ? 0xffff0000u : 0u);
     return p.lo & ~drop;
 }
-
-// largest |v| of a 256-thread workgroup, in every thread
-__device__ __forceinline__ float block_absmax(float m, float* red) {
-    m = row16_max(m);
-    const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(m), __float_as_uint(m), false, false);
-    m = fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
-    const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
-    m = fmaxf(__uint_as_float(q[0]), __uint_as_float(q[1]));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-    __syncthreads();
-    return fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-}
-
-__device__ __forceinline__ float silu_times(float g, float u) {
-    return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-g * kLog2e)) * u;
-}
-
 
 // Rows of 32 fp16 (64 bytes) in LDS: the 16-byte unit u of row R sits at u ^ swizzle(R). A read of lane l: row l % 16,
 // unit l / 16, is served 16 lanes at a time, rows 0-3 and 12-15 of one unit with rows 4-11 of the next, and these then

@@ -16,13 +16,11 @@
 // and a 1024-weight K-split, one quarter of the split per wave, so each wave requests all its weights at once (no
 // loop over K) and reuses every activation piece it reads from LDS across its row tiles. Splits of one row group
 // are added by the last workgroup to finish (see linear_rows_kernel).
-#include "rk_device.h"
-#include "rk_internal.h"
+#include "linear_operands.h"
 
 namespace rk {
 namespace {
 
-constexpr int kQB = 32;            // weights per quantization block = the MFMA k-extent
 constexpr int kCols = 16;          // activation rows per launch (MFMA columns)
 
 struct LinArgs {
@@ -52,72 +50,12 @@ template <> struct WTraits<RK_W_BF16> { static constexpr int BPB = 64; };
 template <> struct WTraits<RK_W_INT8> { static constexpr int BPB = 32; };
 template <> struct WTraits<RK_W_INT4> { static constexpr int BPB = 16; };
 
-__device__ __forceinline__ float half_to_f32(uint16_t h) { return (float)__builtin_bit_cast(_Float16, h); }
-
-// silu(g) * u = g / (1 + exp(-g)) * u with the hardware exp2 and reciprocal: SwiGLU's product, in the one form that
-// both the silu * up input transform (XF 1) and the paired [gate; up] output (glu) compute, so they give equal bits.
-// The result is the rounded fp32 product, as the reference hands silu * up to the next op as an fp32 tensor: the
-// empty asm makes it opaque, since an inlined product would otherwise be contracted into the activation split that
-// consumes it (x - hi as fma(a, u, -hi)), whose pieces would then carry the unrounded product.
-__device__ __forceinline__ float silu_times(float g, float u) {
-    const float d = 1.0f + __builtin_amdgcn_exp2f(-g * 1.4426950408889634f);
-    float h = g * __builtin_amdgcn_rcpf(d) * u;
-    asm("" : "+v"(h));
-    return h;
-}
-
 // the weight row behind output row lr of the kernel: lr itself, or with glu (W = [gate; up], N = 2F rows, F % 8 == 0)
 // gate rows 8T .. 8T+7 then up rows F + 8T .. F + 8T+7 for 16-row tile T, so that in the MFMA result each gate
 // output's up partner is 8 lanes away and the tile's 8 outputs silu(gate) * up are columns 8T .. 8T+7 of y
 __device__ __forceinline__ size_t weight_row(const LinArgs& a, int lr) {
     const int c = lr & 15, base = 8 * (lr >> 4) + (c & 7);
     return (size_t)(a.glu ? (c < 8 ? base : (a.N >> 1) + base) : lr);
-}
-
-// 8 INT8 codes (one lane's MFMA slots of one block: bytes of lo then hi) as bf16 bits; q in [-127, 127] is exact in
-// bf16, and the top half of the fp32 value is its bf16 pattern
-__device__ __forceinline__ u32x4 int8_bf16(uint32_t lo, uint32_t hi) {
-    u32x4 o;
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            const uint32_t w = h ? hi : lo;
-            const float f0 = (float)(int)__builtin_amdgcn_sbfe(w, 16 * e, 8);
-            const float f1 = (float)(int)__builtin_amdgcn_sbfe(w, 16 * e + 8, 8);
-            o[2 * h + e] = pack_hi2(__float_as_uint(f0), __float_as_uint(f1));
-        }
-    return o;
-}
-
-// 8 INT4 codes (4 bytes; byte j holds elements 2j in the low nibble, 2j+1 in the high one) as bf16 bits, in the
-// element order 0 2 4 6 1 3 5 7 (kInt4Order; the activations are staged in the same order, so the MFMA's k-sum
-// is unchanged). A code q alone in a byte, read as an fp8 e4m3 pattern 0000qqqq, is exactly q * 2^-9 (codes 0-7
-// are subnormals m * 2^-9, 8-15 the first normal binade (8 + m) * 2^-9), so v_cvt_scalef32_pk_bf16_fp8 with the
-// scale 2^9 turns two such bytes into two exact bf16 integers: 7 instructions for 8 codes.
-__device__ __forceinline__ u32x4 int4_bf16(uint32_t v) {
-    const uint32_t lo = v & 0x0F0F0F0Fu, hi = (v >> 4) & 0x0F0F0F0Fu;   // codes 0 2 4 6 | 1 3 5 7, one per byte
-    u32x4 o;
-    o[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 512.0f, false));
-    o[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 512.0f, true));
-    o[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 512.0f, false));
-    o[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 512.0f, true));
-    return o;
-}
-// element pairs of the four bf16-pair registers of an INT4 operand (int4_bf16), and of the activation pieces staged
-// against it
-constexpr int kInt4Order[4][2] = {{0, 2}, {4, 6}, {1, 3}, {5, 7}};
-
-// 4 x 4 transpose over the wave's four 16-lane groups: afterwards register d of lane group g holds what register g
-// of lane group d held. v_permlane32_swap exchanges the upper 32 lanes of its first operand with the lower 32 of its
-// second, v_permlane16_swap the odd 16-lane groups of the first with the even ones of the second; all 64 lanes must
-// be active.
-__device__ __forceinline__ u32x4 xpose4(uint32_t a0, uint32_t a1, uint32_t a2, uint32_t a3) {
-    const auto s02 = __builtin_amdgcn_permlane32_swap(a0, a2, false, false);
-    const auto s13 = __builtin_amdgcn_permlane32_swap(a1, a3, false, false);
-    const auto s01 = __builtin_amdgcn_permlane16_swap(s02[0], s13[0], false, false);
-    const auto s23 = __builtin_amdgcn_permlane16_swap(s02[1], s13[1], false, false);
-    return (u32x4){s01[0], s01[1], s23[0], s23[1]};
 }
 
 constexpr int kWaveBlocks = 8;                     // quantization blocks per wave

@@ -5,29 +5,21 @@
 // block-quantized (src/quant.py:1-10, 45-56); and Backend.swiglu (src/backend/base.py:40-41) over a stacked
 // [gate; up] weight.
 //
-// Design: the fp32 matrix rate of gfx950 is 1/16 of its 16-bit rate, so an fp32 product is worth two 16-bit ones if
-// two carry enough bits. Here they do:
-//   x  enters as two fp16 pieces hi + lo of x * 2^a, with 2^a (per row) placing the row's largest value in
-//      [2^14, 2^15): hi = fp16(x 2^a), lo = fp16(x 2^a - hi). A value keeps a relative error of 2^-24, what one fp32
-//      rounding costs, down to 2^-16 of its row's largest, and below that an absolute one of 2^-40 of the largest.
-//   W  is one fp16 operand: INT8 / INT4 codes are exact, a bf16 row times its own 2^b (largest in [2^14, 2^15)) is
-//      exact down to 2^-32 of the row's largest and within 2^-40 of it below.
-// Every product of two pieces is exact in fp32 and accumulates in fp32. A quantization block is one MFMA's k-extent
-// (32), so its scale multiplies the block's sums on the VALU. The powers of two leave in the epilogue (ldexp), exactly.
+// Design: the fp32 matrix rate of gfx950 is 1/16 of its 16-bit rate, so an fp32 product is worth three 16-bit ones, and
+// three carry all its bits: operands are linear_operands.h's, three bf16 pieces of every activation and the weights, all
+// exact (as in linear.hip, so a row is computed alike however many there are). Products accumulate in fp32. A
+// quantization block is one MFMA's k-extent (32), so its scale multiplies the block's sums on the VALU.
 //
-// W is expanded to fp16 rows, a slab at a time, and the product runs on LDS tiles of both. An INT4 weight is
-// s (q - 8) + (8 s + min): the codes enter as q - 8 (small partial sums), and min and 8 s as K / 16 more columns, (min,
-// s) against the block's activation sum (1, 8): pairs in one MFMA, whose near-equal terms of opposite sign cancel
-// inside it. Three launches per slab: split_rows, slab_weights, gemm_rows (four with K-splits: gemm_finish). Up to a few
-// hundred rows linear_mid.hip reads W as stored instead.
+// The product runs on LDS tiles of both operands. split_rows writes the pieces of x. bf16 weights are read as stored;
+// INT8 / INT4 ones are expanded to bf16 rows, a slab at a time (slab_weights). An INT4 weight is s (q - 8) + (8 s + min):
+// the codes enter as q - 8 (small partial sums), and 8 s + min, in its three pieces, as K / 8 more columns against the
+// block's activation sum. Then gemm_rows (and with K-splits gemm_finish). Up to a few hundred rows linear_mid.hip reads
+// quantized weights as stored instead.
 //
-// Measured against the fp32 GEMM on the expanded weight, an MLP of 1777 rows, bf16 weights (12288 x 2048 with silu * up,
-// then 2048 x 6144): 1188 -> 355 us in all; gemm_rows 212 us there (840 TFLOP/s of 16-bit products; a large bf16 GEMM of
-// the BLAS reaches 1270 on this card) and 133 us, the expansions 20 us each, the splits 7 and 20. Error against 64 bits
-// 9.6e-7 -> 1.6e-7 of the result. What bounds gemm_rows: matrix-core issue and the fp32 joins beside it (joins after
-// every stage instead of every other: 374 against 349 us in all; copies without the loads or without the LDS reads were
-// each about 10 % faster), and whole tiles: 224 workgroups on 256 CUs at 2048 columns, 672 at 12288.
-#include "fp16_pieces.h"
+// Measured, an MLP of 1777 rows, bf16 weights (12288 x 2048 with silu * up, then 2048 x 6144): 1188 us as an fp32 GEMM on
+// the expanded weight, 362 on two fp16 pieces of x (23 bits in a range of 2^40 below the row's largest value), 390 so.
+// What bounds gemm_rows: matrix-core issue and the fp32 joins beside it, and whole tiles.
+#include "linear_operands.h"
 
 #include <type_traits>
 
@@ -35,8 +27,8 @@ namespace rk {
 namespace {
 
 constexpr int kBK = 32;                            // k per step
-constexpr int kSumShift = 8;                       // 8 block sums (of 32 values) are scaled by 2^-kSumShift
-constexpr long long kSlabElems = 1ll << 25;        // fp16 weights expanded at a time (64 MiB)
+constexpr int P = 3;                               // pieces of an activation
+constexpr long long kSlabElems = 1ll << 25;        // quantized weights expanded at a time (64 MiB)
 
 // 16 bytes per lane from src into LDS at dst (wave-uniform) + 16 * lane
 __device__ __forceinline__ void load_to_lds(const void* src, char* dst) {
@@ -47,79 +39,60 @@ __device__ __forceinline__ void load4_to_lds(const void* src, char* dst) {   // 
     __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)dst, 4, 0, 0);
 }
 
-// Operand layout of gemm_rows, shared by both operands: rows cut into steps of 32 values, [step][rows][32] fp16 (x:
-// [step][piece][rows][32]), so that a stage of a tile is one contiguous run per operand. The 16-byte unit u of row R
-// sits at u ^ swizzle(R).
+// Rows of 32 bf16 (64 bytes) in LDS: the 16-byte unit u of row R sits at u ^ swizzle(R). A read of lane l: row l % 16,
+// unit l / 16, is served 16 lanes at a time, rows 0-3 and 12-15 of one unit with rows 4-11 of the next, and these then
+// lie on all 16 units of the 256-byte bank line.
+__device__ __forceinline__ int swizzle(int R) { return (0x78 >> (2 * ((R >> 2) & 3))) & 3; }
+
+// Operands of gemm_rows in memory: rows cut into steps of 32 values, x [step][piece][rows][32], an expanded weight slab
+// [step][rows][32], so that a stage of a tile is one contiguous run per operand, in the LDS order.
 // Rows past the matrix (up to whole tiles) are not written: their products are never stored.
 __device__ __forceinline__ size_t unit_at(size_t slice, int rows, int R, int u) {
     return (slice * rows + R) * kBK + 8 * (u ^ swizzle(R));
 }
 
-// One workgroup per row m of x: the row's pieces and its exponent ex[m]. With SUMS, columns K + 2b and K + 2b + 1 are
-// the pieces of block b's sum and of 8 times it, both * 2^-kSumShift, then zeros to the end of the last step. The
-// second pass reads the row from the caches.
+// One workgroup per row m of x: the row's pieces. With SUMS, columns K + 4 b .. + 2 are block b's sum, and zeros to the
+// end of the last step.
 template <bool SUMS>
-__global__ __launch_bounds__(256) void split_rows(uint16_t* a, int* ex, const float* x, long long x_ld, int Mp, int K,
-                                                  int steps) {
-    __shared__ float red[4];
+__global__ __launch_bounds__(256) void split_rows(uint16_t* a, const float* x, long long x_ld, int Mp, int K, int steps) {
     const int m = blockIdx.x, tid = threadIdx.x;
     const float* xr = x + (size_t)m * x_ld;
-    float big = 0.0f;
+    auto put_sum = [&](int b, const Split3& p) {   // eight blocks to a step
+        const uint32_t v[P] = {p.hi, p.mid, p.lo};
+#pragma unroll
+        for (int q = 0; q < P; ++q)
+            *reinterpret_cast<u32x2*>(a + unit_at(P * (size_t)(K / kBK + (b >> 3)) + q, Mp, m, (b & 7) >> 1) + 4 * (b & 1)) =
+                (u32x2){pack_hi2(v[q], v[q]), v[q] >> 16};
+    };
     for (int c = tid; c < K / 8; c += 256) {
         const f32x4 v0 = *reinterpret_cast<const f32x4*>(xr + 8 * c), v1 = *reinterpret_cast<const f32x4*>(xr + 8 * c + 4);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) big = fmaxf(big, fmaxf(fabsf(v0[e]), fabsf(v1[e])));
-    }
-    big = block_absmax(big, red);
-    const int k = top_exponent(big);
-    if (tid == 0) ex[m] = k;
-    for (int c = tid; c < K / 8; c += 256) {
-        const f32x4 v0 = *reinterpret_cast<const f32x4*>(xr + 8 * c), v1 = *reinterpret_cast<const f32x4*>(xr + 8 * c + 4);
-        float v[8];
+        const float v[8] = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
+        u32x4 pc[P];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            v[e] = ldexpf(v0[e], k);
-            v[4 + e] = ldexpf(v1[e], k);
+            const Split3 s0 = split3_any(v[2 * e]), s1 = split3_any(v[2 * e + 1]);
+            pc[0][e] = pack_hi2(s0.hi, s1.hi);
+            pc[1][e] = pack_hi2(s0.mid, s1.mid);
+            pc[2][e] = pack_hi2(s0.lo, s1.lo);
         }
-        u32x4 ph, pl;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const Pieces p = split_pair(v[2 * e], v[2 * e + 1]);
-            ph[e] = p.hi;
-            pl[e] = rest_of(p);
-        }
-        *reinterpret_cast<u32x4*>(a + unit_at(2 * (size_t)(c >> 2), Mp, m, c & 3)) = ph;
-        *reinterpret_cast<u32x4*>(a + unit_at(2 * (size_t)(c >> 2) + 1, Mp, m, c & 3)) = pl;
+        for (int q = 0; q < P; ++q) *reinterpret_cast<u32x4*>(a + unit_at(P * (size_t)(c >> 2) + q, Mp, m, c & 3)) = pc[q];
         if constexpr (SUMS) {                      // the four threads of a block are neighbours in one wave
             float sum = 0.0f;
 #pragma unroll
             for (int e = 0; e < 8; ++e) sum += v[e];
             sum += dpp_f32<0xb1>(sum);             // lane ^ 1
             sum += dpp_f32<0x4e>(sum);             // lane ^ 2
-            if ((c & 3) == 0) {
-                const int b = c >> 2;              // sixteen blocks' pairs to a step
-                sum = ldexpf(sum, -kSumShift);
-                const Pieces p = split_pair(sum, 0.0f);
-                const float h = half_to_f32(p.hi & 0xffffu), l = half_to_f32(rest_of(p) & 0xffffu);
-                const size_t sl = 2 * (size_t)(K / kBK + (b >> 4));
-                *reinterpret_cast<uint32_t*>(a + unit_at(sl, Mp, m, (b & 15) >> 2) + 2 * (b & 3)) = pack_f16(h, 8.0f * h);
-                *reinterpret_cast<uint32_t*>(a + unit_at(sl + 1, Mp, m, (b & 15) >> 2) + 2 * (b & 3)) =
-                    pack_f16(l, 8.0f * l);
-            }
+            if ((c & 3) == 0) put_sum(c >> 2, split3_any(sum));
         }
     }
     if constexpr (SUMS)
-        for (int b = K / kBK + tid; b < 16 * (steps - K / kBK); b += 256) {
-            const size_t sl = 2 * (size_t)(K / kBK + (b >> 4));
-            *reinterpret_cast<uint32_t*>(a + unit_at(sl, Mp, m, (b & 15) >> 2) + 2 * (b & 3)) = 0u;
-            *reinterpret_cast<uint32_t*>(a + unit_at(sl + 1, Mp, m, (b & 15) >> 2) + 2 * (b & 3)) = 0u;
-        }
+        for (int b = K / kBK + tid; b < 8 * (steps - K / kBK); b += 256) put_sum(b, {0u, 0u, 0u});
 }
 
 struct SlabArgs {
-    uint16_t* out;                 // [steps][Np][32] fp16
-    float* sc;                     // quantized: [steps][Np] scales
-    int* ew;                       // bf16: [rows] exponents
+    uint16_t* out;                 // [steps][Np][32] bf16
+    float* sc;                     // [steps][Np] scales
     const void* w;
     const uint16_t* scales;
     const uint16_t* mins;
@@ -127,97 +100,66 @@ struct SlabArgs {
     int F;                         // glu: rows of each half; 0: plain
 };
 
-// the weight row behind slab row j: row0 + j, or with glu sixteen gate rows, then the sixteen up rows of the same
-// outputs, in turn, so that an output's gate and up sums meet in one lane (rows past F, in the last pair of
-// sixteens, repeat row F - 1: their outputs are not stored)
-__device__ __forceinline__ size_t slab_row(const SlabArgs& a, int j) {
-    if (!a.F) return (size_t)(a.row0 + j);
-    const int f = min(a.row0 + 16 * (j >> 5) + (j & 15), a.F - 1);
-    return (size_t)((j & 16) ? a.F + f : f);
+// the weight row behind tile row j from row0 on: row0 + j, or with glu (F rows in each half) sixteen gate rows, then the
+// sixteen up rows of the same outputs, in turn, so that an output's gate and up sums meet in one lane (rows past F, in
+// the last pair of sixteens, repeat row F - 1: their outputs are not stored)
+__device__ __forceinline__ size_t weight_row(int row0, int F, int j) {
+    if (!F) return (size_t)(row0 + j);
+    const int f = min(row0 + 16 * (j >> 5) + (j & 15), F - 1);
+    return (size_t)((j & 16) ? F + f : f);
 }
 
-// One workgroup per slab row: fp16 operands of the row (codes, or bf16 * 2^b) and its scales; INT4 codes minus 8, then
-// the row's (min, scale) pairs.
+// One workgroup per slab row: the row's codes and scales; INT4: codes minus 8, then the pieces of 8 s + min.
 template <int WT>
 __global__ __launch_bounds__(256) void slab_weights(SlabArgs a) {
-    __shared__ float red[4];
     const int j = blockIdx.x, tid = threadIdx.x;
-    const size_t n = slab_row(a, j);
+    const size_t n = weight_row(a.row0, a.F, j);
     const int nblk = a.K / kQB;
-    int k = 0;
-    if constexpr (WT == RK_W_BF16) {
-        const uint16_t* w = static_cast<const uint16_t*>(a.w) + n * a.K;
-        float big = 0.0f;
-        for (int c = tid; c < a.K / 8; c += 256) {
-            const u32x4 q = *reinterpret_cast<const u32x4*>(w + 8 * c);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) big = fmaxf(big, fmaxf(fabsf(bf16_lo(q[e])), fabsf(bf16_hi(q[e]))));
-        }
-        k = top_exponent(block_absmax(big, red));
-        if (tid == 0) a.ew[j] = k;
-    }
     for (int c = tid; c < a.K / 8; c += 256) {
         u32x4 o;
-        if constexpr (WT == RK_W_BF16) {
-            const u32x4 q = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.w) + n * a.K + 8 * c);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = pack_f16(ldexpf(bf16_lo(q[e]), k), ldexpf(bf16_hi(q[e]), k));
-        } else if constexpr (WT == RK_W_INT8) {
+        if constexpr (WT == RK_W_INT8) {
             const u32x2 q = *reinterpret_cast<const u32x2*>(static_cast<const int8_t*>(a.w) + n * a.K + 8 * c);
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                o[e] = pack_f16((float)(int)__builtin_amdgcn_sbfe(q[e >> 1], 16 * (e & 1), 8),
-                                (float)(int)__builtin_amdgcn_sbfe(q[e >> 1], 16 * (e & 1) + 8, 8));
+            o = int8_bf16(q[0], q[1]);
         } else {
             const uint32_t q = *reinterpret_cast<const uint32_t*>(static_cast<const uint8_t*>(a.w) + n * (a.K / 2) + 4 * c);
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                o[e] = pack_f16((float)__builtin_amdgcn_ubfe(q, 8 * e, 4) - 8.0f,
-                                (float)__builtin_amdgcn_ubfe(q, 8 * e + 4, 4) - 8.0f);
+                o[e] = pack_hi2(__float_as_uint((float)__builtin_amdgcn_ubfe(q, 8 * e, 4) - 8.0f),
+                                __float_as_uint((float)__builtin_amdgcn_ubfe(q, 8 * e + 4, 4) - 8.0f));
         }
         *reinterpret_cast<u32x4*>(a.out + unit_at(c >> 2, a.Np, j, c & 3)) = o;
     }
-    if constexpr (WT != RK_W_BF16) {
-        const uint16_t* s = a.scales + n * nblk;
-        for (int t = tid; t < a.steps; t += 256)   // the pairs' steps: 2^kSumShift
-            a.sc[(size_t)t * a.Np + j] = t < nblk ? half_to_f32(s[t]) : (float)(1 << kSumShift);
-        if constexpr (WT == RK_W_INT4) {
-            const uint16_t* mn = a.mins + n * nblk;
-            for (int b = tid; b < 16 * (a.steps - nblk); b += 256)
-                *reinterpret_cast<uint32_t*>(a.out + unit_at(nblk + (b >> 4), a.Np, j, (b & 15) >> 2) + 2 * (b & 3)) =
-                    b < nblk ? mn[b] | (uint32_t)s[b] << 16 : 0u;
+    const uint16_t* s = a.scales + n * nblk;
+    for (int t = tid; t < a.steps; t += 256) a.sc[(size_t)t * a.Np + j] = t < nblk ? half_to_f32(s[t]) : 1.0f;
+    if constexpr (WT == RK_W_INT4) {
+        const uint16_t* mn = a.mins + n * nblk;
+        for (int b = tid; b < 8 * (a.steps - nblk); b += 256) {
+            const Split3 p = split3(b < nblk ? fmaf(8.0f, half_to_f32(s[b]), half_to_f32(mn[b])) : 0.0f);
+            *reinterpret_cast<u32x2*>(a.out + unit_at(nblk + (b >> 3), a.Np, j, (b & 7) >> 1) + 4 * (b & 1)) =
+                (u32x2){pack_hi2(p.hi, p.mid), p.lo >> 16};
         }
     }
 }
 
 struct GemmArgs {
     float* y;
-    const uint16_t* a;             // [steps][2][Mp][32]
-    const uint16_t* w;             // [steps][Np][32], the slab
+    const uint16_t* a;             // [steps][3][Mp][32]
+    const uint16_t* w;             // SCALED: [steps][Np][32], the slab; else [N][K] as stored
     const float* sc;               // [steps][Np]
-    const int* ex;
-    const int* ew;
     const float* bias;             // [columns of y] or null
     const float* res;              // as y, or null
     long long y_ld;
-    int M, N, Mp, Np, steps;
+    int M, N, Mp, Np, steps;       // N: weight rows of this slab
+    int F;                         // bf16 glu: rows of each half; 0: plain
     int col0, cols;                // first column of y this slab gives; columns of y
     int tm, tn;                    // tiles
     int S;                         // K-splits
     float* part;                   // S > 1: [S][M][Np] sums, to be finished by gemm_finish
 };
 
-// weight columns 32 q + r and 32 q + 16 + r (v, u) of row m: powers of two, then bias and residual or silu * up
-template <bool SCALED, bool GLU>
+// weight columns 32 q + r and 32 q + 16 + r (v, u) of row m: bias and residual or silu * up
+template <bool GLU>
 __device__ __forceinline__ void gemm_store(const GemmArgs& g, int m, int n, float v, float u) {
-    const int em = g.ex[m];
-    int ev = -em, eu = -em;
-    if constexpr (!SCALED) {
-        ev -= g.ew[min(n, g.N - 1)];
-        eu -= g.ew[min(n + 16, g.N - 1)];
-    }
-    v = ldexpf(v, ev);
-    u = ldexpf(u, eu);
     if constexpr (GLU) {
         const int c = g.col0 + ((n & ~31) >> 1) + (n & 15);
         if (c < g.cols && n < g.N) g.y[(size_t)m * g.y_ld + c] = silu_times(v, u);
@@ -234,14 +176,14 @@ __device__ __forceinline__ void gemm_store(const GemmArgs& g, int m, int n, floa
     }
 }
 
-// Workgroup of WM x WN waves, each a 16 TI x 64 tile of y. A stage is one step of 32: 2 BM piece rows and BN
+// Workgroup of WM x WN waves, each a 16 TI x 64 tile of y. A stage is one step of 32: 3 BM piece rows and BN
 // weight rows of 64 bytes (and each wave's 64 scales), straight from memory into LDS by global_load_lds, 1 KB per
-// instruction, kStages buffers in turn. Per stage and wave 12 operand reads feed 32 MFMAs, each read one group of
-// sixteen rows ahead, across the stages' barriers too. The loop has no other memory reads, and a wave's loads complete
+// instruction, kStages buffers in turn. Per stage and wave 16 operand reads feed 48 MFMAs (TI = 4), each read one group
+// of sixteen rows ahead, across the stages' barriers too. The loop has no other memory reads, and a wave's loads complete
 // in order, so waiting for all but the newest (kStages - 3) x loads-per-stage leaves this stage and the next in LDS.
 template <int WM, int WN, int TI, bool SCALED>
 struct Tile {
-    static constexpr int NW = WM * WN, BM = 16 * TI * WM, BN = 64 * WN, ROWS = 2 * BM + BN, NI = ROWS / 16 / NW;
+    static constexpr int NW = WM * WN, BM = 16 * TI * WM, BN = 64 * WN, ROWS = P * BM + BN, NI = ROWS / 16 / NW;
     static constexpr int kLoads = NI + (SCALED ? 1 : 0);
     static constexpr int kBytes = ROWS * 2 * kBK + (SCALED ? 256 * NW : 0);
     static constexpr int kStages = 160 * 1024 / kBytes < 6 ? 160 * 1024 / kBytes : 6;
@@ -267,17 +209,24 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_rows(GemmArgs g) {
 
     // this split's steps
     const int s0 = (int)((long long)g.steps * blockIdx.y / g.S), S = (int)((long long)g.steps * (blockIdx.y + 1) / g.S) - s0;
-    // load instruction i of this wave: stage rows 16 (NI wave + i) .. + 15 (hi piece rows, lo piece rows, weight rows);
-    // wave-uniform addresses, 16 bytes per lane from there
+    // load instruction i of this wave: stage rows 16 (NI wave + i) .. + 15 (hi, mid, lo piece rows, weight rows);
+    // lane l brings unit (l % 4) ^ swizzle of row l / 4 of the sixteen (operands laid out in the LDS order: 16 l on)
     const char* src[NI];
     size_t hop[NI];
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
         const int R = 16 * (NI * wave + i);
-        const bool pc = R < 2 * BM;
-        const size_t row = pc ? (size_t)(R / BM) * g.Mp + m0 + R % BM : (size_t)(n0 + R - 2 * BM);
-        src[i] = reinterpret_cast<const char*>((pc ? g.a : g.w) + row * kBK);
-        hop[i] = (size_t)(pc ? 2 * g.Mp : g.Np) * kBK * 2;
+        const bool pc = R < P * BM;
+        if (pc || SCALED) {
+            const size_t row = pc ? (size_t)(R / BM) * g.Mp + m0 + R % BM : (size_t)(n0 + R - P * BM);
+            src[i] = reinterpret_cast<const char*>((pc ? g.a : g.w) + row * kBK) + 16 * lane;
+            hop[i] = (size_t)(pc ? P * g.Mp : g.Np) * kBK * 2;
+        } else {
+            const int j = n0 + R - P * BM + (lane >> 2);
+            const size_t row = weight_row(g.col0, g.F, min(j, g.N - 1));
+            src[i] = reinterpret_cast<const char*>(g.w + row * (size_t)(g.steps * kBK)) + 16 * ((lane & 3) ^ swizzle(lane >> 2));
+            hop[i] = kBK * 2;
+        }
         src[i] += s0 * hop[i];
     }
     const char* scp = reinterpret_cast<const char*>(g.sc + n0 + 64 * wn) + (size_t)s0 * g.Np * 4;
@@ -285,7 +234,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_rows(GemmArgs g) {
     auto request = [&](int buf) {
         char* dst = smem + buf * TL::kBytes;
 #pragma unroll
-        for (int i = 0; i < NI; ++i) load_to_lds(src[i] + 16 * lane, dst + 1024 * (NI * wave + i));
+        for (int i = 0; i < NI; ++i) load_to_lds(src[i], dst + 1024 * (NI * wave + i));
         if constexpr (SCALED) load4_to_lds(scp + 4 * lane, dst + TL::ROWS * 2 * kBK + 256 * wave);
         if (++ahead < S) {                         // uniform
 #pragma unroll
@@ -299,13 +248,13 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_rows(GemmArgs g) {
     // operand reads: lane (r, grp) takes unit grp of row R0 + r; R0 is a multiple of 16, so the unit's place is the
     // lane's alone
     const int at = 64 * r + 16 * (grp ^ swizzle(r));
-    const int at_a = at + 64 * 16 * TI * wm, at_b = at + 64 * (2 * BM + 64 * wn);
+    const int at_a = at + 64 * 16 * TI * wm, at_b = at + 64 * (P * BM + 64 * wn);
     const int at_s = TL::ROWS * 2 * kBK + 256 * wave + 4 * r;
     auto rd = [&](const char* p) { return *reinterpret_cast<const u32x4*>(p); };
     // the sums in the making: of one group of sixteen rows and the one before (SCALED), or of every group (two stages)
     constexpr int ND = SCALED ? 2 : TI;
     f32x4 acc[TI][4], d[ND][4];
-    u32x4 b[4], bn[4], h[2], l[2];
+    u32x4 b[4], bn[4], x[2][P];
     float f[4], fn[4], fd[4];                      // scales: of this stage, of the next, of d[1]'s stage
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
@@ -315,8 +264,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_rows(GemmArgs g) {
         for (int i = 0; i < TI; ++i) acc[i][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
     }
     // a stage's sums (a pair of stages' where no scales stand between them) start from zero and join the running ones by
-    // an fp32 addition (or fma): a third of the error of MFMAs on the running sums (1777 rows, bf16, K 6144: 2.0e-7 of the
-    // result against 7.1e-7; an fp32 GEMM: 1.4e-6)
+    // an fp32 addition (or fma): a third of the error of MFMAs on the running sums
     auto join = [&](f32x4 (&to)[4], const f32x4 (&from)[4], const float (&by)[4]) {
 #pragma unroll
         for (int t = 0; t < 4; ++t)
@@ -335,8 +283,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_rows(GemmArgs g) {
         b[t] = rd(smem + at_b + 1024 * t);
         if constexpr (SCALED) f[t] = *reinterpret_cast<const float*>(smem + at_s + 64 * t);
     }
-    h[0] = rd(smem + at_a);
-    l[0] = rd(smem + at_a + 64 * BM);
+#pragma unroll
+    for (int q = 0; q < P; ++q) x[0][q] = rd(smem + at_a + 64 * BM * q);
 
     int buf = 0;
     auto stage = [&](int s, auto odd_c) __attribute__((always_inline)) {
@@ -353,13 +301,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_rows(GemmArgs g) {
 #pragma unroll
         for (int i = 0; i < TI; ++i) {
             const int c = i & 1, o = c ^ 1, di = SCALED ? c : i;
-            if (i < TI - 1) {
-                h[o] = rd(cur + at_a + 1024 * (i + 1));
-                l[o] = rd(cur + at_a + 64 * BM + 1024 * (i + 1));
-            } else {
-                h[o] = rd(nxt + at_a);
-                l[o] = rd(nxt + at_a + 64 * BM);
-            }
+#pragma unroll
+            for (int q = 0; q < P; ++q) x[o][q] = rd((i < TI - 1 ? cur + 1024 * (i + 1) : nxt) + at_a + 64 * BM * q);
             if (i >= TI - 2) {
 #pragma unroll
                 for (int t = 2 * (i - TI + 2); t < 2 * (i - TI + 3); ++t) {
@@ -371,14 +314,16 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_rows(GemmArgs g) {
             if (i == 0 && (SCALED || !kOdd)) join(acc[TI - 1], d[ND - 1], fd);
 #pragma unroll
             for (int t = 0; t < 4; ++t)
-                d[di][t] = mfma_f16(l[c], b[t], kOdd ? d[di][t] : (f32x4){0.f, 0.f, 0.f, 0.f});
+                d[di][t] = mfma16x16x32(x[c][P - 1], b[t], kOdd ? d[di][t] : (f32x4){0.f, 0.f, 0.f, 0.f});
 #pragma unroll
-            for (int t = 0; t < 4; ++t) d[di][t] = mfma_f16(h[c], b[t], d[di][t]);
+            for (int q = P - 2; q >= 0; --q)
+#pragma unroll
+                for (int t = 0; t < 4; ++t) d[di][t] = mfma16x16x32(x[c][q], b[t], d[di][t]);
             if (i && (SCALED || kOdd)) join(acc[i - 1], d[SCALED ? o : i - 1], f);
-            if (i < TI - 2) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-            else __builtin_amdgcn_sched_group_barrier(0x100, SCALED ? 6 : 4, 0);
+            if (i < TI - 2) __builtin_amdgcn_sched_group_barrier(0x100, P, 0);
+            else __builtin_amdgcn_sched_group_barrier(0x100, P + (SCALED ? 4 : 2), 0);
 #pragma unroll
-            for (int q = 0; q < 8; ++q) {
+            for (int q = 0; q < 4 * P; ++q) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
             }
@@ -421,15 +366,15 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_rows(GemmArgs g) {
 #pragma unroll
                 for (int t = 0; t < 4; ++t) g.part[((size_t)blockIdx.y * g.M + m) * g.Np + n + 16 * t] = acc[i][t][e];
             } else {
-                gemm_store<SCALED, GLU>(g, m, n, acc[i][0][e], acc[i][1][e]);
-                gemm_store<SCALED, GLU>(g, m, n + 32, acc[i][2][e], acc[i][3][e]);
+                gemm_store<GLU>(g, m, n, acc[i][0][e], acc[i][1][e]);
+                gemm_store<GLU>(g, m, n + 32, acc[i][2][e], acc[i][3][e]);
             }
         }
     }
 }
 
 // The splits' sums of row blockIdx.y, in order; a thread per pair of columns 16 apart.
-template <bool SCALED, bool GLU>
+template <bool GLU>
 __global__ __launch_bounds__(256) void gemm_finish(GemmArgs g) {
     const int q = 256 * blockIdx.x + threadIdx.x, m = blockIdx.y;
     const int n = 32 * (q >> 4) + (q & 15);
@@ -441,13 +386,14 @@ __global__ __launch_bounds__(256) void gemm_finish(GemmArgs g) {
         v += p[0];
         u += p[16];
     }
-    gemm_store<SCALED, GLU>(g, m, n, v, u);
+    gemm_store<GLU>(g, m, n, v, u);
 }
 
 struct Layout {
-    int Mp, Np, steps, slab;       // slab: output columns expanded at a time; Np: its weight rows, in whole tiles
+    int Mp, Np, steps, slab;       // rows of x in whole tiles; slab: output columns at a time; Np: its weight rows, in
+                                   // whole tiles
     int form, S;                   // gemm_rows' tile: 0 128 x 256, 1 128 x 128, 2 64 x 128; K-splits
-    size_t pieces, ex, slab_w, slab_sc, ew, part, total;
+    size_t slab_w, slab_sc, part, total;
 };
 
 size_t up256(size_t n) { return (n + 255) / 256 * 256; }
@@ -457,24 +403,23 @@ int slab_rows(int cols, bool glu) { return glu ? (cols + 15) / 16 * 32 : cols; }
 
 Layout layout(int M, int N, int K, int w_type, bool glu) {
     Layout l;
+    l.steps = K / kBK + (w_type == RK_W_INT4 ? (K / kQB + 7) / 8 : 0);
     l.Mp = (M + 127) / 128 * 128;
-    l.steps = K / kBK + (w_type == RK_W_INT4 ? (K / 16 + kBK - 1) / kBK : 0);
     const int cols = glu ? N / 2 : N;
-    long long s = kSlabElems / (l.steps * kBK) / (glu ? 2 : 1) / 256 * 256;
-    if (s < 256) s = 256;
-    l.slab = s < cols ? (int)s : cols;
+    l.slab = cols;
+    if (w_type != RK_W_BF16) {
+        long long s = kSlabElems / (l.steps * kBK) / (glu ? 2 : 1) / 256 * 256;
+        if (s < 256) s = 256;
+        if (s < cols) l.slab = (int)s;
+    }
     const size_t rows = (size_t)slab_rows(l.slab, glu);
     l.Np = (int)up256(rows);
-    l.pieces = 0;
-    l.ex = (size_t)l.steps * 2 * l.Mp * kBK * 2;
-    l.slab_w = l.ex + up256((size_t)M * 4);
-    l.slab_sc = l.slab_w + (size_t)l.steps * l.Np * kBK * 2;
-    l.ew = l.slab_sc + (w_type == RK_W_BF16 ? 0 : (size_t)l.steps * l.Np * 4);
-    l.part = l.ew + up256(rows * 4);
+    l.slab_w = (size_t)l.Mp * l.steps * P * kBK * 2;
+    l.slab_sc = l.slab_w + (w_type == RK_W_BF16 ? 0 : (size_t)l.steps * l.Np * kBK * 2);
+    l.part = l.slab_sc + (w_type == RK_W_BF16 ? 0 : (size_t)l.steps * l.Np * 4);
     // 128 x 256 tiles where they give every CU two of them, else 128 x 128 (1777 x 2048 outputs: 112 tiles of 256
-    // columns leave half the CUs idle), else 64 x 128; eight waves of 32 x 64 beat four of 64 x 64 there (157 against
-    // 168 us in all at 1777 x 2048 x 6144: two waves per SIMD). Fewer than half as many tiles as CUs: K-splits of at least
-    // 16 steps, until the tiles fill the CUs (2048 columns, K 6144: 384 rows 133 -> 56 us, 256 rows 132 -> 45)
+    // columns leave half the CUs idle), else 64 x 128. Fewer than half as many tiles as CUs: K-splits of at least
+    // 16 steps, until the tiles fill the CUs
     int cus = device_cus();
     if (cus <= 0) cus = 256;
     auto tiles = [&](int bm, int bn) { return (long long)((M + bm - 1) / bm) * (((long long)rows + bn - 1) / bn); };
@@ -502,8 +447,7 @@ int launch_gemm(const GemmArgs& in, bool scaled, bool glu, hipStream_t s) {
     hipLaunchKernelGGL(fn, dim3((unsigned)(g.tm * g.tn), (unsigned)g.S), dim3(64 * WM * WN), lds, s, g);
     if (int rc = check_launch("gemm_rows")) return rc;
     if (g.S == 1) return RK_OK;
-    const auto fin = scaled ? (glu ? gemm_finish<true, true> : gemm_finish<true, false>)
-                            : (glu ? gemm_finish<false, true> : gemm_finish<false, false>);
+    const auto fin = glu ? gemm_finish<true> : gemm_finish<false>;
     hipLaunchKernelGGL(fin, dim3((unsigned)((g.Np / 2 + 255) / 256), (unsigned)g.M), dim3(256), 0, s, g);
     return check_launch("gemm_finish");
 }
@@ -545,27 +489,29 @@ int rk_linear_gemm(float* y, const float* x, long long x_ld, int M, int N, int K
     const Layout l = layout(M, N, K, w_type, glu != 0);
     char* ws = static_cast<char*>(workspace);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    uint16_t* pieces = reinterpret_cast<uint16_t*>(ws + l.pieces);
-    int* ex = reinterpret_cast<int*>(ws + l.ex);
+    uint16_t* pieces = reinterpret_cast<uint16_t*>(ws);
     const auto split = w_type == RK_W_INT4 ? split_rows<true> : split_rows<false>;
-    hipLaunchKernelGGL(split, dim3((unsigned)M), dim3(256), 0, st, pieces, ex, x, x_ld, l.Mp, K, l.steps);
-    if (int rc = check_launch("split_rows")) return rc;
     const int cols = glu ? N / 2 : N;
+    hipLaunchKernelGGL(split, dim3((unsigned)M), dim3(256), 0, st, pieces, x, x_ld, l.Mp, K, l.steps);
+    if (int rc = check_launch("split_rows")) return rc;
     for (int c0 = 0; c0 < cols; c0 += l.slab) {
         const int nc = l.slab < cols - c0 ? l.slab : cols - c0;
-        SlabArgs sa{};
-        sa.out = reinterpret_cast<uint16_t*>(ws + l.slab_w);
-        sa.sc = reinterpret_cast<float*>(ws + l.slab_sc);
-        sa.ew = reinterpret_cast<int*>(ws + l.ew);
-        sa.w = w; sa.scales = static_cast<const uint16_t*>(scales); sa.mins = static_cast<const uint16_t*>(mins);
-        sa.Np = l.Np; sa.row0 = c0; sa.K = K; sa.steps = l.steps; sa.F = glu ? cols : 0;
         const int rows = slab_rows(nc, glu != 0);
-        const auto expand = w_type == RK_W_BF16 ? slab_weights<RK_W_BF16>
-                            : w_type == RK_W_INT8 ? slab_weights<RK_W_INT8> : slab_weights<RK_W_INT4>;
-        hipLaunchKernelGGL(expand, dim3((unsigned)rows), dim3(256), 0, st, sa);
-        if (int rc = check_launch("slab_weights")) return rc;
         GemmArgs g{};
-        g.y = y; g.a = pieces; g.w = sa.out; g.sc = sa.sc; g.ex = ex; g.ew = sa.ew; g.bias = bias; g.res = residual;
+        g.w = static_cast<const uint16_t*>(w);
+        g.F = glu ? cols : 0;
+        if (quant) {
+            SlabArgs sa{};
+            sa.out = reinterpret_cast<uint16_t*>(ws + l.slab_w);
+            sa.sc = reinterpret_cast<float*>(ws + l.slab_sc);
+            sa.w = w; sa.scales = static_cast<const uint16_t*>(scales); sa.mins = static_cast<const uint16_t*>(mins);
+            sa.Np = l.Np; sa.row0 = c0; sa.K = K; sa.steps = l.steps; sa.F = g.F;
+            const auto expand = w_type == RK_W_INT8 ? slab_weights<RK_W_INT8> : slab_weights<RK_W_INT4>;
+            hipLaunchKernelGGL(expand, dim3((unsigned)rows), dim3(256), 0, st, sa);
+            if (int rc = check_launch("slab_weights")) return rc;
+            g.w = sa.out; g.sc = sa.sc;
+        }
+        g.y = y; g.a = pieces; g.bias = bias; g.res = residual;
         g.y_ld = cols; g.M = M; g.N = rows; g.Mp = l.Mp; g.Np = l.Np; g.steps = l.steps; g.col0 = c0; g.cols = cols;
         g.S = l.S;
         g.part = reinterpret_cast<float*>(ws + l.part);

@@ -4,29 +4,26 @@
 // launches, so W is read once, as stored, straight into MFMA operands, and the whole chip shares it: a workgroup takes
 // 16 NT weight rows and one K-split, its eight waves an eighth of the split each, and every wave multiplies its blocks
 // with all the activation rows of a row block (48 or 64). The activations come as operand-ready pieces from memory
-// (the L2s hold them: 4 bytes per value, 0.5 MB for 64 x 2048), written once by split_operands; they pass through no
-// LDS, since no two waves of a workgroup use the same ones. INT8 / INT4: two fp16 pieces, codes exact in fp16, a
-// block's scale on the VALU, INT4 mins and 8 scales as one more MFMA per 8 blocks; bf16: three bf16 pieces
-// (exact), so that W needs no conversion. The waves' sums meet in LDS; K-splits meet in memory, added in order by
-// mid_finish.
+// (the L2s hold them: 6 bytes per value, 0.8 MB for 64 x 2048), written once by split_operands; they pass through no
+// LDS, since no two waves of a workgroup use the same ones. Operands are linear_operands.h's: three bf16 pieces of every
+// activation and the weights, all exact. A block's scale multiplies its sums on the VALU; an INT4 weight is
+// s (q - 8) + (8 s + min), whose second term, times the block's activation sum, is one more MFMA per 4 blocks. The
+// waves' sums meet in LDS; K-splits meet in memory, added in order by mid_finish.
 //
-// Measured (64 rows, INT4, all launches): 12288 x 2048 with silu * up 23 us, 2048 x 6144 23 us (gemm_rows 45 and 36, the
-// fp32 GEMM on the expanded weight 100 and 110); mid_rows itself 20.6 and 15.4 us in a trace. The mins on the VALU, four
-// fmas a block and tile, had cost 10 of 55 us for the two; one chunk of weights in flight instead of two 2.
-#include "fp16_pieces.h"
+// Measured (64 rows, INT4, all launches): 12288 x 2048 with silu * up 26 us, 2048 x 6144 28 us (gemm_rows 48 and 37, the
+// fp32 GEMM on the expanded weight 100 and 110; two fp16 pieces of x 23 and 23).
+#include "linear_operands.h"
 
 namespace rk {
 namespace {
 
 constexpr int kWaves = 8;
-
-template <int WT> constexpr int pieces_of() { return WT == RK_W_BF16 ? 3 : 2; }
+constexpr int P = 3;               // pieces of an activation
 
 struct MidArgs {
     float* y;
     const uint16_t* a;             // [row block][K / 32][piece][MT][64 lanes][8]: MFMA operands
-    const uint16_t* sums;          // INT4: [row block][K / 64][16 MT rows][2 blocks][4] block sums (split_operands)
-    const int* ex;                 // [M] exponents (INT8 / INT4)
+    const uint16_t* sums;          // INT4: [row block][K / 32][MT][16 rows][8] block sums (split_operands)
     const void* w;
     const uint16_t* scales;
     const uint16_t* mins;
@@ -39,18 +36,15 @@ struct MidArgs {
 };
 
 // Row m of x as operands of the row block m / (16 MT): lane (r, g) of tile i takes row 16 i + r's values 8g .. 8g + 7
-// of a block. fp16 pairs of x * 2^ex (INT4: in the order of int4_f16) or bf16 thirds. INT4: also each block's sum b of the
-// scaled values, as the fp16 pieces (b hi, 8 b hi, b lo, 8 b lo) * 2^-kSumShift, against (min, scale, min, scale).
-constexpr int kSumShift = 8;
+// of a block, in three pieces (INT4: in the order of int4_bf16). INT4: also each block's sum, in pieces b1 b2 b3 as
+// (b1, b1, b1, b2, b2, b2, b3, b3), against the pieces of 8 s + min as (c1, c2, c3, c1, c2, c3, c1, c2): all products but
+// the last, 2^-32 of the whole.
 template <int WT, int MT>
-__global__ __launch_bounds__(256) void split_operands(uint16_t* a, uint16_t* sums, int* ex, const float* x, long long x_ld,
-                                                      int K) {
-    constexpr int P = pieces_of<WT>();
-    __shared__ float red[4];
+__global__ __launch_bounds__(256) void split_operands(uint16_t* a, uint16_t* sums, const float* x, long long x_ld, int K) {
     const int m = blockIdx.x, tid = threadIdx.x;
     const int mb = m / (16 * MT), i = m % (16 * MT) / 16, r = m % 16, nblk = K / kQB;
     const float* xr = x + (size_t)m * x_ld;
-    // a thread's first kHeld groups of 8 values stay in registers (rows of up to 8192: read once, all at the start)
+    // a thread's first kHeld groups of 8 values are requested together
     constexpr int kHeld = 4;
     f32x4 held[kHeld][2];
 #pragma unroll
@@ -59,44 +53,16 @@ __global__ __launch_bounds__(256) void split_operands(uint16_t* a, uint16_t* sum
         held[j][0] = *reinterpret_cast<const f32x4*>(p);
         held[j][1] = *reinterpret_cast<const f32x4*>(p + 4);
     }
-    int k = 0;
-    if constexpr (WT != RK_W_BF16) {
-        float big = 0.0f;
-#pragma unroll
-        for (int j = 0; j < kHeld; ++j)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) big = fmaxf(big, fmaxf(fabsf(held[j][0][e]), fabsf(held[j][1][e])));
-        for (int c = tid + 256 * kHeld; c < K / 8; c += 256) {
-            const f32x4 v0 = *reinterpret_cast<const f32x4*>(xr + 8 * c), v1 = *reinterpret_cast<const f32x4*>(xr + 8 * c + 4);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) big = fmaxf(big, fmaxf(fabsf(v0[e]), fabsf(v1[e])));
-        }
-        k = top_exponent(block_absmax(big, red));
-        if (tid == 0) ex[m] = k;
-    }
     auto put = [&](int c, f32x4 v0, f32x4 v1) __attribute__((always_inline)) {
-        float v[8];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            v[e] = WT == RK_W_BF16 ? v0[e] : ldexpf(v0[e], k);
-            v[4 + e] = WT == RK_W_BF16 ? v1[e] : ldexpf(v1[e], k);
-        }
+        const float v[8] = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
         u32x4 pc[P];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const int e0 = WT == RK_W_INT4 ? q : 2 * q, e1 = WT == RK_W_INT4 ? q + 4 : 2 * q + 1;
-            if constexpr (WT == RK_W_BF16) {
-                Split3 s0 = split3(v[e0]), s1 = split3(v[e1]);
-                if (!__builtin_isfinite(v[e0])) s0.mid = s0.lo = 0u;   // an infinity has no rest
-                if (!__builtin_isfinite(v[e1])) s1.mid = s1.lo = 0u;
-                pc[0][q] = pack_hi2(s0.hi, s1.hi);
-                pc[1][q] = pack_hi2(s0.mid, s1.mid);
-                pc[2][q] = pack_hi2(s0.lo, s1.lo);
-            } else {
-                const Pieces p = split_pair(v[e0], v[e1]);
-                pc[0][q] = p.hi;
-                pc[1][q] = rest_of(p);
-            }
+            const Split3 s0 = split3_any(v[WT == RK_W_INT4 ? kInt4Order[q][0] : 2 * q]);
+            const Split3 s1 = split3_any(v[WT == RK_W_INT4 ? kInt4Order[q][1] : 2 * q + 1]);
+            pc[0][q] = pack_hi2(s0.hi, s1.hi);
+            pc[1][q] = pack_hi2(s0.mid, s1.mid);
+            pc[2][q] = pack_hi2(s0.lo, s1.lo);
         }
         const size_t blk = (size_t)mb * nblk + (c >> 2);
 #pragma unroll
@@ -109,17 +75,15 @@ __global__ __launch_bounds__(256) void split_operands(uint16_t* a, uint16_t* sum
             sum += dpp_f32<0xb1>(sum);             // lane ^ 1
             sum += dpp_f32<0x4e>(sum);             // lane ^ 2
             if ((c & 3) == 0) {
-                const Pieces p = split_pair(ldexpf(sum, -kSumShift), 0.0f);
-                const float h = half_to_f32(p.hi & 0xffffu), l = half_to_f32(rest_of(p) & 0xffffu);
-                const size_t pair = (size_t)mb * (nblk / 2) + (c >> 3);
-                *reinterpret_cast<u32x2*>(sums + (pair * (16 * MT) + 16 * i + r) * 8 + 4 * ((c >> 2) & 1)) =
-                    (u32x2){pack_f16(h, 8.0f * h), pack_f16(l, 8.0f * l)};
+                const Split3 b = split3_any(sum);
+                *reinterpret_cast<u32x4*>(sums + ((blk * MT + i) * 16 + r) * 8) =
+                    (u32x4){pack_hi2(b.hi, b.hi), pack_hi2(b.hi, b.mid), pack_hi2(b.mid, b.mid), pack_hi2(b.lo, b.lo)};
             }
         }
     };
 #pragma unroll
     for (int j = 0; j < kHeld; ++j)
-        if (tid + 256 * j < K / 8) put(tid + 256 * j, held[j][0], held[j][1]);   // the four threads of a block together
+        if (tid + 256 * j < K / 8) put(tid + 256 * j, held[j][0], held[j][1]);
     for (int c = tid + 256 * kHeld; c < K / 8; c += 256)
         put(c, *reinterpret_cast<const f32x4*>(xr + 8 * c), *reinterpret_cast<const f32x4*>(xr + 8 * c + 4));
 }
@@ -131,16 +95,12 @@ __device__ __forceinline__ size_t mid_row(const MidArgs& a, int lr) {
     return (size_t)((lr & 8) ? F + f : f);
 }
 
-// rows 4g .. 4g + 3 of tile i, column c of tile t (lane l = 16 g + c of item (i, t)): powers of two, bias, residual or
-// silu * up, store; whole waves enter
-template <int WT, int MT, int NT>
+// rows 4g .. 4g + 3 of tile i, column c of tile t (lane l = 16 g + c of item (i, t)): bias, residual or silu * up, store;
+// whole waves enter
+template <int MT, int NT>
 __device__ __forceinline__ void mid_store(const MidArgs& a, f32x4 v, int mb, int rg, int item) {
     const int i = item / (64 * NT), t = item / 64 % NT, l = item & 63, c = l & 15;
     const int m0 = 16 * MT * mb + 16 * i + 4 * (l >> 4);
-    if constexpr (WT != RK_W_BF16) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = ldexpf(v[e], -a.ex[min(m0 + e, a.M - 1)]);
-    }
     if (a.glu) {                                   // uniform
         f32x4 u;
 #pragma unroll
@@ -165,48 +125,12 @@ __device__ __forceinline__ void mid_store(const MidArgs& a, f32x4 v, int mb, int
     }
 }
 
-// 4 x 4 transpose over the wave's 16-lane groups: register d of group g <- register g of group d
-__device__ __forceinline__ u32x4 xpose4(uint32_t a0, uint32_t a1, uint32_t a2, uint32_t a3) {
-    const auto s02 = __builtin_amdgcn_permlane32_swap(a0, a2, false, false);
-    const auto s13 = __builtin_amdgcn_permlane32_swap(a1, a3, false, false);
-    const auto s01 = __builtin_amdgcn_permlane16_swap(s02[0], s13[0], false, false);
-    const auto s23 = __builtin_amdgcn_permlane16_swap(s02[1], s13[1], false, false);
-    return (u32x4){s01[0], s01[1], s23[0], s23[1]};
-}
-
-// 8 INT4 codes minus 8 as fp16, in the order 0 4 1 5 2 6 3 7: a code q as the low bits of 0x6400 is the fp16 value
-// 1024 + q; the subtraction is exact
-__device__ __forceinline__ u32x4 int4_f16(uint32_t v) {
-    const f16x2 off = {(_Float16)1032.0f, (_Float16)1032.0f};
-    u32x4 o;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const uint32_t p = (v >> (4 * q) & 0x000F000Fu) | 0x64006400u;
-        o[q] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, p) - off);
-    }
-    return o;
-}
-
-// 8 INT8 codes as fp16: q + 128 as the low byte of 0x6400 is the fp16 value 1152 + q; the subtraction is exact
-__device__ __forceinline__ u32x4 int8_f16(uint32_t lo, uint32_t hi) {
-    const f16x2 off = {(_Float16)1152.0f, (_Float16)1152.0f};
-    u32x4 o;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const uint32_t u = (q < 2 ? lo : hi) ^ 0x80808080u;
-        const uint32_t p = __builtin_amdgcn_perm(0x64646464u, u, q & 1 ? 0x04030402u : 0x04010400u);
-        o[q] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, p) - off);
-    }
-    return o;
-}
-
 // One workgroup per (row group, K-split, row block). A wave walks its blocks four at a time (a chunk: 16-byte weight
 // loads of whole blocks, transposed over the lane groups as in linear.hip), the next chunk's weights and scales and the
 // next block's activations requested ahead. Chunks past the wave's range repeat loaded addresses and enter with
 // weight 0, so the loop body has no branch.
 template <int WT, int MT, int NT>
 __global__ __launch_bounds__(64 * kWaves) void mid_rows(MidArgs a) {
-    constexpr int P = pieces_of<WT>();
     constexpr int CH = WT == RK_W_INT4 ? 1 : WT == RK_W_INT8 ? 2 : 4;   // 16-byte loads per tile and chunk
     constexpr bool QUANT = WT != RK_W_BF16;
     extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -231,9 +155,10 @@ __global__ __launch_bounds__(64 * kWaves) void mid_rows(MidArgs a) {
         if constexpr (QUANT) srow[t] = a.scales + n * nblk;
         if constexpr (WT == RK_W_INT4) mrow[t] = a.mins + n * nblk;
     }
-    constexpr int DEPTH = WT == RK_W_INT4 ? 2 : 1;   // chunks of weights in flight
+    constexpr int DEPTH = WT == RK_W_INT4 && MT * NT < 12 ? 2 : 1;   // chunks of weights in flight (as registers allow)
     u32x4 wn[DEPTH][NT][CH];
     uint32_t sn[DEPTH][QUANT ? NT : 1][2];
+    uint16_t mn[DEPTH][WT == RK_W_INT4 ? NT : 1];  // min of the lane group's own block of the chunk
     auto load_w = [&](int kb, int set) __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
@@ -251,6 +176,7 @@ __global__ __launch_bounds__(64 * kWaves) void mid_rows(MidArgs a) {
                     sn[set][t][h] = *reinterpret_cast<const uint32_t*>(srow[t] + min(kb + 2 * h, nblk - 2));
                 }
             }
+            if constexpr (WT == RK_W_INT4) mn[set][t] = mrow[t][min(kb + grp, nblk - 1)];
         }
     };
     u32x4 xa[2][P][MT];
@@ -273,36 +199,11 @@ __global__ __launch_bounds__(64 * kWaves) void mid_rows(MidArgs a) {
 #pragma unroll
         for (int i = 0; i < DEPTH; ++i) load_w(min(k0 + 4 * i, k_last), i);
         load_x(k0, 0);
-        // INT4 is s (q - 8) + (8 s + min): the second terms of 8 blocks are one MFMA per tile, with the block sums' pieces
-        // against (min, s) pairs, whose near-equal products of opposite sign cancel inside it
-        if constexpr (WT == RK_W_INT4) {
-            for (int kb = k0; kb < k1; kb += 8) {
-                const int kp = kb + 2 * grp;       // the lane group's two blocks
-                const int kc = min(kp, nblk - 2);
-                const uint32_t in = kp < k1 ? 0xffffffffu : 0u;   // k0 and k1 are even
-                u32x4 sa[MT];
-#pragma unroll
-                for (int i = 0; i < MT; ++i)
-                    sa[i] = *reinterpret_cast<const u32x4*>(a.sums + (((size_t)mb * (nblk / 2) + kc / 2) * (16 * MT) + 16 * i + r) * 8);
-#pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    const uint32_t m = *reinterpret_cast<const uint32_t*>(mrow[t] + kc) & in;
-                    const uint32_t f = *reinterpret_cast<const uint32_t*>(srow[t] + kc) & in;
-                    const uint32_t b0 = __builtin_amdgcn_perm(f, m, 0x05040100u), b1 = __builtin_amdgcn_perm(f, m, 0x07060302u);
-                    const u32x4 b = {b0, b0, b1, b1};
-#pragma unroll
-                    for (int i = 0; i < MT; ++i) {
-                        const f32x4 p = mfma_f16(sa[i], b, (f32x4){0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) acc[i][t][e] = fmaf((float)(1 << kSumShift), p[e], acc[i][t][e]);
-                    }
-                }
-            }
-        }
     }
     for (int kc = k0; kc < k1; kc += 4) {
         u32x4 wc[NT][CH];
         uint32_t sc[QUANT ? NT : 1][2];
+        uint16_t mc[WT == RK_W_INT4 ? NT : 1];
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
             if constexpr (WT == RK_W_INT4) wc[t][0] = xpose4(wn[0][t][0][0], wn[0][t][0][1], wn[0][t][0][2], wn[0][t][0][3]);
@@ -319,6 +220,7 @@ __global__ __launch_bounds__(64 * kWaves) void mid_rows(MidArgs a) {
 #pragma unroll
                 for (int h = 0; h < 2; ++h) sc[t][h] = sn[0][t][h];
             }
+            if constexpr (WT == RK_W_INT4) mc[t] = mn[0][t];
             if constexpr (DEPTH == 2) {
 #pragma unroll
                 for (int c = 0; c < CH; ++c) wn[0][t][c] = wn[1][t][c];
@@ -326,9 +228,17 @@ __global__ __launch_bounds__(64 * kWaves) void mid_rows(MidArgs a) {
 #pragma unroll
                     for (int h = 0; h < 2; ++h) sn[0][t][h] = sn[1][t][h];
                 }
+                if constexpr (WT == RK_W_INT4) mn[0][t] = mn[1][t];
             }
         }
         load_w(min(kc + 4 * DEPTH, k_last), DEPTH - 1);
+        u32x4 bs[WT == RK_W_INT4 ? MT : 1];
+        if constexpr (WT == RK_W_INT4) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+                bs[i] = *reinterpret_cast<const u32x4*>(
+                    a.sums + ((((size_t)mb * nblk + min(kc + grp, nblk - 1)) * MT + i) * 16 + r) * 8);
+        }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
@@ -339,17 +249,16 @@ __global__ __launch_bounds__(64 * kWaves) void mid_rows(MidArgs a) {
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
                 u32x4 b;
-                if constexpr (WT == RK_W_INT4) b = int4_f16(wc[t][0][d]);
-                else if constexpr (WT == RK_W_INT8) b = int8_f16(wc[t][d >> 1][2 * (d & 1)], wc[t][d >> 1][2 * (d & 1) + 1]);
+                if constexpr (WT == RK_W_INT4) b = int4_bf16_centred(wc[t][0][d]);
+                else if constexpr (WT == RK_W_INT8) b = int8_bf16(wc[t][d >> 1][2 * (d & 1)], wc[t][d >> 1][2 * (d & 1) + 1]);
                 else b = wc[t][d] & (u32x4){in, in, in, in};
                 float f = 0.0f;
-                if constexpr (QUANT) f = half_to_f32((sc[t][d >> 1] & in) >> (16 * (d & 1)));
+                if constexpr (QUANT) f = half_to_f32((uint16_t)((sc[t][d >> 1] & in) >> (16 * (d & 1))));
 #pragma unroll
                 for (int i = 0; i < MT; ++i) {
                     f32x4 p = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                    for (int q = P - 1; q >= 0; --q)
-                        p = QUANT ? mfma_f16(xa[s][q][i], b, p) : mfma16x16x32(xa[s][q][i], b, p);
+                    for (int q = P - 1; q >= 0; --q) p = mfma16x16x32(xa[s][q][i], b, p);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         if constexpr (QUANT) acc[i][t][e] = fmaf(f, p[e], acc[i][t][e]);
@@ -358,6 +267,19 @@ __global__ __launch_bounds__(64 * kWaves) void mid_rows(MidArgs a) {
                 }
             }
             __builtin_amdgcn_sched_barrier(0);     // one block ahead: more in flight does not fit the registers
+        }
+        if constexpr (WT == RK_W_INT4) {           // 8 s + min of the lane group's block, in the pieces that meet its sum's
+            const uint32_t in = kc + grp < k1 ? 0xffffffffu : 0u;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                const uint64_t s4 = (uint64_t)sc[t][1] << 32 | sc[t][0];
+                const float c = fmaf(8.0f, half_to_f32((uint16_t)(s4 >> (16 * grp))), half_to_f32(mc[t]));
+                const Split3 p = split3(__uint_as_float(__float_as_uint(c) & in));
+                const u32x4 b = {pack_hi2(p.hi, p.mid), pack_hi2(p.lo, p.hi), pack_hi2(p.mid, p.lo), pack_hi2(p.hi, p.mid)};
+#pragma unroll
+                for (int i = 0; i < MT; ++i) acc[i][t] = mfma16x16x32(bs[i], b, acc[i][t]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
     }
 
@@ -377,13 +299,13 @@ __global__ __launch_bounds__(64 * kWaves) void mid_rows(MidArgs a) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] += o[e];
         }
-        if (a.S == 1) mid_store<WT, MT, NT>(a, v, mb, rg, item);
+        if (a.S == 1) mid_store<MT, NT>(a, v, mb, rg, item);
         else a.part[((size_t)(mb * a.G + rg) * a.S + sp) * ITEMS + item] = v;
     }
 }
 
 // The splits of one (row block, row group, wave of items), in order.
-template <int WT, int MT, int NT>
+template <int MT, int NT>
 __global__ __launch_bounds__(256) void mid_finish(MidArgs a) {
     constexpr int ITEMS = 64 * MT * NT;
     const int item = 256 * blockIdx.y + threadIdx.x;
@@ -395,34 +317,30 @@ __global__ __launch_bounds__(256) void mid_finish(MidArgs a) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] += o[e];
     }
-    mid_store<WT, MT, NT>(a, v, blockIdx.x / a.G, blockIdx.x % a.G, item);
+    mid_store<MT, NT>(a, v, blockIdx.x / a.G, blockIdx.x % a.G, item);
 }
 
 struct MidPlan {
     int MB, MT, NT, G, S, SB, WB;
-    size_t sums, ex, part, total;
+    size_t sums, part, total;
 };
 
-// Rows up to which this form is the faster one (12288 x 2048 with silu * up, 2048 x 6144, 8224 x 2048; us, this form
-// against gemm_rows): INT4 at 192 rows 60 / 40 / 58 against 74 / 44 / 67 and at 256 rows 80 / 42 / 61 against
-// 73 / 47 / 68; INT8 at 256 rows 69 / 41 / 56 against 74 / 44 / 66 and at 384 rows 111 / 59 / 84 against 109 / 54 / 68;
-// bf16 (three pieces and two bytes of W per value here) at 96 rows 46 / 29 / 43 against 51 / 37 / 39 and at 128 rows
-// 54 / 33 / 50 against 52 / 38 / 41.
-int mid_rows_max(int w_type) { return w_type == RK_W_INT8 ? 256 : w_type == RK_W_INT4 ? 192 : 96; }
+// Rows up to which this form is the faster one
+int mid_rows_max(int w_type) { return w_type == RK_W_BF16 ? 96 : 256; }
 
 // NT, S: the least estimated time over the rounds of one workgroup per CU: a block costs a wave its activations from
 // the L2 (1 KB per 16 cycles and CU) or its MFMAs (19 cycles each, two waves per SIMD), whichever is longer, a
 // workgroup a start and an end, a split its partials
 MidPlan mid_plan(int M, int N, int K, int w_type, int glu) {
     MidPlan p{};
-    const int nblk = K / kQB, P = w_type == RK_W_BF16 ? 3 : 2;
+    const int nblk = K / kQB;
     const int tiles = glu ? (N / 2 + 7) / 8 : (N + 15) / 16;
     p.MB = (M + 63) / 64;
     p.MT = (M + 16 * p.MB - 1) / (16 * p.MB) <= 3 ? 3 : 4;
     int cus = device_cus();
     if (cus <= 0) cus = 256;
     double best = 0;
-    for (int nt = 1; nt <= (w_type == RK_W_BF16 ? 2 : w_type == RK_W_INT4 && p.MT == 4 ? 3 : 4); ++nt)
+    for (int nt = 1; nt <= (w_type == RK_W_BF16 ? 2 : p.MT == 4 ? 3 : 4); ++nt)   // as the registers hold
         for (int s = 1; s <= 16 && s <= (nblk + 31) / 32 * 2; ++s) {
             const int sb = ((nblk + s - 1) / s + 1) / 2 * 2;
             const int wb = ((sb + kWaves - 1) / kWaves + 1) / 2 * 2;
@@ -439,8 +357,7 @@ MidPlan mid_plan(int M, int N, int K, int w_type, int glu) {
     const size_t rows = (size_t)p.MB * 16 * p.MT;
     auto up = [](size_t n) { return (n + 255) / 256 * 256; };
     p.sums = up(rows * K * 2 * P);
-    p.ex = p.sums + (w_type == RK_W_INT4 ? up(rows * nblk * 8) : 0);
-    p.part = p.ex + up(rows * 4);
+    p.part = p.sums + (w_type == RK_W_INT4 ? up(rows * nblk * 16) : 0);
     p.total = p.part + (p.S > 1 ? (size_t)p.MB * p.G * p.S * 64 * p.MT * p.NT * sizeof(f32x4) : 0);
     return p;
 }
@@ -462,13 +379,12 @@ int mid_linear(float* y, const float* x, long long x_ld, int M, int N, int K, co
     char* ws = static_cast<char*>(workspace);
     uint16_t* ops = reinterpret_cast<uint16_t*>(ws);
     uint16_t* sums = reinterpret_cast<uint16_t*>(ws + p.sums);
-    int* ex = reinterpret_cast<int*>(ws + p.ex);
     MidArgs a{};
-    a.y = y; a.a = ops; a.sums = sums; a.ex = ex; a.w = w;
+    a.y = y; a.a = ops; a.sums = sums; a.w = w;
     a.scales = static_cast<const uint16_t*>(scales); a.mins = static_cast<const uint16_t*>(mins);
     a.bias = bias; a.res = residual; a.part = reinterpret_cast<f32x4*>(ws + p.part);
     a.M = M; a.N = N; a.K = K; a.S = p.S; a.SB = p.SB; a.WB = p.WB; a.MB = p.MB; a.G = p.G; a.glu = glu ? 1 : 0;
-    using Split = void (*)(uint16_t*, uint16_t*, int*, const float*, long long, int);
+    using Split = void (*)(uint16_t*, uint16_t*, const float*, long long, int);
     using Fn = void (*)(MidArgs);
     Split split = nullptr;
     Fn rows = nullptr, fin = nullptr;
@@ -476,17 +392,17 @@ int mid_linear(float* y, const float* x, long long x_ld, int M, int N, int K, co
     if (w_type == W && p.MT == T && p.NT == C) {                                                               \
         split = split_operands<W, T>;                                                                          \
         rows = mid_rows<W, T, C>;                                                                              \
-        fin = mid_finish<W, T, C>;                                                                             \
+        fin = mid_finish<T, C>;                                                                                \
     }
 #define RK_MIDS(T)                                                                                             \
     RK_MID(RK_W_INT4, T, 1) RK_MID(RK_W_INT4, T, 2) RK_MID(RK_W_INT4, T, 3)                                    \
-    RK_MID(RK_W_INT8, T, 1) RK_MID(RK_W_INT8, T, 2) RK_MID(RK_W_INT8, T, 3) RK_MID(RK_W_INT8, T, 4)            \
+    RK_MID(RK_W_INT8, T, 1) RK_MID(RK_W_INT8, T, 2) RK_MID(RK_W_INT8, T, 3)                                    \
     RK_MID(RK_W_BF16, T, 1) RK_MID(RK_W_BF16, T, 2)
-    RK_MIDS(3) RK_MIDS(4) RK_MID(RK_W_INT4, 3, 4)
+    RK_MIDS(3) RK_MIDS(4) RK_MID(RK_W_INT4, 3, 4) RK_MID(RK_W_INT8, 3, 4)
 #undef RK_MIDS
 #undef RK_MID
     if (!rows) return fail(RK_ERR_ARG, "rk_linear_gemm: no kernel for %d x %d tiles", p.MT, p.NT);
-    hipLaunchKernelGGL(split, dim3((unsigned)M), dim3(256), 0, stream, ops, sums, ex, x, x_ld, K);
+    hipLaunchKernelGGL(split, dim3((unsigned)M), dim3(256), 0, stream, ops, sums, x, x_ld, K);
     if (int rc = check_launch("split_operands")) return rc;
     const size_t lds = (size_t)kWaves * 64 * p.MT * p.NT * sizeof(f32x4);
     if (int rc = allow_dynamic_lds((const void*)rows, lds)) return rc;

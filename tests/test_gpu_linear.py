@@ -288,6 +288,65 @@ def test_many_row_linears_against_64_bits(backend, kind, M, N, K, glu):
     assert over < 1.0
 
 
+@pytest.mark.parametrize("kind", ["bf16", "int8", "int4"])
+@pytest.mark.parametrize("M,N,K", [(48, 200, 256), (90, 100, 1088), (300, 500, 288), (700, 130, 192)])
+def test_many_row_linears_take_every_bit(backend, kind, M, N, K):
+    """Activations and bf16 weights enter with all their bits, however far below the others of their row they are: rows
+    of the weight that pick one value each give it back exactly, and so do activations that pick one weight each."""
+    g = torch.Generator().manual_seed(M + K)
+    wide = lambda *s: torch.randn(*s, generator=g) * torch.exp2(torch.randint(-60, 40, s, generator=g).float())
+    pick = torch.randint(0, K, (N,), generator=g)
+    one = torch.zeros(N, K).scatter_(1, pick[:, None], 1.0)
+    if kind == "bf16":
+        w = one.bfloat16()
+    elif kind == "int8":
+        w = quant.QuantTensor("int8", one.to(torch.int8), torch.ones(N, K // 32).half(), (N, K))
+    else:                                               # 1 * code - 8
+        code = (8 + one).to(torch.uint8)
+        w = quant.QuantTensor("int4", code[:, 0::2] | code[:, 1::2] << 4, torch.ones(N, K // 32).half(), (N, K),
+                              mins=torch.full((N, K // 32), -8.0).half())
+    x = wide(M, K)
+    assert torch.equal(backend.linear(x.to(DEV), to_dev(w)).cpu(), x[:, pick])
+    if kind == "bf16":
+        w, at = wide(N, K).bfloat16(), torch.randint(0, K, (M,), generator=g)
+        x = torch.zeros(M, K).scatter_(1, at[:, None], 1.0)
+        assert torch.equal(backend.linear(x.to(DEV), w.to(DEV)).cpu(), w.float()[:, at].T)
+
+
+@pytest.mark.parametrize("kind", ["bf16", "int8", "int4"])
+@pytest.mark.parametrize("M,glu", [(64, False), (90, True), (300, False), (1000, True)])
+def test_many_row_linears_over_channels_of_different_size(backend, kind, M, glu):
+    """Blocks of channels whose activations are 2^e times the others' and whose weights 2^-e times, so that every channel
+    counts alike. Bound as in test_many_row_linears_against_64_bits."""
+    N, K = 400, 512
+    w, _ = weight(kind, N, K, M)
+    g = torch.Generator().manual_seed(M)
+    e = torch.randint(-8, 19, (K // 32,), generator=g).float()
+    if kind == "bf16":
+        e = 2 * e
+        w = (w.float() * torch.exp2(e).repeat_interleave(32)).bfloat16()
+        deq = w.float()
+    else:
+        w.scales = (w.scales.float() * torch.exp2(e)).half()
+        w.mins = None if w.mins is None else (w.mins.float() * torch.exp2(e)).half()
+        deq = quant_ref.dequantize(w.scheme, w.data, w.scales, w.mins)
+    assert torch.isfinite(deq).all()
+    x = torch.randn(M, K, generator=g) * torch.exp2(-e).repeat_interleave(32)
+    want = x.double() @ deq.double().T
+    bound = (x.double().abs() @ deq.double().abs().T) * (2 + K / 32) * 2.0 ** -24
+    if glu:
+        F = N // 2
+        gate, up, bg, bu = want[:, :F], want[:, F:], bound[:, :F], bound[:, F:]
+        got = backend.swiglu(x.to(DEV), to_dev(w))
+        want, sg = gate * torch.sigmoid(gate) * up, (gate * torch.sigmoid(gate)).abs()
+        bound = 1.1 * bg * up.abs() + sg * bu + bg * bu + 1e-6 * want.abs() + 1e-30
+    else:
+        got = backend.linear(x.to(DEV), to_dev(w))
+    over = ((got.cpu().double() - want).abs() / bound).max()
+    print(f"channels {kind} {M} glu {glu}: {over:.3f} of the bound")
+    assert over < 1.0
+
+
 def test_many_row_linears_take_what_the_row_kernels_take(backend):
     """33 rows with strided activations, a bias and residual that broadcast, and a weight at an odd address; a row that
     holds an infinity gives infinities or NaN and leaves its neighbours alone."""
