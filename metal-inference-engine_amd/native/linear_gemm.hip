@@ -29,6 +29,7 @@ namespace {
 constexpr int kBK = 32;                            // k per step
 constexpr int P = 3;                               // pieces of an activation
 constexpr long long kSlabElems = 1ll << 25;        // quantized weights expanded at a time (64 MiB)
+constexpr long long kPieceBytes = 192ll << 20;     // activation pieces made at a time
 
 // 16 bytes per lane from src into LDS at dst (wave-uniform) + 16 * lane
 __device__ __forceinline__ void load_to_lds(const void* src, char* dst) {
@@ -390,8 +391,8 @@ __global__ __launch_bounds__(256) void gemm_finish(GemmArgs g) {
 }
 
 struct Layout {
-    int Mp, Np, steps, slab;       // rows of x in whole tiles; slab: output columns at a time; Np: its weight rows, in
-                                   // whole tiles
+    int Mc, Mp, Np, steps, slab;   // rows of x at a time, and in whole tiles; slab: output columns at a time; Np: its
+                                   // weight rows, in whole tiles
     int form, S;                   // gemm_rows' tile: 0 128 x 256, 1 128 x 128, 2 64 x 128; K-splits
     size_t slab_w, slab_sc, part, total;
 };
@@ -404,7 +405,13 @@ int slab_rows(int cols, bool glu) { return glu ? (cols + 15) / 16 * 32 : cols; }
 Layout layout(int M, int N, int K, int w_type, bool glu) {
     Layout l;
     l.steps = K / kBK + (w_type == RK_W_INT4 ? (K / kQB + 7) / 8 : 0);
-    l.Mp = (M + 127) / 128 * 128;
+    // rows in pieces of about the same size whose operands fit kPieceBytes
+    const long long row_bytes = (long long)l.steps * P * kBK * 2;
+    long long most = kPieceBytes / row_bytes / 128 * 128;
+    if (most < 128) most = 128;
+    const long long runs = (M + most - 1) / most;
+    l.Mc = runs == 1 ? M : (int)((M + 128 * runs - 1) / (128 * runs) * 128);
+    l.Mp = (l.Mc + 127) / 128 * 128;
     const int cols = glu ? N / 2 : N;
     l.slab = cols;
     if (w_type != RK_W_BF16) {
@@ -414,7 +421,7 @@ Layout layout(int M, int N, int K, int w_type, bool glu) {
     }
     const size_t rows = (size_t)slab_rows(l.slab, glu);
     l.Np = (int)up256(rows);
-    l.slab_w = (size_t)l.Mp * l.steps * P * kBK * 2;
+    l.slab_w = (size_t)l.Mp * row_bytes;
     l.slab_sc = l.slab_w + (w_type == RK_W_BF16 ? 0 : (size_t)l.steps * l.Np * kBK * 2);
     l.part = l.slab_sc + (w_type == RK_W_BF16 ? 0 : (size_t)l.steps * l.Np * 4);
     // 128 x 256 tiles where they give every CU two of them, else 128 x 128 (1777 x 2048 outputs: 112 tiles of 256
@@ -422,13 +429,13 @@ Layout layout(int M, int N, int K, int w_type, bool glu) {
     // 16 steps, until the tiles fill the CUs
     int cus = device_cus();
     if (cus <= 0) cus = 256;
-    auto tiles = [&](int bm, int bn) { return (long long)((M + bm - 1) / bm) * (((long long)rows + bn - 1) / bn); };
-    l.form = tiles(128, 256) >= 2 * cus ? 0 : M > 64 ? 1 : 2;
+    auto tiles = [&](int bm, int bn) { return (long long)((l.Mc + bm - 1) / bm) * (((long long)rows + bn - 1) / bn); };
+    l.form = tiles(128, 256) >= 2 * cus ? 0 : l.Mc > 64 ? 1 : 2;
     const long long t = l.form == 1 ? tiles(128, 128) : tiles(64, 128);
     l.S = 1;
     if (l.form && 2 * t <= cus) l.S = (int)(cus / t < l.steps / 16 ? cus / t : l.steps / 16);
     if (l.S < 1) l.S = 1;
-    l.total = l.part + (l.S > 1 ? (size_t)l.S * M * l.Np * 4 : 0);
+    l.total = l.part + (l.S > 1 ? (size_t)l.S * l.Mc * l.Np * 4 : 0);
     return l;
 }
 
@@ -492,34 +499,38 @@ int rk_linear_gemm(float* y, const float* x, long long x_ld, int M, int N, int K
     uint16_t* pieces = reinterpret_cast<uint16_t*>(ws);
     const auto split = w_type == RK_W_INT4 ? split_rows<true> : split_rows<false>;
     const int cols = glu ? N / 2 : N;
-    hipLaunchKernelGGL(split, dim3((unsigned)M), dim3(256), 0, st, pieces, x, x_ld, l.Mp, K, l.steps);
-    if (int rc = check_launch("split_rows")) return rc;
-    for (int c0 = 0; c0 < cols; c0 += l.slab) {
-        const int nc = l.slab < cols - c0 ? l.slab : cols - c0;
-        const int rows = slab_rows(nc, glu != 0);
-        GemmArgs g{};
-        g.w = static_cast<const uint16_t*>(w);
-        g.F = glu ? cols : 0;
-        if (quant) {
-            SlabArgs sa{};
-            sa.out = reinterpret_cast<uint16_t*>(ws + l.slab_w);
-            sa.sc = reinterpret_cast<float*>(ws + l.slab_sc);
-            sa.w = w; sa.scales = static_cast<const uint16_t*>(scales); sa.mins = static_cast<const uint16_t*>(mins);
-            sa.Np = l.Np; sa.row0 = c0; sa.K = K; sa.steps = l.steps; sa.F = g.F;
-            const auto expand = w_type == RK_W_INT8 ? slab_weights<RK_W_INT8> : slab_weights<RK_W_INT4>;
-            hipLaunchKernelGGL(expand, dim3((unsigned)rows), dim3(256), 0, st, sa);
-            if (int rc = check_launch("slab_weights")) return rc;
-            g.w = sa.out; g.sc = sa.sc;
+    for (int m0 = 0; m0 < M; m0 += l.Mc) {
+        const int rows_x = l.Mc < M - m0 ? l.Mc : M - m0;
+        hipLaunchKernelGGL(split, dim3((unsigned)rows_x), dim3(256), 0, st, pieces, x + (size_t)m0 * x_ld, x_ld, l.Mp, K,
+                           l.steps);
+        if (int rc = check_launch("split_rows")) return rc;
+        for (int c0 = 0; c0 < cols; c0 += l.slab) {
+            const int nc = l.slab < cols - c0 ? l.slab : cols - c0;
+            const int rows = slab_rows(nc, glu != 0);
+            GemmArgs g{};
+            g.w = static_cast<const uint16_t*>(w);
+            g.F = glu ? cols : 0;
+            if (quant) {
+                SlabArgs sa{};
+                sa.out = reinterpret_cast<uint16_t*>(ws + l.slab_w);
+                sa.sc = reinterpret_cast<float*>(ws + l.slab_sc);
+                sa.w = w; sa.scales = static_cast<const uint16_t*>(scales); sa.mins = static_cast<const uint16_t*>(mins);
+                sa.Np = l.Np; sa.row0 = c0; sa.K = K; sa.steps = l.steps; sa.F = g.F;
+                const auto expand = w_type == RK_W_INT8 ? slab_weights<RK_W_INT8> : slab_weights<RK_W_INT4>;
+                hipLaunchKernelGGL(expand, dim3((unsigned)rows), dim3(256), 0, st, sa);
+                if (int rc = check_launch("slab_weights")) return rc;
+                g.w = sa.out; g.sc = sa.sc;
+            }
+            g.y = y + (size_t)m0 * cols; g.a = pieces; g.bias = bias; g.res = residual ? residual + (size_t)m0 * cols : nullptr;
+            g.y_ld = cols; g.M = rows_x; g.N = rows; g.Mp = l.Mp; g.Np = l.Np; g.steps = l.steps; g.col0 = c0; g.cols = cols;
+            g.S = l.S;
+            g.part = reinterpret_cast<float*>(ws + l.part);
+            int rc;
+            if (l.form == 0) rc = launch_gemm<2, 4, 4>(g, quant, glu != 0, st);
+            else if (l.form == 1) rc = launch_gemm<4, 2, 2>(g, quant, glu != 0, st);
+            else rc = launch_gemm<2, 2, 2>(g, quant, glu != 0, st);
+            if (rc) return rc;
         }
-        g.y = y; g.a = pieces; g.bias = bias; g.res = residual;
-        g.y_ld = cols; g.M = M; g.N = rows; g.Mp = l.Mp; g.Np = l.Np; g.steps = l.steps; g.col0 = c0; g.cols = cols;
-        g.S = l.S;
-        g.part = reinterpret_cast<float*>(ws + l.part);
-        int rc;
-        if (l.form == 0) rc = launch_gemm<2, 4, 4>(g, quant, glu != 0, st);
-        else if (l.form == 1) rc = launch_gemm<4, 2, 2>(g, quant, glu != 0, st);
-        else rc = launch_gemm<2, 2, 2>(g, quant, glu != 0, st);
-        if (rc) return rc;
     }
     return RK_OK;
 }

@@ -345,5 +345,9 @@ def test_linear_gemm_checked_on_host(lib):
         assert need > 4 * M * K and call(M=M, N=N, K=K, xld=K, wt=wt, glu=glu, wsb=need - 1) == 3
         assert "workspace" in lib.last_error()
     assert L.rk_linear_gemm_workspace_bytes(0, 64, 64, 1, 0) == 0
-    # weights are expanded a slab at a time: 64 MiB of them at most, however many there are
-    assert L.rk_linear_gemm_workspace_bytes(64, 1 << 22, 2048, 1, 0) < 80 << 20
+    # weights are expanded a slab at a time (64 MiB of them at most, however many there are; bf16 not at all), and pieces
+    # made of some rows at a time (192 MiB)
+    assert L.rk_linear_gemm_workspace_bytes(64, 1 << 22, 2048, 1, 0) < 8 << 20
+    assert L.rk_linear_gemm_workspace_bytes(64, 1 << 22, 2048, 2, 0) < 80 << 20
+    for wt in (1, 2, 3):
+        assert L.rk_linear_gemm_workspace_bytes(1 << 20, 8192, 6144, wt, 0) < 280 << 20

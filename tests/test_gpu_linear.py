@@ -288,6 +288,20 @@ def test_many_row_linears_against_64_bits(backend, kind, M, N, K, glu):
     assert over < 1.0
 
 
+@pytest.mark.parametrize("kind,glu", [("bf16", False), ("bf16", True), ("int8", False), ("int4", True)])
+def test_many_row_linears_in_pieces_of_rows(backend, kind, glu):
+    """More rows than are taken at a time (192 MiB of pieces: 3 of them here): the bits of each part by itself."""
+    M, N, K = 70003, 96, 1024
+    w, _ = weight(kind, N, K, 2)
+    wd, g = to_dev(w), torch.Generator(device=DEV).manual_seed(1)
+    x = torch.randn(M, K, generator=g, device=DEV)
+    f = (lambda a, r: backend.swiglu(a, wd)) if glu else (lambda a, r: backend.linear(a, wd, residual=r))
+    res = torch.randn(M, N, generator=g, device=DEV)
+    y = f(x, res)
+    for m0, m1 in ((0, 20000), (20000, 45000), (45000, M)):
+        assert torch.equal(y[m0:m1], f(x[m0:m1].contiguous(), res[m0:m1].contiguous()))
+
+
 @pytest.mark.parametrize("kind", ["bf16", "int8", "int4"])
 @pytest.mark.parametrize("M,N,K", [(48, 200, 256), (90, 100, 1088), (300, 500, 288), (700, 130, 192)])
 def test_many_row_linears_take_every_bit(backend, kind, M, N, K):
