@@ -17,7 +17,7 @@
 // quantized weights as stored instead.
 //
 // Measured, an MLP of 1777 rows, bf16 weights (12288 x 2048 with silu * up, then 2048 x 6144): 1188 us as an fp32 GEMM on
-// the expanded weight, 362 on two fp16 pieces of x (23 bits in a range of 2^40 below the row's largest value), 390 so.
+// the expanded weight, 362 on two fp16 pieces of x (23 bits in a range of 2^40 below the row's largest value), 377 so.
 // What bounds gemm_rows: matrix-core issue and the fp32 joins beside it, and whole tiles.
 #include "linear_operands.h"
 
@@ -30,6 +30,7 @@ constexpr int kBK = 32;                            // k per step
 constexpr int P = 3;                               // pieces of an activation
 constexpr long long kSlabElems = 1ll << 25;        // quantized weights expanded at a time (64 MiB)
 constexpr long long kPieceBytes = 192ll << 20;     // activation pieces made at a time
+constexpr long long kPartBytes = 64ll << 20;       // partial sums of K-splits
 
 // 16 bytes per lane from src into LDS at dst (wave-uniform) + 16 * lane
 __device__ __forceinline__ void load_to_lds(const void* src, char* dst) {
@@ -393,7 +394,8 @@ __global__ __launch_bounds__(256) void gemm_finish(GemmArgs g) {
 struct Layout {
     int Mc, Mp, Np, steps, slab;   // rows of x at a time, and in whole tiles; slab: output columns at a time; Np: its
                                    // weight rows, in whole tiles
-    int form, S;                   // gemm_rows' tile: 0 128 x 256, 1 128 x 128, 2 64 x 128; K-splits
+    int form, S;                   // gemm_rows' tile (kTiles); K-splits
+    double us;                     // the estimated time
     size_t slab_w, slab_sc, part, total;
 };
 
@@ -401,6 +403,18 @@ size_t up256(size_t n) { return (n + 255) / 256 * 256; }
 
 // rows of W behind `cols` output columns (glu: whole pairs of sixteens)
 int slab_rows(int cols, bool glu) { return glu ? (cols + 15) / 16 * 32 : cols; }
+
+// gemm_rows' tiles, and what its time is made of, in us: a round of one workgroup per CU costs `start`, and for each of
+// its steps `step` and up to `full` more when every CU has one ([1]: with scales). Fitted, with the constants of layout(),
+// to 168 sizes (seven weights of 1024 x 3584 to 12288 x 2048, 64 to 4096 rows, bf16, INT8, INT4) x up to 10 of these
+// forms, 12 to 1200 us: 4.8 % of root mean square error; the form it names is the fastest measured, or within 4 % of it,
+// at all but 9 of them (the worst 13 %).
+constexpr int kTiles[3][2] = {{128, 256}, {128, 128}, {64, 128}};
+struct RoundCost {
+    double start, step, full;
+};
+constexpr RoundCost kRound[2][3] = {{{2.7, 0.88, 0.28}, {2.5, 0.50, 0.17}, {2.2, 0.36, 0.05}},
+                                    {{0.6, 1.10, 0.24}, {1.4, 0.69, 0.12}, {1.6, 0.47, 0.03}}};
 
 Layout layout(int M, int N, int K, int w_type, bool glu) {
     Layout l;
@@ -424,17 +438,29 @@ Layout layout(int M, int N, int K, int w_type, bool glu) {
     l.slab_w = (size_t)l.Mp * row_bytes;
     l.slab_sc = l.slab_w + (w_type == RK_W_BF16 ? 0 : (size_t)l.steps * l.Np * kBK * 2);
     l.part = l.slab_sc + (w_type == RK_W_BF16 ? 0 : (size_t)l.steps * l.Np * 4);
-    // 128 x 256 tiles where they give every CU two of them, else 128 x 128 (1777 x 2048 outputs: 112 tiles of 256
-    // columns leave half the CUs idle), else 64 x 128. Fewer than half as many tiles as CUs: K-splits of at least
-    // 16 steps, until the tiles fill the CUs
+    // the tile and the K-splits of the least estimated time
     int cus = device_cus();
     if (cus <= 0) cus = 256;
-    auto tiles = [&](int bm, int bn) { return (long long)((l.Mc + bm - 1) / bm) * (((long long)rows + bn - 1) / bn); };
-    l.form = tiles(128, 256) >= 2 * cus ? 0 : l.Mc > 64 ? 1 : 2;
-    const long long t = l.form == 1 ? tiles(128, 128) : tiles(64, 128);
-    l.S = 1;
-    if (l.form && 2 * t <= cus) l.S = (int)(cus / t < l.steps / 16 ? cus / t : l.steps / 16);
-    if (l.S < 1) l.S = 1;
+    const bool quant = w_type != RK_W_BF16;
+    l.us = 0.0;
+    for (int f = 0; f < 3; ++f) {
+        const long long t = (long long)((l.Mc + kTiles[f][0] - 1) / kTiles[f][0]) * (((long long)rows + kTiles[f][1] - 1) / kTiles[f][1]);
+        const RoundCost& c = kRound[quant][f];
+        for (int sp = 1; sp <= 16 && (sp == 1 || (l.steps / sp >= 8 && (long long)sp * l.Mc * l.Np * 4 <= kPartBytes)); ++sp) {
+            const long long rounds = (t * sp + cus - 1) / cus;
+            const double full = (double)(t * sp) / (double)(rounds * cus);
+            double us = (double)rounds * (c.start + (c.step + c.full * full) * ((l.steps + sp - 1) / sp));
+            if (sp > 1) us += 1.5 + 1.05e-6 * sp * l.Mc * (double)rows;       // gemm_finish
+            if (l.us == 0.0 || us < l.us) {
+                l.us = us;
+                l.form = f;
+                l.S = sp;
+            }
+        }
+    }
+    const double slabs = (cols + l.slab - 1) / l.slab;
+    if (quant) l.us += 4.8 + 0.75e-6 * (double)rows * K;                     // slab_weights
+    l.us = (double)runs * (slabs * l.us + 6.6 + 1.5e-6 * (double)l.Mc * K);  // split_rows
     l.total = l.part + (l.S > 1 ? (size_t)l.S * l.Mc * l.Np * 4 : 0);
     return l;
 }
@@ -468,10 +494,10 @@ extern "C" {
 
 size_t rk_linear_gemm_workspace_bytes(int M, int N, int K, int w_type, int glu) {
     if (M < 1 || N < 1 || K < kQB || K % kQB) return 0;
-    // either form may run (an odd address of the scales sends a call to the other one)
-    const size_t tiles = layout(M, N, K, w_type, glu != 0).total;
-    const size_t mid = mid_takes(M, K, w_type, nullptr, nullptr) ? mid_workspace_bytes(M, N, K, w_type, glu) : 0;
-    return tiles > mid ? tiles : mid;
+    // either form may run (an odd address of the scales sends a call to this one)
+    const Layout l = layout(M, N, K, w_type, glu != 0);
+    const size_t mid = mid_takes(M, N, K, w_type, glu, nullptr, nullptr, l.us) ? mid_workspace_bytes(M, N, K, w_type, glu) : 0;
+    return l.total > mid ? l.total : mid;
 }
 
 int rk_linear_gemm(float* y, const float* x, long long x_ld, int M, int N, int K, const void* w, int w_type,
@@ -490,10 +516,10 @@ int rk_linear_gemm(float* y, const float* x, long long x_ld, int M, int N, int K
     const size_t need = rk_linear_gemm_workspace_bytes(M, N, K, w_type, glu);
     if (!workspace || workspace_bytes < need)
         return fail(RK_ERR_WORKSPACE, "rk_linear_gemm: workspace %zu bytes (need %zu)", workspace_bytes, need);
-    if (mid_takes(M, K, w_type, scales, mins))
+    const Layout l = layout(M, N, K, w_type, glu != 0);
+    if (mid_takes(M, N, K, w_type, glu, scales, mins, l.us))
         return mid_linear(y, x, x_ld, M, N, K, w, w_type, scales, mins, bias, residual, glu, workspace,
                           static_cast<hipStream_t>(stream));
-    const Layout l = layout(M, N, K, w_type, glu != 0);
     char* ws = static_cast<char*>(workspace);
     hipStream_t st = static_cast<hipStream_t>(stream);
     uint16_t* pieces = reinterpret_cast<uint16_t*>(ws);

@@ -322,15 +322,22 @@ __global__ __launch_bounds__(256) void mid_finish(MidArgs a) {
 
 struct MidPlan {
     int MB, MT, NT, G, S, SB, WB;
+    double us;                     // the estimated time
     size_t sums, part, total;
 };
 
-// Rows up to which this form is the faster one
-int mid_rows_max(int w_type) { return w_type == RK_W_BF16 ? 96 : 256; }
+// What the time is made of, in us: the launches and x's pieces; a round of one workgroup per CU: its start, and for each
+// chunk of four blocks a wave walks a constant, the activations from the L2 (per row tile, more when every CU asks) and
+// the MFMAs (per row and weight tile); mid_finish and the partial sums it reads. Fitted to 14 weights of 1024 x 1024 to
+// 12288 x 2048, 33 to 384 rows, x the NT and S there are: 10 % of root mean square error; NT and S chosen by it cost on
+// average 0.5 % more than the best measured, 9 % at worst.
+struct MidCost {
+    double launch, split, start, item, chunk, x, x_full, mfma, finish, part;
+};
+constexpr MidCost kCost[3] = {{6.7, 5.9e-6, 0.0, 0.37, 1.51, 0.24, 0.17, 0.294, 1.8, 0.0},         // bf16
+                              {6.9, 5.7e-6, 0.0, 0.34, 1.77, 0.08, 0.21, 0.309, 1.8, 0.046e-3},    // INT8
+                              {7.1, 5.3e-6, 1.2, 0.31, 2.35, 0.0, 0.20, 0.320, 1.9, 0.070e-3}};    // INT4
 
-// NT, S: the least estimated time over the rounds of one workgroup per CU: a block costs a wave its activations from
-// the L2 (1 KB per 16 cycles and CU) or its MFMAs (19 cycles each, two waves per SIMD), whichever is longer, a
-// workgroup a start and an end, a split its partials
 MidPlan mid_plan(int M, int N, int K, int w_type, int glu) {
     MidPlan p{};
     const int nblk = K / kQB;
@@ -339,18 +346,20 @@ MidPlan mid_plan(int M, int N, int K, int w_type, int glu) {
     p.MT = (M + 16 * p.MB - 1) / (16 * p.MB) <= 3 ? 3 : 4;
     int cus = device_cus();
     if (cus <= 0) cus = 256;
-    double best = 0;
+    const MidCost& c = kCost[w_type == RK_W_BF16 ? 0 : w_type == RK_W_INT8 ? 1 : 2];
     for (int nt = 1; nt <= (w_type == RK_W_BF16 ? 2 : p.MT == 4 ? 3 : 4); ++nt)   // as the registers hold
         for (int s = 1; s <= 16 && s <= (nblk + 31) / 32 * 2; ++s) {
             const int sb = ((nblk + s - 1) / s + 1) / 2 * 2;
             const int wb = ((sb + kWaves - 1) / kWaves + 1) / 2 * 2;
             const int g = (tiles + nt - 1) / nt, used = (nblk + sb - 1) / sb;
-            const double rounds = (double)((long long)g * used * p.MB + cus - 1) / cus;
-            const double blk = 128.0 * P * p.MT > 38.0 * P * p.MT * nt ? 128.0 * P * p.MT : 38.0 * P * p.MT * nt;
-            const double cost = (double)(long long)rounds * ((wb + 3) / 4 * 4 * (blk + 60.0 * nt) + 3000.0) +
-                                (used > 1 ? 5000.0 + 20.0 * used * p.MB * g * nt * p.MT / 16 : 0.0);
-            if (best == 0 || cost < best) {
-                best = cost;
+            const long long groups = (long long)g * used * p.MB, rounds = (groups + cus - 1) / cus;
+            const double full = (double)groups / (double)(rounds * cus);
+            double us = c.launch + c.split * (double)M * K +
+                        (double)rounds * (c.start + c.item * p.MT * nt +
+                                          (wb + 3) / 4 * (c.chunk + p.MT * (c.x + c.x_full * full + c.mfma * nt)));
+            if (used > 1) us += c.finish + c.part * (double)groups * nt * p.MT;
+            if (p.us == 0.0 || us < p.us) {
+                p.us = us;
                 p.NT = nt; p.G = g; p.S = used; p.SB = sb; p.WB = wb;
             }
         }
@@ -364,10 +373,12 @@ MidPlan mid_plan(int M, int N, int K, int w_type, int glu) {
 
 }  // namespace
 
-bool mid_takes(int M, int K, int w_type, const void* scales, const void* mins) {
+// kMost: the estimates end there; no weight measured was faster here at 512 rows
+bool mid_takes(int M, int N, int K, int w_type, int glu, const void* scales, const void* mins, double gemm_us) {
+    constexpr int kMost = 384;
     // scales and mins are read two blocks at a time
-    return M <= mid_rows_max(w_type) && K % (2 * kQB) == 0 && reinterpret_cast<uintptr_t>(scales) % 4 == 0 &&
-           reinterpret_cast<uintptr_t>(mins) % 4 == 0;
+    return M <= kMost && K % (2 * kQB) == 0 && reinterpret_cast<uintptr_t>(scales) % 4 == 0 &&
+           reinterpret_cast<uintptr_t>(mins) % 4 == 0 && mid_plan(M, N, K, w_type, glu).us < gemm_us;
 }
 
 size_t mid_workspace_bytes(int M, int N, int K, int w_type, int glu) { return mid_plan(M, N, K, w_type, glu).total; }
