@@ -18,7 +18,7 @@
 extern "C" {
 #endif
 
-#define RK_ABI_VERSION 18
+#define RK_ABI_VERSION 19
 
 /* status codes */
 #define RK_OK 0
@@ -342,7 +342,11 @@ int rk_swiglu_rows(float* y, const float* x, long long x_ld, int x_op, const flo
  *   rk_linear_rows; K a multiple of 32. x and the weights enter exactly (three bf16 pieces of every x; bf16 weights and
  *   INT8 / INT4 codes as they are), products are exact, sums fp32. An infinite or NaN value of x makes its row's outputs
  *   infinite or NaN, one of W its column's.
- *   workspace: rk_linear_gemm_workspace_bytes(M, N, K, w_type, glu) bytes, 256-byte aligned, no zeroing needed. */
+ *   workspace: rk_linear_gemm_workspace_bytes(M, N, K, w_type, glu) bytes, 256-byte aligned, no zeroing needed.
+ * rk_linear_gemm_plan: how such a call is worked (with scales and mins 4-byte aligned), on the current device:
+ *   plan[0] 0 the weight as stored (linear_mid.hip), 1 tiles of 128 x 256, 2 of 128 x 128, 3 of 64 x 128; plan[1]
+ *   K-splits; plan[2] parts the weight is expanded in; plan[3] parts the rows are taken in. */
+int rk_linear_gemm_plan(int M, int N, int K, int w_type, int glu, int* plan);
 size_t rk_linear_gemm_workspace_bytes(int M, int N, int K, int w_type, int glu);
 int rk_linear_gemm(float* y, const float* x, long long x_ld, int M, int N, int K, const void* w, int w_type,
                    const void* scales, const void* mins, const float* bias, const float* residual, int glu,

@@ -500,6 +500,19 @@ size_t rk_linear_gemm_workspace_bytes(int M, int N, int K, int w_type, int glu) 
     return l.total > mid ? l.total : mid;
 }
 
+int rk_linear_gemm_plan(int M, int N, int K, int w_type, int glu, int* plan) {
+    if (M < 1 || N < 1 || K < kQB || K % kQB || (glu && N % 2) || !plan)
+        return fail(RK_ERR_ARG, "rk_linear_gemm_plan: M %d, N %d, K %d", M, N, K);
+    const Layout l = layout(M, N, K, w_type, glu != 0);
+    const bool mid = mid_takes(M, N, K, w_type, glu, nullptr, nullptr, l.us);
+    const int cols = glu ? N / 2 : N;
+    plan[0] = mid ? 0 : 1 + l.form;
+    plan[1] = mid ? mid_splits(M, N, K, w_type, glu) : l.S;
+    plan[2] = mid ? 1 : (cols + l.slab - 1) / l.slab;
+    plan[3] = mid ? 1 : (M + l.Mc - 1) / l.Mc;
+    return RK_OK;
+}
+
 int rk_linear_gemm(float* y, const float* x, long long x_ld, int M, int N, int K, const void* w, int w_type,
                    const void* scales, const void* mins, const float* bias, const float* residual, int glu,
                    void* workspace, size_t workspace_bytes, void* stream) {

@@ -381,6 +381,8 @@ bool mid_takes(int M, int N, int K, int w_type, int glu, const void* scales, con
            reinterpret_cast<uintptr_t>(mins) % 4 == 0 && mid_plan(M, N, K, w_type, glu).us < gemm_us;
 }
 
+int mid_splits(int M, int N, int K, int w_type, int glu) { return mid_plan(M, N, K, w_type, glu).S; }
+
 size_t mid_workspace_bytes(int M, int N, int K, int w_type, int glu) { return mid_plan(M, N, K, w_type, glu).total; }
 
 int mid_linear(float* y, const float* x, long long x_ld, int M, int N, int K, const void* w, int w_type,

@@ -11,7 +11,7 @@ from pathlib import Path
 HERE = Path(__file__).resolve().parent
 LIB_PATH = HERE / "librk_path.so"
 HEADER = HERE.parent.parent / "include" / "rk_path.h"
-ABI_VERSION = 18
+ABI_VERSION = 19
 
 RK_F32, RK_BF16 = 0, 1
 RK_W_BF16, RK_W_INT8, RK_W_INT4 = 1, 2, 3
@@ -64,6 +64,7 @@ SIGNATURES = {
                                    P, P, P, P, P, c_size_t, P, c_int, P]),
     "rk_swiglu_rows": (c_int, [P, P, c_longlong, c_int, P, c_longlong, P, c_float, c_int, c_int, c_int, P, c_int, P, P,
                                P, c_size_t, P, c_int, P]),
+    "rk_linear_gemm_plan": (c_int, [c_int] * 5 + [P]),
     "rk_linear_gemm_workspace_bytes": (c_size_t, [c_int] * 5),
     "rk_linear_gemm": (c_int, [P, P, c_longlong, c_int, c_int, c_int, P, c_int, P, P, P, P, c_int, P, c_size_t, P]),
     "rk_rms_norm": (c_int, [P, P, c_int, c_longlong, P, c_int, c_int, c_int, c_float, P]),

@@ -351,3 +351,28 @@ def test_linear_gemm_checked_on_host(lib):
     assert L.rk_linear_gemm_workspace_bytes(64, 1 << 22, 2048, 2, 0) < 80 << 20
     for wt in (1, 2, 3):
         assert L.rk_linear_gemm_workspace_bytes(1 << 20, 8192, 6144, wt, 0) < 280 << 20
+
+
+def test_linear_gemm_cases_reach_every_form(lib):
+    """The parity cases of the many-row linears cover rk_linear_gemm's forms: each tile and the weight as stored, with
+    K-splits and without, with gate and up and without; and a quantized weight expanded in parts, the last one smaller."""
+    from test_gpu_linear import MANY_ROWS
+    seen, parts = set(), set()
+    for M, N, K, glu in MANY_ROWS:
+        for wt, kind in ((1, "bf16"), (2, "int8"), (3, "int4")):
+            p = (ctypes.c_int * 4)()
+            assert lib.lib.rk_linear_gemm_plan(M, N, K, wt, int(glu), p) == 0
+            seen.add((kind, p[0], p[1] > 1, glu))
+            if p[2] > 1:
+                parts.add((kind, glu))
+    for kind in ("bf16", "int8", "int4"):
+        for form in range(4):
+            for split in (False, True):
+                assert any((kind, form, split, glu) in seen for glu in (False, True)), (kind, form, split)
+            assert any((kind, form, split, True) in seen for split in (False, True)), (kind, form)
+            assert any((kind, form, split, False) in seen for split in (False, True)), (kind, form)
+    assert parts == {(k, g) for k in ("int8", "int4") for g in (False, True)}
+    p = (ctypes.c_int * 4)()
+    assert lib.lib.rk_linear_gemm_plan(70003, 96, 1024, 1, 0, p) == 0 and p[3] == 3     # rows in parts
+    assert lib.lib.rk_linear_gemm_plan(64, 512, 2048, 3, 0, p) == 0 and p[0] == 0
+    assert lib.lib.rk_linear_gemm_plan(64, 512, 2040, 3, 0, p) == 1

@@ -252,17 +252,33 @@ def test_long_int8_matrix_on_the_persistent_grid(backend, N, K):
     assert torch.equal(rows[1][0], rows[8][0]) and torch.equal(rows[3], rows[8][:3])
 
 
+# (M, N, K, glu) at the edges of rk_linear_gemm's forms: rows and columns around 48, 64, 96, 128 and 256, odd numbers of
+# 32-value steps, glu halves that are not whole sixteens, K-splits, wave shares and weight parts with a remainder
+MANY_ROWS = [(33, 100, 96, False), (64, 130, 2080, False), (65, 272, 64, False), (129, 1000, 512, False),
+             (257, 515, 1056, False), (600, 4352, 256, False), (48, 17, 192, False), (49, 300, 3072, False),
+             (97, 2064, 448, False), (33, 2 * 20, 256, True), (96, 2 * 700, 1920, True), (250, 2 * 36, 320, True),
+             (140, 2 * 1000, 544, True), (513, 2 * 2200, 128, True), (33, 18, 2048, False), (40, 2 * 9, 2048, True),
+             (1100, 15000, 96, False), (1090, 2 * 7500, 160, True), (600, 2 * 700, 2080, True), (777, 4100, 288, False),
+             (200, 2066, 2048, False), (390, 2 * 1500, 2048, True), (1100, 260, 2048, False), (600, 1400, 2080, False),
+             (390, 5000, 8192, False), (390, 2 * 2200, 8192, True), (33, 2 * 16400, 1056, True),
+             (33, 33000, 1056, False)]
+
+
+def products_64(x, deq):
+    """(x @ deq^T in 64 bits, the bound of test_many_row_linears_against_64_bits)."""
+    M, K = x.shape
+    at = DEV if M * K * deq.shape[0] > 1 << 30 else "cpu"
+    x, d = x.double().to(at), deq.double().to(at)
+    return (x @ d.T).cpu(), (x.abs() @ d.abs().T).cpu() * (2 + K / 32) * 2.0 ** -24
+
+
 @pytest.mark.parametrize("kind", ["bf16", "int8", "int4"])
-@pytest.mark.parametrize("M,N,K,glu", [(33, 100, 96, False), (64, 130, 2080, False), (65, 272, 64, False),
-                                       (129, 1000, 512, False), (257, 515, 1056, False), (600, 4352, 256, False),
-                                       (48, 17, 192, False), (49, 300, 3072, False), (97, 2064, 448, False),
-                                       (33, 2 * 20, 256, True), (96, 2 * 700, 1920, True), (250, 2 * 36, 320, True),
-                                       (140, 2 * 1000, 544, True), (513, 2 * 2200, 128, True)])
+@pytest.mark.parametrize("M,N,K,glu", MANY_ROWS)
 def test_many_row_linears_against_64_bits(backend, kind, M, N, K, glu):
-    """rk_linear_gemm at the edges of its forms and tiles (rows and columns around 48, 64, 96, 128 and 256, odd numbers
-    of 32-value steps, glu halves that are not whole sixteens, K-splits and wave shares with a remainder), with rows of
-    very different magnitude and values of very different magnitude in one row, against the products in 64 bits. Bound: each output's sum of |x w| times 2^-24 for the
-    rounding of x and the same for every 32-value partial sum's fp32 rounding, of which there are K / 32 in sequence."""
+    """rk_linear_gemm in every form it has (test_abi.py checks that these reach them), with rows of very different magnitude
+    and values of very different magnitude in one row, against the products in 64 bits. Bound: each output's sum of |x w|
+    times 2^-24 for the rounding of x and the same for every 32-value partial sum's fp32 rounding, of which there are
+    K / 32 in sequence."""
     w, deq = weight(kind, N, K, N + K)
     g = torch.Generator().manual_seed(M)
     x = torch.randn(M, K, generator=g) * torch.exp2(torch.randint(-60, 40, (M, 1), generator=g).float())
@@ -271,8 +287,7 @@ def test_many_row_linears_against_64_bits(backend, kind, M, N, K, glu):
     b, r = (None, None) if glu else (torch.randn(N, generator=g), torch.randn(M, N, generator=g))
     if glu:
         x = x.sign() * x.abs().clamp(1e-6, 1e3)         # silu's tails are not what is tested
-    want = x.double() @ deq.double().T
-    bound = (x.double().abs() @ deq.double().abs().T) * (2 + K / 32) * 2.0 ** -24
+    want, bound = products_64(x, deq)
     if glu:
         F = N // 2
         gate, up, bg, bu = want[:, :F], want[:, F:], bound[:, :F], bound[:, F:]
@@ -346,8 +361,7 @@ def test_many_row_linears_over_channels_of_different_size(backend, kind, M, glu)
         deq = quant_ref.dequantize(w.scheme, w.data, w.scales, w.mins)
     assert torch.isfinite(deq).all()
     x = torch.randn(M, K, generator=g) * torch.exp2(-e).repeat_interleave(32)
-    want = x.double() @ deq.double().T
-    bound = (x.double().abs() @ deq.double().abs().T) * (2 + K / 32) * 2.0 ** -24
+    want, bound = products_64(x, deq)
     if glu:
         F = N // 2
         gate, up, bg, bu = want[:, :F], want[:, F:], bound[:, :F], bound[:, F:]
@@ -359,6 +373,23 @@ def test_many_row_linears_over_channels_of_different_size(backend, kind, M, glu)
     over = ((got.cpu().double() - want).abs() / bound).max()
     print(f"channels {kind} {M} glu {glu}: {over:.3f} of the bound")
     assert over < 1.0
+
+
+@pytest.mark.parametrize("part", ["scales", "mins"])
+def test_many_row_linears_with_parameters_at_odd_addresses(backend, part):
+    """The form that reads the weight as stored takes scales and mins two at a time; at an address that is not a multiple
+    of four the other form runs (64 x 512 x 2048 INT4 takes the first one otherwise), in the same workspace."""
+    w, deq = weight("int4", 512, 2048, 6)
+    x = torch.randn(64, 2048, generator=torch.Generator().manual_seed(6))
+    want, bound = products_64(x, deq)
+    wd = to_dev(w)
+    t = getattr(wd, part)
+    flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=DEV)
+    setattr(wd, part, flat[1:].view(t.shape).copy_(t))
+    assert getattr(wd, part).data_ptr() % 4 == 2
+    for weights in (wd, to_dev(w)):
+        got = backend.linear(x.to(DEV), weights).cpu().double()
+        assert ((got - want).abs() / bound).max() < 1.0
 
 
 def test_many_row_linears_take_what_the_row_kernels_take(backend):
