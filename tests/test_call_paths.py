@@ -25,7 +25,7 @@ class _General:
 
 
 class _Watch:
-    """The C++ calls, noting which of them answered."""
+    """The C++ calls, noting each by name and whether it answered."""
 
     def __init__(self, mod):
         self.mod, self.answered = mod, []
@@ -33,20 +33,26 @@ class _Watch:
     def __getattr__(self, name):
         def call(*a):
             r = getattr(self.mod, name)(*a)
-            self.answered.append(r is not None)
+            self.answered.append((name, r is not None))
             return r
         return call
 
 
 def both(monkeypatch, fn):
     """(result with the C++ calls, result the general way, whether a C++ call answered)."""
+    fast, slow, calls = both_calls(monkeypatch, fn)
+    return fast, slow, any(answered for _, answered in calls)
+
+
+def both_calls(monkeypatch, fn):
+    """(result with the C++ calls, result the general way, [(C++ call, whether it answered)])."""
     watch = _Watch(kernels._calls())
     monkeypatch.setattr(kernels, "_native_calls", watch)
     fast = fn()
     monkeypatch.setattr(kernels, "_native_calls", _General())
     slow = fn()
     monkeypatch.setattr(kernels, "_native_calls", watch.mod)
-    return fast, slow, any(watch.answered)
+    return fast, slow, watch.answered
 
 
 def equal(a, b):
@@ -95,10 +101,16 @@ def test_linears(backend, monkeypatch, kind, M, N, K):
     for f in forms:
         fast, slow, used = both(monkeypatch, f)
         assert used and equal(fast, slow)
-    fast, slow, used = both(monkeypatch, lambda: backend.rms_norm_linear(x, ss, nw, 1e-6, w, b))
-    assert equal(fast, slow) and used == (M <= 8 and K % 256 == 0 and K <= 2048 or M <= 16)   # or its two parts answered
-    fast, slow, _ = both(monkeypatch, lambda: backend.rms_norm_swiglu(x, ss, nw, 1e-6, w))
-    assert equal(fast, slow)
+    # the norm inside the linear: one call, answered; elsewhere that call is declined, and the two parts follow
+    inside = M <= 8 and K % 256 == 0 and K <= 2048
+    for f, whole in ((lambda: backend.rms_norm_linear(x, ss, nw, 1e-6, w, b), inside),
+                     (lambda: backend.rms_norm_swiglu(x, ss, nw, 1e-6, w), inside and N % 16 == 0)):
+        fast, slow, calls = both_calls(monkeypatch, f)
+        assert equal(fast, slow)
+        if whole:
+            assert calls == [("linear", True)]
+        else:
+            assert calls[0] == ("linear", False) and ("norm" in [n for n, _ in calls]) == (not inside)
     # left to the general way
     for f in (lambda: backend.linear(x.double(), w), lambda: backend.linear(wide[:, 1:K + 1], w),
               lambda: backend.linear(x, w, b.bfloat16()), lambda: backend.linear(x, w, None, res.double())):
