@@ -32,12 +32,11 @@ __device__ __forceinline__ Pieces split_pair(float a, float b) {
     const f16x2 l = __builtin_convertvector((f32x2_t){a - (float)h[0], b - (float)h[1]}, f16x2);
     return {__builtin_bit_cast(uint32_t, h), __builtin_bit_cast(uint32_t, l)};
 }
-// the same where a value may be infinite: an infinite hi has no rest (inf - inf would make it NaN)
-__device__ __forceinline__ uint32_t rest_of(Pieces p) {
-    const uint32_t e = p.hi & 0x7c007c00u, m = p.hi & 0x03ff03ffu;   // exponent 31 with mantissa 0
-    const uint32_t drop = ((e & 0xffffu) == 0x7c00u && !(m & 0xffffu) ? 0xffffu : 0u) |
-                          (e >> 16 == 0x7c00u && !(m >> 16) ? 0xffff0000u : 0u);
-    return p.lo & ~drop;
+// Where a value was infinite: it has no rest (inf - inf would make it NaN).
+__device__ __forceinline__ Pieces infinite_alone(Pieces p) {
+    const uint32_t m = p.hi & 0x7fff7fffu;           // exponent 31 with mantissa 0
+    const uint32_t inf = ((m & 0xffffu) == 0x7c00u ? 0xffffu : 0u) | (m >> 16 == 0x7c00u ? 0xffff0000u : 0u);
+    return {p.hi, p.lo & ~inf};
 }
 
 // Rows of 32 fp16 (64 bytes) in LDS: the 16-byte unit u of row R sits at u ^ swizzle(R). A read of lane l: row l % 16,

@@ -27,6 +27,7 @@
 
 #include <cfloat>
 #include <climits>
+#include <type_traits>
 
 namespace rk {
 namespace {
@@ -572,12 +573,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // ---- 3. attention with fp32 operands: the same work list, masks, splits and gate as prefill_attention, for an
 // fp32 q or pool and for exact requests (any group size, D = 64 / 128 / 256). The reference computes attention in fp32
 // on widened inputs (src/ops.py:84-87, 91-103). The fp32 matrix rate is 1/16 of the fp16 one, so the products are made
-// of fp16 pieces (fp16_pieces.h): every operand x, scaled by a power of two that puts its neighbourhood's largest value
-// into [2^14, 2^15), is hi + lo to 2^-24 of itself (2^-40 of that largest value where it is tiny), and a product is
-// lo hi + hi lo + hi hi (lo lo, 2^-24 of the product, is the rounding an fp32 product has too), summed in fp32:
-// 3/16 of the fp32 matrix time. The neighbourhoods: a query row; a group of 4 keys (its exponent multiplies the group's
-// scores, held 4 to a lane); a group of 4 value rows, whose exponent, with a common one E for the accumulators, scales
-// the group's probabilities. Probabilities enter as two pieces as well.
+// of fp16 pieces (fp16_pieces.h): every operand x, scaled by a power of two that puts its row's largest value into
+// [2^14, 2^15), is hi + lo within 2^-23 of itself, and below 2^-16 of that largest value within 2^-40 of it; a product is
+// lo hi + hi lo + hi hi (lo lo is at most 2^-22 of it), summed in fp32: 3/16 of the fp32 matrix time. The rows: of the
+// queries, of the keys (whose exponents scale the scores, held 8 to a lane) and of the values (whose sizes w weigh the
+// probabilities). A query's probabilities enter as p w 2^E, E its own: the largest p w it has seen, as the running maximum
+// stands, bounds the others. So keys that a query does not see, or of no weight for it, cost it no bits.
 // blockDim = 512: wave w takes query head (chunk * 4 + w % 4) of the group (none past the group's end: that
 // wave only helps stage) and queries 16 (w / 4) .. + 15 of the work item's 32. All 8 waves stage each tile of 32
 // keys into a 2-stage LDS ring, requested a whole tile ahead, split into pieces on the way: K rows and V^T rows
@@ -588,20 +589,28 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 //                 16 + 4 (l / 16) + j - 4, the keys of the lane's own scores, so B is the lane's 8 probabilities.
 // So every lane keeps its own query's softmax state, and O^T is rescaled per lane. LDS reads are conflict-free.
 // Measured (8 packed segments, 8/2 heads x 256, up to 2,048 new tokens on up to 16,384 cached ones; fp32): 4,985 us on
-// fp32 MFMA (111 TFLOP/s of 157) -> 2,050 us; error against 64 bits 1.2e-6 -> 7.2e-7 of the result. What bounds it: per
+// fp32 MFMA (111 TFLOP/s of 157) -> 2,020 us; error against 64 bits 1.2e-6 -> 8.3e-7 of the result, and smaller than fp32
+// MFMA's where masked or negligible values are far larger than the others, below a sink, after a jump of the maximum
+// (with one E for a wave, from all values, it was 10^3 times larger there). What bounds it: per
 // tile the MFMAs take 43 % of the time, the LDS reads (64 KB per wave) and the VALU (softmax, splits, addresses) as
 // much each; copies without the loads / the splits / the LDS writes / the softmax are 13 / 11 / 8 / 6 % faster, one
 // without staging 30 %.
 constexpr int kF32QW = 16;      // queries per wave
 constexpr int kF32Heads = 4;    // query heads per workgroup
+constexpr int kDown = 5;        // a value row's size 2^(kTop - exponent) enters a probability's weight as 2^(kDown - exponent)
+constexpr int kNone = 140;      // E while nothing is held
+constexpr int kRoom = 4;        // a new E leaves the largest probability 2^kRoom below where it would change again
 
-// largest x over groups of N neighbouring lanes (8, 16, 32 or 64), in every lane
+// The largest m[r] over each group of N neighbouring lanes (8, 16, 32 or 64), for row r = l % 4 in lane l: the first two
+// exchanges halve the rows a lane keeps.
 template <int N>
-__device__ __forceinline__ float lanes_max(float x) {
-    x = fmaxf(x, dpp_f32<0xb1>(x));                  // quad_perm 1 0 3 2
-    x = fmaxf(x, dpp_f32<0x4e>(x));                  // quad_perm 2 3 0 1
-    x = fmaxf(x, dpp_f32<0x141>(x));                 // row_half_mirror: the other four of eight
-    if constexpr (N >= 16) x = fmaxf(x, dpp_f32<0x140>(x));   // row_mirror: the other eight of sixteen
+__device__ __forceinline__ float row_max4(const float (&m)[4], int lane) {
+    const bool odd = lane & 1, high = lane & 2;
+    const float a = fmaxf(odd ? m[1] : m[0], dpp_f32<0xb1>(odd ? m[0] : m[1]));   // quad_perm 1 0 3 2
+    const float b = fmaxf(odd ? m[3] : m[2], dpp_f32<0xb1>(odd ? m[2] : m[3]));
+    float x = fmaxf(high ? b : a, dpp_f32<0x4e>(high ? a : b));                   // quad_perm 2 3 0 1
+    x = fmaxf(x, dpp_f32<0x1b>(dpp_f32<0x141>(x)));  // lane ^ 4: row_half_mirror, then each quad reversed
+    if constexpr (N >= 16) x = fmaxf(x, dpp_f32<0x128>(x));   // row_ror:8 (lane ^ 8)
     if constexpr (N >= 32) {
         const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
         x = fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
@@ -628,14 +637,14 @@ __device__ __forceinline__ int v_row(int dim) {
 }
 
 // The lazy running maximum of a 16-query wave (scores s[kt][r] of lane l: query l % 16, keys 16 kt + 4 (l / 16) + r):
-// m is raised to the tile's maximum (sub-tile kt scaled by scale_kt > 0) only where that exceeds m by more than kLazy, so
-// p = 2^(s scale - m) stays <= 2^kLazy (exact in fp32, representable in bf16). Each lane first compares its own 8
+// m is raised to the tile's maximum (scaled by qscale) only where that exceeds m by more than kLazy, so
+// p = 2^(s qscale - m) stays <= 2^kLazy (exact in fp32, representable in bf16). Each lane first compares its own 8
 // scores; only when some lane of the wave exceeds the bound is the maximum over the query's 4 lanes formed, so the
-// result equals max-then-compare over all 32 keys while the common case needs no cross-lane exchange (scaling by a
-// positive factor is monotonic, so it commutes with max).
-__device__ __forceinline__ void lazy_max(const f32x4 (&s)[2], float& m, float scale0, float scale1) {
-    float t = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])) * scale0,
-                    fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])) * scale1);
+// result equals max-then-compare over all 32 keys while the common case needs no cross-lane exchange (scaling by
+// qscale > 0 is monotonic, so it commutes with max).
+__device__ __forceinline__ void lazy_max(const f32x4 (&s)[2], float& m, float qscale) {
+    float t = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])),
+                    fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3]))) * qscale;
     if (__any(t > m + kLazy)) {
         t = fmaxf(t, __shfl_xor(t, 16));
         t = fmaxf(t, __shfl_xor(t, 32));
@@ -752,9 +761,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                   "each unit slot of a wave must take one tensor");
     constexpr int NC = D / 32, ND = D / 16;          // 32-dim steps of the scores, 16-dim tiles of the output
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    float* ksc = reinterpret_cast<float*>(smem + 2 * STAGE);                   // [2 stages][8] 2^-(a key group's exponent)
-    int* vex = reinterpret_cast<int*>(ksc + 2 * GROUPS);                       // [2 stages][8] a value group's exponent
-    int* tab = vex + 2 * GROUPS;                                               // [kTabCache] block ids
+    float* ksc = reinterpret_cast<float*>(smem + 2 * STAGE);                   // [2 stages][32] 2^-(a key row's exponent)
+    float* vsc = ksc + 2 * kBKP;                                               // [2 stages][32] 2^(kDown - a value row's)
+    int* tab = reinterpret_cast<int*>(vsc + 2 * kBKP);                               // [kTabCache] block ids
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const WorkSlot ws = work_slot(a.Hkv, (a.G + kF32Heads - 1) / kF32Heads);
@@ -840,73 +849,78 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             }
         }
     };
-    auto stash = [&](int stage) __attribute__((always_inline)) {
+    // Splits and writes unit j: true if an infinite value was among its wave's. Then a second pass, INF, takes the rows'
+    // exponents from their finite values, and the infinities as infinite_alone does: they stay infinities without taking
+    // the others along. (Both in one pass, by branches, cost 5 % of the kernel.)
+    auto split = [&](int j, int stage, auto inf_c) __attribute__((always_inline)) {
+        constexpr bool INF = decltype(inf_c)::value;
         char* s = smem + stage * STAGE;
+        int g, pc;
+        const bool is_v = unit_of(j, g, pc);
+        float v[4][EL], big[4];
 #pragma unroll
-        for (int j = 0; j < NU; ++j) {
-            if (tid + 512 * j >= 2 * UNITS_T) continue;
-            int g, pc;
-            const bool is_v = unit_of(j, g, pc);
-            float v[4][EL];
-            float big = 0.0f;
+        for (int r = 0; r < 4; ++r) {
+            big[r] = 0.0f;
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-#pragma unroll
-                for (int d = 0; d < EL; ++d) {
-                    if constexpr (sizeof(TP) == 4) v[r][d] = __uint_as_float(st[j][r][d]);
-                    else v[r][d] = d & 1 ? bf16_hi(st[j][r][d >> 1]) : bf16_lo(st[j][r][d >> 1]);
-                    big = fmaxf(big, fabsf(v[r][d]));
-                }
-            // the group's exponent, from its finite values: an infinity stays one without taking its neighbours along
-            const bool odd = __any(big == INFINITY);
-            if (odd) {
-                big = 0.0f;
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-#pragma unroll
-                    for (int d = 0; d < EL; ++d) big = fmaxf(big, __builtin_isfinite(v[r][d]) ? fabsf(v[r][d]) : 0.0f);
+            for (int d = 0; d < EL; ++d) {
+                if constexpr (sizeof(TP) == 4) v[r][d] = __uint_as_float(st[j][r][d]);
+                else v[r][d] = d & 1 ? bf16_hi(st[j][r][d >> 1]) : bf16_lo(st[j][r][d >> 1]);
+                const float m = fabsf(v[r][d]);
+                big[r] = fmaxf(big[r], INF && m == INFINITY ? 0.0f : m);
             }
-            big = lanes_max<PER_ROW>(big);
-            const int e = big == 0.0f && is_v ? 126 : top_exponent(big);   // zero values: no bound on the others
-            const float f = __uint_as_float((uint32_t)(127 + e) << 23);
-            if (pc == 0) {
-                if (is_v) vex[stage * GROUPS + g] = e;
-                else ksc[stage * GROUPS + g] = __uint_as_float((uint32_t)(127 - e) << 23);
+        }
+        const float top = row_max4<PER_ROW>(big, lane);          // of row lane % 4, as pc % 4
+        const uint32_t size = __float_as_uint(fmaxf(top, 0x1p-112f)) & 0x7f800000u;
+        const float fl = __uint_as_float(((127u + 127u + kTop) << 23) - size);   // puts top into [2^kTop, 2^(kTop + 1))
+        if (pc < 4) {
+            const float out = __uint_as_float(size - ((uint32_t)(kTop - (is_v ? kDown : 0)) << 23));
+            (is_v ? vsc : ksc)[stage * kBKP + 4 * g + pc] = is_v && top == 0.0f ? 0.0f : out;   // zero values weigh 0
+        }
+        const float f[4] = {dpp_f32<0x00>(fl), dpp_f32<0x55>(fl), dpp_f32<0xaa>(fl), dpp_f32<0xff>(fl)};
+        // pieces of pairs: values of two keys (V^T rows hold keys side by side), of two dims (K)
+        Pieces pr[2 * EL];
+#pragma unroll
+        for (int i = 0; i < 2 * EL; ++i) {
+            const int d = i >> 1, r = 2 * (i & 1);          // V: dim d, keys r, r + 1
+            const int kr = i / (EL / 2), kd = 2 * (i % (EL / 2));   // K: key kr, dims kd, kd + 1
+            pr[i] = is_v ? split_pair(v[r][d] * f[r], v[r + 1][d] * f[r + 1])
+                         : split_pair(v[kr][kd] * f[kr], v[kr][kd + 1] * f[kr]);
+            if constexpr (INF) pr[i] = infinite_alone(pr[i]);
+        }
+        if (is_v) {                                  // V^T[row of the dim][the group's 4 keys]
+            char* dst = s + 2 * KPC + 8 * (g >> 2);
+#pragma unroll
+            for (int d = 0; d < EL; ++d) {
+                const int R = v_row<D>(pc * EL + d);
+                char* q = dst + 64 * R + 16 * ((g & 3) ^ swizzle(R));
+                *reinterpret_cast<u32x2*>(q) = (u32x2){pr[2 * d].hi, pr[2 * d + 1].hi};
+                *reinterpret_cast<u32x2*>(q + KPC) = (u32x2){pr[2 * d].lo, pr[2 * d + 1].lo};
             }
-            // pieces of pairs: values of two keys (V^T rows hold keys side by side), of two dims (K)
-            Pieces pr[2 * EL];
+        } else {                                     // K[key][dims pc EL ..]
 #pragma unroll
-            for (int i = 0; i < 2 * EL; ++i) {
-                const int d = i >> 1, r = 2 * (i & 1);          // V: dim d, keys r, r + 1
-                const int kr = i / (EL / 2), kd = 2 * (i % (EL / 2));   // K: key kr, dims kd, kd + 1
-                pr[i] = is_v ? split_pair(v[r][d] * f, v[r + 1][d] * f) : split_pair(v[kr][kd] * f, v[kr][kd + 1] * f);
-            }
-            if (odd) {
+            for (int r = 0; r < 4; ++r) {
+                const int row = 4 * g + r;
+                char* q = s + 2 * D * row + 16 * k_unit<D>(row, pc * EL / 8) + 2 * (pc * EL % 8);
 #pragma unroll
-                for (int i = 0; i < 2 * EL; ++i) pr[i].lo = rest_of(pr[i]);
-            }
-            if (is_v) {                              // V^T[row of the dim][the group's 4 keys]
-                char* dst = s + 2 * KPC + 8 * (g >> 2);
-#pragma unroll
-                for (int d = 0; d < EL; ++d) {
-                    const int R = v_row<D>(pc * EL + d);
-                    char* q = dst + 64 * R + 16 * ((g & 3) ^ swizzle(R));
-                    *reinterpret_cast<u32x2*>(q) = (u32x2){pr[2 * d].hi, pr[2 * d + 1].hi};
-                    *reinterpret_cast<u32x2*>(q + KPC) = (u32x2){pr[2 * d].lo, pr[2 * d + 1].lo};
-                }
-            } else {                                 // K[key][dims pc EL ..]
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int row = 4 * g + r;
-                    char* q = s + 2 * D * row + 16 * k_unit<D>(row, pc * EL / 8) + 2 * (pc * EL % 8);
-#pragma unroll
-                    for (int d = 0; d < EL; d += 4) {
-                        const int i = (r * EL + d) / 2;
-                        *reinterpret_cast<u32x2*>(q + 2 * d) = (u32x2){pr[i].hi, pr[i + 1].hi};
-                        *reinterpret_cast<u32x2*>(q + 2 * d + KPC) = (u32x2){pr[i].lo, pr[i + 1].lo};
-                    }
+                for (int d = 0; d < EL; d += 4) {
+                    const int i = (r * EL + d) / 2;
+                    *reinterpret_cast<u32x2*>(q + 2 * d) = (u32x2){pr[i].hi, pr[i + 1].hi};
+                    *reinterpret_cast<u32x2*>(q + 2 * d + KPC) = (u32x2){pr[i].lo, pr[i + 1].lo};
                 }
             }
+        }
+        return !INF && __any(top == INFINITY);
+    };
+    auto stash = [&](int t_rel, int stage) __attribute__((always_inline)) {
+        bool any = false;
+#pragma unroll
+        for (int j = 0; j < NU; ++j)
+            if (tid + 512 * j < 2 * UNITS_T) any |= split(j, stage, std::false_type{});
+        if (any) {                                   // its rows again (held through the first pass they would cost spills)
+            issue(t_rel);
+#pragma unroll
+            for (int j = 0; j < NU; ++j)
+                if (tid + 512 * j < 2 * UNITS_T) split(j, stage, std::true_type{});
         }
     };
 
@@ -919,9 +933,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int qlast = a.causal ? p0 + min(half * kF32QW + kF32QW, nq) - 1 : n_keys - 1;
     const int lo_edge = a.window > 0 ? qlast - a.window : INT_MIN;
     u32x4 qh[NC], ql[NC];                            // Q[query][32 c + 8 qq .. + 7] * 2^(its exponent), two pieces
-    f32x4 o[ND];                                     // O^T[row 16 dt + 4 qq + r][query] * 2^E
+    f32x4 o[ND];                                     // O^T[row 16 dt + 4 qq + r][query] * 2^(E + kDown)
     float m_run = -INFINITY, l_run = 0.0f, qs = a.qscale;
-    int E = 0;
+    int E = kNone;
     if (active) {
         const long long qb = ((long long)(row0 + (qi < nq ? qi : nq - 1)) * a.Hq + head) * D + 8 * qq;
         float q[NC][8], big = 0.0f;
@@ -948,9 +962,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int c = 0; c < NC; ++c)
 #pragma unroll
             for (int d = 0; d < 4; ++d) {
-                const Pieces p = split_pair(ldexpf(q[c][2 * d], e), ldexpf(q[c][2 * d + 1], e));
+                const Pieces p = infinite_alone(split_pair(ldexpf(q[c][2 * d], e), ldexpf(q[c][2 * d + 1], e)));
                 qh[c][d] = p.hi;
-                ql[c][d] = rest_of(p);
+                ql[c][d] = p.lo;
             }
 #pragma unroll
         for (int dt = 0; dt < ND; ++dt) o[dt] = f32x4{};
@@ -978,17 +992,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
             for (int kt = 0; kt < 2; ++kt) x[kt] = mfma_f16(kh[kt], ql[c], x[kt]);
         }
-        // never 0: a masked score's product must stay -inf
-        const float f0 = fmaxf(qs * ksc[stage * GROUPS + qq], FLT_MIN);
-        const float f1 = fmaxf(qs * ksc[stage * GROUPS + 4 + qq], FLT_MIN);
-        int ve[GROUPS], vmin = 126;
+        f32x4 f[2], w[2];                            // the scales of the lane's scores, and of its probabilities
 #pragma unroll
-        for (int g = 0; g < GROUPS; ++g) {
-            ve[g] = __builtin_amdgcn_readfirstlane(vex[stage * GROUPS + g]);
-            vmin = min(vmin, ve[g]);
+        for (int kt = 0; kt < 2; ++kt) {
+            f[kt] = *reinterpret_cast<const f32x4*>(ksc + stage * kBKP + 16 * kt + 4 * qq);
+            w[kt] = *reinterpret_cast<const f32x4*>(vsc + stage * kBKP + 16 * kt + 4 * qq);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) f[kt][r] = fmaxf(qs * f[kt][r], FLT_MIN);   // never 0: -inf must stay -inf
+            s[kt] += x[kt];
         }
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt) s[kt] += x[kt];
         // lane (qc, qq), register r of sub-tile kt: key k0 + 16 kt + 4 qq + r
         if (k0 + kBKP - 1 > qfirst || k0 <= lo_edge) {
 #pragma unroll
@@ -1000,45 +1012,45 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 }
         }
         const float m_prev = m_run;
-        lazy_max(s, m_run, f0, f1);
+        const f32x4 sf[2] = {s[0] * f[0], s[1] * f[1]};
+        lazy_max(sf, m_run, 1.0f);
         const float mb = m_run == -INFINITY ? 0.0f : m_run;
-        // probabilities (at most 2^kLazy) enter as p 2^(E - a value group's exponent) < 2^(kTop + 1): E falls when a
-        // group of larger values comes
-        const int e_new = min(E, vmin + kTop + 1 - (int)kLazy);
-        const bool first = t_rel == 0;
-        if (first) E = vmin + kTop + 1 - (int)kLazy;
-        else if (e_new < E) {                        // uniform
+        // probabilities enter as p w 2^E < 2^(kTop + 1), w the size of the key's values: only what counts for the query
+        // bounds the others (a masked key's p is 0, zero values' w)
+        float p[8], sum = 0.0f, top = 0.0f;
 #pragma unroll
-            for (int dt = 0; dt < ND; ++dt)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) o[dt][r] = ldexpf(o[dt][r], e_new - E);
-            E = e_new;
+        for (int i = 0; i < 8; ++i) {
+            p[i] = fast_exp2(fmaf(s[i >> 2][i & 3], f[i >> 2][i & 3], -mb));
+            sum += p[i];                             // this lane's keys; the 4 lanes of a query are summed at the end
         }
-        if (__any(m_run != m_prev)) {
-            const float alpha = fast_exp2(m_prev - mb);     // 0 on the first tile (m_prev = -inf)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            p[i] *= w[i >> 2][i & 3];
+            top = fmaxf(top, p[i]);
+        }
+        if (__any(m_run != m_prev || top >= ldexpf(1.0f, kTop + 1 - E))) {
+            // what is held shrinks by alpha (0 on the first tile: m_prev = -inf), and E rises with it; E falls where
+            // something larger comes, with room for more
+            const float alpha = fast_exp2(m_prev - mb);
+            int e_new = min(E + 127 - (int)(__float_as_uint(alpha) >> 23), kNone);
+            top = fmaxf(top, __shfl_xor(top, 16));
+            top = fmaxf(top, __shfl_xor(top, 32));
+            if (top >= ldexpf(1.0f, kTop + 1 - e_new)) e_new = kTop - kRoom - ((int)(__float_as_uint(top) >> 23) - 127);
+            const float by = ldexpf(alpha, e_new - E);
+            E = e_new;
             l_run *= alpha;
 #pragma unroll
-            for (int dt = 0; dt < ND; ++dt) o[dt] *= alpha;
+            for (int dt = 0; dt < ND; ++dt) o[dt] *= by;
         }
+        l_run += sum;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) p[i] = ldexpf(p[i], E);
         u32x4 ph, pl;
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt) {
-            int g = ve[4 * kt];
-#pragma unroll
-            for (int i = 1; i < 4; ++i) g = qq == i ? ve[4 * kt + i] : g;
-            float p[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                p[r] = fast_exp2(fmaf(s[kt][r], kt ? f1 : f0, -mb));
-                l_run += p[r];                       // this lane's keys; the 4 lanes of a query are summed at the end
-                p[r] = ldexpf(p[r], E - g);
-            }
-#pragma unroll
-            for (int r = 0; r < 2; ++r) {
-                const Pieces pp = split_pair(p[2 * r], p[2 * r + 1]);
-                ph[2 * kt + r] = pp.hi;
-                pl[2 * kt + r] = pp.lo;
-            }
+        for (int i = 0; i < 4; ++i) {
+            const Pieces pp = split_pair(p[2 * i], p[2 * i + 1]);
+            ph[i] = pp.hi;
+            pl[i] = pp.lo;
         }
 #pragma unroll
         for (int d0 = 0; d0 < ND; d0 += 2) {
@@ -1063,12 +1075,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // stages before it computes, the other after, so that one's splits (VALU) run beside the other's MFMAs.
     if (n_tiles > 0) {
         issue(0);
-        stash(0);
+        stash(0, 0);
         if (n_tiles > 1) issue(1);
         lds_barrier();
         auto produce = [&](int t) __attribute__((always_inline)) {
             if (t + 1 < n_tiles) {
-                stash((t + 1) & 1);
+                stash(t + 1, (t + 1) & 1);
                 if (t + 2 < n_tiles) issue(t + 2);
             }
         };
@@ -1091,7 +1103,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int r = 0; r < 4; ++r)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) od[4 * q + r][i] = ldexpf(o[q + D / 64 * i][r], -E);
+            for (int i = 0; i < 4; ++i) od[4 * q + r][i] = ldexpf(o[q + D / 64 * i][r], -kDown - E);
     finish_queries<D, true>(a, we, od, m_run, l_run, head, half, row0, nq);
 }
 
@@ -1332,7 +1344,7 @@ __global__ __launch_bounds__(kB16Threads) void prefill_attention_b16(PrefillArgs
         for (int i = 0; i < kB16Ahead; ++i) va[i] = vread(i);
         __builtin_amdgcn_sched_barrier(0);
         const float m_prev = m_run;
-        lazy_max(s, m_run, a.qscale, a.qscale);
+        lazy_max(s, m_run, a.qscale);
         const float mb = m_run == -INFINITY ? 0.0f : m_run;
         if (__any(m_run != m_prev)) {
             const float alpha = fast_exp2(m_prev - mb);     // 0 on the first tile (m_prev = -inf)
@@ -1469,7 +1481,7 @@ int rk_paged_prefill(float* out, const void* q, int q_dtype, const void* k_new, 
         hipLaunchKernelGGL(fn, dim3(n_work * Hkv * chunks), dim3(kB16Threads), lds, s, a);
         return check_launch("prefill_attention_b16");
     }
-    const size_t lds = (size_t)2 * 4 * kBKP * D * sizeof(uint16_t) + 2 * (kBKP / 4) * 2 * sizeof(int) +
+    const size_t lds = (size_t)2 * 4 * kBKP * D * sizeof(uint16_t) + 4 * kBKP * sizeof(float) +
                        (tab_lds ? kTabCache * sizeof(int) : 0);
     const bool f32_pool = pool_dtype == RK_F32;
 #define RK_F32_PICK(DD)                                                                                      \

@@ -246,3 +246,81 @@ def test_fp32_operands_over_magnitudes(backend, Hq, Hkv, d, pool):
         over = ((got[:, h].double() - want).abs() / bound)[:, ~held].max()
         assert over < 1.0, (h, float(over))
         assert not torch.isfinite(got[:, h][:, held]).any()
+
+
+def one_segment(q, k, v, past, pool, bs=16):
+    """A PrefillCase of one segment of len(q) queries after `past` cached positions, K and V [S, Hkv, d] in the pool type
+    (an fp32 q with a bf16 pool takes fp32 operands)."""
+    S, n = k.shape[0], q.shape[0]
+    case = wl.prefill_case([n], [past], q.shape[1], k.shape[1], q.shape[2], bs, torch.float32, seed=1)
+    rows = (case.tables[0].long()[:, None] * bs + torch.arange(bs)).flatten()[:S]
+    case.q, (k, v) = q, (k.to(pool), v.to(pool))
+    case.k_pool, case.v_pool = case.k_pool.to(pool), case.v_pool.to(pool)
+    case.k_pool.view(-1, *k.shape[1:])[rows[:past]], case.v_pool.view(-1, *k.shape[1:])[rows[:past]] = k[:past], v[:past]
+    case.k_new, case.v_new = k[past:].clone(), v[past:].clone()
+    return case, k, v
+
+
+def in_64_bits(q, k, v, past):
+    """Causal attention [n, Hq, d] in 64 bits, and the bound of test_fp32_operands_over_magnitudes, in which only the keys
+    a query sees count: its scores' largest rounding and the probabilities' mass over |v|."""
+    n, Hq, d = q.shape
+    S, G = k.shape[0], Hq // k.shape[1]
+    kd, vd, qd = k.double().repeat_interleave(G, 1), v.double().repeat_interleave(G, 1), q.double()
+    hidden = torch.arange(S)[None, :] > torch.arange(past, past + n)[:, None]
+    want, bound = torch.empty_like(qd), torch.empty_like(qd)
+    for h in range(Hq):
+        s = (qd[:, h] @ kd[:, h].T) / d ** 0.5
+        ds = (qd[:, h].abs() @ kd[:, h].abs().T) / d ** 0.5 * (4 + d / 32) * 2.0 ** -24
+        pr = torch.softmax(s.masked_fill(hidden, float("-inf")), -1)
+        ds = (ds + s.abs() * 2.0 ** -24).masked_fill(hidden | (pr < 2.0 ** -80), 0.0).amax(1, keepdim=True)
+        want[:, h], bound[:, h] = pr @ vd[:, h], (2 * ds + (8 + 3 * S / 32) * 2.0 ** -24) * (pr @ vd[:, h].abs())
+    return want, bound
+
+
+def aligned(n, S, Hq, Hkv, d, g):
+    """Queries near one vector, and what to add to a key for a score of 1: scores that can be chosen."""
+    u = torch.randn(d, generator=g)
+    q = u + 1e-3 * torch.randn(n, Hq, d, generator=g)
+    return q, u * d ** 0.5 / u.dot(u), 1e-2 * torch.randn(S, Hkv, d, generator=g), torch.randn(S, Hkv, d, generator=g)
+
+
+@pytest.mark.parametrize("Hq,Hkv,d,pool", [(8, 2, 256, torch.float32), (16, 4, 128, torch.float32),
+                                           (14, 2, 64, torch.float32), (8, 2, 256, torch.bfloat16),
+                                           (8, 8, 64, torch.bfloat16)])
+@pytest.mark.parametrize("kind", ["masked values", "masked keys", "negligible", "sink", "jump", "channels"])
+def test_fp32_operands_see_only_what_counts(backend, Hq, Hkv, d, pool, kind):
+    """The fp32-operand kernel where values that do not count are far larger than those that do: keys masked for some
+    queries of a block with values (or keys) 2^24 times the others', a visible key of probability 2^-60 with values 2^20
+    times the others', a sink of zero values 2^24 times as probable as the rest, values 2^20 times the others' whose keys
+    are outweighed 2^100 times by later ones; and q and k channels 2^12 up and down. Each output is held to the bound
+    over what the query sees alone."""
+    g = torch.Generator().manual_seed(d + Hq)
+    n, past = 64, 448
+    S = n + past
+    q, unit, k, v = aligned(n, S, Hq, Hkv, d, g)
+    ln2 = 0.6931471805599453
+    if kind == "masked values":
+        v[past + 5::7] *= 2.0 ** 24
+        k[past + 5::7] -= 60 * ln2 * unit                   # of no weight where they are visible
+    elif kind == "masked keys":
+        k[past + 5::7] -= 2.0 ** 24 * unit
+    elif kind == "negligible":
+        k[[9, 200]] -= 60 * ln2 * unit
+        v[[9, 200]] *= 2.0 ** 20
+    elif kind == "sink":
+        k[0] += 24 * ln2 * unit
+        v[0] = 0.0
+    elif kind == "jump":
+        v[:40] *= 2.0 ** 20
+        k[300:] += 100 * ln2 * unit
+    else:
+        e = torch.exp2(torch.randint(-6, 7, (d,), generator=g).float())
+        q, k = torch.randn(n, Hq, d, generator=g) * e, torch.randn(S, Hkv, d, generator=g) / e
+    case, k, v = one_segment(q, k, v, past, pool)
+    got, _, _ = run_gpu(backend, case, gate=False, exact=True)
+    want, bound = in_64_bits(q, k, v, past)
+    over = ((got.double() - want).abs() / bound).max()
+    print(f"{kind} {Hq}/{Hkv} x {d} {pool}: {float(over):.3f} of the bound, rel err "
+          f"{float((got.double() - want).abs().max() / want.abs().max()):.1e}")
+    assert over < 1.0
