@@ -32,11 +32,12 @@ __device__ __forceinline__ Pieces split_pair(float a, float b) {
     const f16x2 l = __builtin_convertvector((f32x2_t){a - (float)h[0], b - (float)h[1]}, f16x2);
     return {__builtin_bit_cast(uint32_t, h), __builtin_bit_cast(uint32_t, l)};
 }
-// Where a value was infinite: it has no rest (inf - inf would make it NaN).
-__device__ __forceinline__ Pieces infinite_alone(Pieces p) {
+// Where a value was infinite: it is all in lo, which meets only the other operand's hi, whose sign is the value's (hi times
+// the other's lo, of either sign or 0, would make it NaN).
+__device__ __forceinline__ Pieces infinite_in_lo(Pieces p) {
     const uint32_t m = p.hi & 0x7fff7fffu;           // exponent 31 with mantissa 0
     const uint32_t inf = ((m & 0xffffu) == 0x7c00u ? 0xffffu : 0u) | (m >> 16 == 0x7c00u ? 0xffff0000u : 0u);
-    return {p.hi, p.lo & ~inf};
+    return {p.hi & ~inf, (p.lo & ~inf) | (p.hi & inf)};
 }
 
 // Rows of 32 fp16 (64 bytes) in LDS: the 16-byte unit u of row R sits at u ^ swizzle(R). A read of lane l: row l % 16,

@@ -763,7 +763,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     extern __shared__ __attribute__((aligned(16))) char smem[];
     float* ksc = reinterpret_cast<float*>(smem + 2 * STAGE);                   // [2 stages][32] 2^-(a key row's exponent)
     float* vsc = ksc + 2 * kBKP;                                               // [2 stages][32] 2^(kDown - a value row's)
-    int* tab = reinterpret_cast<int*>(vsc + 2 * kBKP);                               // [kTabCache] block ids
+    char* inf = reinterpret_cast<char*>(vsc + 2 * kBKP);                       // [2 stages][8 waves] infinities staged
+    int* tab = reinterpret_cast<int*>(inf + 16);                               // [kTabCache] block ids
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const WorkSlot ws = work_slot(a.Hkv, (a.G + kF32Heads - 1) / kF32Heads);
@@ -850,7 +851,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
     };
     // Splits and writes unit j: true if an infinite value was among its wave's. Then a second pass, INF, takes the rows'
-    // exponents from their finite values, and the infinities as infinite_alone does: they stay infinities without taking
+    // exponents from their finite values, and the infinities as infinite_in_lo does: they stay infinities without taking
     // the others along. (Both in one pass, by branches, cost 5 % of the kernel.)
     auto split = [&](int j, int stage, auto inf_c) __attribute__((always_inline)) {
         constexpr bool INF = decltype(inf_c)::value;
@@ -885,7 +886,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             const int kr = i / (EL / 2), kd = 2 * (i % (EL / 2));   // K: key kr, dims kd, kd + 1
             pr[i] = is_v ? split_pair(v[r][d] * f[r], v[r + 1][d] * f[r + 1])
                          : split_pair(v[kr][kd] * f[kr], v[kr][kd + 1] * f[kr]);
-            if constexpr (INF) pr[i] = infinite_alone(pr[i]);
+            if constexpr (INF) pr[i] = infinite_in_lo(pr[i]);
         }
         if (is_v) {                                  // V^T[row of the dim][the group's 4 keys]
             char* dst = s + 2 * KPC + 8 * (g >> 2);
@@ -922,6 +923,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             for (int j = 0; j < NU; ++j)
                 if (tid + 512 * j < 2 * UNITS_T) split(j, stage, std::true_type{});
         }
+        if (lane == 0) inf[8 * stage + wave] = any;
     };
 
     // ---- per-wave query state
@@ -962,7 +964,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int c = 0; c < NC; ++c)
 #pragma unroll
             for (int d = 0; d < 4; ++d) {
-                const Pieces p = infinite_alone(split_pair(ldexpf(q[c][2 * d], e), ldexpf(q[c][2 * d + 1], e)));
+                const Pieces p = infinite_in_lo(split_pair(ldexpf(q[c][2 * d], e), ldexpf(q[c][2 * d + 1], e)));
                 qh[c][d] = p.hi;
                 ql[c][d] = p.lo;
             }
@@ -992,6 +994,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
             for (int kt = 0; kt < 2; ++kt) x[kt] = mfma_f16(kh[kt], ql[c], x[kt]);
         }
+        const u32x2 any = *reinterpret_cast<const u32x2*>(inf + 8 * stage);
         f32x4 f[2], w[2];                            // the scales of the lane's scores, and of its probabilities
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt) {
@@ -1028,7 +1031,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             p[i] *= w[i >> 2][i & 3];
             top = fmaxf(top, p[i]);
         }
-        if (__any(m_run != m_prev || top >= ldexpf(1.0f, kTop + 1 - E))) {
+        if (__any(m_run != m_prev || top >= ldexpf(1.0f, kTop + 1 - E) || (any[0] | any[1]))) {
             // what is held shrinks by alpha (0 on the first tile: m_prev = -inf), and E rises with it; E falls where
             // something larger comes, with room for more
             const float alpha = fast_exp2(m_prev - mb);
@@ -1041,6 +1044,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             l_run *= alpha;
 #pragma unroll
             for (int dt = 0; dt < ND; ++dt) o[dt] *= by;
+            if (any[0] | any[1]) {                   // infinite values: a probability above 0 keeps them, as the least fp16
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    if (fast_exp2(fmaf(s[i >> 2][i & 3], f[i >> 2][i & 3], -mb)) > 0.0f) p[i] = fmaxf(p[i], ldexpf(0x1p-24f, -E));
+            }
         }
         l_run += sum;
 #pragma unroll
@@ -1481,7 +1489,7 @@ int rk_paged_prefill(float* out, const void* q, int q_dtype, const void* k_new, 
         hipLaunchKernelGGL(fn, dim3(n_work * Hkv * chunks), dim3(kB16Threads), lds, s, a);
         return check_launch("prefill_attention_b16");
     }
-    const size_t lds = (size_t)2 * 4 * kBKP * D * sizeof(uint16_t) + 4 * kBKP * sizeof(float) +
+    const size_t lds = (size_t)2 * 4 * kBKP * D * sizeof(uint16_t) + 4 * kBKP * sizeof(float) + 16 +
                        (tab_lds ? kTabCache * sizeof(int) : 0);
     const bool f32_pool = pool_dtype == RK_F32;
 #define RK_F32_PICK(DD)                                                                                      \

@@ -324,3 +324,35 @@ def test_fp32_operands_see_only_what_counts(backend, Hq, Hkv, d, pool, kind):
     print(f"{kind} {Hq}/{Hkv} x {d} {pool}: {float(over):.3f} of the bound, rel err "
           f"{float((got.double() - want).abs().max() / want.abs().max()):.1e}")
     assert over < 1.0
+
+
+@pytest.mark.parametrize("Hq,Hkv,d,pool", [(8, 2, 256, torch.float32), (16, 4, 128, torch.bfloat16),
+                                           (14, 2, 64, torch.float32)])
+def test_fp32_operands_and_infinities(backend, Hq, Hkv, d, pool):
+    """An infinite value gives the queries that see its key an infinity of its sign in its dim, however small the
+    probability (2^-60 here for one) and whatever its row's other values, and nothing else; a key whose score is -inf
+    drops out."""
+    g = torch.Generator().manual_seed(d)
+    n, past = 40, 100
+    S = n + past
+    q, unit, k, v = aligned(n, S, Hq, Hkv, d, g)
+    q[..., 7] = q[..., 7].abs() + 0.1
+    k[50] -= 60 * 0.6931471805599453 * unit
+    v[60] = 0.0
+    marks = [(3, 0, 5, 1), (20, 1, 9, -1), (50, 0, 11, 1), (60, 1, 13, -1), (past - 1, 0, 15, 1)]
+    for j, h, dim, sign in marks:
+        v[j, h, dim] = sign * float("inf")
+    dropped = [17, 33, 90]
+    for j in dropped:
+        k[j, :, 7] = float("-inf")
+        v[j] = 1e6
+    case, k, v = one_segment(q, k, v, past, pool)
+    got, _, _ = run_gpu(backend, case, gate=False, exact=True)
+    seen = [j for j in range(S) if j not in dropped]
+    vf = torch.where(torch.isinf(v), torch.zeros_like(v), v)
+    want, bound = in_64_bits(q, k[seen], vf[seen], past - len(dropped))
+    G, finite = Hq // Hkv, torch.ones(n, Hq, d, dtype=torch.bool)
+    for _, h, dim, sign in marks:
+        assert (got[:, h * G:(h + 1) * G, dim] == sign * float("inf")).all(), (h, dim)
+        finite[:, h * G:(h + 1) * G, dim] = False
+    assert ((got.double() - want).abs() / bound)[finite].max() < 1.0
