@@ -297,7 +297,7 @@ PREFILL_BLOCK = 32          # queries per work item of rk_paged_prefill
 PREFILL_TILE = 32           # key positions per tile of rk_paged_prefill
 PREFILL_SPLIT_TILES = None  # None: split only when the blocks x KV heads leave CUs idle; an int forces a split size
 PREFILL_MIN_SPLIT = 32      # the smallest automatic piece, in tiles (1024 keys: the merge stays a small fraction)
-PREFILL_BALANCE_PIECES = 2  # balance split: no piece above half a CU's share of the tiles
+PREFILL_BALANCE_PIECES = 3  # balance split: no piece above a third of a CU's share of the tiles
 
 
 def prefill_split_tiles(spans: list[int], heads: int, n_cu: int, balance: bool = False) -> int:
@@ -308,10 +308,11 @@ def prefill_split_tiles(spans: list[int], heads: int, n_cu: int, balance: bool =
     unless balance: then blocks longer than 1/PREFILL_BALANCE_PIECES of a CU's share are cut to that size (at least
     2 PREFILL_MIN_SPLIT tiles), so that the last workgroups to start end close together. balance is for the
     fp32-operand kernel (one workgroup per CU, where a packed batch like config 5's 632 uneven workgroups on 256
-    CUs leaves ~14% of the CU time idle at the end): 8 segments of 552 GFLOP take 2,056-2,157 us at a whole share,
-    2,070-2,077 at a half, 2,121-2,210 at a quarter, 2,276-2,285 at an eighth; 4 segments at 16/4 heads x 128 879-902 /
-    894-898 / 919 / 965. A piece costs a partial record and its share of the merge, and on the bf16-operand kernel the longer start-up
-    of its producer pipeline outweighs the gain."""
+    CUs leaves ~14% of the CU time idle at the end). Over six packs (2 to 16 segments, 8k to 80k keys) at each of 8/2
+    heads x 256, 16/4 x 128 and 14/2 x 64, 0.14 to 4 ms, a whole share, a half, a third, a quarter and an eighth sum to
+    17.2, 17.1, 17.0, 17.0 and 17.1 ms, and are at worst 10, 7, 5, 4 and 8 % above the best of them; a pack of 552
+    GFLOP takes 2,020, 2,020 and 2,085 us at a half, a third and a quarter. A piece costs a partial record and its share
+    of the merge, and on the bf16-operand kernel the longer start-up of its producer pipeline outweighs the gain."""
     if not spans:
         return 0
     total = sum(spans) * heads

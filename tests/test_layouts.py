@@ -132,7 +132,7 @@ def test_prefill_auto_split():
 
 def test_prefill_balance_split():
     """The balance split of the fp32-operand kernel: with enough workgroups to fill the CUs, blocks longer than a
-    quarter of a CU's share of the tiles are cut to that size (never below two minimum pieces), and nothing is cut
+    third of a CU's share of the tiles are cut to that size (never below two minimum pieces), and nothing is cut
     when every block is already that short."""
     from native import kernels
     gen = torch.Generator().manual_seed(5)                                  # config 5's draw
