@@ -155,3 +155,29 @@ def test_chunked_delta_calls_replay_in_order():
         torch.cuda.synchronize()
         for got, ref in zip(outs + [S], want):
             assert torch.equal(got, ref)
+
+
+@pytest.mark.parametrize("kind,M", [("int4", 64), ("int8", 300), ("bf16", 40), ("bf16", 600)])
+def test_many_row_linears_in_a_graph(backend, kind, M):
+    """An MLP past the row kernels' 32 rows (each form of rk_linear_gemm, with K-splits), whose workspaces are tensors of
+    the calls: every replay gives the eager bits for the inputs it finds, with eager work and synchronizations between."""
+    g = torch.Generator(device=DEV).manual_seed(M)
+    r = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    fmt = lambda w: w.bfloat16() if kind == "bf16" else quant.quantize(w, kind)
+    w_gu, w_dn = fmt(r(2 * 1536, 1024) / 32), fmt(r(1024, 1536) / 40)
+    x, res = r(M, 1024), r(M, 1024)
+    run = lambda: backend.linear(backend.swiglu(x, w_gu), w_dn, residual=res)
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        run()
+        stream.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            y = run()
+    for _ in range(4):
+        x.copy_(r(M, 1024))
+        want = run()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)

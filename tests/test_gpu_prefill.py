@@ -210,7 +210,7 @@ def test_split_item_with_an_empty_piece(backend, dtype, Hq, Hkv, d, tol):
                                            (4, 4, 64, torch.bfloat16)])
 def test_fp32_operands_over_magnitudes(backend, Hq, Hkv, d, pool):
     """The fp32-operand kernel on keys, values and queries whose rows differ by powers of two (its operands are scaled by
-    row and by group of four rows), with groups of zero values, large values that come late, and an infinite value,
+    row), with groups of zero values, large values that come late, and an infinite value,
     against attention in 64 bits. Bound, per output: the scores' rounding (each |q k| to 2^-22, the sum of D of them in
     D / 32 steps) moves every probability by that much twice (numerator and sum), and the products p v are rounded to
     2^-22 each and summed in as many fp32 steps as there are tiles."""
