@@ -39,9 +39,9 @@ def _stream(dev: torch.device) -> int:
 
 
 CALLS_PATH = Path(__file__).resolve().parent / "rk_calls.so"
-CALLED = ("rk_abi_version", "rk_linear_workspace_bytes", "rk_linear_rows_ex2", "rk_swiglu_rows", "rk_rms_norm", "rk_layer_norm",
-          "rk_paged_decode_workspace_bytes", "rk_paged_decode", "rk_paged_decode_planned", "rk_deltanet_decode",
-          "rk_attn_prep")
+CALLED = ("rk_abi_version", "rk_linear_workspace_bytes", "rk_linear_rows_ex2", "rk_swiglu_rows", "rk_rms_norm",
+          "rk_layer_norm", "rk_paged_decode_workspace_bytes", "rk_paged_decode", "rk_paged_decode_planned",
+          "rk_deltanet_decode", "rk_attn_prep")
 _native_calls = None
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)      # the current stream's handle of a device index
 

@@ -446,7 +446,9 @@ Layout layout(int M, int N, int K, int w_type, bool glu) {
     for (int f = 0; f < 3; ++f) {
         const long long t = (long long)((l.Mc + kTiles[f][0] - 1) / kTiles[f][0]) * (((long long)rows + kTiles[f][1] - 1) / kTiles[f][1]);
         const RoundCost& c = kRound[quant][f];
-        for (int sp = 1; sp <= 16 && (sp == 1 || (l.steps / sp >= 8 && (long long)sp * l.Mc * l.Np * 4 <= kPartBytes)); ++sp) {
+        for (int sp = 1; sp <= 16; ++sp) {
+            // splits of at least 8 steps, for at most two rounds of workgroups, their sums within kPartBytes
+            if (sp > 1 && (l.steps < 8 * sp || t * sp > 2 * cus || (long long)sp * l.Mc * l.Np * 4 > kPartBytes)) break;
             const long long rounds = (t * sp + cus - 1) / cus;
             const double full = (double)(t * sp) / (double)(rounds * cus);
             double us = (double)rounds * (c.start + (c.step + c.full * full) * ((l.steps + sp - 1) / sp));
@@ -463,6 +465,23 @@ Layout layout(int M, int N, int K, int w_type, bool glu) {
     l.us = (double)runs * (slabs * l.us + 6.6 + 1.5e-6 * (double)l.Mc * K);  // split_rows
     l.total = l.part + (l.S > 1 ? (size_t)l.S * l.Mc * l.Np * 4 : 0);
     return l;
+}
+
+// Which form takes a call, and the workspace for it (scales or mins at an odd address send a call to the tiles)
+struct Choice {
+    Layout l;
+    MidPlan p;
+    bool mid;
+    size_t total;
+};
+
+Choice choose(int M, int N, int K, int w_type, int glu) {
+    Choice c;
+    c.l = layout(M, N, K, w_type, glu != 0);
+    c.p = mid_plan(M, N, K, w_type, glu);
+    c.mid = c.p.us > 0.0 && c.p.us < c.l.us;
+    c.total = c.mid && c.p.total > c.l.total ? c.p.total : c.l.total;
+    return c;
 }
 
 template <int WM, int WN, int TI>
@@ -494,22 +513,18 @@ extern "C" {
 
 size_t rk_linear_gemm_workspace_bytes(int M, int N, int K, int w_type, int glu) {
     if (M < 1 || N < 1 || K < kQB || K % kQB) return 0;
-    // either form may run (an odd address of the scales sends a call to this one)
-    const Layout l = layout(M, N, K, w_type, glu != 0);
-    const size_t mid = mid_takes(M, N, K, w_type, glu, nullptr, nullptr, l.us) ? mid_workspace_bytes(M, N, K, w_type, glu) : 0;
-    return l.total > mid ? l.total : mid;
+    return choose(M, N, K, w_type, glu).total;
 }
 
 int rk_linear_gemm_plan(int M, int N, int K, int w_type, int glu, int* plan) {
     if (M < 1 || N < 1 || K < kQB || K % kQB || (glu && N % 2) || !plan)
         return fail(RK_ERR_ARG, "rk_linear_gemm_plan: M %d, N %d, K %d", M, N, K);
-    const Layout l = layout(M, N, K, w_type, glu != 0);
-    const bool mid = mid_takes(M, N, K, w_type, glu, nullptr, nullptr, l.us);
+    const Choice c = choose(M, N, K, w_type, glu);
     const int cols = glu ? N / 2 : N;
-    plan[0] = mid ? 0 : 1 + l.form;
-    plan[1] = mid ? mid_splits(M, N, K, w_type, glu) : l.S;
-    plan[2] = mid ? 1 : (cols + l.slab - 1) / l.slab;
-    plan[3] = mid ? 1 : (M + l.Mc - 1) / l.Mc;
+    plan[0] = c.mid ? 0 : 1 + c.l.form;
+    plan[1] = c.mid ? c.p.S : c.l.S;
+    plan[2] = c.mid ? 1 : (cols + c.l.slab - 1) / c.l.slab;
+    plan[3] = c.mid ? 1 : (M + c.l.Mc - 1) / c.l.Mc;
     return RK_OK;
 }
 
@@ -526,13 +541,13 @@ int rk_linear_gemm(float* y, const float* x, long long x_ld, int M, int N, int K
     if (glu && (bias || residual)) return fail(RK_ERR_ARG, "rk_linear_gemm: no bias or residual with glu");
     if (reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(w) % 16 || x_ld < K || x_ld % 4)
         return fail(RK_ERR_ARG, "rk_linear_gemm: x and w must be 16-byte aligned, x rows at a stride >= K of 4n");
-    const size_t need = rk_linear_gemm_workspace_bytes(M, N, K, w_type, glu);
-    if (!workspace || workspace_bytes < need)
-        return fail(RK_ERR_WORKSPACE, "rk_linear_gemm: workspace %zu bytes (need %zu)", workspace_bytes, need);
-    const Layout l = layout(M, N, K, w_type, glu != 0);
-    if (mid_takes(M, N, K, w_type, glu, scales, mins, l.us))
-        return mid_linear(y, x, x_ld, M, N, K, w, w_type, scales, mins, bias, residual, glu, workspace,
+    const Choice c = choose(M, N, K, w_type, glu);
+    if (!workspace || workspace_bytes < c.total)
+        return fail(RK_ERR_WORKSPACE, "rk_linear_gemm: workspace %zu bytes (need %zu)", workspace_bytes, c.total);
+    if (c.mid && mid_reads(scales, mins))
+        return mid_linear(c.p, y, x, x_ld, M, N, K, w, w_type, scales, mins, bias, residual, glu, workspace,
                           static_cast<hipStream_t>(stream));
+    const Layout& l = c.l;
     char* ws = static_cast<char*>(workspace);
     hipStream_t st = static_cast<hipStream_t>(stream);
     uint16_t* pieces = reinterpret_cast<uint16_t*>(ws);

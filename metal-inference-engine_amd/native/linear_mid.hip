@@ -320,12 +320,6 @@ __global__ __launch_bounds__(256) void mid_finish(MidArgs a) {
     mid_store<MT, NT>(a, v, blockIdx.x / a.G, blockIdx.x % a.G, item);
 }
 
-struct MidPlan {
-    int MB, MT, NT, G, S, SB, WB;
-    double us;                     // the estimated time
-    size_t sums, part, total;
-};
-
 // What the time is made of, in us: the launches and x's pieces; a round of one workgroup per CU: its start, and for each
 // chunk of four blocks a wave walks a constant, the activations from the L2 (per row tile, more when every CU asks) and
 // the MFMAs (per row and weight tile); mid_finish and the partial sums it reads. Fitted to 14 weights of 1024 x 1024 to
@@ -338,8 +332,14 @@ constexpr MidCost kCost[3] = {{6.7, 5.9e-6, 0.0, 0.37, 1.51, 0.24, 0.17, 0.294, 
                               {6.9, 5.7e-6, 0.0, 0.34, 1.77, 0.08, 0.21, 0.309, 1.8, 0.046e-3},    // INT8
                               {7.1, 5.3e-6, 1.2, 0.31, 2.35, 0.0, 0.20, 0.320, 1.9, 0.070e-3}};    // INT4
 
+}  // namespace
+
+// kMost: the estimates end there; no weight measured was faster here at 512 rows. Scales and mins are read two blocks at
+// a time.
 MidPlan mid_plan(int M, int N, int K, int w_type, int glu) {
+    constexpr int kMost = 384;
     MidPlan p{};
+    if (M > kMost || K % (2 * kQB)) return p;
     const int nblk = K / kQB;
     const int tiles = glu ? (N / 2 + 7) / 8 : (N + 15) / 16;
     p.MB = (M + 63) / 64;
@@ -371,24 +371,13 @@ MidPlan mid_plan(int M, int N, int K, int w_type, int glu) {
     return p;
 }
 
-}  // namespace
-
-// kMost: the estimates end there; no weight measured was faster here at 512 rows
-bool mid_takes(int M, int N, int K, int w_type, int glu, const void* scales, const void* mins, double gemm_us) {
-    constexpr int kMost = 384;
-    // scales and mins are read two blocks at a time
-    return M <= kMost && K % (2 * kQB) == 0 && reinterpret_cast<uintptr_t>(scales) % 4 == 0 &&
-           reinterpret_cast<uintptr_t>(mins) % 4 == 0 && mid_plan(M, N, K, w_type, glu).us < gemm_us;
+bool mid_reads(const void* scales, const void* mins) {
+    return reinterpret_cast<uintptr_t>(scales) % 4 == 0 && reinterpret_cast<uintptr_t>(mins) % 4 == 0;
 }
 
-int mid_splits(int M, int N, int K, int w_type, int glu) { return mid_plan(M, N, K, w_type, glu).S; }
-
-size_t mid_workspace_bytes(int M, int N, int K, int w_type, int glu) { return mid_plan(M, N, K, w_type, glu).total; }
-
-int mid_linear(float* y, const float* x, long long x_ld, int M, int N, int K, const void* w, int w_type,
+int mid_linear(const MidPlan& p, float* y, const float* x, long long x_ld, int M, int N, int K, const void* w, int w_type,
                const void* scales, const void* mins, const float* bias, const float* residual, int glu,
                void* workspace, hipStream_t stream) {
-    const MidPlan p = mid_plan(M, N, K, w_type, glu);
     char* ws = static_cast<char*>(workspace);
     uint16_t* ops = reinterpret_cast<uint16_t*>(ws);
     uint16_t* sums = reinterpret_cast<uint16_t*>(ws + p.sums);

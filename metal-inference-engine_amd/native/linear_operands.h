@@ -8,12 +8,15 @@
 
 namespace rk {
 
-// linear_mid.hip: the form for up to a few hundred rows, behind rk_linear_gemm; taken where it can run and is estimated
-// to be faster than gemm_us
-bool mid_takes(int M, int N, int K, int w_type, int glu, const void* scales, const void* mins, double gemm_us);
-int mid_splits(int M, int N, int K, int w_type, int glu);
-size_t mid_workspace_bytes(int M, int N, int K, int w_type, int glu);
-int mid_linear(float* y, const float* x, long long x_ld, int M, int N, int K, const void* w, int w_type,
+// linear_mid.hip: the form for up to a few hundred rows, behind rk_linear_gemm
+struct MidPlan {
+    int MB, MT, NT, G, S, SB, WB;  // row blocks and their tiles; weight tiles and groups of them; K-splits and their blocks
+    double us;                     // the estimated time; 0: not for this form
+    size_t sums, part, total;      // the workspace
+};
+MidPlan mid_plan(int M, int N, int K, int w_type, int glu);
+bool mid_reads(const void* scales, const void* mins);   // their addresses allow it
+int mid_linear(const MidPlan& p, float* y, const float* x, long long x_ld, int M, int N, int K, const void* w, int w_type,
                const void* scales, const void* mins, const float* bias, const float* residual, int glu,
                void* workspace, hipStream_t stream);
 
