@@ -180,11 +180,11 @@ int rk_deltanet_decode(float* out, const float* qkv, const float* z, const float
  *   pool both bf16 takes bf16 MFMA operands (q, K, V as stored, the probabilities rounded to bf16; fp32
  *   accumulation): bf16-level results, on 32 queries per wave at group size 4, D in {128, 256}, block_size >= 2 and
  *   max_nb * block_size^2 < 2^32 (config 5), on 16 queries per wave otherwise. exact = 1 or an fp32 q or pool takes
- *   fp32 operands: two fp16 pieces of every value of q, K and V, within 2^-23 of it, and within 2^-40 of the largest
- *   value of its row (of D) where it lies more than 2^16 below; three products each, fp32 sums; probabilities fp32, as
- *   two pieces against V, within 2^-34 of the largest product a query has of them. Keys a query does not see cost it
- *   nothing. An infinite value of V gives an infinity of its sign, a score of -inf (K infinite, q not within 2^-39 of 0
- *   in that dim) drops out.
+ *   fp32 operands: two fp16 pieces of every value of q, K and V, within 2^-23 of it, and where it lies more than 2^28 (V:
+ *   2^16) below the largest value of its row (of D), within 2^-52 (V: 2^-40) of that one; three products each, fp32
+ *   sums; probabilities fp32, as two pieces against V, within 2^-34 of the largest product a query has of them. Keys a
+ *   query does not see cost it nothing. An infinite value of V gives an infinity of its sign, a score of -inf (K
+ *   infinite, q not below 2^-39 of its row's largest value in that dim) drops out.
  *   window 0 or W >= 1 (causal only): query i also sees only positions above start[s] + i - W (the sliding-window
  *   prefill of src/models/cohere2.py:155-163; ops.attention's window, src/ops.py:77-81, 97-98); blocks wholly below
  *   every query's window are never read. causal 0: every query of segment s sees positions 0 .. start[s]+n[s]-1

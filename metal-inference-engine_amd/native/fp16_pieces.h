@@ -23,13 +23,15 @@ __device__ __forceinline__ int top_exponent(float m) {
     return m == 0.0f ? 0 : kTop - max(min(e, 127), -112);
 }
 
-// hi and lo pieces of a pair (already scaled), packed: hi = fp16(v), lo = fp16(v - hi)
+// hi and lo pieces of a pair (already scaled), packed: hi = fp16(v), lo = fp16((v - hi) up). up = 2^kUp, where lo's
+// products have sums of their own, keeps its bits 2^kUp further down
+constexpr int kUp = 12;
 struct Pieces {
     uint32_t hi, lo;
 };
-__device__ __forceinline__ Pieces split_pair(float a, float b) {
+__device__ __forceinline__ Pieces split_pair(float a, float b, float up = 1.0f) {
     const f16x2 h = __builtin_convertvector((f32x2_t){a, b}, f16x2);
-    const f16x2 l = __builtin_convertvector((f32x2_t){a - (float)h[0], b - (float)h[1]}, f16x2);
+    const f16x2 l = __builtin_convertvector((f32x2_t){(a - (float)h[0]) * up, (b - (float)h[1]) * up}, f16x2);
     return {__builtin_bit_cast(uint32_t, h), __builtin_bit_cast(uint32_t, l)};
 }
 // Where a value was infinite: it is all in lo, which meets only the other operand's hi, whose sign is the value's (hi times

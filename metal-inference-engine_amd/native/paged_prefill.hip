@@ -574,10 +574,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // fp32 q or pool and for exact requests (any group size, D = 64 / 128 / 256). The reference computes attention in fp32
 // on widened inputs (src/ops.py:84-87, 91-103). The fp32 matrix rate is 1/16 of the fp16 one, so the products are made
 // of fp16 pieces (fp16_pieces.h): every operand x, scaled by a power of two that puts its row's largest value into
-// [2^14, 2^15), is hi + lo within 2^-23 of itself, and below 2^-16 of that largest value within 2^-40 of it; a product is
-// lo hi + hi lo + hi hi (lo lo is at most 2^-22 of it), summed in fp32: 3/16 of the fp32 matrix time. The rows: of the
-// queries, of the keys (whose exponents scale the scores, held 8 to a lane) and of the values (whose sizes w weigh the
-// probabilities). A query's probabilities enter as p w 2^E, E its own: the largest p w it has seen, as the running maximum
+// [2^14, 2^15), is hi + lo within 2^-23 of itself, and a product is lo hi + hi lo + hi hi (lo lo is at most 2^-22 of it),
+// summed in fp32: 3/16 of the fp32 matrix time. The rows: of the queries, of the keys (whose exponents scale the scores,
+// held 8 to a lane) and of the values (whose sizes w weigh the probabilities). The scores' cross products have sums of
+// their own, so q's and K's lo are held 2^12 up: their values keep 23 bits down to 2^-28 of their row's largest, and
+// within 2^-52 of it below; values of V down to 2^-16, and within 2^-40. (q and k channels 2^28 apart: as good as with fp32
+// products; without the 2^12 up to 12 times the bound of fp32 sums off.) A query's
+// probabilities enter as p w 2^E, E its own: the largest p w it has seen, as the running maximum
 // stands, bounds the others. So keys that a query does not see, or of no weight for it, cost it no bits.
 // blockDim = 512: wave w takes query head (chunk * 4 + w % 4) of the group (none past the group's end: that
 // wave only helps stage) and queries 16 (w / 4) .. + 15 of the work item's 32. All 8 waves stage each tile of 32
@@ -884,8 +887,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int i = 0; i < 2 * EL; ++i) {
             const int d = i >> 1, r = 2 * (i & 1);          // V: dim d, keys r, r + 1
             const int kr = i / (EL / 2), kd = 2 * (i % (EL / 2));   // K: key kr, dims kd, kd + 1
-            pr[i] = is_v ? split_pair(v[r][d] * f[r], v[r + 1][d] * f[r + 1])
-                         : split_pair(v[kr][kd] * f[kr], v[kr][kd + 1] * f[kr]);
+            pr[i] = split_pair(is_v ? v[r][d] * f[r] : v[kr][kd] * f[kr], is_v ? v[r + 1][d] * f[r + 1] : v[kr][kd + 1] * f[kr],
+                               is_v ? 1.0f : 1 << kUp);
             if constexpr (INF) pr[i] = infinite_in_lo(pr[i]);
         }
         if (is_v) {                                  // V^T[row of the dim][the group's 4 keys]
@@ -964,7 +967,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int c = 0; c < NC; ++c)
 #pragma unroll
             for (int d = 0; d < 4; ++d) {
-                const Pieces p = infinite_in_lo(split_pair(ldexpf(q[c][2 * d], e), ldexpf(q[c][2 * d + 1], e)));
+                const Pieces p = infinite_in_lo(split_pair(ldexpf(q[c][2 * d], e), ldexpf(q[c][2 * d + 1], e), 1 << kUp));
                 qh[c][d] = p.hi;
                 ql[c][d] = p.lo;
             }
@@ -1002,7 +1005,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             w[kt] = *reinterpret_cast<const f32x4*>(vsc + stage * kBKP + 16 * kt + 4 * qq);
 #pragma unroll
             for (int r = 0; r < 4; ++r) f[kt][r] = fmaxf(qs * f[kt][r], FLT_MIN);   // never 0: -inf must stay -inf
-            s[kt] += x[kt];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) s[kt][r] = fmaf(x[kt][r], 1.0f / (1 << kUp), s[kt][r]);
         }
         // lane (qc, qq), register r of sub-tile kt: key k0 + 16 kt + 4 qq + r
         if (k0 + kBKP - 1 > qfirst || k0 <= lo_edge) {
