@@ -592,7 +592,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 //                 16 + 4 (l / 16) + j - 4, the keys of the lane's own scores, so B is the lane's 8 probabilities.
 // So every lane keeps its own query's softmax state, and O^T is rescaled per lane. LDS reads are conflict-free.
 // Measured (8 packed segments, 8/2 heads x 256, up to 2,048 new tokens on up to 16,384 cached ones; fp32): 4,985 us on
-// fp32 MFMA (111 TFLOP/s of 157) -> 2,020 us; error against 64 bits 1.2e-6 -> 7.4e-7 of the result, and smaller than fp32
+// fp32 MFMA (111 TFLOP/s of 157) -> 2,060 us; error against 64 bits 1.2e-6 -> 7.4e-7 of the result, and smaller than fp32
 // MFMA's where masked or negligible values are far larger than the others, below a sink, after a jump of the maximum
 // (with one E for a wave, from all values, it was 10^3 times larger there). What bounds it: per
 // tile the MFMAs take 43 % of the time, the LDS reads (64 KB per wave) and the VALU (softmax, splits, addresses) as
